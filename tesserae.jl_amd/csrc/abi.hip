@@ -148,6 +148,10 @@ void ctx_drop_caches(tess_ctx* c) {
   c->misplaced_x_ptr = nullptr;
   c->last_misplaced = -1;
   c->rollout.last_kept = false;
+  // the counters a cut-short step may have left unreported
+  c->broken_pending = c->nodes_pending = false;
+  if (c->counters.ptr) (void)hipMemset(c->counters.ptr, 0, 64 * sizeof(uint32_t));
+  if (c->lanes.ptr) (void)hipMemset(c->lanes.ptr, 0, LANE_BYTES);
 }
 
 void check_ctx(const tess_ctx* cctx) {
@@ -261,7 +265,7 @@ tess_ctx* ctx_new(int device, hipStream_t stream) {
   c->stream = stream;
   c->seen_epoch = error_epoch();
   void* pinned = nullptr;
-  // pinned readback slots: counters (words 0-63), mover counts (words 64-319)
+  // pinned readback slots: the device counters' words 0-63
   hipError_t e = hipHostMalloc(&pinned, 512 * sizeof(int64_t), hipHostMallocDefault);
   if (e != hipSuccess) {
     delete c;
@@ -271,6 +275,7 @@ tess_ctx* ctx_new(int device, hipStream_t stream) {
   try {
     // device counters start at zero (the binning reads slots written by the previous P2G)
     TESS_HIP(hipMemset(c->counters.get(64 * sizeof(uint32_t)), 0, 64 * sizeof(uint32_t)));
+    TESS_HIP(hipMemset(c->lanes.get(LANE_BYTES), 0, LANE_BYTES));
   } catch (...) {
     ctx_free(c);
     throw;
@@ -290,14 +295,15 @@ void ctx_free(tess_ctx* ctx) {
   tess::Buffer* bufs[] = {&ctx->keys,      &ctx->keys_sorted, &ctx->vals,         &ctx->keys_alt,
                           &ctx->vals_alt,  &ctx->hist,        &ctx->scan_tmp,     &ctx->tile_start,
                           &ctx->tile_end,  &ctx->tile_flag,   &ctx->tile_slot,    &ctx->active_tiles,
-                          &ctx->nb_flag,   &ctx->nb_slot,     &ctx->nb_list,      &ctx->nb_list_prev,
+                          &ctx->nb_flag,   &ctx->nb_list,     &ctx->nb_list_prev, &ctx->alt_start,
+                          &ctx->alt_end,   &ctx->alt_flag,    &ctx->alt_slot,     &ctx->alt_active,
+                          &ctx->alt_nb_flag, &ctx->alt_nb_list, &ctx->tab_sums,   &ctx->tile_seg,
                           &ctx->partials,  &ctx->counters,    &ctx->host_pinned_dummy, &ctx->reorder_tmp, &ctx->reorder_cnt,
-                          &ctx->per_tile,  &ctx->per_nodeblock, &ctx->skeys2, &ctx->perm2,
-                          &ctx->inc_nk,    &ctx->inc_spos,  &ctx->inc_mkey, &ctx->inc_mj,
-                          &ctx->inc_mks,   &ctx->inc_mr,    &ctx->inc_mjs, &ctx->inc_rng,
+                          &ctx->per_tile,  &ctx->skeys2,    &ctx->perm2,    &ctx->inc_nk,
+                          &ctx->tile_stay, &ctx->tile_tin,  &ctx->inc_out,  &ctx->inc_seg, &ctx->inc_seg2, &ctx->inc_pout, &ctx->inc_rank,
                           &ctx->sp_occ,    &ctx->sp_act,    &ctx->sp_scan,
                           &ctx->adj_partials, &ctx->adj_nodes, &ctx->ro_checkpoints, &ctx->ro_segment,
-                          &ctx->ro_gradv,  &ctx->ro_snapshots, &ctx->ro_grid, &ctx->movers, &ctx->g2p2g_x,
+                          &ctx->ro_gradv,  &ctx->ro_snapshots, &ctx->ro_grid, &ctx->lanes, &ctx->g2p2g_x,
                           &ctx->export_buf};
   for (auto* b : bufs) b->release();
   for (auto ev : ctx->prof.pool) (void)hipEventDestroy(ev);

@@ -19,6 +19,8 @@
 //                          ∂/∂logE += P̄ : P
 // Rollouts keep checkpoints every k steps and replay each segment before
 // reversing it.
+#ifdef TESS_PART
+
 #include "transfer_impl.hpp"
 
 // Reversed steps a segment replay keeps enqueued ahead of its own progress.
@@ -1285,18 +1287,44 @@ struct RolloutAdjointOp {
 
 }  // namespace
 
+namespace TESS_PART {
+
+void step_adjoint(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,
+                  const tess_params& prm, const tess_adjoint& adj) {
+  dispatch<AdjointOp>(basis, mesh, false, ctx, mesh, G, P, prm, adj);
+}
+
+void rollout(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,
+             const tess_params& prm, int nsteps, int every) {
+  dispatch<RolloutOp>(basis, mesh, false, ctx, mesh, G, P, prm, nsteps, every);
+}
+
+void rollout_adjoint(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_params& prm,
+                     const tess_adjoint& adj) {
+  dispatch<RolloutAdjointOp>(basis, mesh, false, ctx, mesh, G, prm, adj);
+}
+
+}  // namespace TESS_PART
+}  // namespace tess
+
+#else
+
+#include "tess_internal.hpp"
+
+namespace tess {
+
 void run_step_adjoint(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,
                       const tess_params& prm, const tess_adjoint& adj) {
   ctx->corr = 0;  // plain kernels only
   ctx->corr_filter = nullptr;
-  dispatch<AdjointOp>(basis, mesh, false, ctx, mesh, G, P, prm, adj);
+  TESS_FORWARD(mesh, step_adjoint(ctx, basis, mesh, G, P, prm, adj));
 }
 
 void run_rollout(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,
                  const tess_params& prm, int nsteps, int every) {
   ctx->corr = 0;
   ctx->corr_filter = nullptr;
-  dispatch<RolloutOp>(basis, mesh, false, ctx, mesh, G, P, prm, nsteps, every);
+  TESS_FORWARD(mesh, rollout(ctx, basis, mesh, G, P, prm, nsteps, every));
 }
 
 void run_rollout_adjoint(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G,
@@ -1308,7 +1336,9 @@ void run_rollout_adjoint(tess_ctx* ctx, int basis, const tess_mesh& mesh, const 
   if (!same) raise(TESS_ERR_ARGUMENT, "mesh, dtype or basis differ from the recorded rollout");
   ctx->corr = 0;
   ctx->corr_filter = nullptr;
-  dispatch<RolloutAdjointOp>(basis, mesh, false, ctx, mesh, G, prm, adj);
+  TESS_FORWARD(mesh, rollout_adjoint(ctx, basis, mesh, G, prm, adj));
 }
 
 }  // namespace tess
+
+#endif

@@ -7,6 +7,8 @@
 // batch.  Tile kernels look their scene up from the tile index
 // (scene_of/bind_scene in transfer_impl.hpp).  An autotuner times the launch
 // variants (waves per tile in P2G and G2P) on the batch itself.
+#ifdef TESS_PART
+
 #include "transfer_impl.hpp"
 
 #include <algorithm>
@@ -62,6 +64,10 @@ void batch_create_impl(tess_ctx* ctx, tess_batch& b) {
                           ctx->stream));
   TESS_HIP(hipMemcpyAsync(b.d_poff.get(b.poff.size() * 8), b.poff.data(), b.poff.size() * 8, hipMemcpyHostToDevice,
                           ctx->stream));
+  std::vector<int32_t> nt;  // tiles per axis of each scene
+  for (const auto& r : recs)
+    for (int d = 0; d < 3; ++d) nt.push_back(d < D ? r.ntiles[d < D ? d : 0] : 1);
+  TESS_HIP(hipMemcpyAsync(b.d_nt.get(nt.size() * 4), nt.data(), nt.size() * 4, hipMemcpyHostToDevice, ctx->stream));
   TESS_HIP(hipStreamSynchronize(ctx->stream));
 }
 
@@ -78,8 +84,18 @@ Args<T, D> batch_args(tess_ctx* ctx, tess_batch& b) {
   return a;
 }
 
-// Full sort of the batch's keys every step (the batch-wide tile space), then the
-// tile runs, active tiles and touched node blocks, as bin_particles does.
+// Arguments that build the batch's tables into the alternate set.
+inline TabArgs batch_tables(tess_ctx* ctx, tess_batch& B) {
+  TabArgs t = table_args(ctx, B.tiles_total);
+  t.scene_toff = static_cast<const int64_t*>(B.d_toff.ptr);
+  t.scene_nt = static_cast<const int32_t*>(B.d_nt.ptr);
+  t.nscenes = B.nscenes;
+  return t;
+}
+
+// Full sort of the batch's keys on a call's first step (the batch-wide tile
+// space), the merge of the changed keys from then on, and the tile tables, as
+// bin_particles does.
 template <typename T, int D, int BASIS>
 void batch_bin_run(tess_ctx* ctx, tess_batch& B, bool keys_from_g2p);
 
@@ -107,87 +123,49 @@ void batch_bin_run(tess_ctx* ctx, tess_batch& B, bool keys_from_g2p) {
   b.valid = false;
   b.state_valid = false;  // the single-scene incremental state does not describe a batch
   b.keys_ready = false;
-  uint32_t* counters = ctx->counters.as<uint32_t>(CNT_SLOTS);
-  uint32_t* hc = reinterpret_cast<uint32_t*>(ctx->counters_host);
-  const int kbits = key_bits_for(ntiles * 64);
-  int64_t movers = -1;
-  if (incremental) {
-    // the last G2P counted the particles whose key changed; with none the
-    // previous order and tile lists stand
-    TESS_HIP(hipMemcpyAsync(hc, counters, CNT_SLOTS * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
-    movers_readback(ctx);
-    TESS_HIP(hipStreamSynchronize(ctx->stream));
-    movers = movers_total(ctx);
-    if (movers == 0) {
-      ctx->last_active_nodes = int64_t(hc[CNT_NODES]);
-      B.kept_binnings += 1;
-      b.valid = true;
-      return;
-    }
-  }
-  TESS_HIP(hipMemsetAsync(counters, 0, CNT_BIN_SLOTS * sizeof(uint32_t), ctx->stream));
-  uint32_t* keys = ctx->keys.as<uint32_t>(size_t(std::max<int64_t>(n, 1)));
-  uint32_t* skeys = ctx->keys_sorted.as<uint32_t>(size_t(std::max<int64_t>(n, 1)));
-  uint32_t* perm = ctx->vals.as<uint32_t>(size_t(std::max<int64_t>(n, 1)));
-  uint32_t* tstart = ctx->tile_start.as<uint32_t>(ntiles);
-  uint32_t* tend = ctx->tile_end.as<uint32_t>(ntiles);
-  uint32_t* tflag = ctx->tile_flag.as<uint32_t>(ntiles);
-  uint32_t* tslot = ctx->tile_slot.as<uint32_t>(ntiles);
-  uint32_t* active = ctx->active_tiles.as<uint32_t>(ntiles);
-  uint32_t* nbflag = ctx->nb_flag.as<uint32_t>(ntiles);
-  uint32_t* nbslot = ctx->nb_slot.as<uint32_t>(ntiles);
-  uint32_t* nblist = ctx->nb_list.as<uint32_t>(ntiles);
-  Args<T, D> a = batch_args<T, D>(ctx, B);
+  uint32_t* counters = ctx->counters.as<uint32_t>(64);
+  const uint32_t* hc = reinterpret_cast<const uint32_t*>(ctx->counters_host);
+  const size_t m = size_t(std::max<int64_t>(n, 1));
+  const TabArgs tab = batch_tables(ctx, B);
   const int tok = prof_begin(ctx, "binning", 0.0);
   if (incremental) {
-    // movers merged into the previous sorted order
-    uint32_t* nk = ctx->inc_nk.as<uint32_t>(size_t(n));
-    uint32_t* spos = ctx->inc_spos.as<uint32_t>(size_t(n) + 1);
-    TESS_HIP(hipMemsetAsync(spos + n, 0, sizeof(uint32_t), ctx->stream));
-    exclusive_scan_u32(ctx, spos, n + 1, counters + CNT_STAY);
-    TESS_HIP(hipMemcpyAsync(hc + CNT_STAY, counters + CNT_STAY, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
+    // the last G2P wrote the keys and counted the particles whose key changed;
+    // with none the previous order and tile lists stand
+    launch_tables(ctx->stream, tab);
     TESS_HIP(hipStreamSynchronize(ctx->stream));
-    const int64_t M = n - int64_t(hc[CNT_STAY]);
-    if (M > 0) merge_movers(ctx, nk, spos, n, M, kbits);
-    skeys = static_cast<uint32_t*>(ctx->keys_sorted.ptr);
-    perm = static_cast<uint32_t*>(ctx->vals.ptr);
+    take_report(ctx);
+    ctx->last_active_nodes = int64_t(hc[CNT_NODES]);
+    if (hc[CNT_MOVED] == 0) {
+      B.kept_binnings += 1;
+      b.valid = true;
+      prof_end(ctx, tok);
+      return;
+    }
+    merge_moves(ctx, n, int64_t(ntiles), b.n_active, b.n_inside);
   } else {
-    hipLaunchKernelGGL((k_bin_keys<T, D, BASIS, false, true>), dim3(blocks_for(n, 256)), dim3(256), 0, ctx->stream, a,
-                       keys, uint32_t(ntiles), counters);
-    TESS_HIP(hipGetLastError());
-    radix_sort_pairs(ctx, keys, nullptr, skeys, perm, n, kbits);
+    Args<T, D> a = batch_args<T, D>(ctx, B);
+    uint32_t* skeys = ctx->keys_sorted.as<uint32_t>(m);
+    uint32_t* perm = ctx->vals.as<uint32_t>(m);
+    if (n > 0) {
+      uint32_t* keys = ctx->keys.as<uint32_t>(m);
+      hipLaunchKernelGGL((k_bin_keys<T, D, BASIS, false, true>), dim3(blocks_for(n, 256)), dim3(256), 0, ctx->stream, a,
+                         keys, uint32_t(ntiles), counters);
+      TESS_HIP(hipGetLastError());
+      radix_sort_pairs(ctx, keys, nullptr, skeys, perm, n, key_bits_for(ntiles * 64));
+    }
+    launch_tile_counts(ctx->stream, skeys, n, int64_t(ntiles), tab.stay, tab.tin);
+    launch_tables(ctx->stream, tab);
+    TESS_HIP(hipStreamSynchronize(ctx->stream));
+    take_report(ctx);
+    ctx->last_active_nodes = int64_t(hc[CNT_NODES]);  // written by the previous step's gather
   }
-  TESS_HIP(hipMemsetAsync(tstart, 0, ntiles * sizeof(uint32_t), ctx->stream));
-  TESS_HIP(hipMemsetAsync(tend, 0, ntiles * sizeof(uint32_t), ctx->stream));
-  hipLaunchKernelGGL(k_tile_runs, dim3(blocks_for(n, 256)), dim3(256), 0, ctx->stream, skeys, n, uint32_t(ntiles),
-                     tstart, tend, counters);
-  TESS_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_tile_flags, dim3(blocks_for(ntiles, 256)), dim3(256), 0, ctx->stream, tstart, tend,
-                     uint32_t(ntiles), tflag, tslot);
-  TESS_HIP(hipGetLastError());
-  exclusive_scan_u32(ctx, tslot, int64_t(ntiles), counters + CNT_ACTIVE);
-  hipLaunchKernelGGL(k_compact, dim3(blocks_for(ntiles, 256)), dim3(256), 0, ctx->stream, tflag, tslot,
-                     uint32_t(ntiles), active);
-  TESS_HIP(hipGetLastError());
-  TESS_HIP(hipMemsetAsync(nbflag, 0, ntiles * sizeof(uint32_t), ctx->stream));
-  hipLaunchKernelGGL((k_nb_mark_batch<T, D>), dim3(blocks_for(ntiles, 256)), dim3(256), 0, ctx->stream, a, tflag,
-                     uint32_t(ntiles), nbflag);
-  TESS_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_copy_u32, dim3(blocks_for(ntiles, 256)), dim3(256), 0, ctx->stream, nbflag, nbslot,
-                     int64_t(ntiles));
-  TESS_HIP(hipGetLastError());
-  exclusive_scan_u32(ctx, nbslot, int64_t(ntiles), counters + CNT_NB);
-  hipLaunchKernelGGL(k_compact, dim3(blocks_for(ntiles, 256)), dim3(256), 0, ctx->stream, nbflag, nbslot,
-                     uint32_t(ntiles), nblist);
-  TESS_HIP(hipGetLastError());
   prof_end(ctx, tok);
-  TESS_HIP(hipMemcpyAsync(hc, counters, CNT_SLOTS * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
-  TESS_HIP(hipStreamSynchronize(ctx->stream));
   if (hc[CNT_ERR] & ERR_GIMP_LENGTH) raise(TESS_ERR_ARGUMENT, "uGIMP requires 0 ≤ pt.l ≤ spacing(mesh)");
-  b.n_inside = n > 0 ? int64_t(hc[CNT_INSIDE]) : 0;
-  ctx->last_active_nodes = int64_t(hc[CNT_NODES]);  // written by the previous step's gather
+  swap_tables(ctx);
+  b.n_inside = int64_t(hc[CNT_INSIDE]);
   b.n_active = int64_t(hc[CNT_ACTIVE]);
   b.n_nodeblocks = int64_t(hc[CNT_NB]);
+  b.generation += 1;
   b.ntiles = int64_t(ntiles);
   b.n = n;
   b.valid = true;
@@ -288,8 +266,8 @@ void batch_reorder(tess_ctx* ctx, tess_batch& B, double threshold) {
   Args<T, D> a = batch_args<T, D>(ctx, B);
   uint32_t* layered = ctx->keys_alt.as<uint32_t>(size_t(n));
   uint32_t* order = ctx->keys.as<uint32_t>(size_t(n));  // the raw keys are dead after the sort
-  uint32_t* pout = ctx->inc_mr.as<uint32_t>(size_t(n));
-  uint32_t* R = ctx->inc_mks.as<uint32_t>(size_t(n) + 1);
+  uint32_t* pout = ctx->inc_pout.as<uint32_t>(size_t(n));
+  uint32_t* R = ctx->inc_rank.as<uint32_t>(size_t(n) + 1);
   uint32_t* broken = ctx->reorder_cnt.as<uint32_t>(size_t(b.n_active));
   uint32_t* counters = ctx->counters.as<uint32_t>(CNT_SLOTS);
   const uint32_t* sk = static_cast<const uint32_t*>(ctx->keys_sorted.ptr);
@@ -341,11 +319,10 @@ void launch_p2g(tess_ctx* ctx, const Args<T, D>& a, int64_t n_active, const uint
 }
 
 template <typename T, int D, int BASIS, int NW>
-void launch_g2p(tess_ctx* ctx, const Args<T, D>& a, int64_t n_active, const uint32_t* sk, uint32_t* nk, uint32_t* stay,
-                uint32_t* movers) {
+void launch_g2p(tess_ctx* ctx, const Args<T, D>& a, int64_t n_active, const uint32_t* sk, const MoveOut& mo) {
   const uint32_t nt = uint32_t(ctx->bin.ntiles);
   hipLaunchKernelGGL((k_g2p_fast<T, D, BASIS, true, NW, true>), dim3(xcd_grid(n_active)), dim3(64 * NW), 0,
-                     ctx->stream, a, sk, nk, stay, nt, movers);
+                     ctx->stream, a, sk, mo, nt);
   TESS_HIP(hipGetLastError());
 }
 
@@ -381,62 +358,48 @@ void batch_step_impl(tess_ctx* ctx, tess_batch& B, int nsteps) {
       TESS_HIP(hipGetLastError());
     }
     const uint32_t* sk = static_cast<const uint32_t*>(ctx->keys_sorted.ptr);
-    uint32_t* counters = static_cast<uint32_t*>(ctx->counters.ptr);
     if (b.n_active > 0) {
       a.partials = ctx->partials.as<T>(size_t(b.n_active) * Part<D, SW>::SIZE);
       const int tok = prof_begin(ctx, "k_p2g_tile", double(b.n_inside) * sizeof(T) * (2 * D + 1 + D * D));
       // with a threshold in (0, 1) P2G counts the broken layered pairs for the
       // next step's reorder test
       const bool count = B.reorder_threshold > 0.0 && B.reorder_threshold < 1.0;
-      uint32_t* broken = count ? ctx->reorder_cnt.as<uint32_t>(size_t(b.n_active)) : nullptr;
+      uint32_t* broken = count ? lane_counters(ctx) : nullptr;
       if (D == 3 || (B.variant & 1)) launch_p2g<T, D, BASIS, SW>(ctx, a, b.n_active, sk, broken);
       else launch_p2g<T, D, BASIS, 1>(ctx, a, b.n_active, sk, broken);
       prof_end(ctx, tok);
-      if (count) {
-        sum_u32(ctx, broken, b.n_active, counters + CNT_MISPLACED);
-        B.counted_pairs = b.n_inside - b.n_active;
-      }
+      if (count) B.counted_pairs = b.n_inside - b.n_active;
       B.counted = count;
     } else {
       B.counted = false;
     }
     if (b.n_nodeblocks > 0) {
-      uint32_t* per_nb = ctx->per_nodeblock.as<uint32_t>(size_t(b.n_nodeblocks));
       const int tok = prof_begin(ctx, "k_gather_grid", 0.0);
       hipLaunchKernelGGL((k_gather_grid<T, D, SW, true, true>), dim3(xcd_grid(b.n_nodeblocks)), dim3(64), 0, ctx->stream,
-                         a, per_nb);
+                         a, lane_counters(ctx));
       TESS_HIP(hipGetLastError());
       prof_end(ctx, tok);
-      sum_u32(ctx, per_nb, b.n_nodeblocks, counters + CNT_NODES);
       uint32_t* prev = B.prev_list.as<uint32_t>(size_t(b.n_nodeblocks));
       TESS_HIP(hipMemcpyAsync(prev, ctx->nb_list.ptr, size_t(b.n_nodeblocks) * sizeof(uint32_t),
                               hipMemcpyDeviceToDevice, ctx->stream));
     }
     B.prev_nb = b.n_nodeblocks;
     // next-step keys at the sorted positions while the call goes on
-    uint32_t* nk = nullptr;
-    uint32_t* stay = nullptr;
-    uint32_t* mv = nullptr;
-    if (s + 1 < nsteps && B.ntot > 0) {
-      nk = ctx->inc_nk.as<uint32_t>(size_t(B.ntot));
-      stay = ctx->inc_spos.as<uint32_t>(size_t(B.ntot) + 1);
-      mv = movers_counters(ctx);
-      movers_zero(ctx);
-    }
+    const MoveOut mo = s + 1 < nsteps && B.ntot > 0 ? move_out(ctx, B.ntot, B.tiles_total) : no_moves();
     if (b.n_active > 0) {
       const int tok = prof_begin(ctx, "k_g2p_tile",
                                  double(b.n_inside) * sizeof(T) * (2 * D + D * D + 2 * D + 3 * D * D + 1));
-      if (B.variant & 4) launch_g2p<T, D, BASIS, 1>(ctx, a, b.n_active, sk, nk, stay, mv);
-      else if (B.variant & 2) launch_g2p<T, D, BASIS, 2>(ctx, a, b.n_active, sk, nk, stay, mv);
-      else launch_g2p<T, D, BASIS, 4>(ctx, a, b.n_active, sk, nk, stay, mv);
+      if (B.variant & 4) launch_g2p<T, D, BASIS, 1>(ctx, a, b.n_active, sk, mo);
+      else if (B.variant & 2) launch_g2p<T, D, BASIS, 2>(ctx, a, b.n_active, sk, mo);
+      else launch_g2p<T, D, BASIS, 4>(ctx, a, b.n_active, sk, mo);
       prof_end(ctx, tok);
     }
     if (B.ntot > b.n_inside) {
       hipLaunchKernelGGL((k_g2p_outside<T, D, true>), dim3(blocks_for(B.ntot - b.n_inside, 256)), dim3(256), 0,
-                         ctx->stream, a, sk, nk, stay);
+                         ctx->stream, a, sk, mo.nk);
       TESS_HIP(hipGetLastError());
     }
-    B.keys_ready = nk != nullptr;
+    B.keys_ready = mo.nk != nullptr;
   }
   // the single-scene zeroing bookkeeping no longer describes any grid
   ctx->last_grid_m = nullptr;
@@ -447,8 +410,8 @@ void batch_step_impl(tess_ctx* ctx, tess_batch& B, int nsteps) {
 //
 // With bit 3 of the variant a batch steps on a private context (its own stream
 // and scratch, so no other call can move the buffers a captured step points
-// at).  Its step reads nothing back to the host: the binning sorts every
-// particle again (every launch size fixed by the batch), the counts of inside
+// at).  Its step reads nothing back to the host: the binning merges the
+// particles whose key changed (every launch size fixed by the batch), the counts of inside
 // particles, active tiles and touched node blocks stay on the device, and the
 // tile and node-block kernels are persistent launches (a grid sized to the
 // device by its occupancy) that walk those lists up to the device-side counts.
@@ -509,12 +472,11 @@ __global__ __launch_bounds__(256) void k_save_list(const uint32_t* __restrict__ 
 // inside particles to n): the update with zero grid increments.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void k_g2p_outside_persist(Args<T, D> a, const uint32_t* __restrict__ skeys,
-                                                             uint32_t* __restrict__ nk, uint32_t* __restrict__ stay,
+                                                             uint32_t* __restrict__ nk,
                                                              const uint32_t* __restrict__ n_inside) {
   const int64_t from = int64_t(*n_inside);
   for (int64_t j = from + int64_t(blockIdx.x) * 256 + threadIdx.x; j < a.n; j += int64_t(gridDim.x) * 256) {
     nk[j] = skeys[j];  // the position does not change: the key stays
-    stay[j] = 1u;
     uint32_t pid = a.perm[j];
     pid -= uint32_t(bind_scene(a, scene_of(a.scene_poff, a.nscenes, pid)).poff);
     T dv[D], L[D * D], dx[D];
@@ -572,22 +534,21 @@ void batch_graph_grids(tess_ctx* g, tess_batch& B) {
                             ceil_div(std::max<int64_t>(B.ntot, 1), int64_t(256)), cus);
 }
 
-__global__ void k_mover_count(const uint32_t* __restrict__ stay_total, int64_t n, uint32_t* __restrict__ movers) {
-  if (threadIdx.x == 0) *movers = uint32_t(n - int64_t(*stay_total));
-}
-
-// Graph mode's binning double buffer: (sorted keys, permutation) in set 0 =
-// (keys_sorted, vals) or set 1 = (skeys2, perm2).
-struct BinSets {
-  uint32_t* keys[2];
-  uint32_t* perm[2];
+// Graph mode's binning double buffer: sorted keys, permutation and tile tables
+// in set 0 (keys_sorted, vals, tile_start, ...) or set 1 (skeys2, perm2,
+// alt_start, ...).
+struct BinSet {
+  uint32_t *keys, *perm, *start, *end, *flag, *slot, *active, *nb_flag, *nb_list;
 };
-inline BinSets bin_sets(tess_ctx* g, int64_t n) {
-  const size_t m = size_t(std::max<int64_t>(n, 1));
-  return BinSets{{g->keys_sorted.as<uint32_t>(m), g->skeys2.as<uint32_t>(m)},
-                 {g->vals.as<uint32_t>(m), g->perm2.as<uint32_t>(m)}};
+inline BinSet bin_set(tess_ctx* g, int64_t n, int64_t ntiles, int which) {
+  const size_t m = size_t(std::max<int64_t>(n, 1)), nt = size_t(ntiles) + 1;
+  auto get = [&](Buffer& a, Buffer& b, size_t k) { return (which ? b : a).as<uint32_t>(k); };
+  return BinSet{get(g->keys_sorted, g->skeys2, m),       get(g->vals, g->perm2, m),
+                get(g->tile_start, g->alt_start, nt),    get(g->tile_end, g->alt_end, nt),
+                get(g->tile_flag, g->alt_flag, nt),      get(g->tile_slot, g->alt_slot, nt),
+                get(g->active_tiles, g->alt_active, nt), get(g->nb_flag, g->alt_nb_flag, nt),
+                get(g->nb_list, g->alt_nb_list, nt)};
 }
-constexpr int CNT_MOVERS = 12;  // counter slot of the mover count (graph mode)
 
 // One step of the batch on context g, every launch size fixed and every count
 // on the device.  full: the binning sorts every particle's key into set 0
@@ -602,102 +563,82 @@ void batch_graph_step(tess_ctx* g, tess_batch& B, bool full, int in) {
   const uint64_t ntiles = uint64_t(B.tiles_total);
   const size_t m = size_t(std::max<int64_t>(n, 1));
   hipStream_t st = g->stream;
-  uint32_t* counters = g->counters.as<uint32_t>(CNT_SLOTS);
+  uint32_t* counters = g->counters.as<uint32_t>(64);
   uint32_t* keys = g->keys.as<uint32_t>(m);
-  const BinSets sets = bin_sets(g, n);
-  uint32_t* nk = g->inc_nk.as<uint32_t>(m);
-  uint32_t* spos = g->inc_spos.as<uint32_t>(m + 1);
-  uint32_t* mkey = g->inc_mkey.as<uint32_t>(m);
-  uint32_t* mj = g->inc_mj.as<uint32_t>(m);
-  uint32_t* mks = g->inc_mks.as<uint32_t>(m + 1);  // the reorder uses it with n + 1 words
-  uint32_t* mr = g->inc_mr.as<uint32_t>(m);
-  uint32_t* mjs = g->inc_mjs.as<uint32_t>(m);
-  const int64_t nsb = blocks_for(std::max<int64_t>(n, 1), STAY_BLOCK);
-  int64_t* ranges = g->inc_rng.as<int64_t>(size_t(2 * nsb));
-  uint32_t* movers = movers_counters(g);  // G2P's mover tally (unused here)
-  uint32_t* tstart = g->tile_start.as<uint32_t>(ntiles);
-  uint32_t* tend = g->tile_end.as<uint32_t>(ntiles);
-  uint32_t* tflag = g->tile_flag.as<uint32_t>(ntiles);
-  uint32_t* tslot = g->tile_slot.as<uint32_t>(ntiles);
-  uint32_t* active = g->active_tiles.as<uint32_t>(ntiles);
-  uint32_t* nbflag = g->nb_flag.as<uint32_t>(ntiles);
-  uint32_t* nbslot = g->nb_slot.as<uint32_t>(ntiles);
-  uint32_t* nblist = g->nb_list.as<uint32_t>(ntiles);
-  uint32_t* per_nb = g->per_nodeblock.as<uint32_t>(ntiles);
+  const int64_t nt64 = int64_t(ntiles);
+  const int out = full ? 0 : 1 - in;
+  const BinSet cur = bin_set(g, n, nt64, out), old = bin_set(g, n, nt64, 1 - out);
+  const MoveOut mo = move_out(g, n, nt64);
+  uint2* seg = g->inc_seg.as<uint2>(m);
+  uint2* seg_alt = g->inc_seg2.as<uint2>(m);
+  uint32_t* lanes = lane_counters(g);
   uint32_t* prev_list = B.g_prev_list.as<uint32_t>(ntiles);
   uint32_t* prev_count = B.g_prev_count.as<uint32_t>(64);
   T* partials = g->partials.as<T>(size_t(ntiles) * Part<D, SW>::SIZE);
-  // the scans' work area at its largest use (spos, the tile lists, the sort's
-  // histograms, the reorder's ranks), so no later call moves it
-  g->scan_tmp.get(std::max({scan_work_bytes(n + 1), scan_work_bytes(int64_t(ntiles)),
-                            scan_work_bytes(int64_t(sort_hist_words(std::max<int64_t>(n, 1))))}));
-  const int out = full ? 0 : 1 - in;
-  uint32_t* skeys = sets.keys[out];
-  uint32_t* perm = sets.perm[out];
+  // the scans' work area at its largest use (the sort's histograms, the
+  // reorder's ranks), so no later call moves it
+  g->scan_tmp.get(std::max(scan_work_bytes(n + 1), scan_work_bytes(int64_t(sort_hist_words(std::max<int64_t>(n, 1))))));
+  uint32_t* skeys = cur.keys;
+  const uint32_t* nblist = cur.nb_list;
   Args<T, D> a = batch_args<T, D>(g, B);
-  a.perm = perm;
+  a.perm = cur.perm;
+  a.tile_start = cur.start;
+  a.tile_end = cur.end;
+  a.active = cur.active;
+  a.tile_flag = cur.flag;
+  a.tile_slot = cur.slot;
+  a.nb_list = cur.nb_list;
+  a.nb_flag = cur.nb_flag;
   a.partials = partials;
-  const int kbits = key_bits_for(ntiles * 64);
-  fill_u32(st, counters, CNT_BIN_SLOTS, 0u);
-  if (n > 0) {
-    if (full) {
+  TabArgs tab = batch_tables(g, B);
+  tab.start = cur.start;
+  tab.end = cur.end;
+  tab.flag = cur.flag;
+  tab.slot = cur.slot;
+  tab.active = cur.active;
+  tab.nb_flag = cur.nb_flag;
+  tab.nb_list = cur.nb_list;
+  tab.keep_err = 1;  // the call's one readback of the error flags comes at its end
+  if (full) {
+    fill_u32(st, counters + CNT_ERR, 1, 0u);
+    if (n > 0) {
       hipLaunchKernelGGL((k_bin_keys<T, D, BASIS, false, true>), dim3(blocks_for(n, 256)), dim3(256), 0, st, a, keys,
                          uint32_t(ntiles), counters);
       TESS_HIP(hipGetLastError());
-      radix_sort_pairs(g, keys, nullptr, skeys, perm, n, kbits);
-    } else {
-      // stayers keep their order; the movers, sorted by (key, previous
-      // position), are merged in (the mover count M stays on the device)
-      const uint32_t* M = counters + CNT_MOVERS;
-      fill_u32(st, spos + n, 1, 0u);
-      exclusive_scan_u32(g, spos, n + 1, counters + CNT_STAY);
-      hipLaunchKernelGGL(k_mover_count, dim3(1), dim3(64), 0, st, static_cast<const uint32_t*>(counters + CNT_STAY), n,
-                         counters + CNT_MOVERS);
-      TESS_HIP(hipGetLastError());
-      hipLaunchKernelGGL(k_compact_movers, dim3(blocks_for(n, 256)), dim3(256), 0, st, static_cast<const uint32_t*>(nk),
-                         static_cast<const uint32_t*>(spos), n, mkey, mj);
-      TESS_HIP(hipGetLastError());
-      radix_sort_pairs(g, mkey, nullptr, mks, mr, n, kbits, M);
-      hipLaunchKernelGGL(k_place_movers, dim3(blocks_for(n, 256)), dim3(256), 0, st, static_cast<const uint32_t*>(mks),
-                         static_cast<const uint32_t*>(mr), static_cast<const uint32_t*>(mj),
-                         static_cast<const uint32_t*>(sets.keys[in]), static_cast<const uint32_t*>(sets.perm[in]),
-                         static_cast<const uint32_t*>(spos), n, n, mjs, skeys, perm, M);
-      TESS_HIP(hipGetLastError());
-      hipLaunchKernelGGL(k_stay_ranges, dim3(blocks_for(nsb, 256)), dim3(256), 0, st,
-                         static_cast<const uint32_t*>(sets.keys[in]), n, static_cast<const uint32_t*>(mks),
-                         static_cast<const uint32_t*>(mjs), n, nsb, ranges, M);
-      TESS_HIP(hipGetLastError());
-      hipLaunchKernelGGL(k_place_stayers, dim3(unsigned(nsb)), dim3(STAY_BLOCK), 0, st,
-                         static_cast<const uint32_t*>(sets.keys[in]), static_cast<const uint32_t*>(sets.perm[in]),
-                         static_cast<const uint32_t*>(spos), n, static_cast<const uint32_t*>(mks),
-                         static_cast<const uint32_t*>(mjs), static_cast<const int64_t*>(ranges), skeys, perm);
-      TESS_HIP(hipGetLastError());
+      radix_sort_pairs(g, keys, nullptr, skeys, cur.perm, n, key_bits_for(ntiles * 64));
     }
+    launch_tile_counts(st, skeys, n, nt64, tab.stay, tab.tin);
+    launch_tables(st, tab);
+  } else {
+    // the particles whose key changed merged into the previous order, every
+    // count on the device
+    launch_tables(st, tab);
+    MergeArgs g2;
+    std::memset(static_cast<void*>(&g2), 0, sizeof(g2));
+    g2.n = n;
+    g2.ntiles = nt64;
+    g2.old_active = old.active;
+    g2.old_start = old.start;
+    g2.old_end = old.end;
+    g2.new_active = cur.active;
+    g2.new_start = cur.start;
+    g2.new_end = cur.end;
+    g2.old_count = counters + CNT_PREV_ACTIVE;
+    g2.new_count = counters + CNT_ACTIVE;
+    g2.old_active_n = g2.new_active_n = nt64;
+    g2.stay = mo.stay;
+    g2.nk = mo.nk;
+    g2.perm_old = old.perm;
+    g2.seg_off = tab.seg;
+    g2.out = mo.out;
+    g2.seg = seg;
+    g2.seg_alt = seg_alt;
+    g2.keys_new = cur.keys;
+    g2.perm_new = cur.perm;
+    g2.counters = counters;
+    g2.pos_bits = key_bits_for(uint64_t(m));
+    launch_merge(st, g2, true, n > 0 ? unsigned(std::min<int64_t>(blocks_for(n, 256), 512)) : 0u);
   }
-  fill_u32(st, tstart, int64_t(ntiles), 0u);
-  fill_u32(st, tend, int64_t(ntiles), 0u);
-  if (n > 0) {
-    hipLaunchKernelGGL(k_tile_runs, dim3(blocks_for(n, 256)), dim3(256), 0, st, skeys, n, uint32_t(ntiles), tstart,
-                       tend, counters);
-    TESS_HIP(hipGetLastError());
-  }
-  hipLaunchKernelGGL(k_tile_flags, dim3(blocks_for(ntiles, 256)), dim3(256), 0, st, tstart, tend, uint32_t(ntiles),
-                     tflag, tslot);
-  TESS_HIP(hipGetLastError());
-  exclusive_scan_u32(g, tslot, int64_t(ntiles), counters + CNT_ACTIVE);
-  hipLaunchKernelGGL(k_compact, dim3(blocks_for(ntiles, 256)), dim3(256), 0, st, tflag, tslot, uint32_t(ntiles),
-                     active);
-  TESS_HIP(hipGetLastError());
-  fill_u32(st, nbflag, int64_t(ntiles), 0u);
-  hipLaunchKernelGGL((k_nb_mark_batch<T, D>), dim3(blocks_for(ntiles, 256)), dim3(256), 0, st, a, tflag,
-                     uint32_t(ntiles), nbflag);
-  TESS_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_copy_u32, dim3(blocks_for(ntiles, 256)), dim3(256), 0, st, nbflag, nbslot, int64_t(ntiles));
-  TESS_HIP(hipGetLastError());
-  exclusive_scan_u32(g, nbslot, int64_t(ntiles), counters + CNT_NB);
-  hipLaunchKernelGGL(k_compact, dim3(blocks_for(ntiles, 256)), dim3(256), 0, st, nbflag, nbslot, uint32_t(ntiles),
-                     nblist);
-  TESS_HIP(hipGetLastError());
   // grids: the previous step's stale node blocks, P2G, the grid-node half
   hipLaunchKernelGGL((k_zero_stale_persist<T, D>), dim3(B.grid_zero), dim3(64), 0, st, a,
                      static_cast<const uint32_t*>(prev_list), static_cast<const uint32_t*>(prev_count));
@@ -726,13 +667,13 @@ void batch_graph_step(tess_ctx* g, tess_batch& B, bool full, int in) {
   }
   TESS_HIP(hipGetLastError());
   if (persist)
-    hipLaunchKernelGGL((k_gather_grid_persist<T, D, SW, true, true>), dim3(B.grid_gather), dim3(64), 0, st, a, per_nb,
+    hipLaunchKernelGGL((k_gather_grid_persist<T, D, SW, true, true>), dim3(B.grid_gather), dim3(64), 0, st, a, lanes,
                        n_nb);
   else
-    hipLaunchKernelGGL((k_gather_grid_grid<T, D, SW, true, true>), all_tiles, dim3(64), 0, st, a, per_nb, n_nb);
+    hipLaunchKernelGGL((k_gather_grid_grid<T, D, SW, true, true>), all_tiles, dim3(64), 0, st, a, lanes, n_nb);
   TESS_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_save_list, dim3(unsigned(std::min<int64_t>(blocks_for(int64_t(ntiles), 256), 1024))), dim3(256),
-                     0, st, static_cast<const uint32_t*>(nblist), n_nb, prev_list, prev_count);
+                     0, st, nblist, n_nb, prev_list, prev_count);
   TESS_HIP(hipGetLastError());
   // G2P over the active tiles (next keys and stayer flags at the sorted
   // positions), then the particles outside every mesh
@@ -742,17 +683,17 @@ void batch_graph_step(tess_ctx* g, tess_batch& B, bool full, int in) {
     constexpr int NW = decltype(nwc)::value;
     if (persist)
       hipLaunchKernelGGL((k_g2p_fast_persist<T, D, BASIS, true, NW, true>), dim3(B.grid_g2p), dim3(64 * NW), 0, st, a,
-                         sk, nk, spos, nt32, movers, n_active);
+                         sk, mo, nt32, n_active);
     else
-      hipLaunchKernelGGL((k_g2p_fast_grid<T, D, BASIS, true, NW, true>), all_tiles, dim3(64 * NW), 0, st, a, sk, nk,
-                         spos, nt32, movers, n_active);
+      hipLaunchKernelGGL((k_g2p_fast_grid<T, D, BASIS, true, NW, true>), all_tiles, dim3(64 * NW), 0, st, a, sk, mo,
+                         nt32, n_active);
   };
   if (nw == 1) g2p(std::integral_constant<int, 1>{});
   else if (nw == 2) g2p(std::integral_constant<int, 2>{});
   else g2p(std::integral_constant<int, 4>{});
   TESS_HIP(hipGetLastError());
   if (n > 0) {
-    hipLaunchKernelGGL((k_g2p_outside_persist<T, D>), dim3(B.grid_out), dim3(256), 0, st, a, sk, nk, spos,
+    hipLaunchKernelGGL((k_g2p_outside_persist<T, D>), dim3(B.grid_out), dim3(256), 0, st, a, sk, mo.nk,
                        static_cast<const uint32_t*>(counters + CNT_INSIDE));
     TESS_HIP(hipGetLastError());
   }
@@ -771,13 +712,14 @@ void graph_release(tess_batch& B) {
 
 // Every buffer a captured step points at, with its address at the capture.
 std::vector<std::pair<const Buffer*, void*>> graph_buffers(tess_ctx* g, tess_batch& B) {
-  const Buffer* bufs[] = {&g->counters,  &g->keys,       &g->keys_sorted,  &g->vals,         &g->skeys2,
-                          &g->perm2,     &g->keys_alt,   &g->vals_alt,     &g->hist,         &g->scan_tmp,
-                          &g->inc_nk,    &g->inc_spos,   &g->inc_mkey,     &g->inc_mj,       &g->inc_mks,
-                          &g->inc_mr,    &g->inc_mjs,    &g->inc_rng,      &g->movers,       &g->tile_start,
-                          &g->tile_end,  &g->tile_flag,  &g->tile_slot,    &g->active_tiles, &g->nb_flag,
-                          &g->nb_slot,   &g->nb_list,    &g->per_nodeblock, &g->partials,    &B.g_prev_list,
-                          &B.g_prev_count, &B.recs,      &B.d_toff,        &B.d_poff};
+  const Buffer* bufs[] = {&g->counters,   &g->lanes,      &g->keys,        &g->keys_sorted, &g->vals,
+                          &g->skeys2,     &g->perm2,      &g->keys_alt,    &g->vals_alt,    &g->hist,
+                          &g->scan_tmp,   &g->inc_nk,     &g->tile_stay,   &g->tile_tin,    &g->inc_out,
+                          &g->inc_seg,    &g->inc_seg2,   &g->tab_sums,    &g->tile_seg,    &g->tile_start,
+                          &g->tile_end,   &g->tile_flag,  &g->tile_slot,   &g->active_tiles, &g->nb_flag,
+                          &g->nb_list,    &g->alt_start,  &g->alt_end,     &g->alt_flag,    &g->alt_slot,
+                          &g->alt_active, &g->alt_nb_flag, &g->alt_nb_list, &g->partials,   &B.g_prev_list,
+                          &B.g_prev_count, &B.recs,       &B.d_toff,       &B.d_poff,       &B.d_nt};
   std::vector<std::pair<const Buffer*, void*>> v;
   for (const Buffer* b : bufs) v.emplace_back(b, b->ptr);
   return v;
@@ -807,6 +749,7 @@ void graph_reorder_check(tess_ctx* g, tess_batch& B, int cur) {
   if (cur == 1) {
     std::swap(g->keys_sorted, g->skeys2);
     std::swap(g->vals, g->perm2);
+    swap_tables(g);
   }
   B.counted = false;
   try {
@@ -815,12 +758,14 @@ void graph_reorder_check(tess_ctx* g, tess_batch& B, int cur) {
     if (cur == 1) {
       std::swap(g->keys_sorted, g->skeys2);
       std::swap(g->vals, g->perm2);
+      swap_tables(g);
     }
     throw;
   }
   if (cur == 1) {
     std::swap(g->keys_sorted, g->skeys2);
     std::swap(g->vals, g->perm2);
+    swap_tables(g);
   }
   b.valid = false;
 }
@@ -918,10 +863,8 @@ void batch_graph_run(tess_ctx* ctx, tess_batch& B, int nsteps) {
   if (hc[CNT_ERR] & ERR_GIMP_LENGTH) raise(TESS_ERR_ARGUMENT, "uGIMP requires 0 ≤ pt.l ≤ spacing(mesh)");
   if (TESS_DEBUG && B.ntot > 0) {
     // the last step's binning, in set `cur` (the graphs' merges checked through it)
-    const BinSets sets = bin_sets(g, B.ntot);
-    debug_check_binning(gs, sets.keys[cur], sets.perm[cur], static_cast<const uint32_t*>(g->tile_start.ptr),
-                        static_cast<const uint32_t*>(g->tile_end.ptr),
-                        static_cast<const uint32_t*>(g->active_tiles.ptr), B.ntot, B.tiles_total,
+    const BinSet last = bin_set(g, B.ntot, B.tiles_total, cur);
+    debug_check_binning(gs, last.keys, last.perm, last.start, last.end, last.active, B.ntot, B.tiles_total,
                         int64_t(hc[CNT_ACTIVE]), int64_t(hc[CNT_INSIDE]), "batch graph step");
   }
   // the eager path's binning and zeroing bookkeeping no longer hold
@@ -956,6 +899,49 @@ struct BatchCreateOp {
   }
 };
 
+}  // namespace
+
+namespace TESS_PART {
+
+void batch_create(tess_ctx* ctx, int basis, const tess_mesh& mesh, tess_batch& b) {
+  dispatch<BatchCreateOp>(basis, mesh, false, ctx, mesh, b);
+}
+
+void batch_step(tess_ctx* ctx, int basis, const tess_mesh& mesh, tess_batch& b, int nsteps) {
+  dispatch<BatchStepOp>(basis, mesh, false, ctx, mesh, b, nsteps);
+}
+
+}  // namespace TESS_PART
+}  // namespace tess
+
+#else
+
+#include <algorithm>
+
+#include "tess_internal.hpp"
+
+namespace tess {
+namespace {
+
+// frees the graphs (and with them every pointer they recorded)
+void graph_release(tess_batch& B) {
+  for (int p = 0; p < 2; ++p) {
+    if (B.graph_exec[p]) (void)hipGraphExecDestroy(B.graph_exec[p]);
+    if (B.graph[p]) (void)hipGraphDestroy(B.graph[p]);
+    B.graph_exec[p] = nullptr;
+    B.graph[p] = nullptr;
+  }
+  B.captured_variant = -1;
+  B.graph_deps.clear();
+}
+
+void forward_create(tess_ctx* ctx, int basis, const tess_mesh& mesh, tess_batch& b) {
+  TESS_FORWARD(mesh, batch_create(ctx, basis, mesh, b));
+}
+void forward_step(tess_ctx* ctx, int basis, const tess_mesh& mesh, tess_batch& b, int nsteps) {
+  TESS_FORWARD(mesh, batch_step(ctx, basis, mesh, b, nsteps));
+}
+
 bool julia_fields(const tess_scene& sc, int D) {
   auto pok = [](const tess_field& f, int nc) { return !f.ptr || (f.comp_stride == 1 && f.elem_stride == nc); };
   const tess_particles& P = sc.particles;
@@ -978,7 +964,7 @@ void run_batch_create(tess_ctx* ctx, int basis, int nscenes, const tess_scene* s
     b->scenes.assign(scenes, scenes + nscenes);
     b->toff.assign(size_t(nscenes) + 1, 0);
     b->poff.assign(size_t(nscenes) + 1, 0);
-    const int LT = b->dim == 3 ? Geo<3>::LT : Geo<2>::LT;
+    const int LT = b->dim == 3 ? 2 : 3;  // log2 cells per tile axis (Geo)
     for (int s = 0; s < nscenes; ++s) {
       const tess_scene& sc = scenes[s];
       if (sc.mesh.dim != b->dim || sc.mesh.dtype != b->dtype)
@@ -998,11 +984,12 @@ void run_batch_create(tess_ctx* ctx, int basis, int nscenes, const tess_scene* s
     b->tiles_total = b->toff.back();
     if (uint64_t(b->tiles_total) * 64 >= uint64_t(UINT32_MAX) || b->ntot >= int64_t(UINT32_MAX))
       raise(TESS_ERR_ARGUMENT, "the batch exceeds the 32-bit binning range");
-    dispatch<BatchCreateOp>(basis, scenes[0].mesh, false, ctx, scenes[0].mesh, *b);
+    forward_create(ctx, basis, scenes[0].mesh, *b);
   } catch (...) {
     b->recs.release();
     b->d_toff.release();
     b->d_poff.release();
+    b->d_nt.release();
     delete b;
     throw;
   }
@@ -1027,7 +1014,7 @@ void run_batch_step(tess_ctx* ctx, tess_batch* b, int nsteps) {
     b->last_graph = false;
     b->seen_epoch = ep;
   }
-  dispatch<BatchStepOp>(b->basis, b->scenes[0].mesh, false, ctx, b->scenes[0].mesh, *b, nsteps);
+  forward_step(ctx, b->basis, b->scenes[0].mesh, *b, nsteps);
 }
 
 void run_batch_set_variant(tess_batch* b, int variant) { b->variant = variant; }
@@ -1056,8 +1043,11 @@ void run_batch_destroy(tess_batch* b) {
   b->recs.release();
   b->d_toff.release();
   b->d_poff.release();
+  b->d_nt.release();
   b->prev_list.release();
   delete b;
 }
 
 }  // namespace tess
+
+#endif

@@ -1,0 +1,509 @@
+// Tile tables and the merge that re-bins particles between two steps.
+//
+// A binning keeps the particles in the stable order of their sort keys
+// (tile * 64 + class) and, per tile, its run in that order.  Between two steps
+// only some keys change.  The kernel that computes the new keys (G2P, or
+// k_rekey from the positions) works on one tile at a time and leaves, per tile,
+// the particles that stay in it (stay), an arrival count of every other tile
+// (tin) and a list of those that leave (out: previous sorted position and rank
+// among the arrivals of the tile they enter).  From these:
+//   k_tab_reduce / k_tab_scan  new runs, active tiles, touched node blocks and
+//                              arrival segments in two launches, and the
+//                              totals straight into pinned host memory
+//   k_scatter_out              the leavers into their tiles' arrival segments
+//   k_merge_tiles              per tile: arrivals sorted by previous position,
+//                              then one stable counting pass by class over
+//                              (arrivals from lower positions, those that
+//                              stay, arrivals from higher positions)
+// The result is the stable sort of the previous order by the new keys, the
+// order a full radix sort of (new key, previous order) gives.
+//
+// What bounds it: each kernel moves 8-20 bytes per particle or per tile and is
+// short, so launches and the one readback bound it below about a million
+// particles and HBM above.  The scan, compaction, radix sort and placement of
+// the movers that this replaces took about 40 launches and three readbacks per
+// step.  A step of two disks (10,048 particles, Float64): 209 us before, 67 us
+// with this; of a falling block (1.7 M, Float32): 676 -> 476 us; one rollout
+// and pullback of 132,651 particles over 40 steps: 16.7 -> 10.6 ms.
+#include <hip/hip_runtime.h>
+
+#include "tess_internal.hpp"
+
+namespace tess {
+namespace {
+
+constexpr int TAB_THREADS = 256, TAB_PER = 4, TAB_TILES = TAB_THREADS * TAB_PER;
+
+__device__ __forceinline__ uint32_t wave_scan_incl(uint32_t v) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t u = __shfl_up(v, off, 64);
+    if (lane >= off) v += u;
+  }
+  return v;
+}
+
+// sum of v over the workgroup's 256 threads, in every thread
+__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* s) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return s[0] + s[1] + s[2] + s[3];
+}
+
+// exclusive prefix of v over the workgroup's 256 threads
+__device__ __forceinline__ uint32_t block_scan_excl(uint32_t v, uint32_t* s) {
+  const uint32_t inc = wave_scan_incl(v);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 63) s[threadIdx.x >> 6] = inc;
+  __syncthreads();
+  uint32_t base = 0;
+  for (int w = 0; w < int(threadIdx.x >> 6); ++w) base += s[w];
+  return base + inc - v;
+}
+
+__device__ __forceinline__ uint32_t tile_count(const TabArgs& a, int64_t t) { return a.stay[t] + a.tin[t]; }
+
+// Node block B holds nodes BW*B .. BW*B+BW-1 per axis; tile t's footprint
+// [BW*t-1, BW*t+BW+1] touches node blocks t-1, t, t+1: block t is touched when
+// a tile within one of it holds a particle (in a batch, of its own scene).
+__device__ __forceinline__ bool touched(const TabArgs& a, int64_t t) {
+  int nx = a.nt[0], ny = a.nt[1], nz = a.nt[2];
+  int64_t t0 = 0;
+  if (a.scene_toff) {
+    int lo = 0, hi = a.nscenes - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (a.scene_toff[mid] <= t) lo = mid;
+      else hi = mid - 1;
+    }
+    t0 = a.scene_toff[lo];
+    nx = a.scene_nt[3 * lo];
+    ny = a.scene_nt[3 * lo + 1];
+    nz = a.scene_nt[3 * lo + 2];
+  }
+  const uint32_t l = uint32_t(t - t0);
+  const int x = int(l % uint32_t(nx)), y = int((l / uint32_t(nx)) % uint32_t(ny)), z = int(l / (uint32_t(nx) * uint32_t(ny)));
+  uint32_t any = 0;
+  for (int dz = max(z - 1, 0); dz <= min(z + 1, nz - 1); ++dz)
+    for (int dy = max(y - 1, 0); dy <= min(y + 1, ny - 1); ++dy)
+      for (int dx = max(x - 1, 0); dx <= min(x + 1, nx - 1); ++dx)
+        any |= tile_count(a, t0 + (int64_t(dz) * ny + dy) * nx + dx);
+  return any != 0;
+}
+
+// Per workgroup of TAB_TILES tiles: particles, arrivals, active tiles and
+// touched node blocks; writes the touched flags.
+__global__ __launch_bounds__(TAB_THREADS) void k_tab_reduce(TabArgs a) {
+  __shared__ uint32_t s[4];
+  const int64_t base = int64_t(blockIdx.x) * TAB_TILES;
+  uint32_t c = 0, in = 0, act = 0, nb = 0;
+#pragma unroll
+  for (int k = 0; k < TAB_PER; ++k) {
+    const int64_t t = base + k * TAB_THREADS + threadIdx.x;
+    if (t < a.ntiles) {
+      const uint32_t ti = a.tin[t], ct = a.stay[t] + ti;
+      const bool f = ct != 0 || touched(a, t);
+      a.nb_flag[t] = f ? 1u : 0u;
+      c += ct;
+      in += ti;
+      act += ct ? 1u : 0u;
+      nb += f ? 1u : 0u;
+    }
+  }
+  c = block_sum(c, s);
+  in = block_sum(in, s);
+  const uint32_t packed = block_sum(act | (nb << 16), s);
+  if (threadIdx.x == 0) {
+    a.sums[4 * blockIdx.x] = c;
+    a.sums[4 * blockIdx.x + 1] = in;
+    a.sums[4 * blockIdx.x + 2] = packed & 0xffffu;
+    a.sums[4 * blockIdx.x + 3] = packed >> 16;
+  }
+}
+
+// The tables of a workgroup's tiles from the sums of the workgroups before it.
+// Workgroup 0 also sums the lane counters (particles whose key changed, broken
+// layered pairs, nodes with mass), the last one holds the totals; both report
+// to pinned host memory and reset what the next step counts into.
+__global__ __launch_bounds__(TAB_THREADS) void k_tab_scan(TabArgs a) {
+  __shared__ uint32_t s[4];
+  uint32_t pre[4] = {0, 0, 0, 0};
+  for (int b = int(threadIdx.x); b < int(blockIdx.x); b += TAB_THREADS)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) pre[q] += a.sums[4 * b + q];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) pre[q] = block_sum(pre[q], s);
+  const int64_t base = int64_t(blockIdx.x) * TAB_TILES + int64_t(threadIdx.x) * TAB_PER;
+  uint32_t ct[TAB_PER], ti[TAB_PER], fl[TAB_PER];
+  uint32_t c = 0, in = 0, pk = 0;
+#pragma unroll
+  for (int k = 0; k < TAB_PER; ++k) {
+    const int64_t t = base + k;
+    const bool ok = t < a.ntiles;
+    ti[k] = ok ? a.tin[t] : 0u;
+    ct[k] = ok ? a.stay[t] + ti[k] : 0u;
+    fl[k] = ok ? a.nb_flag[t] : 0u;
+    c += ct[k];
+    in += ti[k];
+    pk += (ct[k] ? 1u : 0u) | (fl[k] << 16);
+  }
+  uint32_t ec = pre[0] + block_scan_excl(c, s), ei = pre[1] + block_scan_excl(in, s);
+  const uint32_t epk = block_scan_excl(pk, s);
+  uint32_t ea = pre[2] + (epk & 0xffffu), en = pre[3] + (epk >> 16);
+#pragma unroll
+  for (int k = 0; k < TAB_PER; ++k) {
+    const int64_t t = base + k;
+    if (t < a.ntiles) {
+      a.start[t] = ec;
+      a.end[t] = ec + ct[k];
+      a.flag[t] = ct[k] ? 1u : 0u;
+      a.slot[t] = ea;
+      a.seg[t] = ei;
+      if (ct[k]) a.active[ea] = uint32_t(t);
+      if (fl[k]) a.nb_list[en] = uint32_t(t);
+      if (ti[k]) a.tin[t] = 0u;
+      ec += ct[k];
+      ei += ti[k];
+      ea += ct[k] ? 1u : 0u;
+      en += fl[k];
+    }
+  }
+  // the workgroup that holds the last tile: totals, and the particles outside
+  // the mesh (the entry past the tiles)
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == TAB_THREADS - 1) {
+    const uint32_t out_in = a.tin[a.ntiles];
+    a.seg[a.ntiles] = ei;
+    a.start[a.ntiles] = ec;
+    a.stay[a.ntiles] += out_in;
+    a.tin[a.ntiles] = 0u;
+    a.counters[CNT_PREV_ACTIVE] = a.counters[CNT_ACTIVE];
+    a.counters[CNT_INSIDE] = ec;
+    a.counters[CNT_ACTIVE] = ea;
+    a.counters[CNT_NB] = en;
+    a.counters[CNT_OUTIN] = out_in;
+    a.host[CNT_INSIDE] = ec;
+    a.host[CNT_ACTIVE] = ea;
+    a.host[CNT_NB] = en;
+    a.host[CNT_OUTIN] = out_in;
+    a.host[CNT_ARRIVE] = ei + out_in;
+  }
+  if (blockIdx.x == 0) {
+    uint32_t v[3];
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+      uint32_t x = 0;
+      if (threadIdx.x < LANES) {
+        uint32_t* lane = a.lanes + (g * LANES + int(threadIdx.x)) * LANE_STRIDE;
+        x = *lane;
+        *lane = 0u;
+      }
+      v[g] = block_sum(x, s);
+    }
+    if (threadIdx.x == 0) {
+      a.host[CNT_MOVED] = v[LANE_MOVED];
+      a.host[CNT_MISPLACED] = v[LANE_BROKEN];
+      a.host[CNT_NODES] = v[LANE_NODES];
+      a.counters[CNT_NODES] = v[LANE_NODES];
+      a.host[CNT_ERR] = a.counters[CNT_ERR];
+      a.host[CNT_REENTER] = a.counters[CNT_REENTER];
+      if (!a.keep_err) a.counters[CNT_ERR] = 0u;
+      a.counters[CNT_REENTER] = 0u;
+    }
+  }
+  __threadfence_system();
+}
+
+// Particles of each tile in a freshly sorted order (binary searches of the
+// keys; the entry past the tiles counts the particles outside the mesh).
+__global__ __launch_bounds__(256) void k_tile_counts(const uint32_t* __restrict__ skeys, int64_t n, int64_t ntiles,
+                                                     uint32_t* __restrict__ stay, uint32_t* __restrict__ tin) {
+  __shared__ uint32_t s_bound[257];
+  auto bound = [&](int64_t t) {  // first position whose key is not below tile t's
+    int64_t lo = 0, hi = n;
+    const uint32_t key = uint32_t(t) * 64u;
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (skeys[mid] < key) lo = mid + 1;
+      else hi = mid;
+    }
+    return uint32_t(lo);
+  };
+  const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (t <= ntiles) s_bound[threadIdx.x] = bound(t);
+  if (threadIdx.x == 255 && t + 1 <= ntiles) s_bound[256] = bound(t + 1);
+  __syncthreads();
+  if (t > ntiles) return;
+  const uint32_t hi = t == ntiles ? uint32_t(n) : s_bound[threadIdx.x + 1];
+  stay[t] = hi - s_bound[threadIdx.x];
+  tin[t] = 0u;
+}
+
+// The leavers of each previously active tile into the arrival segments of the
+// tiles they enter (a leaver's rank there was drawn when its key was computed).
+__global__ __launch_bounds__(64) void k_scatter_out(MergeArgs a) {
+  const int64_t j = blockIdx.x;
+  if (j >= int64_t(a.old_count ? *a.old_count : a.old_active_n)) return;
+  const uint32_t t = a.old_active[j];
+  const uint32_t start = a.old_start[t], cnt = a.old_end[t] - start;
+  const uint32_t leave = cnt - a.stay[t];
+  for (uint32_t i = threadIdx.x; i < leave; i += 64) {
+    const uint2 o = a.out[start + i];
+    const uint32_t key = a.nk[o.x];
+    a.seg[a.seg_off[key >> 6] + o.y] = make_uint2(key, o.x);
+  }
+}
+
+constexpr int MERGE_THREADS = 256, MERGE_WAVES = MERGE_THREADS / 64, MERGE_CAP = 512;
+
+// Sorts k (key, position) pairs of a segment by position with one workgroup:
+// 8-bit digits of the position, `bits` low bits, between seg and alt; returns
+// the buffer that holds the result.  For segments past the LDS list.
+__device__ uint2* segment_sort(uint2* seg, uint2* alt, uint32_t k, int bits, uint32_t* s_hist, uint32_t (*s_wc)[256]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int shift = 0; shift < bits; shift += 8) {
+    __syncthreads();
+    s_hist[threadIdx.x] = 0;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < k; i += MERGE_THREADS) atomicAdd(&s_hist[(seg[i].y >> shift) & 255u], 1u);
+    __syncthreads();
+    const uint32_t h = s_hist[threadIdx.x];
+    __shared__ uint32_t s4[4];
+    const uint32_t ex = block_scan_excl(h, s4);
+    __syncthreads();
+    s_hist[threadIdx.x] = ex;
+    for (uint32_t b = 0; b < k; b += MERGE_THREADS) {
+      const uint32_t i = b + threadIdx.x;
+      const bool valid = i < k;
+      const uint2 e = valid ? seg[i] : make_uint2(0u, 0u);
+      const uint32_t d = (e.y >> shift) & 255u;
+#pragma unroll
+      for (int w = 0; w < MERGE_WAVES; ++w) s_wc[w][threadIdx.x] = 0;
+      __syncthreads();
+      uint64_t peers = __ballot(valid);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const bool bit = (d >> q) & 1u;
+        const uint64_t m = __ballot(valid && bit);
+        peers &= bit ? m : ~m;
+      }
+      const uint32_t below = uint32_t(__popcll(peers & ((uint64_t(1) << lane) - 1)));
+      if (valid && below == 0) s_wc[wave][d] = uint32_t(__popcll(peers));
+      __syncthreads();
+      if (valid) {
+        uint32_t pos = s_hist[d] + below;
+        for (int w = 0; w < wave; ++w) pos += s_wc[w][d];
+        alt[pos] = e;
+      }
+      __syncthreads();
+      uint32_t add = 0;
+#pragma unroll
+      for (int w = 0; w < MERGE_WAVES; ++w) add += s_wc[w][threadIdx.x];
+      s_hist[threadIdx.x] += add;
+      __syncthreads();
+    }
+    __threadfence_block();
+    __syncthreads();
+    uint2* const x = seg;
+    seg = alt;
+    alt = x;
+  }
+  return seg;
+}
+
+// One workgroup per tile that holds particles now.  The tile's new run is the
+// stable counting sort, by class, of a sequence in order of previous position:
+// arrivals from below its old run, the old run without its leavers, arrivals
+// from above.  The four waves take consecutive quarters of the sequence.
+__global__ __launch_bounds__(MERGE_THREADS) void k_merge_tiles(MergeArgs a) {
+  __shared__ uint2 s_raw[MERGE_CAP], s_in[MERGE_CAP];
+  __shared__ uint32_t s_hist[256], s_wc[MERGE_WAVES][256];
+  __shared__ uint32_t s_base[MERGE_WAVES][64], s_low;
+  const int64_t jt = blockIdx.x;
+  if (jt >= int64_t(a.new_count ? *a.new_count : a.new_active_n)) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const uint32_t t = a.new_active[jt];
+  const uint32_t os = a.old_start[t], oc = a.old_end[t] - os;
+  const uint32_t ns = a.new_start[t], k = a.new_end[t] - ns - a.stay[t];
+  const uint2* in = s_in;
+  if (threadIdx.x == 0) s_low = 0;
+  s_base[wave][lane] = 0;
+  if (k > 0 && k <= MERGE_CAP) {
+    const uint2* seg = a.seg + a.seg_off[t];
+    for (uint32_t i = threadIdx.x; i < k; i += MERGE_THREADS) s_raw[i] = seg[i];
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < k; i += MERGE_THREADS) {
+      const uint2 e = s_raw[i];
+      uint32_t r = 0;
+      for (uint32_t q = 0; q < k; ++q) r += s_raw[q].y < e.y ? 1u : 0u;
+      s_in[r] = e;
+    }
+  } else if (k > 0) {
+    in = segment_sort(a.seg + a.seg_off[t], a.seg_alt + a.seg_off[t], k, a.pos_bits, s_hist, s_wc);
+  }
+  __syncthreads();
+  if (k > 0) {
+    uint32_t low = 0;
+    for (uint32_t i = threadIdx.x; i < k; i += MERGE_THREADS) low += in[i].y < os ? 1u : 0u;
+    if (low) atomicAdd(&s_low, low);
+    __syncthreads();
+  }
+  const uint32_t klow = s_low, len = k + oc;
+  // element i of the sequence: its key (in *valid elements) and previous position
+  auto element = [&](uint32_t i, uint32_t& key, uint32_t& pos) {
+    if (i >= len) return false;
+    if (i >= klow && i < klow + oc) {
+      pos = os + (i - klow);
+      key = a.nk[pos];
+      return (key >> 6) == t;
+    }
+    const uint2 e = in[i < klow ? i : i - oc];
+    key = e.x;
+    pos = e.y;
+    return true;
+  };
+  const uint32_t quarter = ((len + 255u) / 256u) * 64u;
+  const uint32_t i0 = uint32_t(wave) * quarter;
+  auto match = [&](uint32_t c, bool valid) {
+    uint64_t peers = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+      const bool bit = (c >> b) & 1u;
+      const uint64_t m = __ballot(valid && bit);
+      peers &= bit ? m : ~m;
+    }
+    return peers;
+  };
+  const uint64_t lt = (uint64_t(1) << lane) - 1;
+  // class counts of the wave's quarter; the first chunks stay in registers
+  constexpr int KEEP = 4;
+  uint32_t kk[KEEP], kp[KEEP];
+  bool kv[KEEP];
+#pragma unroll
+  for (int r = 0; r < KEEP; ++r) {
+    kk[r] = kp[r] = 0u;
+    kv[r] = uint32_t(r) * 64u < quarter && element(i0 + uint32_t(r) * 64u + uint32_t(lane), kk[r], kp[r]);
+  }
+  uint32_t* mine = s_base[wave];
+#pragma unroll
+  for (int r = 0; r < KEEP; ++r) {
+    if (uint32_t(r) * 64u >= quarter) break;  // uniform
+    const uint64_t peers = match(kk[r] & 63u, kv[r]);
+    if (kv[r] && (peers & lt) == 0) mine[kk[r] & 63u] += uint32_t(__popcll(peers));
+    __asm__ volatile("" ::: "memory");  // the next chunk's counts in program order
+  }
+  for (uint32_t o = KEEP * 64u; o < quarter; o += 64u) {
+    uint32_t key = 0u, pos = 0u;
+    const bool v = element(i0 + o + uint32_t(lane), key, pos);
+    const uint64_t peers = match(key & 63u, v);
+    if (v && (peers & lt) == 0) mine[key & 63u] += uint32_t(__popcll(peers));
+    __asm__ volatile("" ::: "memory");
+  }
+  __syncthreads();
+  // where each (class, wave) starts: classes ascending, waves in order
+  if (wave == 0) {
+    uint32_t tot = 0, w[MERGE_WAVES];
+#pragma unroll
+    for (int q = 0; q < MERGE_WAVES; ++q) {
+      w[q] = s_base[q][lane];
+      tot += w[q];
+    }
+    uint32_t run = wave_scan_incl(tot) - tot;
+#pragma unroll
+    for (int q = 0; q < MERGE_WAVES; ++q) {
+      s_base[q][lane] = run;
+      run += w[q];
+    }
+  }
+  __syncthreads();
+  auto place = [&](uint32_t key, uint32_t pos, bool v) {
+    const uint64_t peers = match(key & 63u, v);
+    const uint32_t below = uint32_t(__popcll(peers & lt));
+    // the leader of each class draws its peers' slots (the LDS executes one
+    // wave's accesses in order; the shuffle hands the base to the peers)
+    uint32_t base = 0u;
+    if (v && below == 0) {
+      base = mine[key & 63u];
+      mine[key & 63u] = base + uint32_t(__popcll(peers));
+    }
+    __asm__ volatile("" ::: "memory");  // the next chunk draws after this one
+    base = __shfl(base, v ? __ffsll((unsigned long long)peers) - 1 : lane, 64);
+    if (v) {
+      a.keys_new[ns + base + below] = key;
+      a.perm_new[ns + base + below] = a.perm_old[pos];
+    }
+  };
+#pragma unroll
+  for (int r = 0; r < KEEP; ++r) {
+    if (uint32_t(r) * 64u >= quarter) break;  // uniform
+    place(kk[r], kp[r], kv[r]);
+  }
+  for (uint32_t o = KEEP * 64u; o < quarter; o += 64u) {
+    uint32_t key = 0u, pos = 0u;
+    const bool v = element(i0 + o + uint32_t(lane), key, pos);
+    place(key, pos, v);
+  }
+}
+
+// Particles outside the mesh: those that were outside keep their order behind
+// the arrivals (whose previous positions are all lower).  Workgroup 0 places
+// the arrivals, sorted by previous position.
+__global__ __launch_bounds__(MERGE_THREADS) void k_merge_outside(MergeArgs a) {
+  __shared__ uint32_t s_hist[256], s_wc[MERGE_WAVES][256];
+  const uint32_t k = a.counters ? a.counters[CNT_OUTIN] : a.out_in;
+  const uint32_t ns = a.new_start[a.ntiles], os = a.old_start[a.ntiles];
+  if (blockIdx.x == 0 && k > 0) {
+    const uint32_t off = a.seg_off[a.ntiles];
+    const uint2* in = segment_sort(a.seg + off, a.seg_alt + off, k, a.pos_bits, s_hist, s_wc);
+    for (uint32_t i = threadIdx.x; i < k; i += MERGE_THREADS) {
+      a.keys_new[ns + i] = in[i].x;
+      a.perm_new[ns + i] = a.perm_old[in[i].y];
+    }
+  }
+  const uint32_t stayed = uint32_t(a.n) - os;
+  for (uint32_t i = blockIdx.x * MERGE_THREADS + threadIdx.x; i < stayed; i += gridDim.x * MERGE_THREADS) {
+    a.keys_new[ns + k + i] = a.nk[os + i];
+    a.perm_new[ns + k + i] = a.perm_old[os + i];
+  }
+}
+
+}  // namespace
+
+int64_t tab_blocks(int64_t ntiles) { return ceil_div(ntiles, int64_t(TAB_TILES)); }
+
+void launch_tables(hipStream_t st, const TabArgs& a) {
+  const unsigned nb = unsigned(tab_blocks(a.ntiles));
+  hipLaunchKernelGGL(k_tab_reduce, dim3(nb), dim3(TAB_THREADS), 0, st, a);
+  TESS_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_tab_scan, dim3(nb), dim3(TAB_THREADS), 0, st, a);
+  TESS_HIP(hipGetLastError());
+}
+
+void launch_tile_counts(hipStream_t st, const uint32_t* skeys, int64_t n, int64_t ntiles, uint32_t* stay, uint32_t* tin) {
+  hipLaunchKernelGGL(k_tile_counts, dim3(unsigned(ceil_div(ntiles + 1, int64_t(256)))), dim3(256), 0, st, skeys, n, ntiles,
+                     stay, tin);
+  TESS_HIP(hipGetLastError());
+}
+
+// arrivals: whether any particle entered a tile; the launch counts are those of
+// the host, or upper bounds of the device counts the args point at.
+void launch_merge(hipStream_t st, const MergeArgs& a, bool arrivals, unsigned outside_blocks) {
+  if (arrivals && a.old_active_n > 0) {
+    hipLaunchKernelGGL(k_scatter_out, dim3(unsigned(a.old_active_n)), dim3(64), 0, st, a);
+    TESS_HIP(hipGetLastError());
+  }
+  if (a.new_active_n > 0) {
+    hipLaunchKernelGGL(k_merge_tiles, dim3(unsigned(a.new_active_n)), dim3(MERGE_THREADS), 0, st, a);
+    TESS_HIP(hipGetLastError());
+  }
+  if (outside_blocks > 0) {
+    hipLaunchKernelGGL(k_merge_outside, dim3(outside_blocks), dim3(MERGE_THREADS), 0, st, a);
+    TESS_HIP(hipGetLastError());
+  }
+}
+
+}  // namespace tess

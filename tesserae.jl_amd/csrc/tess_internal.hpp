@@ -57,8 +57,11 @@ struct Binning {
   bool state_valid = false;
   int64_t state_n = -1, state_ntiles = -1;
   int32_t state_dim = 0;
-  // the last G2P wrote the next keys and stay flags at the sorted positions
+  // the last G2P wrote the next keys at the sorted positions and the counts
+  // and leavers of every tile
   bool keys_ready = false;
+  // counts the binnings that built new tile lists
+  uint64_t generation = 0;
 };
 
 // Per-kernel timing with HIP events on the context's stream.  Disabled by
@@ -101,6 +104,71 @@ struct Rollout {
 
 }  // namespace tess
 
+namespace tess {
+
+// device counters (words of tess_ctx::counters, reported to the same words of
+// counters_host): totals of a binning, error flags, and sums over the lanes
+enum {
+  CNT_INSIDE = 0, CNT_ACTIVE = 1, CNT_NB = 2, CNT_ERR = 3, CNT_BIN_SLOTS = 4,
+  CNT_MISPLACED = 8, CNT_NODES = 9, CNT_ARRIVE = 10, CNT_P2GERR = 11, CNT_MOVED = 12, CNT_OUTIN = 13, CNT_REENTER = 14,
+  CNT_PREV_ACTIVE = 15, CNT_SLOTS = 16
+};
+// Kernels count into lanes, one per 128-byte line, chosen by workgroup (no
+// single contended address): particles whose key changed, layered neighbour
+// pairs not consecutive in storage, nodes with m > 0.
+enum { LANE_MOVED = 0, LANE_BROKEN = 1, LANE_NODES = 2, LANE_GROUPS = 3 };
+constexpr int LANES = 32, LANE_STRIDE = 32;
+constexpr size_t LANE_BYTES = size_t(LANE_GROUPS) * LANES * LANE_STRIDE * sizeof(uint32_t);
+
+// What a kernel that computes next keys writes (see binning.hip): the keys at
+// the sorted positions (nullptr: nothing is written), per tile the particles
+// that stay and the arrivals, and the leavers of each tile from its run's start.
+struct MoveOut {
+  uint32_t* nk;
+  uint32_t* stay;
+  uint32_t* tin;
+  uint2* out;
+  uint32_t* lanes;
+};
+
+// The tile tables of a binning, from the per-tile counts (binning.hip).
+struct TabArgs {
+  uint32_t* stay;  // ntiles + 1: particles that stay, the last entry those outside the mesh
+  uint32_t* tin;   // ntiles + 1: arrivals (reset)
+  int64_t ntiles;
+  int32_t nt[3];
+  const int64_t* scene_toff;  // a batch: first tile and tiles per axis of each scene
+  const int32_t* scene_nt;
+  int32_t nscenes;
+  uint32_t* sums;  // 4 words per workgroup
+  uint32_t *start, *end, *flag, *slot, *active, *nb_flag, *nb_list, *seg;
+  uint32_t* lanes;
+  uint32_t* counters;
+  uint32_t* host;
+  int32_t keep_err;
+};
+
+// The merge of the particles whose key changed into the previous order.
+struct MergeArgs {
+  int64_t n, ntiles;
+  const uint32_t *old_active, *old_start, *old_end, *new_active, *new_start, *new_end;
+  const uint32_t* old_count;  // device counts for launches sized by an upper bound, or nullptr
+  const uint32_t* new_count;
+  int64_t old_active_n, new_active_n;
+  const uint32_t* stay;
+  const uint32_t* nk;
+  const uint32_t* perm_old;
+  const uint32_t* seg_off;
+  const uint2* out;
+  uint2 *seg, *seg_alt;
+  uint32_t *keys_new, *perm_new;
+  const uint32_t* counters;  // device count of arrivals outside the mesh, or nullptr: out_in
+  uint32_t out_in;
+  int32_t pos_bits;
+};
+
+}  // namespace tess
+
 struct tess_ctx {
   tess::Profiler prof;
   int device = 0;
@@ -109,11 +177,16 @@ struct tess_ctx {
   // *_alt ping-pong buffers of the radix sort
   tess::Buffer keys, keys_sorted, vals, keys_alt, vals_alt, hist, scan_tmp;
   tess::Buffer tile_start, tile_end, tile_flag, tile_slot, active_tiles;
-  tess::Buffer nb_flag, nb_slot, nb_list, nb_list_prev;
+  tess::Buffer nb_flag, nb_list, nb_list_prev;
+  // the tables being built while the ones above are in use
+  tess::Buffer alt_start, alt_end, alt_flag, alt_slot, alt_active, alt_nb_flag, alt_nb_list;
+  tess::Buffer tab_sums, tile_seg;
   tess::Buffer partials;
-  tess::Buffer per_tile, per_nodeblock;  // per-workgroup counts summed by a reduction
-  // incremental re-binning scratch
-  tess::Buffer skeys2, perm2, inc_nk, inc_spos, inc_mkey, inc_mj, inc_mks, inc_mr, inc_mjs, inc_rng;
+  tess::Buffer per_tile;  // per-workgroup counts of the partition's contiguity score
+  // re-binning scratch: the other half of (keys_sorted, vals), next keys,
+  // per-tile counts, leavers, arrival segments
+  tess::Buffer skeys2, perm2, inc_nk, tile_stay, tile_tin, inc_out, inc_seg, inc_seg2;
+  tess::Buffer inc_pout, inc_rank;  // a batch reorder's new indices and ranks
   int64_t last_movers = -1;
   int64_t kept_binnings = 0;  // binnings that kept the previous layout (no particle changed its key)
   tess::Buffer counters;   // small device scalars
@@ -123,13 +196,14 @@ struct tess_ctx {
   // TESS_POLY_MULTILINEAR bits, 0 for a plain kernel) and its node filter
   int32_t corr = 0;
   const uint8_t* corr_filter = nullptr;
-  tess::Buffer movers;     // G2P's changed-key counts (spread over cache lines)
+  tess::Buffer lanes;      // counts spread over cache lines (LANE_GROUPS groups of LANES)
   tess::Buffer host_pinned_dummy;
   int64_t* counters_host = nullptr;  // pinned readback slots
   tess::Binning bin;
   // zeroing bookkeeping for the grid of the previous P2G
   const void* last_grid_m = nullptr;
   int64_t prev_nodeblocks = 0;
+  uint64_t prev_generation = 0;  // the binning nb_list_prev is of
   int32_t prev_tile_log2 = -1;
   int64_t prev_ntiles = -1;
   int64_t prev_nnodes = -1;
@@ -140,6 +214,9 @@ struct tess_ctx {
   int64_t misplaced_pairs = 0;  // layered neighbour pairs of that P2G's binning
   int64_t last_misplaced = -1;  // of them, pairs not consecutive in storage
   int64_t reorders = 0;
+  // a P2G has counted broken pairs (nodes) since the last report of the lanes
+  bool broken_pending = false, nodes_pending = false;
+  int64_t broken_count = 0;
   // nodes with m > 0 written by the last gather (read back with the next binning)
   int64_t last_active_nodes = -1;
   // SpGrid block activation scratch (occupied flags, active flags, scan)
@@ -168,7 +245,7 @@ struct tess_batch {
   int64_t ntot = 0, tiles_total = 0, max_nodes = 0;
   std::vector<tess_scene> scenes;
   std::vector<int64_t> toff, poff;
-  tess::Buffer recs, d_toff, d_poff, prev_list;
+  tess::Buffer recs, d_toff, d_poff, d_nt, prev_list;
   int64_t prev_nb = 0;
   bool zeroed = false;
   // the binning in the context is this batch's, and the last G2P wrote every
@@ -240,6 +317,12 @@ size_t scan_work_bytes(int64_t n);
 void radix_sort_pairs_ws(const SortWork& w, const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out,
                          uint32_t* vals_out, int64_t n, int key_bits, const uint32_t* n_dev = nullptr);
 
+// ---- tile tables and the merge between two steps (binning.hip) ----
+int64_t tab_blocks(int64_t ntiles);
+void launch_tables(hipStream_t st, const TabArgs& a);
+void launch_tile_counts(hipStream_t st, const uint32_t* skeys, int64_t n, int64_t ntiles, uint32_t* stay, uint32_t* tin);
+void launch_merge(hipStream_t st, const MergeArgs& a, bool arrivals, unsigned outside_blocks);
+
 // ---- reference-layout weights and partition (partition.hip) ----
 void launch_update_weights(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_particles& P,
                            const tess_weights& W);
@@ -309,6 +392,48 @@ void run_batch_stats(const tess_batch* b, int64_t* out, int n);
 void run_batch_destroy(tess_batch* b);
 // Moves every particle field so that slot k receives particle order[k].
 void permute_particles(tess_ctx* ctx, const tess_mesh& mesh, const tess_particles& P, const uint32_t* order);
+
+// ---- scalar type and dimension parts ------------------------------------------
+// The templated files (transfer, batch, adjoint) are compiled once per (scalar
+// type, dimension), in parallel: each part's functions live in the namespace
+// named TESS_PART, and the same file compiled without it forwards to them.
+#define TESS_PART_DECLARE(NS)                                                                                        \
+  namespace NS {                                                                                                     \
+  void p2g(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,             \
+           const tess_weights* W, const tess_params& prm, const tess_sparsity* sp);                                  \
+  void g2p(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,             \
+           const tess_weights* W, const tess_params& prm, const tess_sparsity* sp);                                  \
+  void g2p2g(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,           \
+             const tess_weights* W, const tess_params& prm);                                                         \
+  void g2p2g_steps(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,     \
+                   const tess_params& prm, int nsteps, double reorder_threshold);                                    \
+  void step(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,            \
+            const tess_params& prm, int nsteps, double reorder_threshold, tess_sparsity* sp, int* done);             \
+  void step_adjoint(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,    \
+                    const tess_params& prm, const tess_adjoint& adj);                                                \
+  void rollout(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,         \
+               const tess_params& prm, int nsteps, int every);                                                       \
+  void rollout_adjoint(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_params& prm,  \
+                       const tess_adjoint& adj);                                                                     \
+  void batch_create(tess_ctx* ctx, int basis, const tess_mesh& mesh, tess_batch& b);                                 \
+  void batch_step(tess_ctx* ctx, int basis, const tess_mesh& mesh, tess_batch& b, int nsteps);                       \
+  }
+TESS_PART_DECLARE(part_f32_2d)
+TESS_PART_DECLARE(part_f32_3d)
+TESS_PART_DECLARE(part_f64_2d)
+TESS_PART_DECLARE(part_f64_3d)
+#undef TESS_PART_DECLARE
+#define TESS_FORWARD(mesh, ...)                                  \
+  do {                                                           \
+    if ((mesh).dtype == TESS_FLOAT32) {                          \
+      if ((mesh).dim == 2) return part_f32_2d::__VA_ARGS__;      \
+      if ((mesh).dim == 3) return part_f32_3d::__VA_ARGS__;      \
+    } else {                                                     \
+      if ((mesh).dim == 2) return part_f64_2d::__VA_ARGS__;      \
+      if ((mesh).dim == 3) return part_f64_3d::__VA_ARGS__;      \
+    }                                                            \
+    raise(TESS_ERR_UNSUPPORTED, "unsupported (dim, dtype, basis) combination"); \
+  } while (0)
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 

@@ -9,8 +9,8 @@
 // touches each node at most once, so the sums follow a fixed order):
 //   k_bin_keys      particle -> tile whose footprint holds its support window
 //   radix sort      stable (tile, particle id) order -> perm
-//   k_tile_runs / k_tile_flags / scan / k_active_list   tile ranges + slots
-//   k_nb_mark / scan / k_nb_list    node blocks touched by some footprint
+//   k_tile_counts / k_tab_reduce / k_tab_scan   tile ranges + slots, node blocks
+//                   touched by some footprint (binning.hip)
 //   k_p2g_tile      one wave per tile: lanes own the 64 window-start classes of
 //                   the tile, accumulate their particles' contributions in
 //                   registers and add them into an LDS tile of the
@@ -90,35 +90,12 @@ struct Pow<N, 0> {
   static constexpr int v = 1;
 };
 
-// device counters: binning totals (zeroed per binning), error flags, and the
-// misplaced-particle count of the last P2G (zeroed per P2G)
-enum {
-  CNT_INSIDE = 0, CNT_ACTIVE = 1, CNT_NB = 2, CNT_ERR = 3, CNT_BIN_SLOTS = 4,
-  CNT_MISPLACED = 8, CNT_NODES = 9, CNT_STAY = 10, CNT_P2GERR = 11, CNT_SLOTS = 16
-};
-// G2P counts the particles whose key changed into MOVER_LANES counters, one per
-// 128-byte line, chosen by workgroup (no single contended address)
-constexpr int MOVER_LANES = 8, MOVER_STRIDE = 32;
-
-inline uint32_t* movers_counters(tess_ctx* ctx) {
-  return ctx->movers.as<uint32_t>(size_t(MOVER_LANES * MOVER_STRIDE));
+// the lane counters (zero between their reports)
+inline uint32_t* lane_counters(tess_ctx* ctx) {
+  return ctx->lanes.as<uint32_t>(size_t(LANE_GROUPS) * LANES * LANE_STRIDE);
 }
-// zero them (before a G2P that counts)
-inline void movers_zero(tess_ctx* ctx) {
-  TESS_HIP(hipMemsetAsync(movers_counters(ctx), 0, MOVER_LANES * MOVER_STRIDE * sizeof(uint32_t), ctx->stream));
-}
-// enqueue their readback into the pinned slots after the counters
-inline void movers_readback(tess_ctx* ctx) {
-  uint32_t* hc = reinterpret_cast<uint32_t*>(ctx->counters_host) + 64;
-  TESS_HIP(hipMemcpyAsync(hc, movers_counters(ctx), MOVER_LANES * MOVER_STRIDE * sizeof(uint32_t),
-                          hipMemcpyDeviceToHost, ctx->stream));
-}
-// the sum, after a synchronisation that followed movers_readback
-inline int64_t movers_total(tess_ctx* ctx) {
-  const uint32_t* hc = reinterpret_cast<const uint32_t*>(ctx->counters_host) + 64;
-  int64_t t = 0;
-  for (int i = 0; i < MOVER_LANES; ++i) t += hc[i * MOVER_STRIDE];
-  return t;
+__device__ __forceinline__ uint32_t* lane_of(uint32_t* lanes, int group) {
+  return lanes + (group * LANES + int(blockIdx.x) % LANES) * LANE_STRIDE;
 }
 enum { ERR_GIMP_LENGTH = 1, ERR_WINDOW = 2, ERR_INACTIVE = 4 };
 
@@ -412,218 +389,81 @@ __global__ __launch_bounds__(256) void k_bin_keys(Args<T, D> a, uint32_t* __rest
   keys[p] = particle_key<T, D, BASIS, STORED>(a, p, ntiles, counters + CNT_ERR);
 }
 
-// ---- incremental re-binning ---------------------------------------------------
-// New keys are taken in the previous sorted order j; the new order is the
-// stable sort of that order by the new keys.  Particles whose key is unchanged
-// ("stayers") keep their relative order; the few "movers" are sorted among
-// themselves and merged.  The full radix sort of (new key, previous order) is
-// the fallback when many particles move; both give the same permutation.
+// ---- re-binning ----------------------------------------------------------------
+// New keys are taken in the previous sorted order; the new order is the stable
+// sort of that order by the new keys (the merge of binning.hip).
 
-template <typename T, int D, int BASIS, bool STORED>
-__global__ __launch_bounds__(256) void k_keys_sorted(Args<T, D> a, const uint32_t* __restrict__ perm,
-                                                     const uint32_t* __restrict__ skeys, uint32_t ntiles,
-                                                     uint32_t* __restrict__ nk, uint32_t* __restrict__ stay,
-                                                     uint32_t* __restrict__ counters) {
-  const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (j > a.n) return;
-  if (j == a.n) {
-    stay[j] = 0;  // scan slot holding the stayer total
-    return;
-  }
-  const uint32_t k = particle_key<T, D, BASIS, STORED>(a, perm[j], ntiles, counters + CNT_ERR);
-  nk[j] = k;
-  stay[j] = k == skeys[j] ? 1u : 0u;
-}
+// The counters of a workgroup that computes its tile's next keys.
+struct TileMoves {
+  uint32_t leave, moved;
+};
 
-__global__ void k_compact_movers(const uint32_t* __restrict__ nk, const uint32_t* __restrict__ spos, int64_t n,
-                                 uint32_t* __restrict__ mkey, uint32_t* __restrict__ mj) {
-  const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (j >= n || spos[j + 1] != spos[j]) return;
-  const int64_t r = j - spos[j];
-  mkey[r] = nk[j];
-  mj[r] = uint32_t(j);
-}
-
-// number of i in [lo, hi) with (k[i], jj[i]) < (K, J) for lexicographically sorted pairs
-__device__ __forceinline__ int64_t lower_bound_pair(const uint32_t* k, const uint32_t* jj, int64_t lo, int64_t hi,
-                                                    uint32_t K, uint32_t J) {
-  while (lo < hi) {
-    const int64_t mid = (lo + hi) >> 1;
-    const bool less = k[mid] < K || (k[mid] == K && jj[mid] < J);
-    if (less) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
-}
-
-__device__ __forceinline__ int64_t bound_key(const uint32_t* k, int64_t n, uint32_t K, bool upper) {
-  int64_t lo = 0, hi = n;
-  while (lo < hi) {
-    const int64_t mid = (lo + hi) >> 1;
-    const bool go = upper ? k[mid] <= K : k[mid] < K;
-    if (go) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
-}
-
-// Sorted mover i (key K, previous position j) lands after every stayer with a
-// smaller key or an equal key and smaller previous position, and after the
-// movers before it.
-// (M_dev, when set: the mover count read on the device, at most M.)
-__global__ void k_place_movers(const uint32_t* __restrict__ mks, const uint32_t* __restrict__ mr,
-                               const uint32_t* __restrict__ mj, const uint32_t* __restrict__ skeys_old,
-                               const uint32_t* __restrict__ perm_old, const uint32_t* __restrict__ spos, int64_t n,
-                               int64_t M, uint32_t* __restrict__ mjs, uint32_t* __restrict__ skeys_new,
-                               uint32_t* __restrict__ perm_new, const uint32_t* __restrict__ M_dev) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (M_dev) M = int64_t(*M_dev);
-  if (i >= M) return;
-  const uint32_t K = mks[i];
-  const int64_t j = mj[mr[i]];
-  mjs[i] = uint32_t(j);
-  const int64_t lb = bound_key(skeys_old, n, K, false), ub = bound_key(skeys_old, n, K, true);
-  const int64_t c = j < lb ? lb : (j > ub ? ub : j);
-  const int64_t pos = i + int64_t(spos[c]);
-  skeys_new[pos] = K;
-  perm_new[pos] = perm_old[j];
-}
-
-// Stayer j moves back by the movers removed before it and forward by the
-// movers inserted before it (sorted movers with a pair (key, j') < (key, j)).
-constexpr int STAY_BLOCK = 256, STAY_CAP = 2048;
-// The movers [ranges[2b], ranges[2b+1]) that fall among the stayers of
-// k_place_stayers' workgroup b, one thread per workgroup (the binary searches
-// run in parallel instead of at the start of every workgroup).
-__global__ void k_stay_ranges(const uint32_t* __restrict__ skeys_old, int64_t n, const uint32_t* __restrict__ mks,
-                              const uint32_t* __restrict__ mjs, int64_t M, int64_t nblocks,
-                              int64_t* __restrict__ ranges, const uint32_t* __restrict__ M_dev) {
-  const int64_t b = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (b >= nblocks) return;
-  if (M_dev) M = int64_t(*M_dev);
-  const int64_t j0 = b * STAY_BLOCK;
-  const int64_t j1 = j0 + STAY_BLOCK < n ? j0 + STAY_BLOCK : n;
-  const int64_t lo = lower_bound_pair(mks, mjs, 0, M, skeys_old[j0], uint32_t(j0));
-  ranges[2 * b] = lo;
-  ranges[2 * b + 1] = lower_bound_pair(mks, mjs, lo, M, skeys_old[j1 - 1], uint32_t(j1));
-}
-
-__global__ __launch_bounds__(STAY_BLOCK) void k_place_stayers(
-    const uint32_t* __restrict__ skeys_old, const uint32_t* __restrict__ perm_old, const uint32_t* __restrict__ spos,
-    int64_t n, const uint32_t* __restrict__ mks, const uint32_t* __restrict__ mjs, const int64_t* __restrict__ ranges,
-    uint32_t* __restrict__ skeys_new, uint32_t* __restrict__ perm_new) {
-  __shared__ uint32_t s_k[STAY_CAP], s_j[STAY_CAP];
-  const int64_t j0 = int64_t(blockIdx.x) * STAY_BLOCK;
-  const int64_t j1 = j0 + STAY_BLOCK < n ? j0 + STAY_BLOCK : n;
-  const int64_t a0 = ranges[2 * int64_t(blockIdx.x)], cnt = ranges[2 * int64_t(blockIdx.x) + 1] - a0;
-  const bool in_lds = cnt <= STAY_CAP;
-  if (in_lds)
-    for (int64_t t = threadIdx.x; t < cnt; t += STAY_BLOCK) {
-      s_k[t] = mks[a0 + t];
-      s_j[t] = mjs[a0 + t];
+// One particle's next key at sorted position jj of the tile whose run starts at
+// `start`: written out, counted, and listed with its rank among the arrivals
+// when it enters another tile (or leaves the mesh: tile ntiles).
+__device__ __forceinline__ void next_key(const MoveOut& mo, uint32_t key, uint32_t old_key, uint32_t jj, uint32_t tile,
+                                         uint32_t start, TileMoves* s_mv, uint32_t& moved) {
+  mo.nk[jj] = key;
+  if (key != old_key) {
+    ++moved;
+    if ((key >> 6) != tile) {
+      const uint32_t r = atomicAdd(&mo.tin[key >> 6], 1u);
+      mo.out[start + atomicAdd(&s_mv->leave, 1u)] = make_uint2(jj, r);
     }
+  }
+}
+
+// The tile's counts, by every thread of the workgroup after its last key.
+__device__ __forceinline__ void tile_moves_end(const MoveOut& mo, uint32_t tile, int cnt, TileMoves* s_mv,
+                                               uint32_t moved) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) moved += __shfl_xor(moved, off, 64);
+  if ((threadIdx.x & 63) == 0 && moved) atomicAdd(&s_mv->moved, moved);
   __syncthreads();
-  const int64_t j = j0 + threadIdx.x;
-  if (j >= j1 || spos[j + 1] == spos[j]) return;  // past the end, or a mover
-  const uint32_t K = skeys_old[j];
-  const int64_t ins = in_lds ? a0 + lower_bound_pair(s_k, s_j, 0, cnt, K, uint32_t(j))
-                             : lower_bound_pair(mks, mjs, a0, a0 + cnt, K, uint32_t(j));
-  const int64_t pos = int64_t(spos[j]) + ins;
-  skeys_new[pos] = K;
-  perm_new[pos] = perm_old[j];
-}
-
-__global__ void k_tile_runs(const uint32_t* __restrict__ skeys, int64_t n, uint32_t ntiles,
-                            uint32_t* __restrict__ tile_start, uint32_t* __restrict__ tile_end,
-                            uint32_t* __restrict__ counters) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t k = skeys[i] >> 6;  // tile
-  const bool first = i == 0 || (skeys[i - 1] >> 6) != k;
-  const bool last = i == n - 1 || (skeys[i + 1] >> 6) != k;
-  if (k < ntiles) {
-    if (first) tile_start[k] = uint32_t(i);
-    if (last) tile_end[k] = uint32_t(i + 1);
-    if (i == n - 1) counters[CNT_INSIDE] = uint32_t(n);
-  } else if (first) {
-    counters[CNT_INSIDE] = uint32_t(i);
+  if (threadIdx.x == 0) {
+    mo.stay[tile] = uint32_t(cnt) - s_mv->leave;
+    if (s_mv->moved) atomicAdd(lane_of(mo.lanes, LANE_MOVED), s_mv->moved);
   }
 }
 
-__global__ void k_tile_flags(const uint32_t* __restrict__ tile_start, const uint32_t* __restrict__ tile_end,
-                             uint32_t ntiles, uint32_t* __restrict__ flag, uint32_t* __restrict__ slot) {
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= ntiles) return;
-  const uint32_t f = tile_end[t] > tile_start[t] ? 1u : 0u;
-  flag[t] = f;
-  slot[t] = f;
-}
-
-__global__ void k_compact(const uint32_t* __restrict__ flag, const uint32_t* __restrict__ slot, uint32_t count,
-                          uint32_t* __restrict__ list) {
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= count) return;
-  if (flag[t]) list[slot[t]] = uint32_t(t);
-}
-
-// Node block B holds nodes BW*B .. BW*B+BW-1 per axis; tile t's footprint
-// [BW*t-1, BW*t+BW+1] touches node blocks t-1, t, t+1.
-template <int D>
-__global__ void k_nb_mark(const uint32_t* __restrict__ tile_flag, uint32_t ntiles, int3 nt,
-                          uint32_t* __restrict__ nb_flag) {
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= ntiles || !tile_flag[t]) return;
-  const int dims[3] = {nt.x, nt.y, nt.z};
-  int I[3] = {0, 0, 0};
-  int64_t r = t;
-  for (int d = 0; d < D; ++d) {
-    I[d] = int(r % dims[d]);
-    r /= dims[d];
+// Next keys from the positions: one workgroup per active tile of the previous
+// binning (whose keys may belong to other positions, or another particle set
+// of the same size).
+template <typename T, int D, int BASIS, bool STORED>
+__global__ __launch_bounds__(256) void k_rekey(Args<T, D> a, const uint32_t* __restrict__ skeys, uint32_t ntiles,
+                                               MoveOut mo, uint32_t* __restrict__ counters) {
+  __shared__ TileMoves s_mv;
+  const int64_t j = xcd_remap(blockIdx.x, a.n_active);
+  if (j >= a.n_active) return;
+  const uint32_t tile = a.active[j];
+  const uint32_t start = a.tile_start[tile];
+  const int cnt = int(a.tile_end[tile] - start);
+  if (threadIdx.x == 0) s_mv = TileMoves{0u, 0u};
+  __syncthreads();
+  uint32_t moved = 0;
+  for (int i = int(threadIdx.x); i < cnt; i += 256) {
+    const uint32_t jj = start + uint32_t(i);
+    const uint32_t key = particle_key<T, D, BASIS, STORED>(a, a.perm[jj], ntiles, counters + CNT_ERR);
+    next_key(mo, key, skeys[jj], jj, tile, start, &s_mv, moved);
   }
-  for (int dz = (D == 3 ? -1 : 0); dz <= (D == 3 ? 1 : 0); ++dz)
-    for (int dy = -1; dy <= 1; ++dy)
-      for (int dx = -1; dx <= 1; ++dx) {
-        const int J[3] = {I[0] + dx, I[1] + dy, I[2] + dz};
-        bool ok = true;
-        for (int d = 0; d < D; ++d) ok = ok && J[d] >= 0 && J[d] < dims[d];
-        if (!ok) continue;
-        int64_t l = J[D - 1];
-        for (int d = D - 2; d >= 0; --d) l = l * dims[d] + J[d];
-        nb_flag[l] = 1u;
-      }
+  tile_moves_end(mo, tile, cnt, &s_mv, moved);
 }
 
-// The same for a batch: neighbours are taken in the tile's own scene.
-template <typename T, int D>
-__global__ void k_nb_mark_batch(Args<T, D> a, const uint32_t* __restrict__ tile_flag, uint32_t ntiles,
-                                uint32_t* __restrict__ nb_flag) {
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= ntiles || !tile_flag[t]) return;
-  uint32_t poff;
-  const uint32_t lt = bind_tile<true>(a, uint32_t(t), poff);
-  const uint32_t toff = uint32_t(t) - lt;
-  int I[3] = {0, 0, 0};
-  int64_t r = lt;
-  for (int d = 0; d < D; ++d) {
-    I[d] = int(r % a.ntiles[d]);
-    r /= a.ntiles[d];
+// The same for the particles that were outside the mesh; one that came back is
+// reported (the caller then sorts every key again).
+template <typename T, int D, int BASIS, bool STORED>
+__global__ __launch_bounds__(256) void k_rekey_outside(Args<T, D> a, uint32_t ntiles, MoveOut mo,
+                                                       uint32_t* __restrict__ counters) {
+  const int64_t jj = a.n_inside + int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (jj >= a.n) return;
+  const uint32_t key = particle_key<T, D, BASIS, STORED>(a, a.perm[jj], ntiles, counters + CNT_ERR);
+  mo.nk[jj] = key;
+  if ((key >> 6) != ntiles) {
+    atomicAdd(&mo.tin[key >> 6], 1u);
+    atomicSub(&mo.stay[ntiles], 1u);
+    atomicAdd(lane_of(mo.lanes, LANE_MOVED), 1u);
+    atomicOr(counters + CNT_REENTER, 1u);
   }
-  for (int dz = (D == 3 ? -1 : 0); dz <= (D == 3 ? 1 : 0); ++dz)
-    for (int dy = -1; dy <= 1; ++dy)
-      for (int dx = -1; dx <= 1; ++dx) {
-        const int J[3] = {I[0] + dx, I[1] + dy, I[2] + dz};
-        bool ok = true;
-        for (int d = 0; d < D; ++d) ok = ok && J[d] >= 0 && J[d] < a.ntiles[d];
-        if (!ok) continue;
-        int64_t l = J[D - 1];
-        for (int d = D - 2; d >= 0; --d) l = l * a.ntiles[d] + J[d];
-        nb_flag[toff + l] = 1u;
-      }
-}
-
-__global__ void k_copy_u32(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, int64_t n) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[i];
 }
 
 template <typename T, int D>
@@ -855,7 +695,7 @@ __global__ __launch_bounds__(64) void k_p2g_tile(Args<T, D> a, const uint32_t* _
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) bad += __shfl_xor(bad, off, 64);
-    if (lane == 0) misplaced[j] = bad;  // per tile, summed later
+    if (lane == 0 && bad) atomicAdd(lane_of(misplaced, LANE_BROKEN), bad);
   }
   const T mp = a.mp, hinv = a.mesh.h_inv;
   for (int pass = 0; pass < NPASS; ++pass) {
@@ -1569,7 +1409,7 @@ __device__ __forceinline__ void k_p2g_fast_body(Args<T, D>& a, const uint32_t* _
   if (misplaced && wave == 0) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) bad += __shfl_xor(bad, off, 64);
-    if (lane == 0) misplaced[j] = bad;  // per tile, summed later
+    if (lane == 0 && bad) atomicAdd(lane_of(misplaced, LANE_BROKEN), bad);
   }
   if constexpr (SHJ)
     p2g_write_partial_slabs<T, D, SW, KN, NPASS, NT>(a, j, s_sums);
@@ -1696,15 +1536,15 @@ __device__ __forceinline__ void g2p_stage_store(const Args<T, D>& a, const int* 
 // One particle's G2P and update (README.md:81-86) from the tile's staged
 // footprint (s_n: v and v - vⁿ per component; s_nodex: node coordinates): its
 // axis jets at its class window, the axis-factored sums of Δv, ∇v and the x
-// rate, the writes of v, ∇v, x, F, σ, V and, with nk, of the next sort key and
-// the stayer flag at its sorted slot jj.  emit(val, der, v, σ, V) receives the
+// rate, the writes of v, ∇v, x, F, σ, V and, with mo.nk, of the next sort key
+// at its sorted slot jj (next_key).  emit(val, der, v, σ, V) receives the
 // jets and the updated state.
 template <typename T, int D, int BASIS, bool AOS, bool SEP, typename Emit>
 __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T, D, AOS>& cur,
                                              const T (*s_n)[Geo<D>::PSZ], const T (*s_nodex)[Geo<D>::TS],
                                              const uint32_t jj, const uint32_t tile, const uint32_t ltile,
-                                             uint32_t* __restrict__ nk, uint32_t* __restrict__ stay,
-                                             const uint32_t ntiles, uint32_t* __restrict__ movers, Emit&& emit) {
+                                             const uint32_t start, const MoveOut& mo, TileMoves* s_mv,
+                                             uint32_t& moved, const uint32_t ntiles, Emit&& emit) {
   using G = Geo<D>;
   constexpr int SW = support_width(BASIS);
   const T hinv = a.mesh.h_inv, dt = a.dt;
@@ -1819,20 +1659,13 @@ __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T,
 #pragma unroll
     for (int c = 0; c < D; ++c) a.x_keep[int64_t(pid) * D + c] = cur.x[c];
   }
-  if (nk) {
+  if (mo.nk) {
     uint32_t nl = 1;  // the scene's tiles; in a batch its keys start at its first global tile
 #pragma unroll
     for (int d = 0; d < D; ++d) nl *= uint32_t(a.ntiles[d]);
     const uint32_t kl = key_of_position<T, D, BASIS>(a, xn, cur.l, nl);
     const uint32_t key = kl == nl * 64u ? ntiles * 64u : kl + (tile - ltile) * 64u;
-    nk[jj] = key;
-    const bool moved = key != cur.key;
-    stay[jj] = moved ? 0u : 1u;
-    // particles whose key changed, counted per wave by its lowest live lane
-    // (no atomic in the common case of none)
-    const uint64_t mv = __ballot(moved);
-    if (mv && (__ballot(true) & lanemask_lt64()) == 0)
-      atomicAdd(movers + (blockIdx.x % MOVER_LANES) * MOVER_STRIDE, uint32_t(__popcll(mv)));
+    next_key(mo, key, cur.key, jj, tile, start, s_mv, moved);
   }
   T Fn[D * D];
 #pragma unroll
@@ -1854,9 +1687,9 @@ __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T,
   emit(val, der, vn, sg, Vn);
 }
 
-// With nk != nullptr the kernel also writes, at each particle's sorted position
-// j, the sort key of its new position (nk[j]) and whether it equals the
-// current one (stay[j]): the next step's incremental binning starts from them.
+// With mo.nk != nullptr the kernel also writes, at each particle's sorted
+// position, the sort key of its new position, and per tile what the next
+// step's binning starts from (MoveOut).
 // waves per SIMD the Float32 G2P is compiled for (VGPR budget 512 / n), and
 // waves per tile of the single-scene G2P
 #ifndef TESS_G2P_WAVES_PER_SIMD
@@ -1867,8 +1700,7 @@ __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T,
 #endif
 template <typename T, int D, int BASIS, bool AOS, int NW, bool BATCH, bool SEP>
 __device__ __forceinline__ void k_g2p_fast_body(Args<T, D>& a, const uint32_t* __restrict__ skeys,
-                                                       uint32_t* __restrict__ nk, uint32_t* __restrict__ stay,
-                                                       uint32_t ntiles, uint32_t* __restrict__ movers, const int64_t j) {
+                                                       const MoveOut mo, uint32_t ntiles, const int64_t j) {
   using G = Geo<D>;
   constexpr int SW = support_width(BASIS);
   const int lane = threadIdx.x & 63;
@@ -1887,6 +1719,9 @@ __device__ __forceinline__ void k_g2p_fast_body(Args<T, D>& a, const uint32_t* _
   __shared__ T s_n[2 * D][G::PSZ];
   __shared__ T s_nodex[D][G::TS];
   __shared__ uint32_t s_cnt[64];
+  __shared__ TileMoves s_mv;
+  uint32_t moved = 0;
+  if (threadIdx.x == 0) s_mv = TileMoves{0u, 0u};  // before the barriers below
   G2PStage<T, D, 64 * NW> stage;
   g2p_stage_load<T, D, 64 * NW>(a, origin, stage);
   int ccount, coff, maxcnt;
@@ -1945,8 +1780,8 @@ __device__ __forceinline__ void k_g2p_fast_body(Args<T, D>& a, const uint32_t* _
     q_after = ahead(k + 2 * NW, staged);
     fetch(k + NW, q_next, nxt);
     if (!act) return;
-    g2p_particle<T, D, BASIS, AOS, SEP>(a, cur, s_n, s_nodex, nk ? slot(k) : 0u, tile, ltile, nk, stay, ntiles,
-                                        movers, [](const auto&...) {});
+    g2p_particle<T, D, BASIS, AOS, SEP>(a, cur, s_n, s_nodex, mo.nk ? slot(k) : 0u, tile, ltile, start, mo, &s_mv,
+                                        moved, ntiles, [](const auto&...) {});
   };
   auto walk = [&](auto staged) {
     Ahead qa = ahead(wave + NW, staged), qb{0u, 0u};
@@ -1960,14 +1795,14 @@ __device__ __forceinline__ void k_g2p_fast_body(Args<T, D>& a, const uint32_t* _
     walk(std::true_type{});
   else
     walk(std::false_type{});
+  if (mo.nk) tile_moves_end(mo, tile, cnt, &s_mv, moved);
 }
 
 template <typename T, int D, int BASIS, bool AOS, int NW, bool BATCH = false, bool SEP = false>
 __global__ __launch_bounds__(64 * NW, sizeof(T) == 4 ? TESS_G2P_WAVES_PER_SIMD : 1) void k_g2p_fast(Args<T, D> a, const uint32_t* __restrict__ skeys,
-                                                       uint32_t* __restrict__ nk, uint32_t* __restrict__ stay,
-                                                       uint32_t ntiles, uint32_t* __restrict__ movers) {
+                                                       const MoveOut mo, uint32_t ntiles) {
   const int64_t j = item_of<BATCH>(blockIdx.x, a.n_active);
-  if (j < a.n_active) k_g2p_fast_body<T, D, BASIS, AOS, NW, BATCH, SEP>(a, skeys, nk, stay, ntiles, movers, j);
+  if (j < a.n_active) k_g2p_fast_body<T, D, BASIS, AOS, NW, BATCH, SEP>(a, skeys, mo, ntiles, j);
 }
 
 // Forms whose item count is read on the device at `count` (launch sizes fixed
@@ -1977,21 +1812,19 @@ __global__ __launch_bounds__(64 * NW, sizeof(T) == 4 ? TESS_G2P_WAVES_PER_SIMD :
 // them, as xcd_remap does for one workgroup per item).
 template <typename T, int D, int BASIS, bool AOS, int NW, bool BATCH = false, bool SEP = false>
 __global__ __launch_bounds__(64 * NW, sizeof(T) == 4 ? TESS_G2P_WAVES_PER_SIMD : 1) void k_g2p_fast_grid(Args<T, D> a, const uint32_t* __restrict__ skeys,
-                                                       uint32_t* __restrict__ nk, uint32_t* __restrict__ stay,
-                                                       uint32_t ntiles, uint32_t* __restrict__ movers, const uint32_t* __restrict__ count) {
+                                                       const MoveOut mo, uint32_t ntiles, const uint32_t* __restrict__ count) {
   const int64_t N = int64_t(*count), R = ((N + 7) >> 3) << 3;
   // xcd_remap is a bijection of [0, R) only: workgroups past R end here
   const int64_t j = item_of<BATCH>(blockIdx.x, N);
-  if (int64_t(blockIdx.x) < R && j < N) k_g2p_fast_body<T, D, BASIS, AOS, NW, BATCH, SEP>(a, skeys, nk, stay, ntiles, movers, j);
+  if (int64_t(blockIdx.x) < R && j < N) k_g2p_fast_body<T, D, BASIS, AOS, NW, BATCH, SEP>(a, skeys, mo, ntiles, j);
 }
 template <typename T, int D, int BASIS, bool AOS, int NW, bool BATCH = false, bool SEP = false>
 __global__ __launch_bounds__(64 * NW, sizeof(T) == 4 ? TESS_G2P_WAVES_PER_SIMD : 1) void k_g2p_fast_persist(Args<T, D> a, const uint32_t* __restrict__ skeys,
-                                                       uint32_t* __restrict__ nk, uint32_t* __restrict__ stay,
-                                                       uint32_t ntiles, uint32_t* __restrict__ movers, const uint32_t* __restrict__ count) {
+                                                       const MoveOut mo, uint32_t ntiles, const uint32_t* __restrict__ count) {
   const int64_t N = int64_t(*count), R = ((N + 7) >> 3) << 3;
   for (int64_t it = blockIdx.x; it < R; it += gridDim.x) {
     const int64_t j = item_of<BATCH>(it, N);
-    if (j < N) k_g2p_fast_body<T, D, BASIS, AOS, NW, BATCH, SEP>(a, skeys, nk, stay, ntiles, movers, j);
+    if (j < N) k_g2p_fast_body<T, D, BASIS, AOS, NW, BATCH, SEP>(a, skeys, mo, ntiles, j);
     __syncthreads();  // the next item reuses the workgroup's LDS
   }
 }
@@ -2053,8 +1886,7 @@ struct G2P2GShape {
 
 template <typename T, int D, int BASIS, bool AOS, int NP, int NC>
 __device__ __forceinline__ void k_g2p2g_fast_body(Args<T, D>& a, const uint32_t* __restrict__ skeys,
-                                                  uint32_t* __restrict__ nk, uint32_t* __restrict__ stay,
-                                                  uint32_t ntiles, uint32_t* __restrict__ movers,
+                                                  const MoveOut mo, uint32_t ntiles,
                                                   uint32_t* __restrict__ misplaced, const int64_t j) {
   using G = Geo<D>;
   using SH = G2P2GShape<T, D, BASIS>;
@@ -2077,6 +1909,9 @@ __device__ __forceinline__ void k_g2p2g_fast_body(Args<T, D>& a, const uint32_t*
   __shared__ T s_nodex[D][G::TS];
   __shared__ uint32_t s_cnt[64];
   __shared__ uint32_t s_pid[PID_CAP], s_key[PID_CAP];
+  __shared__ TileMoves s_mv;
+  uint32_t moved = 0;
+  if (threadIdx.x == 0) s_mv = TileMoves{0u, 0u};  // before the barriers below
   // [round parity][producer][row][class lane]; after the last round the
   // tile's node sums take its place: the consumers' slabs (several consumers)
   // or one array per component over the footprint (one)
@@ -2135,7 +1970,7 @@ __device__ __forceinline__ void k_g2p2g_fast_body(Args<T, D>& a, const uint32_t*
         T(*xr)[64] = s_x[r & 1][wave];
         if (k < ccount) {
           g2p_particle<T, D, BASIS, AOS, false>(
-              a, cur, s_n, s_nodex, start + uint32_t(coff + k), tile, ltile, nk, stay, ntiles, movers,
+              a, cur, s_n, s_nodex, start + uint32_t(coff + k), tile, ltile, start, mo, &s_mv, moved, ntiles,
               [&](const auto&, const auto&, const auto& vn, const auto& sg, const T Vn) {
 #pragma unroll
                 for (int d = 0; d < D; ++d) xr[d][lane] = cur.x[d];
@@ -2261,25 +2096,26 @@ __device__ __forceinline__ void k_g2p2g_fast_body(Args<T, D>& a, const uint32_t*
     if (misplaced && pass == 0) {
 #pragma unroll
       for (int off = 32; off >= 1; off >>= 1) bad += __shfl_xor(bad, off, 64);
-      if (lane == 0) misplaced[j] = bad;  // per tile, summed later
+      if (lane == 0 && bad) atomicAdd(lane_of(misplaced, LANE_BROKEN), bad);
     }
   }
   if constexpr (NC > 1)
     p2g_write_partial_slabs<T, D, SW, KN, NC, NT>(a, j, s_xraw);
   else
     p2g_write_partial<T, D, SW, NT>(a, j, s_tile);
+  if (mo.nk) tile_moves_end(mo, tile, cnt, &s_mv, moved);
 }
 
 template <typename T, int D, int BASIS, bool AOS, int NP, int NC>
 __global__ __launch_bounds__(64 * (NP + NC), (G2P2GShape<T, D, BASIS>::wps(NP))) void k_g2p2g_fast(
-    Args<T, D> a, const uint32_t* __restrict__ skeys, uint32_t* __restrict__ nk, uint32_t* __restrict__ stay,
-    uint32_t ntiles, uint32_t* __restrict__ movers, uint32_t* __restrict__ misplaced) {
+    Args<T, D> a, const uint32_t* __restrict__ skeys, const MoveOut mo, uint32_t ntiles,
+    uint32_t* __restrict__ misplaced) {
   const int64_t j = item_of<false>(blockIdx.x, a.n_active);
-  if (j < a.n_active) k_g2p2g_fast_body<T, D, BASIS, AOS, NP, NC>(a, skeys, nk, stay, ntiles, movers, misplaced, j);
+  if (j < a.n_active) k_g2p2g_fast_body<T, D, BASIS, AOS, NP, NC>(a, skeys, mo, ntiles, misplaced, j);
 }
 
 template <typename T, int D, int SW, bool GAOS, bool BATCH>
-__device__ __forceinline__ void k_gather_grid_body(Args<T, D>& a, uint32_t* __restrict__ nodes_per_block, const int64_t j) {
+__device__ __forceinline__ void k_gather_grid_body(Args<T, D>& a, uint32_t* __restrict__ lanes, const int64_t j) {
   using G = Geo<D>;
   using PT = Part<D, SW>;
   constexpr int NV = 1 + 2 * D;
@@ -2362,10 +2198,10 @@ __device__ __forceinline__ void k_gather_grid_body(Args<T, D>& a, uint32_t* __re
   const double md = double(acc[0]);
   const bool has = md > 0.0;
   {
-    // nodes with m > 0 in this block (one plain store per block, summed later)
+    // nodes with m > 0 in this block
     const uint64_t m = __ballot(has);
-    if ((threadIdx.x & 63) == __ffsll((unsigned long long)__ballot(true)) - 1)
-      nodes_per_block[j] = uint32_t(__popcll(m));
+    if (m && (threadIdx.x & 63) == __ffsll((unsigned long long)__ballot(true)) - 1)
+      atomicAdd(lane_of(lanes, LANE_NODES), uint32_t(__popcll(m)));
   }
   const double minv = has ? 1.0 / md : 0.0;
   if (i < 0) return;  // SpGrid node of an inactive block: no storage (and no support, checked by P2G)
@@ -2395,9 +2231,9 @@ __device__ __forceinline__ void k_gather_grid_body(Args<T, D>& a, uint32_t* __re
 }
 
 template <typename T, int D, int SW, bool GAOS, bool BATCH = false>
-__global__ __launch_bounds__(64) void k_gather_grid(Args<T, D> a, uint32_t* __restrict__ nodes_per_block) {
+__global__ __launch_bounds__(64) void k_gather_grid(Args<T, D> a, uint32_t* __restrict__ lanes) {
   const int64_t j = item_of<BATCH>(blockIdx.x, a.n_nb);
-  if (j < a.n_nb) k_gather_grid_body<T, D, SW, GAOS, BATCH>(a, nodes_per_block, j);
+  if (j < a.n_nb) k_gather_grid_body<T, D, SW, GAOS, BATCH>(a, lanes, j);
 }
 
 // Forms whose item count is read on the device at `count` (launch sizes fixed
@@ -2406,18 +2242,18 @@ __global__ __launch_bounds__(64) void k_gather_grid(Args<T, D> a, uint32_t* __re
 // (_persist; a multiple of 8 workgroups keeps each XCD on a contiguous run of
 // them, as xcd_remap does for one workgroup per item).
 template <typename T, int D, int SW, bool GAOS, bool BATCH = false>
-__global__ __launch_bounds__(64) void k_gather_grid_grid(Args<T, D> a, uint32_t* __restrict__ nodes_per_block, const uint32_t* __restrict__ count) {
+__global__ __launch_bounds__(64) void k_gather_grid_grid(Args<T, D> a, uint32_t* __restrict__ lanes, const uint32_t* __restrict__ count) {
   const int64_t N = int64_t(*count), R = ((N + 7) >> 3) << 3;
   // xcd_remap is a bijection of [0, R) only: workgroups past R end here
   const int64_t j = item_of<BATCH>(blockIdx.x, N);
-  if (int64_t(blockIdx.x) < R && j < N) k_gather_grid_body<T, D, SW, GAOS, BATCH>(a, nodes_per_block, j);
+  if (int64_t(blockIdx.x) < R && j < N) k_gather_grid_body<T, D, SW, GAOS, BATCH>(a, lanes, j);
 }
 template <typename T, int D, int SW, bool GAOS, bool BATCH = false>
-__global__ __launch_bounds__(64) void k_gather_grid_persist(Args<T, D> a, uint32_t* __restrict__ nodes_per_block, const uint32_t* __restrict__ count) {
+__global__ __launch_bounds__(64) void k_gather_grid_persist(Args<T, D> a, uint32_t* __restrict__ lanes, const uint32_t* __restrict__ count) {
   const int64_t N = int64_t(*count), R = ((N + 7) >> 3) << 3;
   for (int64_t it = blockIdx.x; it < R; it += gridDim.x) {
     const int64_t j = item_of<BATCH>(it, N);
-    if (j < N) k_gather_grid_body<T, D, SW, GAOS, BATCH>(a, nodes_per_block, j);
+    if (j < N) k_gather_grid_body<T, D, SW, GAOS, BATCH>(a, lanes, j);
     __syncthreads();  // the next item reuses the workgroup's LDS
   }
 }
@@ -2601,15 +2437,12 @@ __global__ __launch_bounds__(64) void k_g2p_tile(Args<T, D> a, const uint32_t* _
 // the particle equations run (g2p.jl:123-153).
 template <typename T, int D, bool BATCH = false>
 __global__ __launch_bounds__(256) void k_g2p_outside(Args<T, D> a, const uint32_t* __restrict__ skeys,
-                                                     uint32_t* __restrict__ nk, uint32_t* __restrict__ stay) {
+                                                     uint32_t* __restrict__ nk) {
   const int64_t j = a.n_inside + int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (j >= a.n) return;
   uint32_t pid = a.perm[j];
   if constexpr (BATCH) pid -= uint32_t(bind_scene(a, scene_of(a.scene_poff, a.nscenes, pid)).poff);
-  if (nk) {  // the position does not change: the key stays
-    nk[j] = skeys[j];
-    stay[j] = 1u;
-  }
+  if (nk) nk[j] = skeys[j];  // the position does not change: the key stays
   T dv[D], L[D * D], dx[D];
 #pragma unroll
   for (int c = 0; c < D; ++c) {
@@ -2716,39 +2549,94 @@ int key_bits_for(uint64_t maxkey) {
   return b;
 }
 
-// Incremental re-binning with M > 0 movers: nk[j] is the new key of the
-// particle at sorted position j, spos[j] its stayer rank (exclusive scan of the
-// stayer flags, spos[n] = stayers).  Few movers are sorted among themselves
-// and merged into the stayers' previous order; many are sorted with the
-// stayers.  The merged order replaces (keys_sorted, vals).
-inline void merge_movers(tess_ctx* ctx, const uint32_t* nk, const uint32_t* spos, int64_t n, int64_t M, int kbits) {
-  uint32_t* skeys = static_cast<uint32_t*>(ctx->keys_sorted.ptr);
-  uint32_t* perm = static_cast<uint32_t*>(ctx->vals.ptr);
-  uint32_t* skeys2 = ctx->skeys2.as<uint32_t>(size_t(n));
-  uint32_t* perm2 = ctx->perm2.as<uint32_t>(size_t(n));
-  if (M <= n / 8) {
-    uint32_t* mkey = ctx->inc_mkey.as<uint32_t>(size_t(M));
-    uint32_t* mj = ctx->inc_mj.as<uint32_t>(size_t(M));
-    uint32_t* mks = ctx->inc_mks.as<uint32_t>(size_t(M));
-    uint32_t* mr = ctx->inc_mr.as<uint32_t>(size_t(M));
-    uint32_t* mjs = ctx->inc_mjs.as<uint32_t>(size_t(M));
-    hipLaunchKernelGGL(k_compact_movers, dim3(blocks_for(n, 256)), dim3(256), 0, ctx->stream, nk, spos, n, mkey, mj);
-    TESS_HIP(hipGetLastError());
-    radix_sort_pairs(ctx, mkey, nullptr, mks, mr, M, kbits);
-    hipLaunchKernelGGL(k_place_movers, dim3(blocks_for(M, 256)), dim3(256), 0, ctx->stream, mks, mr, mj, skeys, perm,
-                       spos, n, M, mjs, skeys2, perm2, static_cast<const uint32_t*>(nullptr));
-    TESS_HIP(hipGetLastError());
-    const int64_t nsb = blocks_for(n, STAY_BLOCK);
-    int64_t* ranges = ctx->inc_rng.as<int64_t>(size_t(2 * nsb));
-    hipLaunchKernelGGL(k_stay_ranges, dim3(blocks_for(nsb, 256)), dim3(256), 0, ctx->stream, skeys, n, mks, mjs, M,
-                       nsb, ranges, static_cast<const uint32_t*>(nullptr));
-    TESS_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_place_stayers, dim3(unsigned(nsb)), dim3(STAY_BLOCK), 0, ctx->stream, skeys, perm, spos, n,
-                       mks, mjs, ranges, skeys2, perm2);
-    TESS_HIP(hipGetLastError());
-  } else {
-    radix_sort_pairs(ctx, nk, perm, skeys2, perm2, n, kbits);
-  }
+// The re-binning's buffers for n particles and the context's current tables.
+inline MoveOut move_out(tess_ctx* ctx, int64_t n, int64_t ntiles) {
+  const size_t m = size_t(std::max<int64_t>(n, 1));
+  MoveOut mo;
+  mo.nk = ctx->inc_nk.as<uint32_t>(m);
+  mo.stay = ctx->tile_stay.as<uint32_t>(size_t(ntiles) + 1);
+  mo.tin = ctx->tile_tin.as<uint32_t>(size_t(ntiles) + 1);
+  mo.out = ctx->inc_out.as<uint2>(m);
+  mo.lanes = lane_counters(ctx);
+  return mo;
+}
+inline MoveOut no_moves() { return MoveOut{nullptr, nullptr, nullptr, nullptr, nullptr}; }
+
+// Arguments that build the tables of ntiles tiles into the alternate set.
+inline TabArgs table_args(tess_ctx* ctx, int64_t ntiles) {
+  TabArgs t;
+  std::memset(static_cast<void*>(&t), 0, sizeof(t));
+  const size_t nt = size_t(ntiles) + 1;
+  t.stay = ctx->tile_stay.as<uint32_t>(nt);
+  t.tin = ctx->tile_tin.as<uint32_t>(nt);
+  t.ntiles = ntiles;
+  t.sums = ctx->tab_sums.as<uint32_t>(size_t(tab_blocks(ntiles)) * 4);
+  t.start = ctx->alt_start.as<uint32_t>(nt);
+  t.end = ctx->alt_end.as<uint32_t>(nt);
+  t.flag = ctx->alt_flag.as<uint32_t>(nt);
+  t.slot = ctx->alt_slot.as<uint32_t>(nt);
+  t.active = ctx->alt_active.as<uint32_t>(nt);
+  t.nb_flag = ctx->alt_nb_flag.as<uint32_t>(nt);
+  t.nb_list = ctx->alt_nb_list.as<uint32_t>(nt);
+  t.seg = ctx->tile_seg.as<uint32_t>(nt);
+  t.lanes = lane_counters(ctx);
+  t.counters = ctx->counters.as<uint32_t>(64);
+  t.host = reinterpret_cast<uint32_t*>(ctx->counters_host);
+  return t;
+}
+
+// The alternate tables become the current ones.
+inline void swap_tables(tess_ctx* ctx) {
+  std::swap(ctx->tile_start, ctx->alt_start);
+  std::swap(ctx->tile_end, ctx->alt_end);
+  std::swap(ctx->tile_flag, ctx->alt_flag);
+  std::swap(ctx->tile_slot, ctx->alt_slot);
+  std::swap(ctx->active_tiles, ctx->alt_active);
+  std::swap(ctx->nb_flag, ctx->alt_nb_flag);
+  std::swap(ctx->nb_list, ctx->alt_nb_list);
+}
+
+// What a report of the lanes says about the last P2G, once.
+inline void take_report(tess_ctx* ctx) {
+  const uint32_t* hc = reinterpret_cast<const uint32_t*>(ctx->counters_host);
+  if (ctx->broken_pending) ctx->broken_count = int64_t(hc[CNT_MISPLACED]);
+  if (ctx->nodes_pending) ctx->last_active_nodes = int64_t(hc[CNT_NODES]);
+  ctx->broken_pending = false;
+  ctx->nodes_pending = false;
+}
+
+// The merge of the particles whose key changed (counts in the report, tables
+// built in the alternate set): (keys_sorted, vals) and the tables become the
+// new ones.
+inline void merge_moves(tess_ctx* ctx, int64_t n, int64_t ntiles, int64_t old_active, int64_t old_inside) {
+  const uint32_t* hc = reinterpret_cast<const uint32_t*>(ctx->counters_host);
+  const size_t m = size_t(std::max<int64_t>(n, 1));
+  MergeArgs g;
+  std::memset(static_cast<void*>(&g), 0, sizeof(g));
+  g.n = n;
+  g.ntiles = ntiles;
+  g.old_active = static_cast<const uint32_t*>(ctx->active_tiles.ptr);
+  g.old_start = static_cast<const uint32_t*>(ctx->tile_start.ptr);
+  g.old_end = static_cast<const uint32_t*>(ctx->tile_end.ptr);
+  g.new_active = static_cast<const uint32_t*>(ctx->alt_active.ptr);
+  g.new_start = static_cast<const uint32_t*>(ctx->alt_start.ptr);
+  g.new_end = static_cast<const uint32_t*>(ctx->alt_end.ptr);
+  g.old_active_n = old_active;
+  g.new_active_n = int64_t(hc[CNT_ACTIVE]);
+  g.stay = static_cast<const uint32_t*>(ctx->tile_stay.ptr);
+  g.nk = static_cast<const uint32_t*>(ctx->inc_nk.ptr);
+  g.perm_old = static_cast<const uint32_t*>(ctx->vals.ptr);
+  g.seg_off = static_cast<const uint32_t*>(ctx->tile_seg.ptr);
+  g.out = static_cast<const uint2*>(ctx->inc_out.ptr);
+  g.seg = ctx->inc_seg.as<uint2>(m);
+  g.seg_alt = ctx->inc_seg2.as<uint2>(m);
+  g.keys_new = ctx->skeys2.as<uint32_t>(m);
+  g.perm_new = ctx->perm2.as<uint32_t>(m);
+  g.out_in = hc[CNT_OUTIN];
+  g.pos_bits = key_bits_for(uint64_t(m));
+  const int64_t outside = n - int64_t(hc[CNT_INSIDE]);
+  launch_merge(ctx->stream, g, hc[CNT_ARRIVE] != 0,
+               outside > 0 ? unsigned(std::min<int64_t>(blocks_for(n - old_inside, 256), 2048)) : 0u);
   std::swap(ctx->keys_sorted, ctx->skeys2);
   std::swap(ctx->vals, ctx->perm2);
 }
@@ -2832,125 +2720,86 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
     raise(TESS_ERR_ARGUMENT, "mesh or particle count exceeds the 32-bit binning range");
   Binning& b = ctx->bin;
   b.valid = false;
-  uint32_t* counters = ctx->counters.as<uint32_t>(CNT_SLOTS);
-  uint32_t* keys = ctx->keys.as<uint32_t>(size_t(std::max<int64_t>(n, 1)));
-  uint32_t* skeys = ctx->keys_sorted.as<uint32_t>(size_t(std::max<int64_t>(n, 1)));
-  uint32_t* perm = ctx->vals.as<uint32_t>(size_t(std::max<int64_t>(n, 1)));
-  uint32_t* tstart = ctx->tile_start.as<uint32_t>(ntiles);
-  uint32_t* tend = ctx->tile_end.as<uint32_t>(ntiles);
-  uint32_t* tflag = ctx->tile_flag.as<uint32_t>(ntiles);
-  uint32_t* tslot = ctx->tile_slot.as<uint32_t>(ntiles);
-  uint32_t* active = ctx->active_tiles.as<uint32_t>(ntiles);
-  uint32_t* nbflag = ctx->nb_flag.as<uint32_t>(ntiles);
-  uint32_t* nbslot = ctx->nb_slot.as<uint32_t>(ntiles);
-  uint32_t* nblist = ctx->nb_list.as<uint32_t>(ntiles);
+  const size_t m = size_t(std::max<int64_t>(n, 1));
+  uint32_t* counters = ctx->counters.as<uint32_t>(64);
   const int tok = prof_begin(ctx, "binning", 0.0);
   const int kbits = key_bits_for(ntiles * 64);
   const bool incremental = b.state_valid && b.state_n == n && b.state_ntiles == int64_t(ntiles) &&
                            b.state_dim == D && n > 0;
-  const bool precomputed = keys_from_g2p && b.keys_ready;
+  const bool precomputed = keys_from_g2p && b.keys_ready && b.x_ptr == P.x.ptr && b.tile_log2 == Geo<D>::LT &&
+                           b.basis == BASIS && b.dtype == mesh.dtype;
   b.keys_ready = false;
-  if (n > 0 && incremental && precomputed && b.x_ptr == P.x.ptr && b.tile_log2 == Geo<D>::LT &&
-      b.basis == BASIS && b.dtype == mesh.dtype) {
-    // The previous G2P counted the particles whose key changed.  With none,
-    // the sorted keys, the order and every tile and node-block list of the
-    // previous binning are what binning again would produce: keep them.
-    uint32_t* hc = reinterpret_cast<uint32_t*>(ctx->counters_host);
-    TESS_HIP(hipMemcpyAsync(hc, counters, CNT_SLOTS * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
-    movers_readback(ctx);
-    TESS_HIP(hipStreamSynchronize(ctx->stream));
-    if (movers_total(ctx) == 0) {
-      ctx->last_movers = 0;
-      ctx->last_active_nodes = int64_t(hc[CNT_NODES]);
-      ctx->last_misplaced = (ctx->misplaced_x_ptr == P.x.ptr && ctx->misplaced_n == n) ? int64_t(hc[CNT_MISPLACED]) : -1;
-      ctx->kept_binnings += 1;
-      b.valid = true;
-      prof_end(ctx, tok);
-      return;
+  TabArgs tab = table_args(ctx, int64_t(ntiles));
+  for (int d = 0; d < 3; ++d) tab.nt[d] = d < D ? a.ntiles[d] : 1;
+  const uint32_t* hc = reinterpret_cast<const uint32_t*>(ctx->counters_host);
+  if (incremental) {
+    // keys in the previous sorted order, from the previous G2P of the same step
+    // loop or from the positions; the tables they give; one readback
+    const MoveOut mo = move_out(ctx, n, int64_t(ntiles));
+    if (!precomputed) {
+      fill_binning_ptrs<T, D>(ctx, a);
+      const uint32_t* skeys = static_cast<const uint32_t*>(ctx->keys_sorted.ptr);
+      if (b.n_active > 0) {
+        hipLaunchKernelGGL((k_rekey<T, D, BASIS, STORED>), dim3(xcd_grid(b.n_active)), dim3(256), 0, ctx->stream, a,
+                           skeys, uint32_t(ntiles), mo, counters);
+        TESS_HIP(hipGetLastError());
+      }
+      if (n > b.n_inside) {
+        hipLaunchKernelGGL((k_rekey_outside<T, D, BASIS, STORED>), dim3(blocks_for(n - b.n_inside, 256)), dim3(256),
+                           0, ctx->stream, a, uint32_t(ntiles), mo, counters);
+        TESS_HIP(hipGetLastError());
+      }
     }
-  }
-  TESS_HIP(hipMemsetAsync(counters, 0, CNT_BIN_SLOTS * sizeof(uint32_t), ctx->stream));
-  if (n > 0 && incremental) {
-    // keys in the previous sorted order, stayer flags -> stayer ranks; the
-    // previous G2P of the same step loop may have written them already
-    uint32_t* nk = ctx->inc_nk.as<uint32_t>(size_t(n));
-    uint32_t* spos = ctx->inc_spos.as<uint32_t>(size_t(n) + 1);
-    if (precomputed) {
-      TESS_HIP(hipMemsetAsync(spos + n, 0, sizeof(uint32_t), ctx->stream));
-    } else {
-      hipLaunchKernelGGL((k_keys_sorted<T, D, BASIS, STORED>), dim3(blocks_for(n + 1, 256)), dim3(256), 0,
-                         ctx->stream, a, perm, skeys, uint32_t(ntiles), nk, spos, counters);
-      TESS_HIP(hipGetLastError());
-    }
-    exclusive_scan_u32(ctx, spos, n + 1, counters + CNT_STAY);
-    uint32_t* hc = reinterpret_cast<uint32_t*>(ctx->counters_host);
-    TESS_HIP(hipMemcpyAsync(hc, counters, CNT_SLOTS * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
+    launch_tables(ctx->stream, tab);
     TESS_HIP(hipStreamSynchronize(ctx->stream));
-    const int64_t M = n - int64_t(hc[CNT_STAY]);
-    ctx->last_movers = M;
-    if (M == 0 && b.tile_log2 == Geo<D>::LT && b.basis == BASIS && b.dtype == mesh.dtype &&
-        !(hc[CNT_ERR] & ERR_GIMP_LENGTH)) {
+    take_report(ctx);
+    ctx->last_movers = int64_t(hc[CNT_MOVED]);
+    const bool same_kind = b.tile_log2 == Geo<D>::LT && b.basis == BASIS && b.dtype == mesh.dtype;
+    if (ctx->last_movers == 0 && same_kind && !(hc[CNT_ERR] & ERR_GIMP_LENGTH)) {
       // no particle changed its key: the previous order and tile lists stand
-      ctx->last_active_nodes = int64_t(hc[CNT_NODES]);
-      ctx->last_misplaced = (ctx->misplaced_x_ptr == P.x.ptr && ctx->misplaced_n == n) ? int64_t(hc[CNT_MISPLACED]) : -1;
+      ctx->last_misplaced = (ctx->misplaced_x_ptr == P.x.ptr && ctx->misplaced_n == n) ? ctx->broken_count : -1;
       ctx->kept_binnings += 1;
       b.x_ptr = P.x.ptr;
       b.valid = true;
       prof_end(ctx, tok);
       return;
     }
-    if (M > 0) {
-      merge_movers(ctx, nk, spos, n, M, kbits);
-      skeys = static_cast<uint32_t*>(ctx->keys_sorted.ptr);
-      perm = static_cast<uint32_t*>(ctx->vals.ptr);
+    if (hc[CNT_REENTER]) {
+      // particles came back into the mesh: every key sorted in the previous order
+      radix_sort_pairs(ctx, mo.nk, static_cast<const uint32_t*>(ctx->vals.ptr), ctx->skeys2.as<uint32_t>(m),
+                       ctx->perm2.as<uint32_t>(m), n, kbits);
+      std::swap(ctx->keys_sorted, ctx->skeys2);
+      std::swap(ctx->vals, ctx->perm2);
+    } else if (ctx->last_movers > 0) {
+      merge_moves(ctx, n, int64_t(ntiles), b.n_active, b.n_inside);
     }
-  } else if (n > 0) {
-    hipLaunchKernelGGL((k_bin_keys<T, D, BASIS, STORED>), dim3(blocks_for(n, 256)), dim3(256), 0, ctx->stream, a,
-                       keys, uint32_t(ntiles), counters);
-    TESS_HIP(hipGetLastError());
-    radix_sort_pairs(ctx, keys, nullptr, skeys, perm, n, kbits);
+  } else {
+    uint32_t* skeys = ctx->keys_sorted.as<uint32_t>(m);
+    uint32_t* perm = ctx->vals.as<uint32_t>(m);
+    if (n > 0) {
+      uint32_t* keys = ctx->keys.as<uint32_t>(m);
+      hipLaunchKernelGGL((k_bin_keys<T, D, BASIS, STORED>), dim3(blocks_for(n, 256)), dim3(256), 0, ctx->stream, a,
+                         keys, uint32_t(ntiles), counters);
+      TESS_HIP(hipGetLastError());
+      radix_sort_pairs(ctx, keys, nullptr, skeys, perm, n, kbits);
+    }
     ctx->last_movers = -1;
+    launch_tile_counts(ctx->stream, skeys, n, int64_t(ntiles), tab.stay, tab.tin);
+    launch_tables(ctx->stream, tab);
+    TESS_HIP(hipStreamSynchronize(ctx->stream));
+    take_report(ctx);
   }
-  TESS_HIP(hipMemsetAsync(tstart, 0, ntiles * sizeof(uint32_t), ctx->stream));
-  TESS_HIP(hipMemsetAsync(tend, 0, ntiles * sizeof(uint32_t), ctx->stream));
-  if (n > 0) {
-    hipLaunchKernelGGL(k_tile_runs, dim3(blocks_for(n, 256)), dim3(256), 0, ctx->stream, skeys, n,
-                       uint32_t(ntiles), tstart, tend, counters);
-    TESS_HIP(hipGetLastError());
-  }
-  hipLaunchKernelGGL(k_tile_flags, dim3(blocks_for(ntiles, 256)), dim3(256), 0, ctx->stream, tstart, tend,
-                     uint32_t(ntiles), tflag, tslot);
-  TESS_HIP(hipGetLastError());
-  exclusive_scan_u32(ctx, tslot, int64_t(ntiles), counters + CNT_ACTIVE);
-  hipLaunchKernelGGL(k_compact, dim3(blocks_for(ntiles, 256)), dim3(256), 0, ctx->stream, tflag, tslot,
-                     uint32_t(ntiles), active);
-  TESS_HIP(hipGetLastError());
-  TESS_HIP(hipMemsetAsync(nbflag, 0, ntiles * sizeof(uint32_t), ctx->stream));
-  const int3 nt = make_int3(a.ntiles[0], a.ntiles[1], D == 3 ? a.ntiles[D == 3 ? 2 : 0] : 1);
-  hipLaunchKernelGGL(k_nb_mark<D>, dim3(blocks_for(ntiles, 256)), dim3(256), 0, ctx->stream, tflag,
-                     uint32_t(ntiles), nt, nbflag);
-  TESS_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_copy_u32, dim3(blocks_for(ntiles, 256)), dim3(256), 0, ctx->stream, nbflag, nbslot,
-                     int64_t(ntiles));
-  TESS_HIP(hipGetLastError());
-  exclusive_scan_u32(ctx, nbslot, int64_t(ntiles), counters + CNT_NB);
-  hipLaunchKernelGGL(k_compact, dim3(blocks_for(ntiles, 256)), dim3(256), 0, ctx->stream, nbflag, nbslot,
-                     uint32_t(ntiles), nblist);
-  TESS_HIP(hipGetLastError());
   prof_end(ctx, tok);
-  // the one host readback of the binning: totals for the launch sizes
-  uint32_t* hc = reinterpret_cast<uint32_t*>(ctx->counters_host);
-  TESS_HIP(hipMemcpyAsync(hc, counters, CNT_SLOTS * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
-  TESS_HIP(hipStreamSynchronize(ctx->stream));
   if (hc[CNT_ERR] & ERR_GIMP_LENGTH) raise(TESS_ERR_ARGUMENT, "uGIMP requires 0 ≤ pt.l ≤ spacing(mesh)");
   if (hc[CNT_ERR] & ERR_WINDOW)
     raise(TESS_ERR_DIMENSION, "stored support window is larger than the basis support width");
-  b.n_inside = n > 0 ? int64_t(hc[CNT_INSIDE]) : 0;
-  ctx->last_active_nodes = int64_t(hc[CNT_NODES]);
+  swap_tables(ctx);
+  b.n_inside = int64_t(hc[CNT_INSIDE]);
   // layout score of the previous P2G on this particle set (consumed by the step driver)
-  ctx->last_misplaced = (ctx->misplaced_x_ptr == P.x.ptr && ctx->misplaced_n == n) ? int64_t(hc[CNT_MISPLACED]) : -1;
+  ctx->last_misplaced = (ctx->misplaced_x_ptr == P.x.ptr && ctx->misplaced_n == n) ? ctx->broken_count : -1;
   b.n_active = int64_t(hc[CNT_ACTIVE]);
   b.n_nodeblocks = int64_t(hc[CNT_NB]);
+  b.generation += 1;
   b.x_ptr = P.x.ptr;
   b.n = n;
   b.dim = D;
@@ -2960,7 +2809,7 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
   b.ntiles = int64_t(ntiles);
   for (int d = 0; d < 3; ++d) b.ntiles_axis[d] = d < D ? a.ntiles[d] : 1;
   b.valid = true;
-  b.state_valid = true;
+  b.state_valid = n > 0;
   b.state_n = n;
   b.state_ntiles = int64_t(ntiles);
   b.state_dim = D;
@@ -3011,7 +2860,8 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
     } else if (fresh) {
       hipLaunchKernelGGL((k_zero_grid<T, D>), dim3(blocks_for(nnodes, 256)), dim3(256), 0, ctx->stream, a, nnodes);
       TESS_HIP(hipGetLastError());
-    } else if (ctx->prev_nodeblocks > 0) {
+    } else if (ctx->prev_nodeblocks > 0 && ctx->prev_generation != ctx->bin.generation) {
+      // (a binning that kept its layout left no node block stale)
       hipLaunchKernelGGL((k_zero_stale<T, D>), dim3(unsigned(ctx->prev_nodeblocks)), dim3(64), 0, ctx->stream, a,
                          static_cast<const uint32_t*>(ctx->nb_list_prev.ptr), ctx->prev_nodeblocks);
       TESS_HIP(hipGetLastError());
@@ -3019,11 +2869,19 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
   };
   if (!sweep) zero_grid();
   const Binning& b = ctx->bin;
+  // broken pairs and nodes with mass are counted into the lanes, which the next
+  // binning's report sums and resets; a count nothing has reported yet (another
+  // P2G, on the same binning) starts over
+  uint32_t* lanes = lane_counters(ctx);
   uint32_t* misplaced = nullptr;
-  uint32_t* per_tile = ctx->per_tile.as<uint32_t>(size_t(std::max<int64_t>(b.n_active, 1)));
-  uint32_t* per_nb = ctx->per_nodeblock.as<uint32_t>(size_t(std::max<int64_t>(b.n_nodeblocks, 1)));
+  if (ctx->broken_pending || ctx->nodes_pending) {
+    TESS_HIP(hipMemsetAsync(lanes + LANE_BROKEN * LANES * LANE_STRIDE, 0, size_t(2) * LANES * LANE_STRIDE * 4, ctx->stream));
+    ctx->broken_pending = ctx->nodes_pending = false;
+  }
+  ctx->nodes_pending = true;
   if (count_misplaced) {
-    misplaced = per_tile;
+    misplaced = lanes;
+    ctx->broken_pending = true;
     ctx->misplaced_x_ptr = P.x.ptr;
     ctx->misplaced_n = P.n;
     ctx->misplaced_pairs = b.n_inside - b.n_active;
@@ -3033,7 +2891,6 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
   if (b.n_active > 0 && sweep) {
     a.partials = ctx->partials.as<T>(size_t(b.n_active) * Part<D, SW>::SIZE);
     (*sweep)(a, static_cast<const uint32_t*>(ctx->keys_sorted.ptr), misplaced);
-    if (misplaced) sum_u32(ctx, misplaced, b.n_active, counters + CNT_MISPLACED);
   } else if (b.n_active > 0) {
     a.partials = ctx->partials.as<T>(size_t(b.n_active) * Part<D, SW>::SIZE);
     // algorithmic bytes: x, v, V, σ per particle
@@ -3072,12 +2929,8 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
     }
     TESS_HIP(hipGetLastError());
     prof_end(ctx, tok);
-    if (misplaced) {
-      sum_u32(ctx, misplaced, b.n_active, counters + CNT_MISPLACED);
-    }
   }
   if (sweep) zero_grid();
-  TESS_HIP(hipMemsetAsync(counters + CNT_NODES, 0, sizeof(uint32_t), ctx->stream));
   if (b.n_nodeblocks > 0) {
     // algorithmic bytes per active node: m, mv, f written, read back by the
     // grid-node half, vⁿ and v written (the node count of the previous call)
@@ -3085,20 +2938,20 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
     const int tok = prof_begin(ctx, "k_gather_grid", nodes * sizeof(T) * (2 * (2 * D + 1) + 2 * D));
     if (grid_julia_layout(G, D))
       hipLaunchKernelGGL((k_gather_grid<T, D, SW, true>), dim3(xcd_grid(b.n_nodeblocks)), dim3(64), 0, ctx->stream, a,
-                         per_nb);
+                         lanes);
     else
       hipLaunchKernelGGL((k_gather_grid<T, D, SW, false>), dim3(xcd_grid(b.n_nodeblocks)), dim3(64), 0, ctx->stream, a,
-                         per_nb);
+                         lanes);
     TESS_HIP(hipGetLastError());
     prof_end(ctx, tok);
-    sum_u32(ctx, per_nb, b.n_nodeblocks, counters + CNT_NODES);
   }
   // remember this call's node blocks for the next call's stale zeroing
   uint32_t* prev = ctx->nb_list_prev.as<uint32_t>(size_t(std::max<int64_t>(b.ntiles, 1)));
-  if (b.n_nodeblocks > 0)
+  if (b.n_nodeblocks > 0 && ctx->prev_generation != b.generation)
     TESS_HIP(hipMemcpyAsync(prev, ctx->nb_list.ptr, size_t(b.n_nodeblocks) * sizeof(uint32_t),
                             hipMemcpyDeviceToDevice, ctx->stream));
   ctx->prev_nodeblocks = b.n_nodeblocks;
+  ctx->prev_generation = b.generation;
   ctx->last_grid_m = sp ? nullptr : G.m.ptr;  // a dense grid after an SpGrid call starts from a full zero
   ctx->prev_tile_log2 = Gm::LT;
   ctx->prev_ntiles = b.ntiles;
@@ -3125,15 +2978,7 @@ void g2p_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
   set_correction<T, D, STORED>(ctx, a);
   // next-step keys at the sorted positions (deferred weights in the fast kernel)
   const bool generic = a.corr && !separable_correction(a.corr, BASIS, a.filter != nullptr);
-  uint32_t* nk = nullptr;
-  uint32_t* stay = nullptr;
-  uint32_t* mv = nullptr;  // movers: particles whose key changes
-  if (write_keys && !STORED && !generic && P.n > 0) {
-    nk = ctx->inc_nk.as<uint32_t>(size_t(P.n));
-    stay = ctx->inc_spos.as<uint32_t>(size_t(P.n) + 1);
-    mv = movers_counters(ctx);
-    movers_zero(ctx);
-  }
+  const MoveOut mo = write_keys && !STORED && !generic && P.n > 0 ? move_out(ctx, P.n, b.ntiles) : no_moves();
   const uint32_t* skeys_now = static_cast<const uint32_t*>(ctx->keys_sorted.ptr);
   const bool aos = julia_layout(P, D);
   if (b.n_active > 0) {
@@ -3158,20 +3003,20 @@ void g2p_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
         if (a.corr) {  // separable corrected basis
           if (aos)
             hipLaunchKernelGGL((k_g2p_fast<T, D, BASIS, true, NW, false, true>), dim3(xcd_grid(b.n_active)),
-                               dim3(64 * NW), 0, ctx->stream, a, sk, nk, stay, nt, mv);
+                               dim3(64 * NW), 0, ctx->stream, a, sk, mo, nt);
           else
             hipLaunchKernelGGL((k_g2p_fast<T, D, BASIS, false, NW, false, true>), dim3(xcd_grid(b.n_active)),
-                               dim3(64 * NW), 0, ctx->stream, a, sk, nk, stay, nt, mv);
+                               dim3(64 * NW), 0, ctx->stream, a, sk, mo, nt);
           done = true;
         }
       }
       if (!done) {
         if (aos)
           hipLaunchKernelGGL((k_g2p_fast<T, D, BASIS, true, NW>), dim3(xcd_grid(b.n_active)), dim3(64 * NW), 0,
-                             ctx->stream, a, sk, nk, stay, nt, mv);
+                             ctx->stream, a, sk, mo, nt);
         else
           hipLaunchKernelGGL((k_g2p_fast<T, D, BASIS, false, NW>), dim3(xcd_grid(b.n_active)), dim3(64 * NW), 0,
-                             ctx->stream, a, sk, nk, stay, nt, mv);
+                             ctx->stream, a, sk, mo, nt);
       }
     }
     TESS_HIP(hipGetLastError());
@@ -3179,11 +3024,11 @@ void g2p_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
   }
   if (P.n > b.n_inside) {
     hipLaunchKernelGGL((k_g2p_outside<T, D>), dim3(blocks_for(P.n - b.n_inside, 256)), dim3(256), 0, ctx->stream,
-                       a, skeys_now, nk, stay);
+                       a, skeys_now, mo.nk);
     TESS_HIP(hipGetLastError());
   }
   ctx->bin.valid = false;  // positions moved
-  ctx->bin.keys_ready = nk != nullptr;
+  ctx->bin.keys_ready = mo.nk != nullptr;
 }
 
 // Layered storage order of the binned particles: inside each tile the k-th
@@ -3298,15 +3143,7 @@ bool g2p2g_sweep(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const
   if (ctx->corr != 0 || !g2p2g_sweep_enabled()) return false;
   using SH = G2P2GShape<T, D, BASIS>;
   const Binning& b = ctx->bin;
-  uint32_t* nk = nullptr;
-  uint32_t* stay = nullptr;
-  uint32_t* mv = nullptr;  // movers: particles whose key changes
-  if (write_keys && P.n > 0) {
-    nk = ctx->inc_nk.as<uint32_t>(size_t(P.n));
-    stay = ctx->inc_spos.as<uint32_t>(size_t(P.n) + 1);
-    mv = movers_counters(ctx);
-    movers_zero(ctx);
-  }
+  const MoveOut mo = write_keys && P.n > 0 ? move_out(ctx, P.n, b.ntiles) : no_moves();
   const bool aos = julia_layout(P, D);
   const uint32_t nt = uint32_t(b.ntiles);
   const SweepFn<T, D> sweep = [&](Args<T, D>& a, const uint32_t* sk, uint32_t* misplaced) {
@@ -3317,11 +3154,11 @@ bool g2p2g_sweep(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const
     const int tok = prof_begin(ctx, "k_g2p2g_tile", double(b.n_inside) * sizeof(T) * per_p + nodes * sizeof(T) * 2 * D);
     const dim3 grid(xcd_grid(b.n_active)), block(64 * (SH::NP + SH::NC));
     if (aos)
-      hipLaunchKernelGGL((k_g2p2g_fast<T, D, BASIS, true, SH::NP, SH::NC>), grid, block, 0, ctx->stream, a, sk, nk,
-                         stay, nt, mv, misplaced);
+      hipLaunchKernelGGL((k_g2p2g_fast<T, D, BASIS, true, SH::NP, SH::NC>), grid, block, 0, ctx->stream, a, sk, mo,
+                         nt, misplaced);
     else
-      hipLaunchKernelGGL((k_g2p2g_fast<T, D, BASIS, false, SH::NP, SH::NC>), grid, block, 0, ctx->stream, a, sk, nk,
-                         stay, nt, mv, misplaced);
+      hipLaunchKernelGGL((k_g2p2g_fast<T, D, BASIS, false, SH::NP, SH::NC>), grid, block, 0, ctx->stream, a, sk, mo,
+                         nt, misplaced);
     TESS_HIP(hipGetLastError());
     prof_end(ctx, tok);
   };
@@ -3330,11 +3167,11 @@ bool g2p2g_sweep(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const
     Args<T, D> a = make_args<T, D>(mesh, &G, P, nullptr, &prm);
     fill_binning_ptrs<T, D>(ctx, a);
     hipLaunchKernelGGL((k_g2p_outside<T, D>), dim3(blocks_for(P.n - b.n_inside, 256)), dim3(256), 0, ctx->stream,
-                       a, static_cast<const uint32_t*>(ctx->keys_sorted.ptr), nk, stay);
+                       a, static_cast<const uint32_t*>(ctx->keys_sorted.ptr), mo.nk);
     TESS_HIP(hipGetLastError());
   }
   ctx->bin.valid = false;  // positions moved
-  ctx->bin.keys_ready = nk != nullptr;
+  ctx->bin.keys_ready = mo.nk != nullptr;
   return true;
 }
 
@@ -3472,13 +3309,9 @@ void dispatch(int basis, const tess_mesh& mesh, bool stored, Args_&&... args) {
   TESS_CASE(T_, D_, TESS_BSPLINE_QUADRATIC)       \
   TESS_CASE(T_, D_, TESS_BSPLINE_CUBIC)           \
   TESS_CASE(T_, D_, TESS_UGIMP)
-  if (mesh.dtype == TESS_FLOAT32) {
-    TESS_CASES(float, 2)
-    TESS_CASES(float, 3)
-  } else {
-    TESS_CASES(double, 2)
-    TESS_CASES(double, 3)
-  }
+#ifdef TESS_PART
+  TESS_CASES(TESS_PART_T, TESS_PART_D)
+#endif
 #undef TESS_CASES
 #undef TESS_CASE
   raise(TESS_ERR_UNSUPPORTED, "unsupported (dim, dtype, basis) combination");
