@@ -303,7 +303,7 @@ void ctx_free(tess_ctx* ctx) {
                           &ctx->tile_stay, &ctx->tile_tin,  &ctx->inc_out,  &ctx->inc_seg, &ctx->inc_seg2, &ctx->inc_pout, &ctx->inc_rank,
                           &ctx->sp_occ,    &ctx->sp_act,    &ctx->sp_scan,
                           &ctx->adj_partials, &ctx->adj_nodes, &ctx->ro_checkpoints, &ctx->ro_segment,
-                          &ctx->ro_gradv,  &ctx->ro_snapshots, &ctx->ro_grid, &ctx->lanes, &ctx->g2p2g_x,
+                          &ctx->ro_gradv,  &ctx->ro_snapshots, &ctx->ro_grid, &ctx->lanes, &ctx->moved, &ctx->g2p2g_x,
                           &ctx->export_buf};
   for (auto* b : bufs) b->release();
   for (auto ev : ctx->prof.pool) (void)hipEventDestroy(ev);

@@ -263,6 +263,28 @@ __global__ void k_scatter_back(U* __restrict__ dst, int64_t es, int64_t cs, int 
   for (int c = 0; c < ncomp; ++c) dst[k * es + c * cs] = tmp[c * n + k];
 }
 
+struct CopyArrays {
+  const void* src[6];
+  void* dst[6];
+  int64_t bytes[6];
+};
+
+// Array blockIdx.y: 16-byte words where both ends are aligned, else 4-byte ones.
+__global__ __launch_bounds__(256) void k_copy_arrays(CopyArrays c) {
+  const char* s = static_cast<const char*>(c.src[blockIdx.y]);
+  char* d = static_cast<char*>(c.dst[blockIdx.y]);
+  const int64_t nb = c.bytes[blockIdx.y];
+  const int64_t i0 = int64_t(blockIdx.x) * 256 + threadIdx.x, stride = int64_t(gridDim.x) * 256;
+  int64_t done = 0;
+  if (((reinterpret_cast<uintptr_t>(s) | reinterpret_cast<uintptr_t>(d)) & 15) == 0) {
+    const int64_t n4 = nb / 16;
+    for (int64_t i = i0; i < n4; i += stride) reinterpret_cast<uint4*>(d)[i] = reinterpret_cast<const uint4*>(s)[i];
+    done = n4 * 4;
+  }
+  for (int64_t i = done + i0; i < nb / 4; i += stride)
+    reinterpret_cast<uint32_t*>(d)[i] = reinterpret_cast<const uint32_t*>(s)[i];
+}
+
 __global__ void k_iota1(int32_t* __restrict__ pidx, int64_t na) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < na) pidx[i] = int32_t(i) + 1;
@@ -542,6 +564,31 @@ void permute_particles(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
     permute_field<uint64_t>(ctx, P.l, 1, perm, n);
     permute_field<uint64_t>(ctx, P.logE, 1, perm, n);
   }
+}
+
+void permute_constants(tess_ctx* ctx, const tess_mesh& mesh, const tess_particles& P, const uint32_t* perm) {
+  if (mesh.dtype == TESS_FLOAT32) {
+    permute_field<uint32_t>(ctx, P.l, 1, perm, P.n);
+    permute_field<uint32_t>(ctx, P.logE, 1, perm, P.n);
+  } else {
+    permute_field<uint64_t>(ctx, P.l, 1, perm, P.n);
+    permute_field<uint64_t>(ctx, P.logE, 1, perm, P.n);
+  }
+}
+
+void copy_arrays(hipStream_t st, const void* const* src, void* const* dst, const int64_t* bytes, int n) {
+  CopyArrays c;
+  int64_t most = 0;
+  for (int i = 0; i < 6; ++i) {
+    c.src[i] = i < n ? src[i] : nullptr;
+    c.dst[i] = i < n ? dst[i] : nullptr;
+    c.bytes[i] = i < n ? bytes[i] : 0;
+    most = std::max(most, c.bytes[i]);
+  }
+  if (most == 0) return;
+  hipLaunchKernelGGL(k_copy_arrays, dim3(unsigned(std::min<int64_t>(ceil_div(most, int64_t(4096)), 65536)), unsigned(n)),
+                     dim3(256), 0, st, c);
+  TESS_HIP(hipGetLastError());
 }
 
 void run_reorder(tess_ctx* ctx, const tess_mesh& mesh, const tess_particles& P, int32_t* pidx, int64_t na,

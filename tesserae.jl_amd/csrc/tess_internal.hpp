@@ -190,6 +190,7 @@ struct tess_ctx {
   int64_t last_movers = -1;
   int64_t kept_binnings = 0;  // binnings that kept the previous layout (no particle changed its key)
   tess::Buffer counters;   // small device scalars
+  tess::Buffer moved;      // the second set of particle arrays of a loop whose reorders ride on G2P
   tess::Buffer g2p2g_x;    // positions before a G2P2G pass (its P2G half's weights)
   tess::Buffer export_buf; // Float32 staging of tess_export_field
   // corrected basis of the current call (TESS_WLS / TESS_KERNEL_CORRECTION /
@@ -392,6 +393,10 @@ void run_batch_stats(const tess_batch* b, int64_t* out, int n);
 void run_batch_destroy(tess_batch* b);
 // Moves every particle field so that slot k receives particle order[k].
 void permute_particles(tess_ctx* ctx, const tess_mesh& mesh, const tess_particles& P, const uint32_t* order);
+// The same for l and log E, which G2P does not write.
+void permute_constants(tess_ctx* ctx, const tess_mesh& mesh, const tess_particles& P, const uint32_t* order);
+// Copies of n <= 6 arrays in one launch (sizes in bytes, multiples of 4).
+void copy_arrays(hipStream_t st, const void* const* src, void* const* dst, const int64_t* bytes, int n);
 
 // ---- scalar type and dimension parts ------------------------------------------
 // The templated files (transfer, batch, adjoint) are compiled once per (scalar

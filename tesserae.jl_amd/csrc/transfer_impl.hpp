@@ -106,6 +106,11 @@ template <typename T, int D>
 struct Args {
   DMesh<T, D> mesh;
   DField<T> x, v, V, gradv, F, sigma, l, logE;
+  // where G2P writes the updated state, and at which index the particle at each
+  // sorted position (nullptr: its own); the fields above unless a reorder moves
+  // the particles to other arrays
+  DField<T> ox, ov, oV, ogradv, oF, osigma;
+  const uint32_t* dest;
   DField<T> gm, gmv, gf, gvn, gv;
   const int64_t* window;
   DField<T> w, gw;
@@ -142,6 +147,18 @@ struct Args {
   T gravity[D];
   int32_t slip;
 };
+
+// G2P writes in place: the state fields are its outputs.
+template <typename T, int D>
+__host__ __device__ __forceinline__ void write_in_place(Args<T, D>& a) {
+  a.ox = a.x;
+  a.ov = a.v;
+  a.oV = a.V;
+  a.ogradv = a.gradv;
+  a.oF = a.F;
+  a.osigma = a.sigma;
+  a.dest = nullptr;
+}
 
 // One scene of a batch: what differs between scenes in Args, plus where the
 // scene's tiles and particles start in the batch-wide index spaces.
@@ -182,6 +199,7 @@ __device__ __forceinline__ const SceneRec<T, D>& bind_scene(Args<T, D>& a, int s
   a.sigma = r.sigma;
   a.l = r.l;
   a.logE = r.logE;
+  write_in_place(a);
   a.gm = r.gm;
   a.gmv = r.gmv;
   a.gf = r.gf;
@@ -1456,6 +1474,7 @@ __global__ __launch_bounds__(64 * NPASS) void k_p2g_fast_persist(Args<T, D> a, c
 template <typename T, int D, bool AOS>
 struct G2PIn {
   uint32_t pid, cls, key;  // particle, window-start class in the tile, sort key at its slot
+  uint32_t dst;            // index its updated state is written at
   T x[D], v[D], F[D * D], l;
 };
 
@@ -1639,25 +1658,25 @@ __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T,
       }
     }
   }
-  const uint32_t pid = cur.pid;
+  const uint32_t pid = cur.pid, dst = cur.dst;
   // particle equations (README.md:81-86)
   T vn[D];
 #pragma unroll
   for (int c = 0; c < D; ++c) {
     vn[c] = cur.v[c] + DV[c];
-    st_g2p(fldw<T, D, AOS>(a.v, pid, c), vn[c]);
+    st_g2p(fldw<T, D, AOS>(a.ov, dst, c), vn[c]);
   }
 #pragma unroll
-  for (int q = 0; q < D * D; ++q) st_g2p(fldw<T, D * D, AOS>(a.gradv, pid, q), L[q]);
+  for (int q = 0; q < D * D; ++q) st_g2p(fldw<T, D * D, AOS>(a.ogradv, dst, q), L[q]);
   T xn[D];
 #pragma unroll
   for (int c = 0; c < D; ++c) {
     xn[c] = cur.x[c] + X[c] * dt;
-    st_g2p(fldw<T, D, AOS>(a.x, pid, c), xn[c]);
+    st_g2p(fldw<T, D, AOS>(a.ox, dst, c), xn[c]);
   }
   if (a.x_keep) {
 #pragma unroll
-    for (int c = 0; c < D; ++c) a.x_keep[int64_t(pid) * D + c] = cur.x[c];
+    for (int c = 0; c < D; ++c) a.x_keep[int64_t(dst) * D + c] = cur.x[c];
   }
   if (mo.nk) {
     uint32_t nl = 1;  // the scene's tiles; in a batch its keys start at its first global tile
@@ -1678,12 +1697,12 @@ __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T,
       Fn[r + D * b] = cur.F[r + D * b] + dt * t;
     }
 #pragma unroll
-  for (int q = 0; q < D * D; ++q) st_g2p(fldw<T, D * D, AOS>(a.F, pid, q), Fn[q]);
+  for (int q = 0; q < D * D; ++q) st_g2p(fldw<T, D * D, AOS>(a.oF, dst, q), Fn[q]);
   T sg[D * D], Vn;
   neo_hookean<T, D>(Fn, a.lambda, a.mu, a.V0, a.logE.p != nullptr, a.logE.p ? a.logE(pid) : T(0), sg, Vn);
 #pragma unroll
-  for (int q = 0; q < D * D; ++q) st_g2p(fldw<T, D * D, AOS>(a.sigma, pid, q), sg[q]);
-  st_g2p(a.V(pid), Vn);
+  for (int q = 0; q < D * D; ++q) st_g2p(fldw<T, D * D, AOS>(a.osigma, dst, q), sg[q]);
+  st_g2p(a.oV(dst), Vn);
   emit(val, der, vn, sg, Vn);
 }
 
@@ -1766,6 +1785,7 @@ __device__ __forceinline__ void k_g2p_fast_body(Args<T, D>& a, const uint32_t* _
   auto fetch = [&](int k, const Ahead& q, G2PIn<T, D, AOS>& in) {
     if (!live(k)) return;
     g2p_load<T, D, BASIS, AOS>(a, q.pid, in);
+    in.dst = a.dest ? a.dest[slot(k)] : q.pid;
     in.key = q.key;
     in.cls = by_sorted ? q.key & 63u : uint32_t(lane);
   };
@@ -1955,6 +1975,7 @@ __device__ __forceinline__ void k_g2p2g_fast_body(Args<T, D>& a, const uint32_t*
     auto fetch = [&](int k, const uint2& q, G2PIn<T, D, AOS>& in) {
       if (k >= ccount) return;
       g2p_load<T, D, BASIS, AOS>(a, q.x, in);
+      in.dst = q.x;
       in.key = q.y;
       in.cls = uint32_t(lane);
     };
@@ -2263,19 +2284,19 @@ __global__ __launch_bounds__(64) void k_gather_grid_persist(Args<T, D> a, uint32
 
 // Particle equations of the README @G2P block (README.md:81-86) after the sums.
 template <typename T, int D>
-__device__ __forceinline__ void particle_update(const Args<T, D>& a, int64_t p, const T* dv, const T* L,
+__device__ __forceinline__ void particle_update(const Args<T, D>& a, int64_t p, int64_t dst, const T* dv, const T* L,
                                                 const T* dx) {
   const T dt = a.dt;
 #pragma unroll
-  for (int c = 0; c < D; ++c) a.v(p, c) += dv[c];
+  for (int c = 0; c < D; ++c) a.ov(dst, c) = a.v(p, c) + dv[c];
 #pragma unroll
-  for (int k = 0; k < D * D; ++k) a.gradv(p, k) = L[k];
-  if (a.x_keep) {
+  for (int k = 0; k < D * D; ++k) a.ogradv(dst, k) = L[k];
 #pragma unroll
-    for (int c = 0; c < D; ++c) a.x_keep[p * D + c] = a.x(p, c);
+  for (int c = 0; c < D; ++c) {
+    const T x = a.x(p, c);
+    if (a.x_keep) a.x_keep[dst * D + c] = x;
+    a.ox(dst, c) = x + dx[c];
   }
-#pragma unroll
-  for (int c = 0; c < D; ++c) a.x(p, c) += dx[c];
   T Fo[D * D], M[D * D], Fn[D * D];
 #pragma unroll
   for (int k = 0; k < D * D; ++k) Fo[k] = a.F(p, k);
@@ -2293,12 +2314,12 @@ __device__ __forceinline__ void particle_update(const Args<T, D>& a, int64_t p, 
       Fn[r + D * b] = s;
     }
 #pragma unroll
-  for (int k = 0; k < D * D; ++k) a.F(p, k) = Fn[k];
+  for (int k = 0; k < D * D; ++k) a.oF(dst, k) = Fn[k];
   T sg[D * D], Vn;
   neo_hookean<T, D>(Fn, a.lambda, a.mu, a.V0, a.logE.p != nullptr, a.logE.p ? a.logE(p) : T(0), sg, Vn);
 #pragma unroll
-  for (int k = 0; k < D * D; ++k) a.sigma(p, k) = sg[k];
-  a.V(p) = Vn;
+  for (int k = 0; k < D * D; ++k) a.osigma(dst, k) = sg[k];
+  a.oV(dst) = Vn;
 }
 
 // One wave per tile, lanes own the tile's classes as in P2G (the walk is
@@ -2429,7 +2450,7 @@ __global__ __launch_bounds__(64) void k_g2p_tile(Args<T, D> a, const uint32_t* _
 #pragma unroll
       for (int c = 0; c < D; ++c) dx[c] += (w * vi[c]) * dt;
     }
-    particle_update<T, D>(a, pid, dv, L, dx);
+    particle_update<T, D>(a, pid, pid, dv, L, dx);
   }
 }
 
@@ -2451,7 +2472,7 @@ __global__ __launch_bounds__(256) void k_g2p_outside(Args<T, D> a, const uint32_
   }
 #pragma unroll
   for (int k = 0; k < D * D; ++k) L[k] = T(0);
-  particle_update<T, D>(a, pid, dv, L, dx);
+  particle_update<T, D>(a, pid, a.dest ? a.dest[j] : pid, dv, L, dx);
 }
 
 // ---- host side ----------------------------------------------------------------
@@ -2482,6 +2503,7 @@ Args<T, D> make_args(const tess_mesh& mesh, const tess_grid* G, const tess_parti
     a.w = dfield<T>(W->w);
     a.gw = dfield<T>(W->grad_w);
   }
+  write_in_place(a);
   a.n = P.n;
   if (prm) {
     a.mp = T(prm->mp);
@@ -2969,10 +2991,19 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
 template <typename T, int D, int BASIS, bool STORED>
 void g2p_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,
                 const tess_weights* W, const tess_params& prm, const tess_sparsity* sp, bool write_keys = false,
-                T* x_keep = nullptr) {
+                T* x_keep = nullptr, const tess_particles* out = nullptr, const uint32_t* dest = nullptr) {
   const Binning& b = ctx->bin;
   Args<T, D> a = make_args<T, D>(mesh, &G, P, W, &prm);
   a.x_keep = x_keep;
+  if (out) {
+    a.ox = dfield<T>(out->x);
+    a.ov = dfield<T>(out->v);
+    a.oV = dfield<T>(out->V);
+    a.ogradv = dfield<T>(out->grad_v);
+    a.oF = dfield<T>(out->F);
+    a.osigma = dfield<T>(out->sigma);
+    a.dest = dest;
+  }
   fill_binning_ptrs<T, D>(ctx, a);
   set_sparse<T, D>(a, mesh, sp);
   set_correction<T, D, STORED>(ctx, a);
@@ -3081,11 +3112,13 @@ inline double layered_contiguity(int64_t broken, int64_t pairs) {
   return pairs > 0 ? 1.0 - double(broken) / double(pairs) : 1.0;
 }
 
+// The layered order of the current binning: order[new index] = particle (in
+// ctx->keys) and the new index of the particle at each sorted position (in
+// ctx->keys_alt, returned).
 template <typename T, int D>
-void layered_reorder(tess_ctx* ctx, const tess_mesh& mesh, const tess_particles& P) {
+uint32_t* layered_maps(tess_ctx* ctx, const tess_mesh& mesh, const tess_particles& P) {
   const Binning& b = ctx->bin;
   const int64_t n = P.n;
-  if (n == 0) return;
   Args<T, D> a = make_args<T, D>(mesh, nullptr, P, nullptr, nullptr);
   fill_binning_ptrs<T, D>(ctx, a);
   uint32_t* order = ctx->keys.as<uint32_t>(size_t(n));        // raw keys are dead after the sort
@@ -3100,9 +3133,122 @@ void layered_reorder(tess_ctx* ctx, const tess_mesh& mesh, const tess_particles&
                        static_cast<const uint32_t*>(ctx->vals.ptr), b.n_inside, n, order, perm_new);
     TESS_HIP(hipGetLastError());
   }
-  permute_particles(ctx, mesh, P, order);
-  TESS_HIP(hipMemcpyAsync(ctx->vals.ptr, perm_new, size_t(n) * sizeof(uint32_t), hipMemcpyDeviceToDevice,
-                          ctx->stream));
+  return perm_new;
+}
+
+// Moves the particles into the layered order where they are stored.
+template <typename T, int D>
+void layered_reorder(tess_ctx* ctx, const tess_mesh& mesh, const tess_particles& P) {
+  if (P.n == 0) return;
+  layered_maps<T, D>(ctx, mesh, P);
+  permute_particles(ctx, mesh, P, static_cast<const uint32_t*>(ctx->keys.ptr));
+  std::swap(ctx->vals, ctx->keys_alt);
+}
+
+// ---- reorders that ride on G2P -------------------------------------------------
+//
+// G2P rewrites every particle field but l and log E, so a step that reorders
+// lets it write the particles at their layered places into a second set of
+// arrays instead of moving them before the step: nothing is read or written
+// twice.  P2G and the gather half of that step read the particles where they
+// were, in the same order, so every sum is the same.  The loop then goes on
+// with the second set; a call's last step writes the caller's arrays again (in
+// place of the second set, at no cost), and only a reorder in that last step,
+// or an error, leaves a copy to make.
+//
+// Moving the 31 scalars of a particle before the step took a gather and a
+// write-back pass: 3.3 ms for 13.4 M particles (Float32), beside 1.5 ms for the
+// step.  What is left is the pair of maps (0.1 ms) and the copy of at most one
+// reorder per call (0.6 ms).
+class MovingParticles {
+ public:
+  // allowed: the step's G2P is the one that can write elsewhere
+  MovingParticles(tess_ctx* ctx, const tess_particles& P, int D, size_t scalar, bool allowed)
+      : ctx_(ctx), home_(P), cur_(P), D_(D), scalar_(scalar), can_(allowed && P.n > 0) {
+    for (int f = 0; f < 6; ++f) {
+      const tess_field& a = field(home_, f);
+      const int nc = comps(f);
+      const bool aos = a.elem_stride == nc && (nc == 1 || a.comp_stride == 1);
+      const bool soa = a.elem_stride == 1 && a.comp_stride == P.n;
+      can_ = can_ && a.ptr && (aos || soa);
+    }
+  }
+  bool can_move() const { return can_; }
+  const tess_particles& now() const { return cur_; }
+  bool home() const { return cur_.x.ptr == home_.x.ptr; }
+  // the set the particles are not in (same layout)
+  tess_particles other() {
+    if (!home()) return home_;
+    tess_particles q = home_;
+    size_t off = 0;
+    for (int f = 0; f < 6; ++f) off += span(f);
+    char* p = static_cast<char*>(ctx_->moved.get(off));
+    for (int f = 0; f < 6; ++f) {
+      const_cast<tess_field&>(field(q, f)).ptr = p;
+      p += span(f);
+    }
+    return q;
+  }
+  // the particles have been written to `to`
+  void moved_to(const tess_particles& to) {
+    if (to.x.ptr == cur_.x.ptr) return;
+    rename(cur_.x.ptr, to.x.ptr);
+    cur_ = to;
+  }
+  // back into the caller's arrays
+  void settle() {
+    if (home()) return;
+    const void* src[6];
+    void* dst[6];
+    int64_t bytes[6];
+    for (int f = 0; f < 6; ++f) {
+      src[f] = field(cur_, f).ptr;
+      dst[f] = field(home_, f).ptr;
+      bytes[f] = home_.n * comps(f) * int64_t(scalar_);
+    }
+    rename(cur_.x.ptr, home_.x.ptr);
+    cur_ = home_;
+    copy_arrays(ctx_->stream, src, dst, bytes, 6);
+  }
+
+ private:
+  static const tess_field& field(const tess_particles& P, int f) {
+    const tess_field* t[6] = {&P.x, &P.v, &P.V, &P.grad_v, &P.F, &P.sigma};
+    return *t[f];
+  }
+  int comps(int f) const { return f < 2 ? D_ : f == 2 ? 1 : D_ * D_; }
+  size_t span(int f) const { return (size_t(home_.n) * size_t(comps(f)) * scalar_ + 255) & ~size_t(255); }
+  void rename(const void* from, const void* to) {
+    if (ctx_->bin.x_ptr == from) ctx_->bin.x_ptr = to;
+    if (ctx_->misplaced_x_ptr == from) ctx_->misplaced_x_ptr = to;
+  }
+  tess_ctx* ctx_;
+  tess_particles home_, cur_;
+  int D_;
+  size_t scalar_;
+  bool can_;
+};
+
+// After a G2P that wrote the particles at their layered places: the binning's
+// permutation, and the fields G2P does not write.
+template <typename T, int D>
+void take_layered(tess_ctx* ctx, const tess_mesh& mesh, const tess_particles& P) {
+  permute_constants(ctx, mesh, P, static_cast<const uint32_t*>(ctx->keys.ptr));
+  std::swap(ctx->vals, ctx->keys_alt);
+}
+
+// The G2P of a deferred-weight loop is k_g2p_fast (not the general corrected
+// form, whose kernel updates in place).
+template <int BASIS>
+bool fast_g2p(const tess_ctx* ctx) {
+  return !ctx->corr || separable_correction(ctx->corr, BASIS, ctx->corr_filter != nullptr);
+}
+
+// Whether the loop's test asks for a reorder of the binned particles.
+inline bool reorder_wanted(tess_ctx* ctx, double threshold) {
+  if (!(threshold > 0.0) || ctx->bin.n_inside == 0) return false;
+  if (threshold >= 1.0) return true;
+  return ctx->last_misplaced >= 0 && layered_contiguity(ctx->last_misplaced, ctx->misplaced_pairs) < threshold;
 }
 
 template <typename T, int D, int BASIS, bool STORED>
@@ -3210,36 +3356,39 @@ void g2p2g_impl(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
 template <typename T, int D, int BASIS>
 void g2p2g_steps_impl(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,
                       const tess_params& prm, int nsteps, double reorder_threshold) {
-  for (int s = 0; s < nsteps; ++s) {
-    bin_particles<T, D, BASIS, false>(ctx, mesh, P, nullptr, s > 0);
-    const Binning& b = ctx->bin;
-    if (reorder_threshold > 0.0 && b.n_inside > 0) {
-      bool go = reorder_threshold >= 1.0;
-      if (!go && ctx->last_misplaced >= 0) {
-        const double score = layered_contiguity(ctx->last_misplaced, ctx->misplaced_pairs);
-        go = score < reorder_threshold;
-      }
-      if (go) {
-        layered_reorder<T, D>(ctx, mesh, P);
+  const bool sweeps = ctx->corr == 0 && g2p2g_sweep_enabled();
+  MovingParticles mp(ctx, P, D, sizeof(T), !sweeps && fast_g2p<BASIS>(ctx));
+  try {
+    for (int s = 0; s < nsteps; ++s) {
+      const bool last = s + 1 == nsteps;
+      bin_particles<T, D, BASIS, false>(ctx, mesh, mp.now(), nullptr, s > 0);
+      const uint32_t* dest = nullptr;
+      if (reorder_wanted(ctx, reorder_threshold)) {
+        if (mp.can_move()) dest = layered_maps<T, D>(ctx, mesh, mp.now());
+        else layered_reorder<T, D>(ctx, mesh, mp.now());
         ctx->reorders += 1;
       }
-    }
-    if (!g2p2g_sweep<T, D, BASIS>(ctx, mesh, G, P, prm, s + 1 < nsteps, reorder_threshold > 0.0)) {
-      tess_particles Pold = P;
-      T* xo = nullptr;
-      if (P.n > 0) {
-        xo = ctx->g2p2g_x.as<T>(size_t(P.n) * D);
-        Pold.x = tess_field{xo, D, 1};
+      if (!g2p2g_sweep<T, D, BASIS>(ctx, mesh, G, mp.now(), prm, !last, reorder_threshold > 0.0)) {
+        const tess_particles to = dest ? mp.other() : last ? P : mp.now();
+        T* xo = P.n > 0 ? ctx->g2p2g_x.as<T>(size_t(P.n) * D) : nullptr;
+        // the G2P half writes the positions before its update to xo
+        g2p_launch<T, D, BASIS, false>(ctx, mesh, G, mp.now(), nullptr, prm, nullptr, !last, xo, &to, dest);
+        if (dest) take_layered<T, D>(ctx, mesh, mp.now());
+        mp.moved_to(to);
+        tess_particles Pold = mp.now();
+        if (xo) Pold.x = tess_field{xo, D, 1};
+        ctx->bin.valid = true;  // the binning describes the old positions the P2G half reads
+        p2g_launch<T, D, BASIS, false>(ctx, mesh, G, Pold, nullptr, prm, reorder_threshold > 0.0, nullptr);
+        ctx->bin.valid = false;
       }
-      // the G2P half writes the positions before its update to xo
-      g2p_launch<T, D, BASIS, false>(ctx, mesh, G, P, nullptr, prm, nullptr, s + 1 < nsteps, xo);
-      ctx->bin.valid = true;  // the binning describes the old positions the P2G half reads
-      p2g_launch<T, D, BASIS, false>(ctx, mesh, G, Pold, nullptr, prm, reorder_threshold > 0.0, nullptr);
-      ctx->bin.valid = false;
+      // the storage order the P2G half measured is that of the particles themselves
+      if (reorder_threshold > 0.0) ctx->misplaced_x_ptr = mp.now().x.ptr;
     }
-    // the storage order the P2G half measured is that of the particles themselves
-    if (reorder_threshold > 0.0) ctx->misplaced_x_ptr = P.x.ptr;
+  } catch (...) {
+    mp.settle();
+    throw;
   }
+  mp.settle();
 }
 
 // nsteps of the README loop body (deferred weights).  With reorder_threshold
@@ -3262,35 +3411,48 @@ template <typename T, int D, int BASIS, bool STORED>
 void step_impl(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,
                const tess_params& prm, int nsteps, double reorder_threshold, tess_sparsity* sp,
                int* done = nullptr, const std::function<void(int, int)>* hook = nullptr) {
-  for (int s = 0; s < nsteps; ++s) {
-    if (done) *done = s;
-    if (hook) (*hook)(0, s);
-    if (sp) {
-      // update_sparsity!(grid, xₚ) at the top of the SpGrid loop (src/Grids/grid.jl:97-101)
-      run_sparsity_update(ctx, mesh, P.x, P.n, *sp, nullptr);
-      if (sp->storage_len > sp->capacity)
-        raise(TESS_ERR_STATE, "SpGrid storage holds " + std::to_string(sp->capacity) + " nodes but the active blocks need " +
-                                  std::to_string(sp->storage_len) + "; resize the grid arrays and call again");
-    }
-    // from the second step on, the previous G2P wrote the keys (same call, so
-    // nothing else moved the particles in between)
-    bin_particles<T, D, BASIS, false>(ctx, mesh, P, nullptr, s > 0);
-    const Binning& b = ctx->bin;
-    if (reorder_threshold > 0.0 && b.n_inside > 0) {
-      bool go = reorder_threshold >= 1.0;
-      if (!go && ctx->last_misplaced >= 0) {
-        const double score = layered_contiguity(ctx->last_misplaced, ctx->misplaced_pairs);
-        go = score < reorder_threshold;
+  MovingParticles mp(ctx, P, D, sizeof(T), !STORED && fast_g2p<BASIS>(ctx));
+  try {
+    for (int s = 0; s < nsteps; ++s) {
+      const bool last = s + 1 == nsteps;
+      if (done) *done = s;
+      if (hook) (*hook)(0, s);
+      if (sp) {
+        // update_sparsity!(grid, xₚ) at the top of the SpGrid loop (src/Grids/grid.jl:97-101)
+        run_sparsity_update(ctx, mesh, mp.now().x, P.n, *sp, nullptr);
+        if (sp->storage_len > sp->capacity)
+          raise(TESS_ERR_STATE, "SpGrid storage holds " + std::to_string(sp->capacity) + " nodes but the active blocks need " +
+                                    std::to_string(sp->storage_len) + "; resize the grid arrays and call again");
       }
-      if (go) {
-        layered_reorder<T, D>(ctx, mesh, P);
+      // from the second step on, the previous G2P wrote the keys (same call, so
+      // nothing else moved the particles in between)
+      bin_particles<T, D, BASIS, false>(ctx, mesh, mp.now(), nullptr, s > 0);
+      const uint32_t* dest = nullptr;
+      if (reorder_wanted(ctx, reorder_threshold)) {
+        if (mp.can_move()) dest = layered_maps<T, D>(ctx, mesh, mp.now());
+        else layered_reorder<T, D>(ctx, mesh, mp.now());
         ctx->reorders += 1;
       }
+      // (P2G reads the particles where they are; in the layered order that its
+      // G2P gives them no neighbour pair is broken)
+      p2g_launch<T, D, BASIS, false>(ctx, mesh, G, mp.now(), nullptr, prm, reorder_threshold > 0.0 && !dest, sp);
+      if (dest) {
+        ctx->misplaced_x_ptr = mp.now().x.ptr;
+        ctx->misplaced_n = P.n;
+        ctx->misplaced_pairs = ctx->bin.n_inside - ctx->bin.n_active;
+        ctx->broken_count = 0;
+      }
+      if (hook) (*hook)(1, s);
+      const tess_particles to = dest ? mp.other() : last ? P : mp.now();
+      g2p_launch<T, D, BASIS, false>(ctx, mesh, G, mp.now(), nullptr, prm, sp, !last, nullptr, &to, dest);
+      if (dest) take_layered<T, D>(ctx, mesh, mp.now());
+      mp.moved_to(to);
     }
-    p2g_launch<T, D, BASIS, false>(ctx, mesh, G, P, nullptr, prm, reorder_threshold > 0.0, sp);
-    if (hook) (*hook)(1, s);
-    g2p_launch<T, D, BASIS, false>(ctx, mesh, G, P, nullptr, prm, sp, s + 1 < nsteps);
+  } catch (...) {
+    mp.settle();
+    throw;
   }
+  mp.settle();
   if (done) *done = nsteps;
 }
 

@@ -75,3 +75,65 @@ def test_rebinning_of_replaced_positions(dim, n):
         assert ctx.stats()["node_blocks"] == ref_ctx.stats()["node_blocks"]
         ref_ctx.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("dim,basis,n", [(2, th.BSpline(th.Quadratic()), 1), (2, th.uGIMP(), 900),
+                                         (3, th.BSpline(th.Cubic()), 65), (3, th.BSpline(th.Quadratic()), 4000)])
+@pytest.mark.parametrize("layout", ["julia", "soa"])
+@pytest.mark.parametrize("threshold,steps", [(1.0, 5), (1.0, 4), (0.85, 6)])
+def test_reorders_of_a_loop(dim, basis, n, layout, threshold, steps):
+    """Reorders in a loop (the G2P of the step writes the particles at their new places): one call equals calls of one
+    step bit for bit where every step reorders, and either gives each particle (told apart by its log E) the state it
+    has without reorders.  Some particles leave the mesh; odd and even numbers of reorders end a call."""
+    sc = random_box(dim, n, 5 + n, basis, dtype=torch.float64, h=0.1, vscale=20.0, lo=0.03, hi=0.97,
+                    with_l=basis.kernel == 16)
+    sc.logE = 0.1 * uniform01(99, n)
+    if sc.l is not None:
+        sc.l = sc.l * (0.5 + uniform01(98, n))
+
+    def run(calls, per, thr):
+        mesh, P, G = to_gpu(sc, layout=layout)
+        ctx = th.Context(library=_abi.DEBUG_LIB_PATH)
+        for _ in range(calls):
+            th.step(G, P, sc.basis, sc.params, nsteps=per, reorder_threshold=thr, ctx=ctx)
+        ctx.sync()
+        st = ctx.stats()
+        ctx.close()
+        return particles_np(P), grid_np(G), st
+
+    got, ggrid, st = run(1, steps, threshold)
+    plain, pgrid, _ = run(1, steps, 0.0)
+    if threshold == 1.0:
+        assert st["reorders"] == steps
+        one, ogrid, _ = run(steps, 1, threshold)
+        for k in got:
+            assert np.array_equal(got[k], one[k]), k
+        for k in ggrid:
+            assert np.array_equal(ggrid[k], ogrid[k]), k
+    ia, ib = np.argsort(got["logE"]), np.argsort(plain["logE"])
+    for k in got:
+        assert rel_err(got[k][ia], plain[k][ib]) <= 1e-9, k
+    assert rel_err(ggrid["m"], pgrid["m"]) <= 1e-12
+
+
+@pytest.mark.parametrize("layout", ["julia", "soa"])
+@pytest.mark.parametrize("passes", [3, 4])
+def test_reorders_of_a_g2p2g_loop(layout, passes):
+    """The same for @G2P2G passes, whose P2G half follows the G2P that moves the particles."""
+    sc = random_box(3, 2000, 8, th.BSpline(th.Quadratic()), dtype=torch.float64, h=0.1, vscale=10.0, lo=0.1, hi=0.9)
+    sc.logE = 0.1 * uniform01(99, sc.n)
+    out = []
+    for thr in (0.0, 1.0):
+        mesh, P, G = to_gpu(sc, layout=layout)
+        ctx = th.Context(library=_abi.DEBUG_LIB_PATH)
+        th.P2G(G, P, sc.basis, sc.params, ctx=ctx)
+        th.g2p2g_steps(G, P, sc.basis, sc.params, nsteps=passes, reorder_threshold=thr, ctx=ctx)
+        ctx.sync()
+        assert ctx.stats()["reorders"] == (passes if thr else 0)
+        out.append((particles_np(P), grid_np(G)))
+        ctx.close()
+    (a, ga), (b, gb) = out
+    ia, ib = np.argsort(a["logE"]), np.argsort(b["logE"])
+    for k in a:
+        assert rel_err(b[k][ib], a[k][ia]) <= 1e-9, k
+    assert rel_err(gb["m"], ga["m"]) <= 1e-12
