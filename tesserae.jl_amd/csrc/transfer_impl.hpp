@@ -574,6 +574,9 @@ __device__ __forceinline__ uint64_t lanemask_lt64() { return (uint64_t(1) << (th
 // bits), by wave-level matching; lane c gets count and offset of class c.
 // sorted slots per tile whose particle ids the transfer kernels stage in LDS
 constexpr int PID_CAP = 1024;
+// G2P's own: a 3D tile of 27 particles per cell holds 1728
+template <int D>
+constexpr int G2P_PID_CAP = D == 3 ? 2048 : 1024;
 
 template <int NW = 1>
 // With s_pid, also stages the particle ids (perm - poff) of the tile's first
@@ -904,21 +907,17 @@ __device__ __forceinline__ T& fldw(const DField<T>& f, int64_t e, int c) {
   else return f(e, c);
 }
 
-// Cache policy of the G2P particle stream (x, v, F read; v, ∇v, x, F, σ, V
-// written; gigabytes per launch, far beyond the L2 and the Infinity Cache):
-// 0 plain accesses, 1 non-temporal stores, 2 non-temporal loads and stores.
-#ifndef TESS_G2P_STREAM
-#define TESS_G2P_STREAM 1
-#endif
-template <typename T>
+// Stores of the G2P particle stream (v, ∇v, x, F, σ, V): non-temporal (NT)
+// where the particles are known to lie in the layered order, so that a wave's
+// stores fill whole lines.  Where they do not, the pieces of a line are written
+// by different waves, and only the L2 can put them together: the block at 1.7 M
+// particles in generation order took 355 us non-temporal and 132 us plain, the
+// falling 13.4 M-particle block (contiguity 0.85-1) 884 and 840 us; the same
+// block in layered order 805 us non-temporal and 843 us plain.
+template <bool NT, typename T>
 __device__ __forceinline__ void st_g2p(T& dst, T v) {
-  if constexpr (TESS_G2P_STREAM >= 1) __builtin_nontemporal_store(v, &dst);
+  if constexpr (NT) __builtin_nontemporal_store(v, &dst);
   else dst = v;
-}
-template <typename T>
-__device__ __forceinline__ T ld_g2p(T& src) {
-  if constexpr (TESS_G2P_STREAM >= 2) return __builtin_nontemporal_load(&src);
-  else return src;
 }
 // P2G's particle reads (x, v, V, σ): 0 plain, 1 non-temporal
 #ifndef TESS_P2G_STREAM
@@ -1216,6 +1215,17 @@ __device__ __forceinline__ void p2g_write_partial_slabs(const Args<T, D>& a, con
   }
 }
 
+// Float64 in 3D with three offsets per axis: one register set, the layer loaded
+// as it is needed.  The set loaded ahead took the kernel to 298 registers, one
+// wave per SIMD and one workgroup per CU, with nothing to run while it waits;
+// without it two workgroups share a CU.  Taylor rod (1.48 M particles): 288 us
+// with two sets, 319 us with one set and one wave per SIMD, 204 us with one set
+// and two.  (Four offsets per axis spill hundreds of registers at two waves.)
+template <typename T, int D, int BASIS>
+constexpr bool p2g_single() {
+  return sizeof(T) == 8 && D == 3 && support_width(BASIS) == 3;
+}
+
 // NPASS waves per tile: wave w accumulates the offsets w*KN .. w*KN+KN-1
 // along the last axis for every class (the particles are read by each wave;
 // the registers of one wave hold 1/NPASS of the stencil, which keeps several
@@ -1248,6 +1258,7 @@ __device__ __forceinline__ void k_p2g_fast_body(Args<T, D>& a, const uint32_t* _
   // Several: one slab per wave (Slab), in LDS that the per-layer jet exchange
   // and the staged particle ids use before.
   constexpr bool SHJ = NPASS > 1;
+  constexpr bool SINGLE = p2g_single<T, D, BASIS>();
   using SL = Slab<T, D, SW, KN>;
   constexpr int JET_WORDS = SHJ ? 2 * D * 2 * SW * 64 : 0;  // [layer parity][axis][val SW, der SW][lane]
   constexpr int PID_WORDS = PID_CAP * int(sizeof(uint32_t)) / int(sizeof(T));
@@ -1319,8 +1330,10 @@ __device__ __forceinline__ void k_p2g_fast_body(Args<T, D>& a, const uint32_t* _
     // the compiler copy all accumulators at each iteration)
     auto layer = [&](int k, const P2GIn<T, D>& cur, P2GIn<T, D>& nxt, uint32_t q_next, uint32_t& q_after,
                      auto staged) {
-      q_after = pid_of(k + 2, staged);
-      if (k + 1 < ccount) p2g_load<T, D, BASIS, AOS>(a, q_next, nxt);
+      if constexpr (!SINGLE) {
+        q_after = pid_of(k + 2, staged);
+        if (k + 1 < ccount) p2g_load<T, D, BASIS, AOS>(a, q_next, nxt);
+      }
       const uint64_t has = __ballot(k < ccount);
       const bool act = k < ccount;
       if (misplaced && pass == 0) bad += broken_pair(has, k, act ? cur.pid : 0u, last);
@@ -1394,6 +1407,14 @@ __device__ __forceinline__ void k_p2g_fast_body(Args<T, D>& a, const uint32_t* _
       p2g_accumulate<T, D, SW, KN>(val, der, vl, dl, mpe, mpv, A, am, amv, af);
     };
     auto walk = [&](auto staged) {
+      if constexpr (SINGLE) {
+        uint32_t qa = 0u, qb = 0u;
+        for (int k = 0; k < maxcnt; ++k) {
+          if (k < ccount) p2g_load<T, D, BASIS, AOS>(a, pid_of(k, staged), pa);
+          layer(k, pa, pb, qa, qb, staged);
+        }
+        return;
+      }
       uint32_t qa = pid_of(1, staged), qb = 0u;
       if (ccount > 0) p2g_load<T, D, BASIS, AOS>(a, pid_of(0, staged), pa);
       for (int k = 0; k < maxcnt; k += 2) {
@@ -1436,7 +1457,7 @@ __device__ __forceinline__ void k_p2g_fast_body(Args<T, D>& a, const uint32_t* _
 }
 
 template <typename T, int D, int BASIS, int NPASS, bool AOS, bool BATCH = false, bool SEP = false>
-__global__ __launch_bounds__(64 * NPASS) void k_p2g_fast(Args<T, D> a, const uint32_t* __restrict__ skeys,
+__global__ __launch_bounds__(64 * NPASS, (p2g_single<T, D, BASIS>() ? 2 : 1)) void k_p2g_fast(Args<T, D> a, const uint32_t* __restrict__ skeys,
                                                           uint32_t* __restrict__ misplaced) {
   const int64_t j = item_of<BATCH>(blockIdx.x, a.n_active);
   if (j < a.n_active) k_p2g_fast_body<T, D, BASIS, NPASS, AOS, BATCH, SEP>(a, skeys, misplaced, j);
@@ -1482,11 +1503,11 @@ template <typename T, int D, int BASIS, bool AOS>
 __device__ __forceinline__ void g2p_load(const Args<T, D>& a, uint32_t pid, G2PIn<T, D, AOS>& in) {
   in.pid = pid;
 #pragma unroll
-  for (int c = 0; c < D; ++c) in.x[c] = ld_g2p(fldw<T, D, AOS>(a.x, pid, c));
+  for (int c = 0; c < D; ++c) in.x[c] = fldw<T, D, AOS>(a.x, pid, c);
 #pragma unroll
-  for (int c = 0; c < D; ++c) in.v[c] = ld_g2p(fldw<T, D, AOS>(a.v, pid, c));
+  for (int c = 0; c < D; ++c) in.v[c] = fldw<T, D, AOS>(a.v, pid, c);
 #pragma unroll
-  for (int q = 0; q < D * D; ++q) in.F[q] = ld_g2p(fldw<T, D * D, AOS>(a.F, pid, q));
+  for (int q = 0; q < D * D; ++q) in.F[q] = fldw<T, D * D, AOS>(a.F, pid, q);
   in.l = T(0);
   if constexpr (BASIS == TESS_UGIMP) in.l = a.l(pid) / a.mesh.h;
 }
@@ -1552,18 +1573,60 @@ __device__ __forceinline__ void g2p_stage_store(const Args<T, D>& a, const int* 
   }
 }
 
+// Writes of one field of NC components from a wave's particles through LDS, in
+// storage order: lane l holds the components of the particle written at index
+// dst, and the wave stores NC times 64 consecutive scalars of the sequence
+// (particle of lane 0, 1, ...).  Where the particles of neighbouring lanes are
+// neighbours in storage, each store instruction covers whole lines.
+//
+// A 3D particle's Mat is 9 scalars: stored straight from registers, every
+// instruction touched 64 pieces of 8-16 bytes, each a write request of its own
+// (6.3 requests per particle in Float32, 20 in Float64), and the address unit
+// was busy throughout the kernel.
+template <typename T, int NC>
+struct RowStore {
+  uint32_t off[NC];  // scalar offsets this lane writes, ~0: none
+  // dst0: index * NC of the lane's particle; act: whether the lane has one
+  __device__ __forceinline__ void prepare(uint32_t dst, bool act) {
+    const int lane = int(threadIdx.x & 63);
+    const uint32_t q = act ? uint32_t(NC) * (dst - uint32_t(lane)) : ~0u;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int w = i * 64 + lane;
+      const uint32_t ql = uint32_t(__shfl(int(q), w / NC, 64));
+      off[i] = ql == ~0u ? ~0u : ql + uint32_t(w);
+    }
+  }
+  __device__ __forceinline__ void store(T* __restrict__ base, const T* v, T* s) const {
+    const int lane = int(threadIdx.x & 63);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) s[lane * NC + c] = v[c];
+    __asm__ volatile("" ::: "memory");  // the LDS executes one wave's accesses in order
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const T t = s[i * 64 + lane];
+      if (off[i] != ~0u) base[off[i]] = t;
+    }
+    __asm__ volatile("" ::: "memory");
+  }
+};
+
 // One particle's G2P and update (README.md:81-86) from the tile's staged
 // footprint (s_n: v and v - vⁿ per component; s_nodex: node coordinates): its
 // axis jets at its class window, the axis-factored sums of Δv, ∇v and the x
 // rate, the writes of v, ∇v, x, F, σ, V and, with mo.nk, of the next sort key
 // at its sorted slot jj (next_key).  emit(val, der, v, σ, V) receives the
-// jets and the updated state.
-template <typename T, int D, int BASIS, bool AOS, bool SEP, typename Emit>
+// jets and the updated state.  ROWS: called by the whole wave (act: the lane
+// has a particle; a lane without one computes on what it holds and writes
+// nothing), the Vec and Mat fields are written through s_row (64 D² scalars of
+// the wave's own).
+template <typename T, int D, int BASIS, bool AOS, bool SEP, bool ROWS, bool NT, typename Emit>
 __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T, D, AOS>& cur,
                                              const T (*s_n)[Geo<D>::PSZ], const T (*s_nodex)[Geo<D>::TS],
                                              const uint32_t jj, const uint32_t tile, const uint32_t ltile,
                                              const uint32_t start, const MoveOut& mo, TileMoves* s_mv,
-                                             uint32_t& moved, const uint32_t ntiles, Emit&& emit) {
+                                             uint32_t& moved, const uint32_t ntiles, const bool act, T* s_row,
+                                             Emit&& emit) {
   using G = Geo<D>;
   constexpr int SW = support_width(BASIS);
   const T hinv = a.mesh.h_inv, dt = a.dt;
@@ -1577,6 +1640,17 @@ __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T,
     }
   }
   T val[D][SW], der[D][SW];
+  T X[D], DV[D], L[D * D];
+#pragma unroll
+  for (int c = 0; c < D; ++c) {
+    X[c] = T(0);
+    DV[c] = T(0);
+  }
+#pragma unroll
+  for (int q = 0; q < D * D; ++q) L[q] = T(0);
+  // (a branch of its own: hoisted among the loads of the next particle and the
+  // stores below, the gather's LDS reads took 175 registers to scratch)
+  if (act) {
   bool corrects = false;
   if constexpr (SEP) corrects = sep_corrects<T, D, BASIS>(a, cur.x);
 #pragma unroll
@@ -1592,14 +1666,6 @@ __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T,
                                 der[d]);
   }
   // X = Σ w v_i, DV = Σ w (v_i - vⁿ_i), L = Σ v_i ⊗ ∇w, factored by axis
-  T X[D], DV[D], L[D * D];
-#pragma unroll
-  for (int c = 0; c < D; ++c) {
-    X[c] = T(0);
-    DV[c] = T(0);
-  }
-#pragma unroll
-  for (int q = 0; q < D * D; ++q) L[q] = T(0);
   if constexpr (D == 3) {
 #pragma unroll
     for (int kz = 0; kz < SW; ++kz)
@@ -1658,23 +1724,41 @@ __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T,
       }
     }
   }
+  }
   const uint32_t pid = cur.pid, dst = cur.dst;
+  RowStore<T, D> rows;
+  RowStore<T, D * D> mats;
+  if constexpr (ROWS) {
+    rows.prepare(dst, act);
+    mats.prepare(dst, act);
+  }
+  auto put_vec = [&](const DField<T>& f, const T* v) {
+    if constexpr (ROWS) {
+      rows.store(f.p, v, s_row);
+    } else {
+#pragma unroll
+      for (int c = 0; c < D; ++c) st_g2p<NT>(fldw<T, D, AOS>(f, dst, c), v[c]);
+    }
+  };
+  auto put_mat = [&](const DField<T>& f, const T* v) {
+    if constexpr (ROWS) {
+      mats.store(f.p, v, s_row);
+    } else {
+#pragma unroll
+      for (int q = 0; q < D * D; ++q) st_g2p<NT>(fldw<T, D * D, AOS>(f, dst, q), v[q]);
+    }
+  };
   // particle equations (README.md:81-86)
   T vn[D];
 #pragma unroll
-  for (int c = 0; c < D; ++c) {
-    vn[c] = cur.v[c] + DV[c];
-    st_g2p(fldw<T, D, AOS>(a.ov, dst, c), vn[c]);
-  }
-#pragma unroll
-  for (int q = 0; q < D * D; ++q) st_g2p(fldw<T, D * D, AOS>(a.ogradv, dst, q), L[q]);
+  for (int c = 0; c < D; ++c) vn[c] = cur.v[c] + DV[c];
+  put_vec(a.ov, vn);
+  put_mat(a.ogradv, L);
   T xn[D];
 #pragma unroll
-  for (int c = 0; c < D; ++c) {
-    xn[c] = cur.x[c] + X[c] * dt;
-    st_g2p(fldw<T, D, AOS>(a.ox, dst, c), xn[c]);
-  }
-  if (a.x_keep) {
+  for (int c = 0; c < D; ++c) xn[c] = cur.x[c] + X[c] * dt;
+  put_vec(a.ox, xn);
+  if (a.x_keep && act) {
 #pragma unroll
     for (int c = 0; c < D; ++c) a.x_keep[int64_t(dst) * D + c] = cur.x[c];
   }
@@ -1684,7 +1768,7 @@ __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T,
     for (int d = 0; d < D; ++d) nl *= uint32_t(a.ntiles[d]);
     const uint32_t kl = key_of_position<T, D, BASIS>(a, xn, cur.l, nl);
     const uint32_t key = kl == nl * 64u ? ntiles * 64u : kl + (tile - ltile) * 64u;
-    next_key(mo, key, cur.key, jj, tile, start, s_mv, moved);
+    if (!ROWS || act) next_key(mo, key, cur.key, jj, tile, start, s_mv, moved);
   }
   T Fn[D * D];
 #pragma unroll
@@ -1696,13 +1780,11 @@ __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T,
       for (int kk = 1; kk < D; ++kk) t += L[r + D * kk] * cur.F[kk + D * b];
       Fn[r + D * b] = cur.F[r + D * b] + dt * t;
     }
-#pragma unroll
-  for (int q = 0; q < D * D; ++q) st_g2p(fldw<T, D * D, AOS>(a.oF, dst, q), Fn[q]);
+  put_mat(a.oF, Fn);
   T sg[D * D], Vn;
   neo_hookean<T, D>(Fn, a.lambda, a.mu, a.V0, a.logE.p != nullptr, a.logE.p ? a.logE(pid) : T(0), sg, Vn);
-#pragma unroll
-  for (int q = 0; q < D * D; ++q) st_g2p(fldw<T, D * D, AOS>(a.osigma, dst, q), sg[q]);
-  st_g2p(a.oV(dst), Vn);
+  put_mat(a.osigma, sg);
+  if (!ROWS || act) st_g2p<NT>(a.oV(dst), Vn);
   emit(val, der, vn, sg, Vn);
 }
 
@@ -1717,7 +1799,7 @@ __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T,
 #ifndef TESS_G2P_WAVES_PER_TILE
 #define TESS_G2P_WAVES_PER_TILE 4
 #endif
-template <typename T, int D, int BASIS, bool AOS, int NW, bool BATCH, bool SEP>
+template <typename T, int D, int BASIS, bool AOS, int NW, bool BATCH, bool SEP, bool NT>
 __device__ __forceinline__ void k_g2p_fast_body(Args<T, D>& a, const uint32_t* __restrict__ skeys,
                                                        const MoveOut mo, uint32_t ntiles, const int64_t j) {
   using G = Geo<D>;
@@ -1744,9 +1826,18 @@ __device__ __forceinline__ void k_g2p_fast_body(Args<T, D>& a, const uint32_t* _
   G2PStage<T, D, 64 * NW> stage;
   g2p_stage_load<T, D, 64 * NW>(a, origin, stage);
   int ccount, coff, maxcnt;
-  __shared__ uint32_t s_pid[PID_CAP], s_key[PID_CAP];
+  __shared__ uint32_t s_pid[G2P_PID_CAP<D>], s_key[G2P_PID_CAP<D>];
+  // 3D Float64 Julia-layout fields leave through LDS rows (RowStore): 573 us
+  // without and 260 us with them on the Taylor rod (1.48 M particles).  In
+  // Float32 the rows' instructions and registers cost more than the requests
+  // they save (840 us without, 938 us with them on the 13.4 M-particle block);
+  // a 2D particle's Vec and Mat are 2 and 4 scalars, which the lanes store
+  // contiguously as they are.
+  constexpr bool ROWS = D == 3 && AOS && sizeof(T) == 8;
+  __shared__ T s_rows[ROWS ? NW : 1][ROWS ? 64 * D * D : 1];
+  T* const s_row = s_rows[ROWS ? wave : 0];
   tile_class_counts<NW>(skeys, start, cnt, s_cnt, ccount, coff, maxcnt, a.perm, poff, s_pid, s_key,
-                        PID_CAP);  // barrier after the staging of ids and keys
+                        G2P_PID_CAP<D>);  // barrier after the staging of ids and keys
   g2p_stage_store<T, D, 64 * NW>(a, origin, stage, s_n, s_nodex);
   __syncthreads();
   // Two walks of the tile's particles.  Class order (lane = class, iteration k =
@@ -1766,7 +1857,7 @@ __device__ __forceinline__ void k_g2p_fast_body(Args<T, D>& a, const uint32_t* _
   struct Ahead {
     uint32_t pid, key;
   };
-  // staged: the tile's ids are all in LDS (cnt <= PID_CAP); the walk is
+  // staged: the tile's ids are all in LDS (cnt <= G2P_PID_CAP<D>); the walk is
   // compiled for each case so that neither waits on the other's loads
   auto ahead = [&](int k, auto staged) {
     Ahead r{0u, 0u};
@@ -1799,9 +1890,11 @@ __device__ __forceinline__ void k_g2p_fast_body(Args<T, D>& a, const uint32_t* _
     const bool act = live(k);
     q_after = ahead(k + 2 * NW, staged);
     fetch(k + NW, q_next, nxt);
-    if (!act) return;
-    g2p_particle<T, D, BASIS, AOS, SEP>(a, cur, s_n, s_nodex, mo.nk ? slot(k) : 0u, tile, ltile, start, mo, &s_mv,
-                                        moved, ntiles, [](const auto&...) {});
+    if constexpr (!ROWS) {
+      if (!act) return;
+    }
+    g2p_particle<T, D, BASIS, AOS, SEP, ROWS, NT>(a, cur, s_n, s_nodex, mo.nk ? slot(k) : 0u, tile, ltile, start, mo,
+                                              &s_mv, moved, ntiles, act, s_row, [](const auto&...) {});
   };
   auto walk = [&](auto staged) {
     Ahead qa = ahead(wave + NW, staged), qb{0u, 0u};
@@ -1811,18 +1904,18 @@ __device__ __forceinline__ void k_g2p_fast_body(Args<T, D>& a, const uint32_t* _
       if (k + NW < kend) particle(k + NW, pb, pa, qb, qa, staged);
     }
   };
-  if (cnt <= PID_CAP)
+  if (cnt <= G2P_PID_CAP<D>)
     walk(std::true_type{});
   else
     walk(std::false_type{});
   if (mo.nk) tile_moves_end(mo, tile, cnt, &s_mv, moved);
 }
 
-template <typename T, int D, int BASIS, bool AOS, int NW, bool BATCH = false, bool SEP = false>
-__global__ __launch_bounds__(64 * NW, sizeof(T) == 4 ? TESS_G2P_WAVES_PER_SIMD : 1) void k_g2p_fast(Args<T, D> a, const uint32_t* __restrict__ skeys,
+template <typename T, int D, int BASIS, bool AOS, int NW, bool BATCH = false, bool SEP = false, bool NT = false>
+__global__ __launch_bounds__(64 * NW, sizeof(T) == 4 ? TESS_G2P_WAVES_PER_SIMD : 2) void k_g2p_fast(Args<T, D> a, const uint32_t* __restrict__ skeys,
                                                        const MoveOut mo, uint32_t ntiles) {
   const int64_t j = item_of<BATCH>(blockIdx.x, a.n_active);
-  if (j < a.n_active) k_g2p_fast_body<T, D, BASIS, AOS, NW, BATCH, SEP>(a, skeys, mo, ntiles, j);
+  if (j < a.n_active) k_g2p_fast_body<T, D, BASIS, AOS, NW, BATCH, SEP, NT>(a, skeys, mo, ntiles, j);
 }
 
 // Forms whose item count is read on the device at `count` (launch sizes fixed
@@ -1831,20 +1924,20 @@ __global__ __launch_bounds__(64 * NW, sizeof(T) == 4 ? TESS_G2P_WAVES_PER_SIMD :
 // (_persist; a multiple of 8 workgroups keeps each XCD on a contiguous run of
 // them, as xcd_remap does for one workgroup per item).
 template <typename T, int D, int BASIS, bool AOS, int NW, bool BATCH = false, bool SEP = false>
-__global__ __launch_bounds__(64 * NW, sizeof(T) == 4 ? TESS_G2P_WAVES_PER_SIMD : 1) void k_g2p_fast_grid(Args<T, D> a, const uint32_t* __restrict__ skeys,
+__global__ __launch_bounds__(64 * NW, sizeof(T) == 4 ? TESS_G2P_WAVES_PER_SIMD : 2) void k_g2p_fast_grid(Args<T, D> a, const uint32_t* __restrict__ skeys,
                                                        const MoveOut mo, uint32_t ntiles, const uint32_t* __restrict__ count) {
   const int64_t N = int64_t(*count), R = ((N + 7) >> 3) << 3;
   // xcd_remap is a bijection of [0, R) only: workgroups past R end here
   const int64_t j = item_of<BATCH>(blockIdx.x, N);
-  if (int64_t(blockIdx.x) < R && j < N) k_g2p_fast_body<T, D, BASIS, AOS, NW, BATCH, SEP>(a, skeys, mo, ntiles, j);
+  if (int64_t(blockIdx.x) < R && j < N) k_g2p_fast_body<T, D, BASIS, AOS, NW, BATCH, SEP, false>(a, skeys, mo, ntiles, j);
 }
 template <typename T, int D, int BASIS, bool AOS, int NW, bool BATCH = false, bool SEP = false>
-__global__ __launch_bounds__(64 * NW, sizeof(T) == 4 ? TESS_G2P_WAVES_PER_SIMD : 1) void k_g2p_fast_persist(Args<T, D> a, const uint32_t* __restrict__ skeys,
+__global__ __launch_bounds__(64 * NW, sizeof(T) == 4 ? TESS_G2P_WAVES_PER_SIMD : 2) void k_g2p_fast_persist(Args<T, D> a, const uint32_t* __restrict__ skeys,
                                                        const MoveOut mo, uint32_t ntiles, const uint32_t* __restrict__ count) {
   const int64_t N = int64_t(*count), R = ((N + 7) >> 3) << 3;
   for (int64_t it = blockIdx.x; it < R; it += gridDim.x) {
     const int64_t j = item_of<BATCH>(it, N);
-    if (j < N) k_g2p_fast_body<T, D, BASIS, AOS, NW, BATCH, SEP>(a, skeys, mo, ntiles, j);
+    if (j < N) k_g2p_fast_body<T, D, BASIS, AOS, NW, BATCH, SEP, false>(a, skeys, mo, ntiles, j);
     __syncthreads();  // the next item reuses the workgroup's LDS
   }
 }
@@ -1990,8 +2083,9 @@ __device__ __forceinline__ void k_g2p2g_fast_body(Args<T, D>& a, const uint32_t*
         fetch(k + NP, q_next, nxt);
         T(*xr)[64] = s_x[r & 1][wave];
         if (k < ccount) {
-          g2p_particle<T, D, BASIS, AOS, false>(
-              a, cur, s_n, s_nodex, start + uint32_t(coff + k), tile, ltile, start, mo, &s_mv, moved, ntiles,
+          g2p_particle<T, D, BASIS, AOS, false, false, sizeof(T) == 4>(
+              a, cur, s_n, s_nodex, start + uint32_t(coff + k), tile, ltile, start, mo, &s_mv, moved, ntiles, true,
+              static_cast<T*>(nullptr),
               [&](const auto&, const auto&, const auto& vn, const auto& sg, const T Vn) {
 #pragma unroll
                 for (int d = 0; d < D; ++d) xr[d][lane] = cur.x[d];
@@ -2988,6 +3082,12 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
   }
 }
 
+// fraction of layered neighbour pairs (particles inside the mesh minus active
+// tiles) that are consecutive in storage; 1 with no pairs
+inline double layered_contiguity(int64_t broken, int64_t pairs) {
+  return pairs > 0 ? 1.0 - double(broken) / double(pairs) : 1.0;
+}
+
 template <typename T, int D, int BASIS, bool STORED>
 void g2p_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,
                 const tess_weights* W, const tess_params& prm, const tess_sparsity* sp, bool write_keys = false,
@@ -3011,7 +3111,12 @@ void g2p_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
   const bool generic = a.corr && !separable_correction(a.corr, BASIS, a.filter != nullptr);
   const MoveOut mo = write_keys && !STORED && !generic && P.n > 0 ? move_out(ctx, P.n, b.ntiles) : no_moves();
   const uint32_t* skeys_now = static_cast<const uint32_t*>(ctx->keys_sorted.ptr);
-  const bool aos = julia_layout(P, D);
+  // (rows are addressed by 32-bit scalar offsets; past them the kernel for any strides)
+  const bool aos = julia_layout(P, D) && (D == 2 || sizeof(T) == 4 || P.n < int64_t(UINT32_MAX) / (D * D));
+  // the particles are written in the layered order: this step puts them there,
+  // or the last P2G that counted found nearly every neighbour pair in place
+  const bool layered = dest || (ctx->last_misplaced >= 0 && ctx->misplaced_x_ptr == P.x.ptr &&
+                                layered_contiguity(ctx->last_misplaced, ctx->misplaced_pairs) >= 0.98);
   if (b.n_active > 0) {
     // algorithmic bytes: x, v, F read and v, ∇v, x, F, σ, V written per
     // particle; vⁿ, v read per active node
@@ -3028,27 +3133,31 @@ void g2p_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
                          ctx->stream, a, sk);
     } else {
       constexpr int NW = TESS_G2P_WAVES_PER_TILE;
+      const dim3 grid(xcd_grid(b.n_active)), block(64 * NW);
       const uint32_t nt = uint32_t(b.ntiles);
+      auto launch = [&](auto sep, auto stream) {
+        constexpr bool SEP = decltype(sep)::value, NT = decltype(stream)::value;
+        if (aos)
+          hipLaunchKernelGGL((k_g2p_fast<T, D, BASIS, true, NW, false, SEP, NT>), grid, block, 0, ctx->stream, a, sk,
+                             mo, nt);
+        else
+          hipLaunchKernelGGL((k_g2p_fast<T, D, BASIS, false, NW, false, SEP>), grid, block, 0, ctx->stream, a, sk, mo,
+                             nt);
+      };
+      auto pick = [&](auto sep) {
+        if constexpr (sizeof(T) == 4) {  // (Float64 rows fill lines by themselves: 260 us NT, 252 us plain on the rod)
+          if (layered) return launch(sep, std::true_type{});
+        }
+        launch(sep, std::false_type{});
+      };
       bool done = false;
       if constexpr (BASIS == TESS_BSPLINE_QUADRATIC || BASIS == TESS_BSPLINE_CUBIC) {
         if (a.corr) {  // separable corrected basis
-          if (aos)
-            hipLaunchKernelGGL((k_g2p_fast<T, D, BASIS, true, NW, false, true>), dim3(xcd_grid(b.n_active)),
-                               dim3(64 * NW), 0, ctx->stream, a, sk, mo, nt);
-          else
-            hipLaunchKernelGGL((k_g2p_fast<T, D, BASIS, false, NW, false, true>), dim3(xcd_grid(b.n_active)),
-                               dim3(64 * NW), 0, ctx->stream, a, sk, mo, nt);
+          pick(std::true_type{});
           done = true;
         }
       }
-      if (!done) {
-        if (aos)
-          hipLaunchKernelGGL((k_g2p_fast<T, D, BASIS, true, NW>), dim3(xcd_grid(b.n_active)), dim3(64 * NW), 0,
-                             ctx->stream, a, sk, mo, nt);
-        else
-          hipLaunchKernelGGL((k_g2p_fast<T, D, BASIS, false, NW>), dim3(xcd_grid(b.n_active)), dim3(64 * NW), 0,
-                             ctx->stream, a, sk, mo, nt);
-      }
+      if (!done) pick(std::false_type{});
     }
     TESS_HIP(hipGetLastError());
     prof_end(ctx, tok);
@@ -3104,12 +3213,6 @@ __global__ void k_tail_identity(const uint32_t* __restrict__ perm, int64_t from,
   if (j >= n) return;
   order[j] = perm[j];
   perm_new[j] = uint32_t(j);
-}
-
-// fraction of layered neighbour pairs (particles inside the mesh minus active
-// tiles) that are consecutive in storage; 1 with no pairs
-inline double layered_contiguity(int64_t broken, int64_t pairs) {
-  return pairs > 0 ? 1.0 - double(broken) / double(pairs) : 1.0;
 }
 
 // The layered order of the current binning: order[new index] = particle (in
