@@ -148,6 +148,7 @@ void ctx_drop_caches(tess_ctx* c) {
   c->misplaced_x_ptr = nullptr;
   c->last_misplaced = -1;
   c->rollout.last_kept = false;
+  c->sp_clean = -1;
   // the counters a cut-short step may have left unreported
   c->broken_pending = c->nodes_pending = false;
   if (c->counters.ptr) (void)hipMemset(c->counters.ptr, 0, 64 * sizeof(uint32_t));
@@ -301,7 +302,7 @@ void ctx_free(tess_ctx* ctx) {
                           &ctx->partials,  &ctx->counters,    &ctx->host_pinned_dummy, &ctx->reorder_tmp, &ctx->reorder_cnt,
                           &ctx->per_tile,  &ctx->skeys2,    &ctx->perm2,    &ctx->inc_nk,
                           &ctx->tile_stay, &ctx->tile_tin,  &ctx->inc_out,  &ctx->inc_seg, &ctx->inc_seg2, &ctx->inc_pout, &ctx->inc_rank,
-                          &ctx->sp_occ,    &ctx->sp_act,    &ctx->sp_scan,
+                          &ctx->sp_occ,    &ctx->sp_act,    &ctx->sp_sums,
                           &ctx->adj_partials, &ctx->adj_nodes, &ctx->ro_checkpoints, &ctx->ro_segment,
                           &ctx->ro_gradv,  &ctx->ro_snapshots, &ctx->ro_grid, &ctx->lanes, &ctx->moved, &ctx->g2p2g_x,
                           &ctx->export_buf};

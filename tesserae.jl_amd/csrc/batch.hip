@@ -54,6 +54,14 @@ SceneRec<T, D> scene_record(const tess_scene& sc, int64_t toff, int64_t poff) {
   return r;
 }
 
+// scene of each global tile: the tile kernels start from it (a search of the
+// scenes' first tiles was eight dependent loads at the start of each workgroup)
+__global__ __launch_bounds__(256) void k_tile_scene(const int64_t* __restrict__ toff, int32_t nscenes, int64_t ntiles,
+                                                    uint32_t* __restrict__ tile_scene) {
+  const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (t < ntiles) tile_scene[t] = uint32_t(scene_of(toff, nscenes, t));
+}
+
 template <typename T, int D>
 void batch_create_impl(tess_ctx* ctx, tess_batch& b) {
   std::vector<SceneRec<T, D>> recs;
@@ -68,6 +76,10 @@ void batch_create_impl(tess_ctx* ctx, tess_batch& b) {
   for (const auto& r : recs)
     for (int d = 0; d < 3; ++d) nt.push_back(d < D ? r.ntiles[d < D ? d : 0] : 1);
   TESS_HIP(hipMemcpyAsync(b.d_nt.get(nt.size() * 4), nt.data(), nt.size() * 4, hipMemcpyHostToDevice, ctx->stream));
+  hipLaunchKernelGGL(k_tile_scene, dim3(blocks_for(b.tiles_total, 256)), dim3(256), 0, ctx->stream,
+                     static_cast<const int64_t*>(b.d_toff.ptr), b.nscenes, b.tiles_total,
+                     b.d_tscene.as<uint32_t>(size_t(std::max<int64_t>(b.tiles_total, 1))));
+  TESS_HIP(hipGetLastError());
   TESS_HIP(hipStreamSynchronize(ctx->stream));
 }
 
@@ -78,6 +90,7 @@ Args<T, D> batch_args(tess_ctx* ctx, tess_batch& b) {
   a.scenes = static_cast<const SceneRec<T, D>*>(b.recs.ptr);
   a.scene_toff = static_cast<const int64_t*>(b.d_toff.ptr);
   a.scene_poff = static_cast<const int64_t*>(b.d_poff.ptr);
+  a.tile_scene = static_cast<const uint32_t*>(b.d_tscene.ptr);
   a.nscenes = b.nscenes;
   a.n = b.ntot;
   fill_binning_ptrs<T, D>(ctx, a);
@@ -89,7 +102,7 @@ inline TabArgs batch_tables(tess_ctx* ctx, tess_batch& B) {
   TabArgs t = table_args(ctx, B.tiles_total);
   t.scene_toff = static_cast<const int64_t*>(B.d_toff.ptr);
   t.scene_nt = static_cast<const int32_t*>(B.d_nt.ptr);
-  t.nscenes = B.nscenes;
+  t.tile_scene = static_cast<const uint32_t*>(B.d_tscene.ptr);
   return t;
 }
 
@@ -131,7 +144,7 @@ void batch_bin_run(tess_ctx* ctx, tess_batch& B, bool keys_from_g2p) {
   if (incremental) {
     // the last G2P wrote the keys and counted the particles whose key changed;
     // with none the previous order and tile lists stand
-    launch_tables(ctx->stream, tab);
+    build_tables(ctx, tab);
     TESS_HIP(hipStreamSynchronize(ctx->stream));
     take_report(ctx);
     ctx->last_active_nodes = int64_t(hc[CNT_NODES]);
@@ -154,7 +167,7 @@ void batch_bin_run(tess_ctx* ctx, tess_batch& B, bool keys_from_g2p) {
       radix_sort_pairs(ctx, keys, nullptr, skeys, perm, n, key_bits_for(ntiles * 64));
     }
     launch_tile_counts(ctx->stream, skeys, n, int64_t(ntiles), tab.stay, tab.tin);
-    launch_tables(ctx->stream, tab);
+    build_tables(ctx, tab);
     TESS_HIP(hipStreamSynchronize(ctx->stream));
     take_report(ctx);
     ctx->last_active_nodes = int64_t(hc[CNT_NODES]);  // written by the previous step's gather
@@ -435,27 +448,10 @@ void fill_u32(hipStream_t st, uint32_t* p, int64_t n, uint32_t v) {
 template <typename T, int D>
 __global__ __launch_bounds__(64) void k_zero_stale_persist(Args<T, D> a, const uint32_t* __restrict__ prev_list,
                                                            const uint32_t* __restrict__ prev_count) {
-  using G = Geo<D>;
   const int64_t np = int64_t(*prev_count);
   for (int64_t j = blockIdx.x; j < np; j += gridDim.x) {
     const uint32_t B = prev_list[j];
-    if (a.nb_flag[B]) continue;
-    uint32_t poff;
-    const uint32_t Bl = bind_tile<true>(a, B, poff);
-    int Bi[D], I[D];
-    unlin<D>(Bl, a.ntiles, Bi);
-    int r = int(threadIdx.x);
-    bool in = true;
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      I[d] = Bi[d] * G::BW + r % G::BW;
-      r /= G::BW;
-      in = in && I[d] < a.mesh.dims[d];
-    }
-    if (in) {
-      const int64_t i = grid_slot(a, I);
-      if (i >= 0) zero_node(a, i);
-    }
+    zero_stale_block<T, D, true>(a, B);
   }
 }
 
@@ -637,6 +633,7 @@ void batch_graph_step(tess_ctx* g, tess_batch& B, bool full, int in) {
     g2.perm_new = cur.perm;
     g2.counters = counters;
     g2.pos_bits = key_bits_for(uint64_t(m));
+    g2.small_tiles = n < 256 * nt64;
     launch_merge(st, g2, true, n > 0 ? unsigned(std::min<int64_t>(blocks_for(n, 256), 512)) : 0u);
   }
   // grids: the previous step's stale node blocks, P2G, the grid-node half
@@ -719,7 +716,8 @@ std::vector<std::pair<const Buffer*, void*>> graph_buffers(tess_ctx* g, tess_bat
                           &g->tile_end,   &g->tile_flag,  &g->tile_slot,   &g->active_tiles, &g->nb_flag,
                           &g->nb_list,    &g->alt_start,  &g->alt_end,     &g->alt_flag,    &g->alt_slot,
                           &g->alt_active, &g->alt_nb_flag, &g->alt_nb_list, &g->partials,   &B.g_prev_list,
-                          &B.g_prev_count, &B.recs,       &B.d_toff,       &B.d_poff,       &B.d_nt};
+                          &B.g_prev_count, &B.recs,       &B.d_toff,       &B.d_poff,       &B.d_nt,
+                          &B.d_tscene};
   std::vector<std::pair<const Buffer*, void*>> v;
   for (const Buffer* b : bufs) v.emplace_back(b, b->ptr);
   return v;
@@ -990,6 +988,7 @@ void run_batch_create(tess_ctx* ctx, int basis, int nscenes, const tess_scene* s
     b->d_toff.release();
     b->d_poff.release();
     b->d_nt.release();
+    b->d_tscene.release();
     delete b;
     throw;
   }
@@ -1044,6 +1043,7 @@ void run_batch_destroy(tess_batch* b) {
   b->d_toff.release();
   b->d_poff.release();
   b->d_nt.release();
+  b->d_tscene.release();
   b->prev_list.release();
   delete b;
 }

@@ -32,7 +32,7 @@
 namespace tess {
 namespace {
 
-constexpr int TAB_THREADS = 256, TAB_PER = 4, TAB_TILES = TAB_THREADS * TAB_PER;
+constexpr int TAB_THREADS = 1024, TAB_WAVES = TAB_THREADS / 64;
 
 __device__ __forceinline__ uint32_t wave_scan_incl(uint32_t v) {
   const int lane = threadIdx.x & 63;
@@ -44,177 +44,205 @@ __device__ __forceinline__ uint32_t wave_scan_incl(uint32_t v) {
   return v;
 }
 
-// sum of v over the workgroup's 256 threads, in every thread
+// sum of v over the workgroup's threads, in every thread
 __device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* s) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
   __syncthreads();
-  return s[0] + s[1] + s[2] + s[3];
+  uint32_t t = 0;
+#pragma unroll
+  for (int w = 0; w < TAB_WAVES; ++w) t += s[w];
+  return t;
 }
 
-// exclusive prefix of v over the workgroup's 256 threads
+// exclusive prefix of v over the workgroup's threads
 __device__ __forceinline__ uint32_t block_scan_excl(uint32_t v, uint32_t* s) {
   const uint32_t inc = wave_scan_incl(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 63) s[threadIdx.x >> 6] = inc;
   __syncthreads();
   uint32_t base = 0;
-  for (int w = 0; w < int(threadIdx.x >> 6); ++w) base += s[w];
+#pragma unroll
+  for (int w = 0; w < TAB_WAVES; ++w) base += w < int(threadIdx.x >> 6) ? s[w] : 0u;
   return base + inc - v;
 }
-
-__device__ __forceinline__ uint32_t tile_count(const TabArgs& a, int64_t t) { return a.stay[t] + a.tin[t]; }
 
 // Node block B holds nodes BW*B .. BW*B+BW-1 per axis; tile t's footprint
 // [BW*t-1, BW*t+BW+1] touches node blocks t-1, t, t+1: block t is touched when
 // a tile within one of it holds a particle (in a batch, of its own scene).
+// The neighbours' counts are loaded together (clamped at the mesh's faces).
 __device__ __forceinline__ bool touched(const TabArgs& a, int64_t t) {
   int nx = a.nt[0], ny = a.nt[1], nz = a.nt[2];
   int64_t t0 = 0;
   if (a.scene_toff) {
-    int lo = 0, hi = a.nscenes - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (a.scene_toff[mid] <= t) lo = mid;
-      else hi = mid - 1;
-    }
-    t0 = a.scene_toff[lo];
-    nx = a.scene_nt[3 * lo];
-    ny = a.scene_nt[3 * lo + 1];
-    nz = a.scene_nt[3 * lo + 2];
+    const uint32_t s = a.tile_scene[t];
+    t0 = a.scene_toff[s];
+    nx = a.scene_nt[3 * s];
+    ny = a.scene_nt[3 * s + 1];
+    nz = a.scene_nt[3 * s + 2];
   }
   const uint32_t l = uint32_t(t - t0);
   const int x = int(l % uint32_t(nx)), y = int((l / uint32_t(nx)) % uint32_t(ny)), z = int(l / (uint32_t(nx) * uint32_t(ny)));
+  const int xs[3] = {max(x - 1, 0), x, min(x + 1, nx - 1)};
+  const int ys[3] = {max(y - 1, 0), y, min(y + 1, ny - 1)};
   uint32_t any = 0;
-  for (int dz = max(z - 1, 0); dz <= min(z + 1, nz - 1); ++dz)
-    for (int dy = max(y - 1, 0); dy <= min(y + 1, ny - 1); ++dy)
-      for (int dx = max(x - 1, 0); dx <= min(x + 1, nx - 1); ++dx)
-        any |= tile_count(a, t0 + (int64_t(dz) * ny + dy) * nx + dx);
+  for (int dz = nz > 1 ? -1 : 0; dz <= (nz > 1 ? 1 : 0); ++dz) {
+    const int64_t zb = t0 + int64_t(min(max(z + dz, 0), nz - 1)) * ny * nx;
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int64_t q = zb + int64_t(ys[j]) * nx + xs[i];
+        any |= a.stay[q] | a.tin[q];
+      }
+  }
   return any != 0;
 }
 
-// Per workgroup of TAB_TILES tiles: particles, arrivals, active tiles and
-// touched node blocks; writes the touched flags.
+// Per workgroup of TAB_THREADS tiles: particles, arrivals, active tiles and
+// touched node blocks; writes the touched flags.  One tile per thread: four per
+// thread left a mesh of 36 k tiles on 36 workgroups of 256 threads, each thread
+// walking the 27 neighbours of four tiles in turn (22 us).
 __global__ __launch_bounds__(TAB_THREADS) void k_tab_reduce(TabArgs a) {
-  __shared__ uint32_t s[4];
-  const int64_t base = int64_t(blockIdx.x) * TAB_TILES;
-  uint32_t c = 0, in = 0, act = 0, nb = 0;
-#pragma unroll
-  for (int k = 0; k < TAB_PER; ++k) {
-    const int64_t t = base + k * TAB_THREADS + threadIdx.x;
-    if (t < a.ntiles) {
-      const uint32_t ti = a.tin[t], ct = a.stay[t] + ti;
-      const bool f = ct != 0 || touched(a, t);
-      a.nb_flag[t] = f ? 1u : 0u;
-      c += ct;
-      in += ti;
-      act += ct ? 1u : 0u;
-      nb += f ? 1u : 0u;
-    }
+  __shared__ uint32_t s[TAB_WAVES];
+  const int64_t t = int64_t(blockIdx.x) * TAB_THREADS + threadIdx.x;
+  uint32_t c = 0, in = 0, pk = 0;
+  if (t < a.ntiles) {
+    in = a.tin[t];
+    c = a.stay[t] + in;
+    const bool f = c != 0 || touched(a, t);
+    a.nb_flag[t] = f ? 1u : 0u;
+    pk = (c ? 1u : 0u) | (f ? 0x10000u : 0u);
   }
   c = block_sum(c, s);
   in = block_sum(in, s);
-  const uint32_t packed = block_sum(act | (nb << 16), s);
+  pk = block_sum(pk, s);
   if (threadIdx.x == 0) {
     a.sums[4 * blockIdx.x] = c;
     a.sums[4 * blockIdx.x + 1] = in;
-    a.sums[4 * blockIdx.x + 2] = packed & 0xffffu;
-    a.sums[4 * blockIdx.x + 3] = packed >> 16;
+    a.sums[4 * blockIdx.x + 2] = pk & 0xffffu;
+    a.sums[4 * blockIdx.x + 3] = pk >> 16;
+  }
+}
+
+// Exclusive prefix of the workgroups' sums in place, by one workgroup.  Up to
+// SUMS_DIRECT workgroups the scan kernel adds the sums before its own by itself
+// (at 1024 that reads 8 MB from the L2 altogether); past them that reading
+// would grow with the square of the mesh.
+constexpr int64_t SUMS_DIRECT = 1024;
+__global__ __launch_bounds__(TAB_THREADS) void k_tab_prefix(uint32_t* __restrict__ sums, int64_t nb) {
+  __shared__ uint32_t s[TAB_WAVES], s_last[4];
+  uint32_t carry[4] = {0, 0, 0, 0};
+  for (int64_t b0 = 0; b0 < nb; b0 += TAB_THREADS) {
+    const int64_t b = b0 + threadIdx.x;
+    uint32_t v[4], e[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      v[q] = b < nb ? sums[4 * b + q] : 0u;
+      e[q] = carry[q] + block_scan_excl(v[q], s);
+      if (b < nb) sums[4 * b + q] = e[q];
+      if (threadIdx.x == TAB_THREADS - 1) s_last[q] = e[q] + v[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) carry[q] = s_last[q];
+    __syncthreads();
   }
 }
 
 // The tables of a workgroup's tiles from the sums of the workgroups before it.
 // Workgroup 0 also sums the lane counters (particles whose key changed, broken
 // layered pairs, nodes with mass), the last one holds the totals; both report
-// to pinned host memory and reset what the next step counts into.
+// to pinned host memory and reset what the next step counts into.  A mesh that
+// fits one workgroup needs no sums: this launch alone (ALONE).
+template <bool ALONE>
 __global__ __launch_bounds__(TAB_THREADS) void k_tab_scan(TabArgs a) {
-  __shared__ uint32_t s[4];
+  __shared__ uint32_t s[TAB_WAVES];
   uint32_t pre[4] = {0, 0, 0, 0};
-  for (int b = int(threadIdx.x); b < int(blockIdx.x); b += TAB_THREADS)
+  if constexpr (!ALONE) {
+    if (gridDim.x > SUMS_DIRECT) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) pre[q] += a.sums[4 * b + q];
+      for (int q = 0; q < 4; ++q) pre[q] = a.sums[4 * int64_t(blockIdx.x) + q];
+    } else {
+      for (int b = int(threadIdx.x); b < int(blockIdx.x); b += TAB_THREADS)
 #pragma unroll
-  for (int q = 0; q < 4; ++q) pre[q] = block_sum(pre[q], s);
-  const int64_t base = int64_t(blockIdx.x) * TAB_TILES + int64_t(threadIdx.x) * TAB_PER;
-  uint32_t ct[TAB_PER], ti[TAB_PER], fl[TAB_PER];
-  uint32_t c = 0, in = 0, pk = 0;
+        for (int q = 0; q < 4; ++q) pre[q] += a.sums[4 * b + q];
 #pragma unroll
-  for (int k = 0; k < TAB_PER; ++k) {
-    const int64_t t = base + k;
-    const bool ok = t < a.ntiles;
-    ti[k] = ok ? a.tin[t] : 0u;
-    ct[k] = ok ? a.stay[t] + ti[k] : 0u;
-    fl[k] = ok ? a.nb_flag[t] : 0u;
-    c += ct[k];
-    in += ti[k];
-    pk += (ct[k] ? 1u : 0u) | (fl[k] << 16);
-  }
-  uint32_t ec = pre[0] + block_scan_excl(c, s), ei = pre[1] + block_scan_excl(in, s);
-  const uint32_t epk = block_scan_excl(pk, s);
-  uint32_t ea = pre[2] + (epk & 0xffffu), en = pre[3] + (epk >> 16);
-#pragma unroll
-  for (int k = 0; k < TAB_PER; ++k) {
-    const int64_t t = base + k;
-    if (t < a.ntiles) {
-      a.start[t] = ec;
-      a.end[t] = ec + ct[k];
-      a.flag[t] = ct[k] ? 1u : 0u;
-      a.slot[t] = ea;
-      a.seg[t] = ei;
-      if (ct[k]) a.active[ea] = uint32_t(t);
-      if (fl[k]) a.nb_list[en] = uint32_t(t);
-      if (ti[k]) a.tin[t] = 0u;
-      ec += ct[k];
-      ei += ti[k];
-      ea += ct[k] ? 1u : 0u;
-      en += fl[k];
+      for (int q = 0; q < 4; ++q) pre[q] = block_sum(pre[q], s);
     }
   }
-  // the workgroup that holds the last tile: totals, and the particles outside
-  // the mesh (the entry past the tiles)
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == TAB_THREADS - 1) {
+  const int64_t t = int64_t(blockIdx.x) * TAB_THREADS + threadIdx.x;
+  const bool ok = t < a.ntiles;
+  const uint32_t ti = ok ? a.tin[t] : 0u, ct = ok ? a.stay[t] + ti : 0u;
+  uint32_t fl = 0u;
+  if constexpr (ALONE) {
+    if (ok) {
+      fl = ct != 0 || touched(a, t) ? 1u : 0u;
+      a.nb_flag[t] = fl;
+    }
+    __syncthreads();  // the neighbours' arrivals have been read; they are reset below
+  } else {
+    fl = ok ? a.nb_flag[t] : 0u;
+  }
+  const uint32_t ec = pre[0] + block_scan_excl(ct, s), ei = pre[1] + block_scan_excl(ti, s);
+  const uint32_t epk = block_scan_excl((ct ? 1u : 0u) | (fl << 16), s);
+  const uint32_t ea = pre[2] + (epk & 0xffffu), en = pre[3] + (epk >> 16);
+  if (ok) {
+    a.start[t] = ec;
+    a.end[t] = ec + ct;
+    a.flag[t] = ct ? 1u : 0u;
+    a.slot[t] = ea;
+    a.seg[t] = ei;
+    if (ct) a.active[ea] = uint32_t(t);
+    if (fl) a.nb_list[en] = uint32_t(t);
+    if (ti) a.tin[t] = 0u;
+  }
+  // the thread of the last tile: totals, and the particles outside the mesh
+  // (the entry past the tiles)
+  if (t == a.ntiles - 1) {
+    const uint32_t inside = ec + ct, arrive = ei + ti, act = ea + (ct ? 1u : 0u), nb = en + fl;
     const uint32_t out_in = a.tin[a.ntiles];
-    a.seg[a.ntiles] = ei;
-    a.start[a.ntiles] = ec;
+    a.seg[a.ntiles] = arrive;
+    a.start[a.ntiles] = inside;
     a.stay[a.ntiles] += out_in;
     a.tin[a.ntiles] = 0u;
     a.counters[CNT_PREV_ACTIVE] = a.counters[CNT_ACTIVE];
-    a.counters[CNT_INSIDE] = ec;
-    a.counters[CNT_ACTIVE] = ea;
-    a.counters[CNT_NB] = en;
+    a.counters[CNT_INSIDE] = inside;
+    a.counters[CNT_ACTIVE] = act;
+    a.counters[CNT_NB] = nb;
     a.counters[CNT_OUTIN] = out_in;
-    a.host[CNT_INSIDE] = ec;
-    a.host[CNT_ACTIVE] = ea;
-    a.host[CNT_NB] = en;
+    a.host[CNT_INSIDE] = inside;
+    a.host[CNT_ACTIVE] = act;
+    a.host[CNT_NB] = nb;
     a.host[CNT_OUTIN] = out_in;
-    a.host[CNT_ARRIVE] = ei + out_in;
+    a.host[CNT_ARRIVE] = arrive + out_in;
+    __threadfence_system();
   }
   if (blockIdx.x == 0) {
-    uint32_t v[3];
-#pragma unroll
-    for (int g = 0; g < 3; ++g) {
-      uint32_t x = 0;
-      if (threadIdx.x < LANES) {
-        uint32_t* lane = a.lanes + (g * LANES + int(threadIdx.x)) * LANE_STRIDE;
-        x = *lane;
-        *lane = 0u;
-      }
-      v[g] = block_sum(x, s);
+    // one wave per group of lanes
+    const int g = int(threadIdx.x >> 6), i = int(threadIdx.x & 63);
+    uint32_t x = 0;
+    if (g < LANE_GROUPS && i < LANES) {
+      uint32_t* lane = a.lanes + (g * LANES + i) * LANE_STRIDE;
+      x = *lane;
+      if (x) *lane = 0u;
     }
-    if (threadIdx.x == 0) {
-      a.host[CNT_MOVED] = v[LANE_MOVED];
-      a.host[CNT_MISPLACED] = v[LANE_BROKEN];
-      a.host[CNT_NODES] = v[LANE_NODES];
-      a.counters[CNT_NODES] = v[LANE_NODES];
-      a.host[CNT_ERR] = a.counters[CNT_ERR];
-      a.host[CNT_REENTER] = a.counters[CNT_REENTER];
-      if (!a.keep_err) a.counters[CNT_ERR] = 0u;
-      a.counters[CNT_REENTER] = 0u;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off, 64);
+    if (i == 0 && g < LANE_GROUPS) {
+      a.host[g == LANE_MOVED ? CNT_MOVED : g == LANE_BROKEN ? CNT_MISPLACED : CNT_NODES] = x;
+      if (g == LANE_NODES) {
+        a.counters[CNT_NODES] = x;
+        a.host[CNT_ERR] = a.counters[CNT_ERR];
+        a.host[CNT_REENTER] = a.counters[CNT_REENTER];
+        if (!a.keep_err) a.counters[CNT_ERR] = 0u;
+        a.counters[CNT_REENTER] = 0u;
+      }
+      __threadfence_system();
     }
   }
-  __threadfence_system();
 }
 
 // Particles of each tile in a freshly sorted order (binary searches of the
@@ -257,31 +285,48 @@ __global__ __launch_bounds__(64) void k_scatter_out(MergeArgs a) {
   }
 }
 
-constexpr int MERGE_THREADS = 256, MERGE_WAVES = MERGE_THREADS / 64, MERGE_CAP = 512;
+// The merge runs one workgroup per tile, of 4 waves, or of one where tiles hold
+// few particles (the batch's 256 uneven scenes, 110 per active tile: 227 us with
+// four waves per tile).  Arrivals up to the LDS list are sorted there.
+template <int NW>
+constexpr int MERGE_CAP = NW == 1 ? 128 : 512;
 
 // Sorts k (key, position) pairs of a segment by position with one workgroup:
 // 8-bit digits of the position, `bits` low bits, between seg and alt; returns
 // the buffer that holds the result.  For segments past the LDS list.
+template <int NW>
 __device__ uint2* segment_sort(uint2* seg, uint2* alt, uint32_t k, int bits, uint32_t* s_hist, uint32_t (*s_wc)[256]) {
+  constexpr int NT = 64 * NW;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int shift = 0; shift < bits; shift += 8) {
     __syncthreads();
-    s_hist[threadIdx.x] = 0;
+    for (int d = int(threadIdx.x); d < 256; d += NT) s_hist[d] = 0;
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < k; i += MERGE_THREADS) atomicAdd(&s_hist[(seg[i].y >> shift) & 255u], 1u);
+    for (uint32_t i = threadIdx.x; i < k; i += NT) atomicAdd(&s_hist[(seg[i].y >> shift) & 255u], 1u);
     __syncthreads();
-    const uint32_t h = s_hist[threadIdx.x];
-    __shared__ uint32_t s4[4];
-    const uint32_t ex = block_scan_excl(h, s4);
+    if (wave == 0) {  // exclusive prefix of the 256 digits, four per lane
+      uint32_t h[4], tot = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        h[q] = s_hist[4 * lane + q];
+        tot += h[q];
+      }
+      uint32_t run = wave_scan_incl(tot) - tot;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        s_hist[4 * lane + q] = run;
+        run += h[q];
+      }
+    }
     __syncthreads();
-    s_hist[threadIdx.x] = ex;
-    for (uint32_t b = 0; b < k; b += MERGE_THREADS) {
+    for (uint32_t b = 0; b < k; b += NT) {
       const uint32_t i = b + threadIdx.x;
       const bool valid = i < k;
       const uint2 e = valid ? seg[i] : make_uint2(0u, 0u);
       const uint32_t d = (e.y >> shift) & 255u;
+      for (int q = int(threadIdx.x); q < 256; q += NT)
 #pragma unroll
-      for (int w = 0; w < MERGE_WAVES; ++w) s_wc[w][threadIdx.x] = 0;
+        for (int w = 0; w < NW; ++w) s_wc[w][q] = 0;
       __syncthreads();
       uint64_t peers = __ballot(valid);
 #pragma unroll
@@ -299,10 +344,12 @@ __device__ uint2* segment_sort(uint2* seg, uint2* alt, uint32_t k, int bits, uin
         alt[pos] = e;
       }
       __syncthreads();
-      uint32_t add = 0;
+      for (int q = int(threadIdx.x); q < 256; q += NT) {
+        uint32_t add = 0;
 #pragma unroll
-      for (int w = 0; w < MERGE_WAVES; ++w) add += s_wc[w][threadIdx.x];
-      s_hist[threadIdx.x] += add;
+        for (int w = 0; w < NW; ++w) add += s_wc[w][q];
+        s_hist[q] += add;
+      }
       __syncthreads();
     }
     __threadfence_block();
@@ -317,9 +364,12 @@ __device__ uint2* segment_sort(uint2* seg, uint2* alt, uint32_t k, int bits, uin
 // One workgroup per tile that holds particles now.  The tile's new run is the
 // stable counting sort, by class, of a sequence in order of previous position:
 // arrivals from below its old run, the old run without its leavers, arrivals
-// from above.  The four waves take consecutive quarters of the sequence.
-__global__ __launch_bounds__(MERGE_THREADS) void k_merge_tiles(MergeArgs a) {
-  __shared__ uint2 s_raw[MERGE_CAP], s_in[MERGE_CAP];
+// from above.  The waves take consecutive parts of the sequence.
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_merge_tiles(MergeArgs a) {
+  constexpr int MERGE_THREADS = 64 * NW, MERGE_WAVES = NW;
+  constexpr uint32_t CAP = MERGE_CAP<NW>;
+  __shared__ uint2 s_raw[CAP], s_in[CAP];
   __shared__ uint32_t s_hist[256], s_wc[MERGE_WAVES][256];
   __shared__ uint32_t s_base[MERGE_WAVES][64], s_low;
   const int64_t jt = blockIdx.x;
@@ -332,7 +382,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void k_merge_tiles(MergeArgs a) {
   const uint2* in = s_in;
   if (threadIdx.x == 0) s_low = 0;
   s_base[wave][lane] = 0;
-  if (k > 0 && k <= MERGE_CAP) {
+  if (k > 0 && k <= CAP) {
     const uint2* seg = a.seg + a.seg_off[t];
     for (uint32_t i = threadIdx.x; i < k; i += MERGE_THREADS) s_raw[i] = seg[i];
     __syncthreads();
@@ -343,7 +393,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void k_merge_tiles(MergeArgs a) {
       s_in[r] = e;
     }
   } else if (k > 0) {
-    in = segment_sort(a.seg + a.seg_off[t], a.seg_alt + a.seg_off[t], k, a.pos_bits, s_hist, s_wc);
+    in = segment_sort<NW>(a.seg + a.seg_off[t], a.seg_alt + a.seg_off[t], k, a.pos_bits, s_hist, s_wc);
   }
   __syncthreads();
   if (k > 0) {
@@ -366,7 +416,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void k_merge_tiles(MergeArgs a) {
     pos = e.y;
     return true;
   };
-  const uint32_t quarter = ((len + 255u) / 256u) * 64u;
+  const uint32_t quarter = ((len + MERGE_THREADS - 1) / MERGE_THREADS) * 64u;  // a wave's part
   const uint32_t i0 = uint32_t(wave) * quarter;
   auto match = [&](uint32_t c, bool valid) {
     uint64_t peers = __ballot(valid);
@@ -452,13 +502,14 @@ __global__ __launch_bounds__(MERGE_THREADS) void k_merge_tiles(MergeArgs a) {
 // Particles outside the mesh: those that were outside keep their order behind
 // the arrivals (whose previous positions are all lower).  Workgroup 0 places
 // the arrivals, sorted by previous position.
-__global__ __launch_bounds__(MERGE_THREADS) void k_merge_outside(MergeArgs a) {
+__global__ __launch_bounds__(256) void k_merge_outside(MergeArgs a) {
+  constexpr int MERGE_THREADS = 256, MERGE_WAVES = 4;
   __shared__ uint32_t s_hist[256], s_wc[MERGE_WAVES][256];
   const uint32_t k = a.counters ? a.counters[CNT_OUTIN] : a.out_in;
   const uint32_t ns = a.new_start[a.ntiles], os = a.old_start[a.ntiles];
   if (blockIdx.x == 0 && k > 0) {
     const uint32_t off = a.seg_off[a.ntiles];
-    const uint2* in = segment_sort(a.seg + off, a.seg_alt + off, k, a.pos_bits, s_hist, s_wc);
+    const uint2* in = segment_sort<4>(a.seg + off, a.seg_alt + off, k, a.pos_bits, s_hist, s_wc);
     for (uint32_t i = threadIdx.x; i < k; i += MERGE_THREADS) {
       a.keys_new[ns + i] = in[i].x;
       a.perm_new[ns + i] = a.perm_old[in[i].y];
@@ -473,13 +524,22 @@ __global__ __launch_bounds__(MERGE_THREADS) void k_merge_outside(MergeArgs a) {
 
 }  // namespace
 
-int64_t tab_blocks(int64_t ntiles) { return ceil_div(ntiles, int64_t(TAB_TILES)); }
+int64_t tab_blocks(int64_t ntiles) { return ceil_div(ntiles, int64_t(TAB_THREADS)); }
 
 void launch_tables(hipStream_t st, const TabArgs& a) {
   const unsigned nb = unsigned(tab_blocks(a.ntiles));
+  if (nb == 1) {
+    hipLaunchKernelGGL(k_tab_scan<true>, dim3(1), dim3(TAB_THREADS), 0, st, a);
+    TESS_HIP(hipGetLastError());
+    return;
+  }
   hipLaunchKernelGGL(k_tab_reduce, dim3(nb), dim3(TAB_THREADS), 0, st, a);
   TESS_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_tab_scan, dim3(nb), dim3(TAB_THREADS), 0, st, a);
+  if (int64_t(nb) > SUMS_DIRECT) {
+    hipLaunchKernelGGL(k_tab_prefix, dim3(1), dim3(TAB_THREADS), 0, st, a.sums, int64_t(nb));
+    TESS_HIP(hipGetLastError());
+  }
+  hipLaunchKernelGGL(k_tab_scan<false>, dim3(nb), dim3(TAB_THREADS), 0, st, a);
   TESS_HIP(hipGetLastError());
 }
 
@@ -497,11 +557,14 @@ void launch_merge(hipStream_t st, const MergeArgs& a, bool arrivals, unsigned ou
     TESS_HIP(hipGetLastError());
   }
   if (a.new_active_n > 0) {
-    hipLaunchKernelGGL(k_merge_tiles, dim3(unsigned(a.new_active_n)), dim3(MERGE_THREADS), 0, st, a);
+    if (a.small_tiles)
+      hipLaunchKernelGGL(k_merge_tiles<1>, dim3(unsigned(a.new_active_n)), dim3(64), 0, st, a);
+    else
+      hipLaunchKernelGGL(k_merge_tiles<4>, dim3(unsigned(a.new_active_n)), dim3(256), 0, st, a);
     TESS_HIP(hipGetLastError());
   }
   if (outside_blocks > 0) {
-    hipLaunchKernelGGL(k_merge_outside, dim3(outside_blocks), dim3(MERGE_THREADS), 0, st, a);
+    hipLaunchKernelGGL(k_merge_outside, dim3(outside_blocks), dim3(256), 0, st, a);
     TESS_HIP(hipGetLastError());
   }
 }

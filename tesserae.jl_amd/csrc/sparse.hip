@@ -11,7 +11,7 @@
 namespace tess {
 namespace {
 
-// counter slots of this file inside ctx->counters (uint32)
+// words of the pinned readback slots this file reports to
 enum { SP_COUNT = 32, SP_CHANGED = 33 };
 
 template <int D>
@@ -41,14 +41,17 @@ __global__ __launch_bounds__(256) void k_sp_occupied(DField<T> x, int64_t n, DMe
 }
 
 // act[b] = 1 if any block of the 3^dim neighbourhood is occupied
-// (_activate_block_neighborhood!, sparsity.jl:141-145); flags a change of the
-// active set against the numbering passed in (sparsity.jl:262-267).
+// (_activate_block_neighborhood!, sparsity.jl:141-145), with the workgroup's
+// count of active blocks and whether its part of the active set differs from
+// the numbering passed in (sparsity.jl:262-267).
+constexpr int SP_THREADS = 256;
 template <int D>
-__global__ __launch_bounds__(256) void k_sp_activity(const uint32_t* __restrict__ occ, BlockGrid<D> bg,
-                                                     const int32_t* __restrict__ old_numbering,
-                                                     uint32_t* __restrict__ act, uint32_t* __restrict__ scan,
-                                                     uint32_t* __restrict__ changed) {
-  const int64_t b = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(SP_THREADS) void k_sp_activity(const uint32_t* __restrict__ occ, BlockGrid<D> bg,
+                                                            const int32_t* __restrict__ old_numbering,
+                                                            uint32_t* __restrict__ act,
+                                                            uint2* __restrict__ sums) {
+  __shared__ uint32_t s_n[SP_THREADS / 64], s_c[SP_THREADS / 64];
+  const int64_t b = int64_t(blockIdx.x) * SP_THREADS + threadIdx.x;
   bool a = false, diff = false;
   if (b < bg.total) {
     int I[D];
@@ -59,33 +62,117 @@ __global__ __launch_bounds__(256) void k_sp_activity(const uint32_t* __restrict_
       r /= bg.nb[d];
     }
     constexpr int NN = (D == 3) ? 27 : 9;
-    for (int k = 0; k < NN && !a; ++k) {
-      int q = k;
-      int64_t nb = 0;
-      bool ok = true;
+    uint32_t any = 0;  // the neighbours' flags loaded together, clamped at the faces
 #pragma unroll
-      for (int d = D - 1; d >= 0; --d) {
-        int div = 1;
-        for (int e = 0; e < d; ++e) div *= 3;
-        const int J = I[d] + (q / div) % 3 - 1;
-        ok = ok && J >= 0 && J < bg.nb[d];
-        nb = nb * bg.nb[d] + J;
+    for (int k = 0; k < NN; ++k) {
+      int q = k;
+      int J[D];
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        J[d] = min(max(I[d] + q % 3 - 1, 0), bg.nb[d] - 1);
+        q /= 3;
       }
-      a = ok && occ[nb] != 0u;
+      int64_t nb = J[D - 1];
+#pragma unroll
+      for (int d = D - 2; d >= 0; --d) nb = nb * bg.nb[d] + J[d];
+      any |= occ[nb];
     }
+    a = any != 0;
     act[b] = a ? 1u : 0u;
-    scan[b] = a ? 1u : 0u;
     diff = (old_numbering[b] != 0) != a;
   }
-  // one store per wave that saw a change
-  if (__ballot(diff) != 0 && (threadIdx.x & 63) == 0) *changed = 1u;
+  const uint64_t m = __ballot(a), dm = __ballot(diff);
+  if ((threadIdx.x & 63) == 0) {
+    s_n[threadIdx.x >> 6] = uint32_t(__popcll(m));
+    s_c[threadIdx.x >> 6] = dm ? 1u : 0u;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint2 t = make_uint2(0u, 0u);
+    for (int w = 0; w < SP_THREADS / 64; ++w) {
+      t.x += s_n[w];
+      t.y |= s_c[w];
+    }
+    sums[blockIdx.x] = t;
+  }
 }
 
-__global__ __launch_bounds__(256) void k_sp_number(const uint32_t* __restrict__ act,
-                                                   const uint32_t* __restrict__ excl, int64_t total,
-                                                   int32_t* __restrict__ numbering) {
-  const int64_t b = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (b < total) numbering[b] = act[b] ? int32_t(excl[b] + 1u) : 0;
+// Exclusive prefix of the workgroups' counts (and the OR of their changes) in
+// place, by one workgroup, where there are more of them than k_sp_number should
+// add up by itself.  Entry `wgs` receives the total.
+constexpr int64_t SUMS_DIRECT = 1024;
+__global__ __launch_bounds__(64) void k_sp_prefix(uint2* __restrict__ sums, int64_t wgs) {
+  uint32_t carry = 0, ch = 0;
+  for (int64_t b0 = 0; b0 < wgs; b0 += 64) {
+    const int64_t b = b0 + threadIdx.x;
+    const uint2 v = b < wgs ? sums[b] : make_uint2(0u, 0u);
+    uint32_t inc = v.x;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t u = __shfl_up(inc, off, 64);
+      if (int(threadIdx.x) >= off) inc += u;
+    }
+    if (__ballot(v.y != 0)) ch = 1u;
+    if (b < wgs) sums[b].x = carry + inc - v.x;
+    carry += __shfl(inc, 63, 64);
+  }
+  if (threadIdx.x == 0) sums[wgs] = make_uint2(carry, ch);
+}
+
+// The numbers of a workgroup's active blocks after the counts of the workgroups
+// before it; clears the occupied flags for the next update.  The last workgroup
+// reports the totals to pinned host memory.
+__global__ __launch_bounds__(SP_THREADS) void k_sp_number(const uint32_t* __restrict__ act,
+                                                          const uint2* __restrict__ sums, int64_t total,
+                                                          int32_t* __restrict__ numbering, uint32_t* __restrict__ occ,
+                                                          uint32_t* __restrict__ host) {
+  __shared__ uint32_t s_n[SP_THREADS / 64], s_c[SP_THREADS / 64], s_w[SP_THREADS / 64];
+  const bool last = blockIdx.x == gridDim.x - 1;
+  uint32_t pre = 0, ch = 0;
+  if (int64_t(gridDim.x) > SUMS_DIRECT) {
+    if (threadIdx.x == 0) {
+      pre = sums[blockIdx.x].x;
+      ch = sums[gridDim.x].y;
+    }
+  } else {
+    for (int i = int(threadIdx.x); i < int(blockIdx.x); i += SP_THREADS) {
+      const uint2 t = sums[i];
+      pre += t.x;
+      ch |= t.y;
+    }
+    if (last && threadIdx.x == 0) ch |= sums[blockIdx.x].y;
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    pre += __shfl_xor(pre, off, 64);
+    ch |= __shfl_xor(ch, off, 64);
+  }
+  const int64_t b = int64_t(blockIdx.x) * SP_THREADS + threadIdx.x;
+  const bool a = b < total && act[b] != 0;
+  const uint64_t m = __ballot(a);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (lane == 0) {
+    s_n[wave] = pre;
+    s_c[wave] = ch;
+    s_w[wave] = uint32_t(__popcll(m));
+  }
+  __syncthreads();
+  uint32_t base = 0, own = 0, changed = 0;
+  for (int w = 0; w < SP_THREADS / 64; ++w) {
+    base += s_n[w];
+    changed |= s_c[w];
+    own += s_w[w];
+  }
+  for (int w = 0; w < wave; ++w) base += s_w[w];
+  if (b < total) {
+    numbering[b] = a ? int32_t(base + uint32_t(__popcll(m & ((uint64_t(1) << lane) - 1))) + 1u) : 0;
+    occ[b] = 0u;
+  }
+  if (last && threadIdx.x == 0) {
+    host[SP_COUNT] = base + own;  // thread 0 is in wave 0: base holds the workgroups before
+    host[SP_CHANGED] = changed;
+    __threadfence_system();
+  }
 }
 
 template <int D>
@@ -99,50 +186,66 @@ BlockGrid<D> block_grid(const tess_mesh& mesh) {
   return bg;
 }
 
+}  // namespace
+
+// The totals of an update whose kernels have run.
+void take_sparsity(tess_ctx* ctx, const tess_mesh& mesh, tess_sparsity& sp, int32_t* changed) {
+  const uint32_t* hc = reinterpret_cast<const uint32_t*>(ctx->counters_host);
+  sp.storage_len = int64_t(hc[SP_COUNT]) << (mesh.block_size_log2 * mesh.dim);
+  if (changed) *changed = hc[SP_CHANGED] ? 1 : 0;
+}
+
+namespace {
+
 template <typename T, int D>
 void sparsity_impl(tess_ctx* ctx, const tess_mesh& mesh, tess_field x, int64_t n, tess_sparsity& sp,
-                   int32_t* changed) {
+                   int32_t* changed, bool defer) {
   const BlockGrid<D> bg = block_grid<D>(mesh);
   const int L = mesh.block_size_log2;
   const int64_t nbt = bg.total;
   if (nbt >= (int64_t(1) << 31)) raise(TESS_ERR_UNSUPPORTED, "block table larger than 2^31 blocks");
-  uint32_t* occ = ctx->sp_occ.as<uint32_t>(size_t(nbt));
   uint32_t* act = ctx->sp_act.as<uint32_t>(size_t(nbt));
-  uint32_t* scan = ctx->sp_scan.as<uint32_t>(size_t(nbt));
-  uint32_t* counters = ctx->counters.as<uint32_t>(64);
-  TESS_HIP(hipMemsetAsync(occ, 0, size_t(nbt) * sizeof(uint32_t), ctx->stream));
-  TESS_HIP(hipMemsetAsync(counters + SP_COUNT, 0, 2 * sizeof(uint32_t), ctx->stream));
+  const int64_t wgs = ceil_div(nbt, int64_t(SP_THREADS));
+  uint2* sums = ctx->sp_sums.as<uint2>(size_t(wgs) + 1);
+  uint32_t* occ = static_cast<uint32_t*>(ctx->sp_occ.ptr);
+  if (ctx->sp_clean != nbt || !occ) {
+    // the first update of this many blocks, or one that was cut short
+    occ = ctx->sp_occ.as<uint32_t>(size_t(nbt));
+    TESS_HIP(hipMemsetAsync(occ, 0, size_t(nbt) * sizeof(uint32_t), ctx->stream));
+  }
+  ctx->sp_clean = -1;
   if (n > 0) {
     const DMesh<T, D> dm = dmesh<T, D>(mesh);
     hipLaunchKernelGGL((k_sp_occupied<T, D>), dim3(unsigned(ceil_div(n, 256))), dim3(256), 0, ctx->stream,
                        dfield<T>(x), n, dm, L, bg, occ);
     TESS_HIP(hipGetLastError());
   }
-  hipLaunchKernelGGL((k_sp_activity<D>), dim3(unsigned(ceil_div(nbt, 256))), dim3(256), 0, ctx->stream, occ, bg,
-                     static_cast<const int32_t*>(sp.blocknumbering), act, scan, counters + SP_CHANGED);
+  hipLaunchKernelGGL((k_sp_activity<D>), dim3(unsigned(wgs)), dim3(SP_THREADS), 0, ctx->stream, occ, bg,
+                     static_cast<const int32_t*>(sp.blocknumbering), act, sums);
   TESS_HIP(hipGetLastError());
-  exclusive_scan_u32(ctx, scan, nbt, counters + SP_COUNT);
-  hipLaunchKernelGGL(k_sp_number, dim3(unsigned(ceil_div(nbt, 256))), dim3(256), 0, ctx->stream, act, scan, nbt,
-                     sp.blocknumbering);
+  if (wgs > SUMS_DIRECT) {
+    hipLaunchKernelGGL(k_sp_prefix, dim3(1), dim3(64), 0, ctx->stream, sums, wgs);
+    TESS_HIP(hipGetLastError());
+  }
+  hipLaunchKernelGGL(k_sp_number, dim3(unsigned(wgs)), dim3(SP_THREADS), 0, ctx->stream, act, sums, nbt,
+                     sp.blocknumbering, occ, reinterpret_cast<uint32_t*>(ctx->counters_host));
   TESS_HIP(hipGetLastError());
-  uint32_t* hc = reinterpret_cast<uint32_t*>(ctx->counters_host);
-  TESS_HIP(hipMemcpyAsync(hc + SP_COUNT, counters + SP_COUNT, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                          ctx->stream));
+  ctx->sp_clean = nbt;
+  if (defer) return;
   TESS_HIP(hipStreamSynchronize(ctx->stream));
-  sp.storage_len = int64_t(hc[SP_COUNT]) << (L * D);
-  if (changed) *changed = hc[SP_CHANGED] ? 1 : 0;
+  take_sparsity(ctx, mesh, sp, changed);
 }
 
 }  // namespace
 
 void run_sparsity_update(tess_ctx* ctx, const tess_mesh& mesh, tess_field x, int64_t n, tess_sparsity& sp,
-                         int32_t* changed) {
+                         int32_t* changed, bool defer) {
   if (mesh.dtype == TESS_FLOAT32) {
-    if (mesh.dim == 2) sparsity_impl<float, 2>(ctx, mesh, x, n, sp, changed);
-    else sparsity_impl<float, 3>(ctx, mesh, x, n, sp, changed);
+    if (mesh.dim == 2) sparsity_impl<float, 2>(ctx, mesh, x, n, sp, changed, defer);
+    else sparsity_impl<float, 3>(ctx, mesh, x, n, sp, changed, defer);
   } else {
-    if (mesh.dim == 2) sparsity_impl<double, 2>(ctx, mesh, x, n, sp, changed);
-    else sparsity_impl<double, 3>(ctx, mesh, x, n, sp, changed);
+    if (mesh.dim == 2) sparsity_impl<double, 2>(ctx, mesh, x, n, sp, changed, defer);
+    else sparsity_impl<double, 3>(ctx, mesh, x, n, sp, changed, defer);
   }
 }
 

@@ -137,9 +137,9 @@ struct TabArgs {
   uint32_t* tin;   // ntiles + 1: arrivals (reset)
   int64_t ntiles;
   int32_t nt[3];
-  const int64_t* scene_toff;  // a batch: first tile and tiles per axis of each scene
+  const int64_t* scene_toff;  // a batch: first tile and tiles per axis of each scene, scene of each tile
   const int32_t* scene_nt;
-  int32_t nscenes;
+  const uint32_t* tile_scene;
   uint32_t* sums;  // 4 words per workgroup
   uint32_t *start, *end, *flag, *slot, *active, *nb_flag, *nb_list, *seg;
   uint32_t* lanes;
@@ -165,6 +165,7 @@ struct MergeArgs {
   const uint32_t* counters;  // device count of arrivals outside the mesh, or nullptr: out_in
   uint32_t out_in;
   int32_t pos_bits;
+  int32_t small_tiles;  // one wave per tile
 };
 
 }  // namespace tess
@@ -204,7 +205,11 @@ struct tess_ctx {
   // zeroing bookkeeping for the grid of the previous P2G
   const void* last_grid_m = nullptr;
   int64_t prev_nodeblocks = 0;
-  uint64_t prev_generation = 0;  // the binning nb_list_prev is of
+  // the binning of the last P2G, and where its node-block list is: in the
+  // current tables, in the alternate set they were swapped with, or copied out
+  // before that set was built again
+  uint64_t prev_generation = 0;
+  enum class PrevList { Current, Alternate, Copied } prev_list = PrevList::Copied;
   int32_t prev_tile_log2 = -1;
   int64_t prev_ntiles = -1;
   int64_t prev_nnodes = -1;
@@ -220,8 +225,10 @@ struct tess_ctx {
   int64_t broken_count = 0;
   // nodes with m > 0 written by the last gather (read back with the next binning)
   int64_t last_active_nodes = -1;
-  // SpGrid block activation scratch (occupied flags, active flags, scan)
-  tess::Buffer sp_occ, sp_act, sp_scan;
+  // SpGrid block activation scratch: occupied flags (all clear between updates
+  // of sp_clean blocks), active flags, per-workgroup counts
+  tess::Buffer sp_occ, sp_act, sp_sums;
+  int64_t sp_clean = -1;
   // adjoint: per-tile Float64 partials, node adjoints, rollout checkpoints and replay
   tess::Buffer adj_partials, adj_nodes, ro_checkpoints, ro_segment, ro_gradv, ro_snapshots;
   tess::Rollout rollout;
@@ -246,7 +253,7 @@ struct tess_batch {
   int64_t ntot = 0, tiles_total = 0, max_nodes = 0;
   std::vector<tess_scene> scenes;
   std::vector<int64_t> toff, poff;
-  tess::Buffer recs, d_toff, d_poff, d_nt, prev_list;
+  tess::Buffer recs, d_toff, d_poff, d_nt, d_tscene, prev_list;
   int64_t prev_nb = 0;
   bool zeroed = false;
   // the binning in the context is this batch's, and the last G2P wrote every
@@ -342,9 +349,12 @@ void run_reorder(tess_ctx* ctx, const tess_mesh& mesh, const tess_particles& P, 
 
 // ---- SpGrid block numbering (sparse.hip) ----
 // update_sparsity!(spinds, xₚ, mesh): writes sp.blocknumbering and
-// sp.storage_len, *changed (host, optional) = active set changed.  Synchronises.
+// sp.storage_len, *changed (host, optional) = active set changed.  Synchronises;
+// with defer it only enqueues, and the caller takes the totals (take_sparsity)
+// after a synchronisation of its own.
 void run_sparsity_update(tess_ctx* ctx, const tess_mesh& mesh, tess_field x, int64_t n, tess_sparsity& sp,
-                         int32_t* changed);
+                         int32_t* changed, bool defer = false);
+void take_sparsity(tess_ctx* ctx, const tess_mesh& mesh, tess_sparsity& sp, int32_t* changed);
 
 // ---- transfers (transfer.hip) ----
 void run_p2g(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,

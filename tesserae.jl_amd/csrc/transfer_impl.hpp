@@ -126,6 +126,9 @@ struct Args {
   const uint32_t* nb_list;
   const uint32_t* nb_flag;
   T* partials;
+  // node blocks the last call on the grid wrote (zeroed unless written again)
+  const uint32_t* stale_list;
+  int64_t n_stale;
   // when set, G2P also writes each particle's position before the update here
   // (dense, D per particle): the positions the P2G half of a @G2P2G pass reads
   T* x_keep;
@@ -139,6 +142,7 @@ struct Args {
   const SceneRec<T, D>* scenes;
   const int64_t* scene_toff;
   const int64_t* scene_poff;
+  const uint32_t* tile_scene;  // scene of each global tile
   int32_t nscenes;
   int64_t n, n_inside, n_active, n_nb;
   int32_t ntiles[D];
@@ -227,7 +231,7 @@ __device__ __forceinline__ uint32_t bind_tile(Args<T, D>& a, uint32_t gtile, uin
   if constexpr (!BATCH) {
     return gtile;
   } else {
-    const SceneRec<T, D>& r = bind_scene(a, scene_of(a.scene_toff, a.nscenes, gtile));
+    const SceneRec<T, D>& r = bind_scene(a, int(a.tile_scene[gtile]));
     poff = uint32_t(r.poff);
     return gtile - uint32_t(r.toff);
   }
@@ -289,7 +293,7 @@ __device__ __forceinline__ int64_t grid_slot(const Args<T, D>& a, const int* I) 
 template <typename T, int D, int SW>
 __device__ __forceinline__ void check_sparse_support(const Args<T, D>& a, const int* origin, const int* ccoord,
                                                      int ccount) {
-  if (a.numbering == nullptr || ccount == 0) return;
+  if (a.p2g_err == nullptr || ccount == 0) return;
   const int L = a.spL;
   int blo[D], ext[D], tot = 1;
 #pragma unroll
@@ -510,14 +514,11 @@ __global__ __launch_bounds__(256) void k_zero_grid_batch(Args<T, D> a) {
   if (i < r.nnodes) zero_node(a, i);
 }
 
-// Zero the nodes of node blocks touched last call but not this call.
+// Zero the nodes of node block B, touched by the last call, unless this call
+// touches it (one thread per node).
 template <typename T, int D, bool BATCH = false>
-__global__ __launch_bounds__(64) void k_zero_stale(Args<T, D> a, const uint32_t* __restrict__ prev_list,
-                                                    int64_t n_prev) {
+__device__ __forceinline__ void zero_stale_block(Args<T, D>& a, const uint32_t B) {
   using G = Geo<D>;
-  const int64_t j = blockIdx.x;
-  if (j >= n_prev) return;
-  const uint32_t B = prev_list[j];
   if (a.nb_flag[B]) return;
   uint32_t poff;
   const uint32_t Bl = bind_tile<BATCH>(a, B, poff);
@@ -532,6 +533,11 @@ __global__ __launch_bounds__(64) void k_zero_stale(Args<T, D> a, const uint32_t*
   }
   const int64_t i = grid_slot(a, I);
   if (i >= 0) zero_node(a, i);
+}
+template <typename T, int D, bool BATCH = false>
+__global__ __launch_bounds__(64) void k_zero_stale(Args<T, D> a, const uint32_t* __restrict__ prev_list,
+                                                    int64_t n_prev) {
+  if (int64_t(blockIdx.x) < n_prev) zero_stale_block<T, D, BATCH>(a, prev_list[blockIdx.x]);
 }
 
 template <typename T, int D, int BASIS>
@@ -2347,6 +2353,12 @@ __device__ __forceinline__ void k_gather_grid_body(Args<T, D>& a, uint32_t* __re
 
 template <typename T, int D, int SW, bool GAOS, bool BATCH = false>
 __global__ __launch_bounds__(64) void k_gather_grid(Args<T, D> a, uint32_t* __restrict__ lanes) {
+  // the workgroups past the node blocks zero the stale ones
+  const int64_t past = int64_t(blockIdx.x) - (((a.n_nb + 7) >> 3) << 3);
+  if (past >= 0) {
+    if (past < a.n_stale) zero_stale_block<T, D, BATCH>(a, a.stale_list[past]);
+    return;
+  }
   const int64_t j = item_of<BATCH>(blockIdx.x, a.n_nb);
   if (j < a.n_nb) k_gather_grid_body<T, D, SW, GAOS, BATCH>(a, lanes, j);
 }
@@ -2701,8 +2713,21 @@ inline TabArgs table_args(tess_ctx* ctx, int64_t ntiles) {
   return t;
 }
 
+// Builds the tables into the alternate set, whose node-block list the stale
+// zeroing may still need.
+inline void build_tables(tess_ctx* ctx, const TabArgs& t) {
+  if (ctx->prev_list == tess_ctx::PrevList::Alternate && ctx->prev_nodeblocks > 0) {
+    uint32_t* keep = ctx->nb_list_prev.as<uint32_t>(size_t(ctx->prev_nodeblocks));
+    TESS_HIP(hipMemcpyAsync(keep, ctx->alt_nb_list.ptr, size_t(ctx->prev_nodeblocks) * sizeof(uint32_t),
+                            hipMemcpyDeviceToDevice, ctx->stream));
+    ctx->prev_list = tess_ctx::PrevList::Copied;
+  }
+  launch_tables(ctx->stream, t);
+}
+
 // The alternate tables become the current ones.
 inline void swap_tables(tess_ctx* ctx) {
+  if (ctx->prev_list == tess_ctx::PrevList::Current) ctx->prev_list = tess_ctx::PrevList::Alternate;
   std::swap(ctx->tile_start, ctx->alt_start);
   std::swap(ctx->tile_end, ctx->alt_end);
   std::swap(ctx->tile_flag, ctx->alt_flag);
@@ -2750,6 +2775,7 @@ inline void merge_moves(tess_ctx* ctx, int64_t n, int64_t ntiles, int64_t old_ac
   g.perm_new = ctx->perm2.as<uint32_t>(m);
   g.out_in = hc[CNT_OUTIN];
   g.pos_bits = key_bits_for(uint64_t(m));
+  g.small_tiles = n < 256 * g.new_active_n;
   const int64_t outside = n - int64_t(hc[CNT_INSIDE]);
   launch_merge(ctx->stream, g, hc[CNT_ARRIVE] != 0,
                outside > 0 ? unsigned(std::min<int64_t>(blocks_for(n - old_inside, 256), 2048)) : 0u);
@@ -2866,7 +2892,7 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
         TESS_HIP(hipGetLastError());
       }
     }
-    launch_tables(ctx->stream, tab);
+    build_tables(ctx, tab);
     TESS_HIP(hipStreamSynchronize(ctx->stream));
     take_report(ctx);
     ctx->last_movers = int64_t(hc[CNT_MOVED]);
@@ -2901,7 +2927,7 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
     }
     ctx->last_movers = -1;
     launch_tile_counts(ctx->stream, skeys, n, int64_t(ntiles), tab.stay, tab.tin);
-    launch_tables(ctx->stream, tab);
+    build_tables(ctx, tab);
     TESS_HIP(hipStreamSynchronize(ctx->stream));
     take_report(ctx);
   }
@@ -2943,7 +2969,7 @@ using SweepFn = std::function<void(Args<T, D>&, const uint32_t*, uint32_t*)>;
 template <typename T, int D, int BASIS, bool STORED>
 void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const tess_particles& P,
                 const tess_weights* W, const tess_params& prm, bool count_misplaced, const tess_sparsity* sp,
-                const SweepFn<T, D>* sweep = nullptr) {
+                const SweepFn<T, D>* sweep = nullptr, bool fresh_numbering = false) {
   using Gm = Geo<D>;
   constexpr int NV = 1 + 2 * D;
   constexpr int SW = support_width(BASIS);
@@ -2962,7 +2988,11 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
   // An SpGrid's storage is zeroed whole (its numbering may have changed).
   const bool fresh = ctx->last_grid_m != G.m.ptr || ctx->prev_tile_log2 != Gm::LT ||
                      ctx->prev_ntiles != ctx->bin.ntiles || ctx->prev_nnodes != nnodes;
-  if (sp) {
+  // The numbering was built from these particles (fresh_numbering): with blocks
+  // of at least two nodes every class window lies within the activated blocks,
+  // and there is nothing to check.
+  const bool check = sp && !(fresh_numbering && mesh.block_size_log2 >= 1 && !TESS_DEBUG);
+  if (check) {
     a.p2g_err = counters + CNT_P2GERR;
     TESS_HIP(hipMemsetAsync(a.p2g_err, 0, sizeof(uint32_t), ctx->stream));
   }
@@ -2976,13 +3006,16 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
     } else if (fresh) {
       hipLaunchKernelGGL((k_zero_grid<T, D>), dim3(blocks_for(nnodes, 256)), dim3(256), 0, ctx->stream, a, nnodes);
       TESS_HIP(hipGetLastError());
-    } else if (ctx->prev_nodeblocks > 0 && ctx->prev_generation != ctx->bin.generation) {
-      // (a binning that kept its layout left no node block stale)
-      hipLaunchKernelGGL((k_zero_stale<T, D>), dim3(unsigned(ctx->prev_nodeblocks)), dim3(64), 0, ctx->stream, a,
-                         static_cast<const uint32_t*>(ctx->nb_list_prev.ptr), ctx->prev_nodeblocks);
-      TESS_HIP(hipGetLastError());
     }
   };
+  // stale node blocks are zeroed by the gather's launch (a binning that kept
+  // its layout left none)
+  const bool stale = !sp && !fresh && ctx->prev_nodeblocks > 0 && ctx->prev_generation != ctx->bin.generation;
+  if (stale) {
+    a.stale_list = static_cast<const uint32_t*>(ctx->prev_list == tess_ctx::PrevList::Alternate ? ctx->alt_nb_list.ptr
+                                                                                                : ctx->nb_list_prev.ptr);
+    a.n_stale = ctx->prev_nodeblocks;
+  }
   if (!sweep) zero_grid();
   const Binning& b = ctx->bin;
   // broken pairs and nodes with mass are counted into the lanes, which the next
@@ -3047,32 +3080,28 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
     prof_end(ctx, tok);
   }
   if (sweep) zero_grid();
-  if (b.n_nodeblocks > 0) {
+  if (b.n_nodeblocks > 0 || a.n_stale > 0) {
     // algorithmic bytes per active node: m, mv, f written, read back by the
     // grid-node half, vⁿ and v written (the node count of the previous call)
     const double nodes = double(std::max<int64_t>(ctx->last_active_nodes, 0));
     const int tok = prof_begin(ctx, "k_gather_grid", nodes * sizeof(T) * (2 * (2 * D + 1) + 2 * D));
+    const dim3 grid(xcd_grid(b.n_nodeblocks) + unsigned(a.n_stale));
     if (grid_julia_layout(G, D))
-      hipLaunchKernelGGL((k_gather_grid<T, D, SW, true>), dim3(xcd_grid(b.n_nodeblocks)), dim3(64), 0, ctx->stream, a,
-                         lanes);
+      hipLaunchKernelGGL((k_gather_grid<T, D, SW, true>), grid, dim3(64), 0, ctx->stream, a, lanes);
     else
-      hipLaunchKernelGGL((k_gather_grid<T, D, SW, false>), dim3(xcd_grid(b.n_nodeblocks)), dim3(64), 0, ctx->stream, a,
-                         lanes);
+      hipLaunchKernelGGL((k_gather_grid<T, D, SW, false>), grid, dim3(64), 0, ctx->stream, a, lanes);
     TESS_HIP(hipGetLastError());
     prof_end(ctx, tok);
   }
-  // remember this call's node blocks for the next call's stale zeroing
-  uint32_t* prev = ctx->nb_list_prev.as<uint32_t>(size_t(std::max<int64_t>(b.ntiles, 1)));
-  if (b.n_nodeblocks > 0 && ctx->prev_generation != b.generation)
-    TESS_HIP(hipMemcpyAsync(prev, ctx->nb_list.ptr, size_t(b.n_nodeblocks) * sizeof(uint32_t),
-                            hipMemcpyDeviceToDevice, ctx->stream));
+  // this call's node blocks are what the next call's stale zeroing looks at
   ctx->prev_nodeblocks = b.n_nodeblocks;
   ctx->prev_generation = b.generation;
+  ctx->prev_list = tess_ctx::PrevList::Current;
   ctx->last_grid_m = sp ? nullptr : G.m.ptr;  // a dense grid after an SpGrid call starts from a full zero
   ctx->prev_tile_log2 = Gm::LT;
   ctx->prev_ntiles = b.ntiles;
   ctx->prev_nnodes = nnodes;
-  if (sp) {
+  if (check) {
     uint32_t* hc = reinterpret_cast<uint32_t*>(ctx->counters_host);
     TESS_HIP(hipMemcpyAsync(hc + CNT_P2GERR, counters + CNT_P2GERR, sizeof(uint32_t), hipMemcpyDeviceToHost,
                             ctx->stream));
@@ -3521,15 +3550,19 @@ void step_impl(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const t
       if (done) *done = s;
       if (hook) (*hook)(0, s);
       if (sp) {
-        // update_sparsity!(grid, xₚ) at the top of the SpGrid loop (src/Grids/grid.jl:97-101)
-        run_sparsity_update(ctx, mesh, mp.now().x, P.n, *sp, nullptr);
-        if (sp->storage_len > sp->capacity)
-          raise(TESS_ERR_STATE, "SpGrid storage holds " + std::to_string(sp->capacity) + " nodes but the active blocks need " +
-                                    std::to_string(sp->storage_len) + "; resize the grid arrays and call again");
+        // update_sparsity!(grid, xₚ) at the top of the SpGrid loop (src/Grids/grid.jl:97-101);
+        // the binning's readback brings its totals too
+        run_sparsity_update(ctx, mesh, mp.now().x, P.n, *sp, nullptr, true);
       }
       // from the second step on, the previous G2P wrote the keys (same call, so
       // nothing else moved the particles in between)
       bin_particles<T, D, BASIS, false>(ctx, mesh, mp.now(), nullptr, s > 0);
+      if (sp) {
+        take_sparsity(ctx, mesh, *sp, nullptr);
+        if (sp->storage_len > sp->capacity)
+          raise(TESS_ERR_STATE, "SpGrid storage holds " + std::to_string(sp->capacity) + " nodes but the active blocks need " +
+                                    std::to_string(sp->storage_len) + "; resize the grid arrays and call again");
+      }
       const uint32_t* dest = nullptr;
       if (reorder_wanted(ctx, reorder_threshold)) {
         if (mp.can_move()) dest = layered_maps<T, D>(ctx, mesh, mp.now());
@@ -3538,7 +3571,8 @@ void step_impl(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const t
       }
       // (P2G reads the particles where they are; in the layered order that its
       // G2P gives them no neighbour pair is broken)
-      p2g_launch<T, D, BASIS, false>(ctx, mesh, G, mp.now(), nullptr, prm, reorder_threshold > 0.0 && !dest, sp);
+      p2g_launch<T, D, BASIS, false>(ctx, mesh, G, mp.now(), nullptr, prm, reorder_threshold > 0.0 && !dest, sp, nullptr,
+                                        sp != nullptr);
       if (dest) {
         ctx->misplaced_x_ptr = mp.now().x.ptr;
         ctx->misplaced_n = P.n;
