@@ -571,9 +571,9 @@ void batch_graph_step(tess_ctx* g, tess_batch& B, bool full, int in) {
   uint32_t* prev_list = B.g_prev_list.as<uint32_t>(ntiles);
   uint32_t* prev_count = B.g_prev_count.as<uint32_t>(64);
   T* partials = g->partials.as<T>(size_t(ntiles) * Part<D, SW>::SIZE);
-  // the scans' work area at its largest use (the sort's histograms, the
-  // reorder's ranks), so no later call moves it
-  g->scan_tmp.get(std::max(scan_work_bytes(n + 1), scan_work_bytes(int64_t(sort_hist_words(std::max<int64_t>(n, 1))))));
+  // the scans' work area at its largest use (the reorder's ranks), so no later
+  // call moves it
+  g->scan_tmp.get(scan_work_bytes(n + 1));
   uint32_t* skeys = cur.keys;
   const uint32_t* nblist = cur.nb_list;
   Args<T, D> a = batch_args<T, D>(g, B);

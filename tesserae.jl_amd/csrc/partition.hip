@@ -385,23 +385,18 @@ void partition_typed(tess_ctx* ctx, const tess_mesh& mesh, tess_field x, int64_t
 //
 // tess_partition_update_noalloc runs the partition above over a fixed work area
 // instead of the context's growing buffers: keys, sorted keys, values, the sort's
-// ping-pong keys and values (n words each), the digit histograms, the scan's
-// block sums and one count.  The area is a file-scope device array sized for
-// kNoAllocMaxParticles; every GPU that loads the library holds its own copy
-// until the process ends.  Calls on one GPU share it: calls that overlap on a
-// device race.
+// ping-pong keys and values (n words each), the digit histograms and one count.
+// The area is a file-scope device array sized for kNoAllocMaxParticles; every GPU
+// that loads the library holds its own copy until the process ends.  Calls on one
+// GPU share it: calls that overlap on a device race.
 
 constexpr int64_t kNoAllocMaxParticles = TESS_PARTITION_NOALLOC_MAX;
-static_assert(kNoAllocMaxParticles % 4096 == 0, "the histogram area counts whole 4096-key sort chunks");
 constexpr size_t kAlign = 256;
 constexpr size_t align_up(size_t b) { return (b + kAlign - 1) / kAlign * kAlign; }
 constexpr size_t kNoAllocWords = size_t(kNoAllocMaxParticles) * sizeof(uint32_t);
-// 4096-key sort chunks × 256 digits; the scan of those words has 16 blocks of 4096
-constexpr size_t kNoAllocHistBytes = size_t(kNoAllocMaxParticles / 4096) * 256 * sizeof(uint32_t);
-constexpr size_t kNoAllocScanBytes = 4096;
-static_assert(kNoAllocMaxParticles / 4096 * 256 <= 4096 * 4096, "the histogram scan takes two levels");
-constexpr size_t kNoAllocScratchBytes = 5 * align_up(kNoAllocWords) + align_up(kNoAllocHistBytes) + kNoAllocScanBytes +
-                                        kAlign;
+// 2048-key sort chunks and one row of totals × 1024 digits
+constexpr size_t kNoAllocHistBytes = (size_t(kNoAllocMaxParticles / 2048) + 2) * 1024 * sizeof(uint32_t);
+constexpr size_t kNoAllocScratchBytes = 5 * align_up(kNoAllocWords) + align_up(kNoAllocHistBytes) + kAlign;
 
 static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 
@@ -431,7 +426,7 @@ void partition_noalloc_typed(const tess_mesh& mesh, tess_field x, int64_t n, int
   const uint64_t outside = (uint64_t(1) << D) * nbt;
   if (outside >= uint64_t(UINT32_MAX) || n >= int64_t(INT32_MAX))
     raise(TESS_ERR_ARGUMENT, "Partition block count exceeds packed block id capacity.");
-  // carve the area: five n-word arrays, histograms, scan block sums, the count
+  // carve the area: five n-word arrays, histograms, the count
   uint8_t* q = area;
   auto take = [&](size_t bytes) {
     uint8_t* r = q;
@@ -445,8 +440,9 @@ void partition_noalloc_typed(const tess_mesh& mesh, tess_field x, int64_t n, int
   w.stream = stream;
   w.keys_alt = reinterpret_cast<uint32_t*>(take(kNoAllocWords));
   w.vals_alt = reinterpret_cast<uint32_t*>(take(kNoAllocWords));
+  if (sort_hist_words(n) * sizeof(uint32_t) > kNoAllocHistBytes)
+    raise(TESS_ERR_STATE, "the sort's histograms exceed the fixed work area");
   w.hist = reinterpret_cast<uint32_t*>(take(kNoAllocHistBytes));
-  w.scan_tmp = take(kNoAllocScanBytes);
   uint32_t* cnt = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t)));
   // fill kernels rather than memset nodes, so that a captured graph replays them
   hipLaunchKernelGGL(k_fill_i32, dim3(nblk(int64_t(nbt), 256)), dim3(256), 0, stream, starts, int64_t(nbt), 0);

@@ -2,14 +2,27 @@
 // uint32) used for particle binning.  Integer-only, so results are
 // deterministic; ranking inside a workgroup is stable (index order).
 //
-// Sort pass structure (one 8-bit digit per pass):
-//   1. k_radix_hist   per-workgroup digit histogram of a 4096-key chunk,
-//                     stored digit-major: hist[digit * nchunks + chunk]
-//   2. exclusive scan of hist -> global output offset of each (digit, chunk)
-//   3. k_radix_scatter re-reads the chunk in index order, ranks each key among
-//                     equal digits (wave match via ballots + per-wave counts),
-//                     and writes (key, value) to offset + rank.
+// Sort pass structure (one digit of 8 to 10 bits per pass):
+//   1. k_radix_hist   per-workgroup digit histogram of a chunk, stored
+//                     digit-major: hist[digit * nchunks + chunk]
+//   2. k_radix_rows   one workgroup per digit: exclusive scan of its row, and
+//                     its total
+//   3. k_radix_scatter re-reads the chunk, each wave a consecutive part of it,
+//                     ranks each key among equal digits (wave match via
+//                     ballots and running counts per wave, no barrier between
+//                     rounds), and writes (key, value) to offset + rank.
+//
+// What bounds it: at a million particles the launches and the few hundred
+// workgroups, each a serial chain of rounds; at ten million the scattered
+// writes of 4 bytes.  1.67 M particles with 20-bit keys, unsorted: a pass took
+// 12 us for the histogram, 14 us for a scan of three launches and 22 us with
+// four barriers per 256 keys, and there were three; now there are two of 12 + 5
+// + 31 us (10-bit digits scatter wider), and the block partition that they
+// serve takes 139 us instead of 188.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <type_traits>
 
 #include "tess_internal.hpp"
 
@@ -20,12 +33,22 @@ constexpr int SCAN_THREADS = 256;
 constexpr int SCAN_ITEMS = 16;
 constexpr int SCAN_CHUNK = SCAN_THREADS * SCAN_ITEMS;  // 4096
 
-constexpr int RADIX_BITS = 8;
-constexpr int RADIX = 1 << RADIX_BITS;
+constexpr int RADIX_BITS_MAX = 10;
 constexpr int SORT_THREADS = 256;
 constexpr int SORT_WAVES = SORT_THREADS / 64;
-constexpr int SORT_ROUNDS = 16;
-constexpr int SORT_CHUNK = SORT_THREADS * SORT_ROUNDS;  // 4096
+// Keys per thread: 16 fill the chip from 4 M keys on (1024 chunks); below, 8.
+constexpr int SORT_ROUNDS_LARGE = 16, SORT_ROUNDS_SMALL = 8;
+constexpr int64_t SORT_LARGE = int64_t(4) << 20;
+inline int64_t sort_chunk(int64_t n) {
+  return int64_t(SORT_THREADS) * (n >= SORT_LARGE ? SORT_ROUNDS_LARGE : SORT_ROUNDS_SMALL);
+}
+// Digit bits: as few passes as 10-bit digits give, of equal width.
+inline int sort_passes(int key_bits) { return key_bits <= 0 ? 1 : (key_bits + RADIX_BITS_MAX - 1) / RADIX_BITS_MAX; }
+inline int sort_digit_bits(int key_bits) {
+  const int p = sort_passes(key_bits);
+  const int b = (key_bits + p - 1) / p;
+  return b < 8 ? 8 : b;
+}
 
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
   const int lane = threadIdx.x & 63;
@@ -115,11 +138,12 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
   return (uint64_t(1) << lane) - 1;
 }
 
-// Lanes of the wave whose 8-bit digit equals this lane's (among `valid` lanes).
+// Lanes of the wave whose digit equals this lane's (among `valid` lanes).
+template <int RB>
 __device__ __forceinline__ uint64_t match_digit(uint32_t digit, bool valid) {
   uint64_t peers = __ballot(valid);
 #pragma unroll
-  for (int b = 0; b < RADIX_BITS; ++b) {
+  for (int b = 0; b < RB; ++b) {
     const bool bit = (digit >> b) & 1u;
     const uint64_t m = __ballot(valid && bit);
     peers &= bit ? m : ~m;
@@ -129,70 +153,141 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t digit, bool valid) {
 
 // n_dev (when set): the element count read on the device, at most n; chunks
 // past it hold an empty histogram.
+template <int RB, int ROUNDS>
 __global__ __launch_bounds__(SORT_THREADS) void k_radix_hist(const uint32_t* __restrict__ keys, int64_t n, int shift,
                                                               uint32_t* __restrict__ hist, int64_t nchunks,
                                                               const uint32_t* __restrict__ n_dev) {
+  constexpr int RADIX = 1 << RB;
   __shared__ uint32_t s_hist[RADIX];
   if (n_dev) n = int64_t(*n_dev);
-  const int64_t base = int64_t(blockIdx.x) * SORT_CHUNK;
-  if (base >= n) {
-    hist[int64_t(threadIdx.x) * nchunks + blockIdx.x] = 0u;
-    return;
+  const int64_t base = int64_t(blockIdx.x) * (SORT_THREADS * ROUNDS);
+  uint32_t k[ROUNDS];
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    const int64_t i = base + r * SORT_THREADS + threadIdx.x;
+    k[r] = i < n ? keys[i] : 0u;
   }
-  s_hist[threadIdx.x] = 0;
+  for (int d = int(threadIdx.x); d < RADIX; d += SORT_THREADS) s_hist[d] = 0;
   __syncthreads();
-#pragma unroll 4
-  for (int r = 0; r < SORT_ROUNDS; ++r) {
-    const int64_t i = base + int64_t(r) * SORT_THREADS + threadIdx.x;
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    const int64_t i = base + r * SORT_THREADS + threadIdx.x;
     const bool valid = i < n;
-    const uint32_t digit = valid ? (keys[i] >> shift) & (RADIX - 1) : 0u;
-    const uint64_t peers = match_digit(digit, valid);
-    if (valid && (peers & lanemask_lt()) == 0) atomicAdd(&s_hist[digit], uint32_t(__popcll(peers)));
+    // integer adds, whose order does not matter; a wave whose keys share one
+    // digit (nearly sorted input) adds once
+    const uint32_t digit = (k[r] >> shift) & (RADIX - 1);
+    const uint64_t live = __ballot(valid);
+    if (live == 0) continue;
+    const uint32_t d0 = uint32_t(__shfl(int(digit), __ffsll((unsigned long long)live) - 1, 64));
+    if (__ballot(valid && digit != d0) == 0) {
+      if ((threadIdx.x & 63) == 0) atomicAdd(&s_hist[d0], uint32_t(__popcll(live)));
+    } else if (valid) {
+      atomicAdd(&s_hist[digit], 1u);
+    }
   }
   __syncthreads();
-  hist[int64_t(threadIdx.x) * nchunks + blockIdx.x] = s_hist[threadIdx.x];
+  for (int d = int(threadIdx.x); d < RADIX; d += SORT_THREADS) hist[int64_t(d) * nchunks + blockIdx.x] = s_hist[d];
 }
 
+// Exclusive scan of each digit's row of chunk counts in place; the row total
+// goes to totals[digit].
+__global__ __launch_bounds__(SORT_THREADS) void k_radix_rows(uint32_t* __restrict__ hist, int64_t nchunks,
+                                                              uint32_t* __restrict__ totals) {
+  __shared__ uint32_t s_wave[SORT_THREADS / 64];
+  uint32_t* row = hist + int64_t(blockIdx.x) * nchunks;
+  uint32_t carry = 0;
+  for (int64_t c0 = 0; c0 < nchunks; c0 += SORT_THREADS) {
+    const int64_t c = c0 + threadIdx.x;
+    const uint32_t v = c < nchunks ? row[c] : 0u;
+    uint32_t total;
+    const uint32_t e = block_exclusive_scan(v, total, s_wave);
+    if (c < nchunks) row[c] = carry + e;
+    carry += total;
+  }
+  if (threadIdx.x == 0) totals[blockIdx.x] = carry;
+}
+
+template <int RB, int ROUNDS>
 __global__ __launch_bounds__(SORT_THREADS) void k_radix_scatter(const uint32_t* __restrict__ keys_in,
                                                                  const uint32_t* __restrict__ vals_in,
                                                                  uint32_t* __restrict__ keys_out,
                                                                  uint32_t* __restrict__ vals_out, int64_t n,
-                                                                 int shift, const uint32_t* __restrict__ offsets,
+                                                                 int shift, const uint32_t* __restrict__ rows,
+                                                                 const uint32_t* __restrict__ totals,
                                                                  int64_t nchunks, const uint32_t* __restrict__ n_dev) {
-  __shared__ uint32_t s_base[RADIX];
-  __shared__ uint32_t s_wcount[SORT_WAVES][RADIX];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int RADIX = 1 << RB, PER = RADIX / SORT_THREADS;
+  __shared__ uint32_t s_cnt[SORT_WAVES][RADIX];
+  __shared__ uint32_t s_wave[SORT_THREADS / 64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   if (n_dev) n = int64_t(*n_dev);
-  const int64_t base = int64_t(blockIdx.x) * SORT_CHUNK;
+  const int64_t base = int64_t(blockIdx.x) * (SORT_THREADS * ROUNDS);
   if (base >= n) return;  // uniform
-  s_base[threadIdx.x] = offsets[int64_t(threadIdx.x) * nchunks + blockIdx.x];
-  for (int r = 0; r < SORT_ROUNDS; ++r) {
-    const int64_t i = base + int64_t(r) * SORT_THREADS + threadIdx.x;
-    const bool valid = i < n;
-    const uint32_t key = valid ? keys_in[i] : 0u;
-    const uint32_t val = valid ? (vals_in ? vals_in[i] : uint32_t(i)) : 0u;
-    const uint32_t digit = (key >> shift) & (RADIX - 1);
+  // wave w takes the keys [w*64*ROUNDS, (w+1)*64*ROUNDS) of the chunk in order
+  const int64_t first = base + int64_t(wave) * (64 * ROUNDS) + lane;
+  uint32_t k[ROUNDS], v[ROUNDS], rank[ROUNDS];
 #pragma unroll
-    for (int w = 0; w < SORT_WAVES; ++w) s_wcount[w][threadIdx.x] = 0;
-    __syncthreads();
-    const uint64_t peers = match_digit(digit, valid);
-    const uint32_t below = uint32_t(__popcll(peers & lanemask_lt()));
-    if (valid && below == 0) s_wcount[wave][digit] = uint32_t(__popcll(peers));
-    __syncthreads();
-    if (valid) {
-      uint32_t pos = s_base[digit] + below;
-      for (int w = 0; w < wave; ++w) pos += s_wcount[w][digit];
-      keys_out[pos] = key;
-      vals_out[pos] = val;
-    }
-    __syncthreads();
-    uint32_t add = 0;
-#pragma unroll
-    for (int w = 0; w < SORT_WAVES; ++w) add += s_wcount[w][threadIdx.x];
-    s_base[threadIdx.x] += add;
-    __syncthreads();
+  for (int r = 0; r < ROUNDS; ++r) {
+    const int64_t i = first + r * 64;
+    k[r] = i < n ? keys_in[i] : 0u;
+    v[r] = i < n ? (vals_in ? vals_in[i] : uint32_t(i)) : 0u;
   }
-  (void)lane;
+  // each thread's digits: where the chunk's keys of a digit go
+  uint32_t dbase[PER], tot = 0;
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    dbase[q] = totals[int(threadIdx.x) * PER + q];
+    tot += dbase[q];
+  }
+#pragma unroll
+  for (int w = 0; w < SORT_WAVES; ++w)
+    for (int d = int(threadIdx.x); d < RADIX; d += SORT_THREADS) s_cnt[w][d] = 0;
+  uint32_t all;
+  uint32_t run = block_exclusive_scan(tot, all, s_wave);  // barriers after the clearing
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    const uint32_t t = dbase[q];
+    dbase[q] = run + rows[int64_t(int(threadIdx.x) * PER + q) * nchunks + blockIdx.x];
+    run += t;
+  }
+  // ranks within the wave, in order (the LDS executes one wave's accesses in order)
+  uint32_t* mine = s_cnt[wave];
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    const bool valid = first + r * 64 < n;
+    const uint32_t digit = (k[r] >> shift) & (RADIX - 1);
+    const uint64_t peers = match_digit<RB>(digit, valid);
+    const uint32_t below = uint32_t(__popcll(peers & lanemask_lt()));
+    uint32_t b = 0;
+    if (valid && below == 0) {
+      b = mine[digit];
+      mine[digit] = b + uint32_t(__popcll(peers));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the next round's counts after this one's
+    rank[r] = uint32_t(__shfl(int(b), valid ? __ffsll((unsigned long long)peers) - 1 : lane, 64)) + below;
+  }
+  __syncthreads();
+  // counts -> where each (digit, wave) starts
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    const int d = int(threadIdx.x) * PER + q;
+    uint32_t at = dbase[q];
+#pragma unroll
+    for (int w = 0; w < SORT_WAVES; ++w) {
+      const uint32_t c = s_cnt[w][d];
+      s_cnt[w][d] = at;
+      at += c;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    if (first + r * 64 < n) {
+      const uint32_t pos = mine[(k[r] >> shift) & (RADIX - 1)] + rank[r];
+      keys_out[pos] = k[r];
+      vals_out[pos] = v[r];
+    }
+  }
 }
 
 // *out += sum of v[0..n): grid-stride partial sums, one atomic add per
@@ -297,14 +392,34 @@ void exclusive_scan_u32(tess_ctx* ctx, uint32_t* data, int64_t n, uint32_t* tota
   exclusive_scan_u32_ws(ctx->stream, tmp, data, n, total_dev);
 }
 
-size_t sort_hist_words(int64_t n) { return size_t(ceil_div(n, SORT_CHUNK)) * RADIX; }
+size_t sort_hist_words(int64_t n) {
+  // a row of chunk counts and a total for each digit of the widest kind
+  return (size_t(ceil_div(n, sort_chunk(n))) + 1) << RADIX_BITS_MAX;
+}
+
+namespace {
+template <int RB, int ROUNDS>
+void sort_pass(const SortWork& w, const uint32_t* kin, const uint32_t* vin, uint32_t* kout, uint32_t* vout, int64_t n,
+               int shift, int64_t nchunks, const uint32_t* n_dev) {
+  uint32_t* totals = w.hist + (nchunks << RB);
+  hipLaunchKernelGGL((k_radix_hist<RB, ROUNDS>), dim3(unsigned(nchunks)), dim3(SORT_THREADS), 0, w.stream, kin, n, shift,
+                     w.hist, nchunks, n_dev);
+  TESS_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_radix_rows, dim3(1u << RB), dim3(SORT_THREADS), 0, w.stream, w.hist, nchunks, totals);
+  TESS_HIP(hipGetLastError());
+  hipLaunchKernelGGL((k_radix_scatter<RB, ROUNDS>), dim3(unsigned(nchunks)), dim3(SORT_THREADS), 0, w.stream, kin, vin,
+                     kout, vout, n, shift, w.hist, totals, nchunks, n_dev);
+  TESS_HIP(hipGetLastError());
+}
+}  // namespace
 
 void radix_sort_pairs_ws(const SortWork& w, const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out,
                          uint32_t* vals_out, int64_t n, int key_bits, const uint32_t* n_dev) {
   if (n <= 0) return;
   if (n > int64_t(UINT32_MAX)) raise(TESS_ERR_ARGUMENT, "radix sort: more than 2^32-1 elements");
-  const int passes = key_bits <= 0 ? 1 : (key_bits + RADIX_BITS - 1) / RADIX_BITS;
-  const int64_t nchunks = ceil_div(n, SORT_CHUNK);
+  const int passes = sort_passes(key_bits), bits = sort_digit_bits(key_bits);
+  const int64_t nchunks = ceil_div(n, sort_chunk(n));
+  const bool large = n >= SORT_LARGE;
   // ping-pong so that the last pass writes (keys_out, vals_out)
   const uint32_t* kin = keys_in;
   const uint32_t* vin = vals_in;
@@ -312,14 +427,14 @@ void radix_sort_pairs_ws(const SortWork& w, const uint32_t* keys_in, const uint3
     const bool to_out = ((passes - 1 - p) % 2) == 0;
     uint32_t* kout = to_out ? keys_out : w.keys_alt;
     uint32_t* vout = to_out ? vals_out : w.vals_alt;
-    const int shift = p * RADIX_BITS;
-    hipLaunchKernelGGL(k_radix_hist, dim3(unsigned(nchunks)), dim3(SORT_THREADS), 0, w.stream, kin, n, shift,
-                       w.hist, nchunks, n_dev);
-    TESS_HIP(hipGetLastError());
-    exclusive_scan_u32_ws(w.stream, w.scan_tmp, w.hist, nchunks * RADIX, nullptr);
-    hipLaunchKernelGGL(k_radix_scatter, dim3(unsigned(nchunks)), dim3(SORT_THREADS), 0, w.stream, kin, vin, kout,
-                       vout, n, shift, w.hist, nchunks, n_dev);
-    TESS_HIP(hipGetLastError());
+    auto run = [&](auto rb) {
+      constexpr int RB = decltype(rb)::value;
+      if (large) sort_pass<RB, SORT_ROUNDS_LARGE>(w, kin, vin, kout, vout, n, p * bits, nchunks, n_dev);
+      else sort_pass<RB, SORT_ROUNDS_SMALL>(w, kin, vin, kout, vout, n, p * bits, nchunks, n_dev);
+    };
+    if (bits == 8) run(std::integral_constant<int, 8>{});
+    else if (bits == 9) run(std::integral_constant<int, 9>{});
+    else run(std::integral_constant<int, 10>{});
     kin = kout;
     vin = vout;
   }
@@ -331,12 +446,9 @@ void radix_sort_pairs(tess_ctx* ctx, const uint32_t* keys_in, const uint32_t* va
   if (n > int64_t(UINT32_MAX)) raise(TESS_ERR_ARGUMENT, "radix sort: more than 2^32-1 elements");
   SortWork w;
   w.stream = ctx->stream;
-  const size_t hw = sort_hist_words(n);
-  w.hist = ctx->hist.as<uint32_t>(hw);
+  w.hist = ctx->hist.as<uint32_t>(sort_hist_words(n));
   w.keys_alt = ctx->keys_alt.as<uint32_t>(size_t(n));
   w.vals_alt = ctx->vals_alt.as<uint32_t>(size_t(n));
-  w.scan_tmp = ceil_div(int64_t(hw), SCAN_CHUNK) > 1 ? static_cast<uint8_t*>(ctx->scan_tmp.get(scan_work_bytes(int64_t(hw))))
-                                                      : nullptr;
   radix_sort_pairs_ws(w, keys_in, vals_in, keys_out, vals_out, n, key_bits, n_dev);
 }
 

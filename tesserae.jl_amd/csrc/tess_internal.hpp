@@ -311,14 +311,12 @@ void sum_u32(tess_ctx* ctx, const uint32_t* v, int64_t n, uint32_t* out);
 void radix_sort_pairs(tess_ctx* ctx, const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out,
                       uint32_t* vals_out, int64_t n, int key_bits, const uint32_t* n_dev = nullptr);
 // The same sort over caller-provided work buffers on a stream (no allocation):
-// hist holds sort_hist_words(n) words, keys_alt/vals_alt n words each, scan_tmp
-// scan_work_bytes(sort_hist_words(n)) bytes.
+// hist holds sort_hist_words(n) words, keys_alt/vals_alt n words each.
 struct SortWork {
   hipStream_t stream = nullptr;
   uint32_t* hist = nullptr;
   uint32_t* keys_alt = nullptr;
   uint32_t* vals_alt = nullptr;
-  uint8_t* scan_tmp = nullptr;
 };
 size_t sort_hist_words(int64_t n);
 size_t scan_work_bytes(int64_t n);
