@@ -483,7 +483,7 @@ __global__ __launch_bounds__(256) void k_g2p_outside_persist(Args<T, D> a, const
     }
 #pragma unroll
     for (int k = 0; k < D * D; ++k) L[k] = T(0);
-    particle_update<T, D>(a, pid, pid, dv, L, dx);
+    particle_update<T, D>(a, ParticleIn<T, D>(a, pid), pid, pid, dv, L, dx);
   }
 }
 

@@ -34,6 +34,7 @@ struct WArgs {
   uint32_t* err;
   int32_t corr;            // corrected basis bits (CORR kernels)
   const uint8_t* filter;   // node filter of update!(..., filter), NULL = Trues
+  int32_t rows;            // w and ∇w in the Julia layout: a particle's weights are contiguous
 };
 
 // Per particle: support window, then either the full-support polynomial fill
@@ -118,36 +119,50 @@ __global__ __launch_bounds__(256) void k_update_weights(WArgs<T, D> a) {
       cs.prepare(a.corr, BASIS, true, a.filter, a.mesh.dims, lo, cnt, xin, val, der);
     }
   }
+  // one row of the window at a time; a whole window in the Julia layout is
+  // stored in 16-byte words (a lane's weights lie apart from its neighbours', and
+  // each store instruction costs a request per lane: 168k particles, 2D Float64
+  // quadratic, 29 us scalar by scalar, 19 us so)
+  const bool rows = whole && a.rows;
 #pragma unroll
-  for (int o = 0; o < IPow<SW, D>::v; ++o) {
-    int aa[D], r = o;
-    bool ok = true;
+  for (int o0 = 0; o0 < IPow<SW, D>::v; o0 += SW) {
+    T w[SW], g[SW][D];
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-      aa[d] = r % SW;
-      r /= SW;
-      ok = ok && aa[d] <= hi[d] - lo[d];
+    for (int i = 0; i < SW; ++i) {
+      int aa[D], r = o0 + i;
+      bool ok = true;
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        aa[d] = r % SW;
+        r /= SW;
+        ok = ok && aa[d] <= hi[d] - lo[d];
+      }
+      if (!ok) continue;
+      if (CORR && cs.mode == CORR_GENERAL) {
+        cs.node(val, aa, filter_pass<D>(a.filter, a.mesh.dims, lo, aa), hinv, w[i], g[i]);
+      } else {
+        w[i] = val[0][aa[0]];
+#pragma unroll
+        for (int d = 1; d < D; ++d) w[i] = w[i] * val[d][aa[d]];
+#pragma unroll
+        for (int c = 0; c < D; ++c) {
+          T gc = (c == 0) ? der[0][aa[0]] : val[0][aa[0]];
+#pragma unroll
+          for (int d = 1; d < D; ++d) gc = gc * ((d == c) ? der[d][aa[d]] : val[d][aa[d]]);
+          g[i][c] = gc * hinv;
+        }
+      }
+      if (!rows) {
+        const int64_t e = int64_t(o0 + i) + int64_t(IPow<SW, D>::v) * p;
+        a.w(e) = w[i];
+#pragma unroll
+        for (int c = 0; c < D; ++c) a.gw(e, c) = g[i][c];
+      }
     }
-    if (!ok) continue;
-    const int64_t e = int64_t(o) + int64_t(IPow<SW, D>::v) * p;
-    if (CORR && cs.mode == CORR_GENERAL) {
-      T w, g[D];
-      cs.node(val, aa, filter_pass<D>(a.filter, a.mesh.dims, lo, aa), hinv, w, g);
-      a.w(e) = w;
-#pragma unroll
-      for (int c = 0; c < D; ++c) a.gw(e, c) = g[c];
-      continue;
-    }
-    T w = val[0][aa[0]];
-#pragma unroll
-    for (int d = 1; d < D; ++d) w = w * val[d][aa[d]];
-    a.w(e) = w;
-#pragma unroll
-    for (int c = 0; c < D; ++c) {
-      T g = (c == 0) ? der[0][aa[0]] : val[0][aa[0]];
-#pragma unroll
-      for (int d = 1; d < D; ++d) g = g * ((d == c) ? der[d][aa[d]] : val[d][aa[d]]);
-      a.gw(e, c) = g * hinv;
+    if (rows) {
+      const int64_t e = int64_t(o0) + int64_t(IPow<SW, D>::v) * p;
+      __builtin_memcpy(a.w.p + e, w, sizeof(w));
+      __builtin_memcpy(a.gw.p + e * D, g, sizeof(g));
     }
   }
 #pragma unroll
@@ -301,6 +316,7 @@ void update_weights_typed(tess_ctx* ctx, int basis, const tess_mesh& mesh, const
   a.l = dfield<T>(P.l);
   a.w = dfield<T>(W.w);
   a.gw = dfield<T>(W.grad_w);
+  a.rows = W.w.elem_stride == 1 && W.grad_w.elem_stride == D && W.grad_w.comp_stride == 1;
   a.window = W.window;
   a.n = P.n;
   a.corr = basis & ~0xff;

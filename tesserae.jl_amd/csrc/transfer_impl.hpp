@@ -11,7 +11,7 @@
 //   radix sort      stable (tile, particle id) order -> perm
 //   k_tile_counts / k_tab_reduce / k_tab_scan   tile ranges + slots, node blocks
 //                   touched by some footprint (binning.hip)
-//   k_p2g_tile      one wave per tile: lanes own the 64 window-start classes of
+//   k_p2g_tile      a few waves per tile: lanes own the 64 window-start classes of
 //                   the tile, accumulate their particles' contributions in
 //                   registers and add them into an LDS tile of the
 //                   (BW+3)^dim footprint (distinct targets per instruction),
@@ -114,6 +114,8 @@ struct Args {
   DField<T> gm, gmv, gf, gvn, gv;
   const int64_t* window;
   DField<T> w, gw;
+  // a particle's stored weights, and its Vec and Mat fields, are contiguous (Julia layout)
+  int32_t w_rows, p_rows;
   // corrected basis of deferred weights (0: the plain kernel) and its node filter
   int32_t corr;
   const uint8_t* filter;
@@ -666,21 +668,74 @@ __device__ __forceinline__ uint32_t broken_pair(uint64_t has, int k, uint32_t pi
   return r;
 }
 
-// One wave per tile.  The sort key orders each tile's particles by class
-// (window start relative to the footprint origin), so lane c owns class c: it
-// walks its particles, accumulates their contributions to the sw^dim nodes of
-// the class window in registers, and adds them into the LDS tile.  Lanes hold
-// distinct classes, so every LDS add instruction touches each node at most once
-// and the per-node order of the adds is the fixed program order.
+// NC components of particle p; where they are contiguous (the Julia layout) as
+// 16-byte words: the particles of a wave lie 64 places apart, and the address
+// unit takes one request per lane and instruction.
+template <typename T, int NC>
+__device__ __forceinline__ void get_row(bool rows, const DField<T>& f, int64_t p, T (&v)[NC]) {
+  if (rows) {
+    __builtin_memcpy(v, f.p + p * NC, sizeof(v));
+  } else {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) v[c] = f(p, c);
+  }
+}
+template <typename T, int NC>
+__device__ __forceinline__ void put_row(bool rows, const DField<T>& f, int64_t p, const T (&v)[NC]) {
+  if (rows) {
+    __builtin_memcpy(f.p + p * NC, v, sizeof(v));
+  } else {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) f(p, c) = v[c];
+  }
+}
+
+// N of a particle's stored weights from offset o0 on, likewise.
+template <typename T, int D, int NOFF, int N>
+__device__ __forceinline__ void stored_weights(const Args<T, D>& a, uint32_t pid, int o0, T (&w)[N], T (&g)[N][D]) {
+  const int64_t e0 = int64_t(o0) + int64_t(NOFF) * pid;
+  if (a.w_rows) {
+    __builtin_memcpy(w, a.w.p + e0, sizeof(w));
+    __builtin_memcpy(g, a.gw.p + e0 * D, sizeof(g));
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      w[i] = a.w(e0 + i);
+#pragma unroll
+      for (int c = 0; c < D; ++c) g[i][c] = a.gw(e0 + i, c);
+    }
+  }
+}
+
+// Stored and general corrected weights.  The sort key orders each tile's
+// particles by class (window start relative to the footprint origin), so lane c
+// owns class c: it walks its particles, accumulates their contributions to the
+// sw^dim nodes of the class window in registers, and adds them into the LDS
+// tile.  Lanes hold distinct classes, so every LDS add instruction touches each
+// node at most once; the waves add in turn, so the order of the adds is fixed.
+//
+// A tile has NPASS x NK waves: wave w accumulates the offsets of pass w % NPASS
+// over every NK-th particle of each class.  What bounds it is the latency of the
+// particle loads (each waits for its id) and, for particles in no order, the
+// lines they touch.  168k particles at random places, 2D Float64 quadratic with
+// stored weights, about 250 and up to 1400 particles per tile: one wave per tile
+// 58 and 239 us; four, ids in LDS, 58 and 106 us; with the weights in 16-byte
+// words 46 and 67 us.
+template <int D, int NPASS>
+constexpr int P2G_TILE_SPLIT = NPASS == 1 ? 4 : (D == 2 ? 2 : 1);  // NK
+
 template <typename T, int D, int BASIS, bool STORED, int NPASS, bool CORR = false>
-__global__ __launch_bounds__(64) void k_p2g_tile(Args<T, D> a, const uint32_t* __restrict__ skeys,
-                                                  uint32_t* __restrict__ misplaced) {
+__global__ __launch_bounds__((64 * NPASS * P2G_TILE_SPLIT<D, NPASS>)) void k_p2g_tile(
+    Args<T, D> a, const uint32_t* __restrict__ skeys, uint32_t* __restrict__ misplaced) {
   using G = Geo<D>;
   constexpr int SW = support_width(BASIS);
   constexpr int NV = 1 + 2 * D;
   constexpr int NOFF = Pow<SW, D>::v;
   constexpr int NSL = NOFF / NPASS;  // offsets per pass (NPASS is 1 or SW)
-  const int lane = threadIdx.x;
+  constexpr int NK = P2G_TILE_SPLIT<D, NPASS>, NW = NPASS * NK;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int pass = wave % NPASS, part = wave / NPASS;
   const int64_t j = xcd_remap(blockIdx.x, a.n_active);
   if (j >= a.n_active) return;
   const uint32_t tile = a.active[j];
@@ -694,13 +749,15 @@ __global__ __launch_bounds__(64) void k_p2g_tile(Args<T, D> a, const uint32_t* _
   __shared__ __align__(16) T s_tile[G::NFOOT][8];
   __shared__ T s_nodex[D][G::TS];
   __shared__ uint32_t s_cnt[64];
-  for (int q = lane; q < 8 * G::NFOOT; q += 64) (&s_tile[0][0])[q] = T(0);
-  for (int q = lane; q < D * G::TS; q += 64) {
+  __shared__ uint32_t s_pid[PID_CAP];
+  for (int q = int(threadIdx.x); q < 8 * G::NFOOT; q += 64 * NW) (&s_tile[0][0])[q] = T(0);
+  for (int q = int(threadIdx.x); q < D * G::TS; q += 64 * NW) {
     const int d = q / G::TS, k = q % G::TS;
     s_nodex[d][k] = a.mesh.node(d, origin[d] + k);
   }
   int ccount, coff, maxcnt;
-  tile_class_counts(skeys, start, cnt, s_cnt, ccount, coff, maxcnt);
+  tile_class_counts<NW>(skeys, start, cnt, s_cnt, ccount, coff, maxcnt, a.perm, 0, s_pid, nullptr, PID_CAP);
+  auto id_at = [&](int i) { return cnt <= PID_CAP ? s_pid[i] : a.perm[start + uint32_t(i)]; };
   int ccoord[D];
   {
     int r = lane;
@@ -710,14 +767,14 @@ __global__ __launch_bounds__(64) void k_p2g_tile(Args<T, D> a, const uint32_t* _
       r /= G::BW;
     }
   }
-  check_sparse_support<T, D, SW>(a, origin, ccoord, ccount);
+  if (wave == 0) check_sparse_support<T, D, SW>(a, origin, ccoord, ccount);
   // neighbours in the layered order (k-th particle of every class, classes
   // ascending, then the next k) whose storage indices are not consecutive
-  if (misplaced) {
+  if (misplaced && wave == NW - 1) {
     uint32_t bad = 0, last = 0;
     for (int k = 0; k < maxcnt; ++k) {
       const uint64_t has = __ballot(k < ccount);
-      const uint32_t pid = k < ccount ? a.perm[start + coff + k] : 0u;
+      const uint32_t pid = k < ccount ? id_at(coff + k) : 0u;
       bad += broken_pair(has, k, pid, last);
     }
 #pragma unroll
@@ -725,15 +782,15 @@ __global__ __launch_bounds__(64) void k_p2g_tile(Args<T, D> a, const uint32_t* _
     if (lane == 0 && bad) atomicAdd(lane_of(misplaced, LANE_BROKEN), bad);
   }
   const T mp = a.mp, hinv = a.mesh.h_inv;
-  for (int pass = 0; pass < NPASS; ++pass) {
+  {
     T acc[NSL][NV];
 #pragma unroll
     for (int s2 = 0; s2 < NSL; ++s2)
 #pragma unroll
       for (int v = 0; v < NV; ++v) acc[s2][v] = T(0);
-    for (int k = 0; k < maxcnt; ++k) {
+    for (int k = part; k < maxcnt; k += NK) {
       if (k >= ccount) continue;
-      const uint32_t pid = a.perm[start + coff + k];
+      const uint32_t pid = id_at(coff + k);
       T x[D], l;
       int lo[D], hi[D];
       particle_window<T, D, BASIS, STORED>(a, pid, x, l, lo, hi, nullptr);
@@ -742,12 +799,16 @@ __global__ __launch_bounds__(64) void k_p2g_tile(Args<T, D> a, const uint32_t* _
       for (int d = 0; d < D; ++d) ext[d] = hi[d] - lo[d];
       // hoisted particle factors (p2g.jl:272-307): mₚ*v[p] and (-V[p])*σ[p]
       T mv[D], A[D * D];
-#pragma unroll
-      for (int d = 0; d < D; ++d) mv[d] = mp * a.v(pid, d);
+      get_row(a.p_rows, a.v, pid, mv);
+      get_row(a.p_rows, a.sigma, pid, A);
       const T negV = -a.V(pid);
 #pragma unroll
-      for (int q = 0; q < D * D; ++q) A[q] = negV * a.sigma(pid, q);
+      for (int d = 0; d < D; ++d) mv[d] = mp * mv[d];
+#pragma unroll
+      for (int q = 0; q < D * D; ++q) A[q] = negV * A[q];
       T val[D][SW], der[D][SW];
+      constexpr int NCH = D == 3 ? SW : NSL;  // weights in registers at a time: 3D a row, 2D the pass's
+      T sw[STORED ? NCH : 1], sg[STORED ? NCH : 1][D];
       if constexpr (!STORED) {
 #pragma unroll
         for (int d = 0; d < D; ++d) axis_jets<T, D, BASIS>(x[d], ccoord[d], s_nodex[d], l, hinv, val[d], der[d]);
@@ -757,6 +818,9 @@ __global__ __launch_bounds__(64) void k_p2g_tile(Args<T, D> a, const uint32_t* _
 #pragma unroll
       for (int s2 = 0; s2 < NSL; ++s2) {
         const int o = pass * NSL + s2;
+        if constexpr (STORED) {
+          if (s2 % NCH == 0) stored_weights<T, D, NOFF>(a, pid, o, sw, sg);
+        }
         int aa[D];
         int r = o;
         bool ok = true;
@@ -769,10 +833,9 @@ __global__ __launch_bounds__(64) void k_p2g_tile(Args<T, D> a, const uint32_t* _
         if (!ok) continue;
         T w, g[D];
         if constexpr (STORED) {
-          const int64_t e = int64_t(o) + int64_t(NOFF) * pid;
-          w = a.w(e);
+          w = sw[s2 % NCH];
 #pragma unroll
-          for (int c = 0; c < D; ++c) g[c] = a.gw(e, c);
+          for (int c = 0; c < D; ++c) g[c] = sg[s2 % NCH][c];
         } else if (CORR && cs.mode == CORR_GENERAL) {
           cs.node(val, aa, filter_pass<D>(a.filter, a.mesh.dims, lo, aa), hinv, w, g);
         } else {
@@ -800,7 +863,8 @@ __global__ __launch_bounds__(64) void k_p2g_tile(Args<T, D> a, const uint32_t* _
         }
       }
     }
-    if (ccount > 0) {
+    for (int turn = 0; turn < NW; ++turn) {
+      if (wave == turn && ccount > part) {
 #pragma unroll
       for (int s2 = 0; s2 < NSL; ++s2) {
         int r = pass * NSL + s2, q = 0, mul = 1;
@@ -813,12 +877,13 @@ __global__ __launch_bounds__(64) void k_p2g_tile(Args<T, D> a, const uint32_t* _
 #pragma unroll
         for (int v = 0; v < NV; ++v) atomicAdd(&s_tile[q][v], acc[s2][v]);
       }
+      }
+      __syncthreads();
     }
   }
-  __syncthreads();
   using PT = Part<D, SW>;
   T* out = a.partials + int64_t(j) * PT::SIZE;
-  for (int e = lane; e < PT::SIZE; e += 64) {
+  for (int e = int(threadIdx.x); e < PT::SIZE; e += 64 * NW) {
     const int n = e / NV, v = e % NV;
     const int x = n % PT::E, y = (n / PT::E) % PT::E, z = D == 3 ? n / (PT::E * PT::E) : 0;
     out[e] = s_tile[x + G::TS * (y + G::TS * z)][v];
@@ -2388,24 +2453,34 @@ __global__ __launch_bounds__(64) void k_gather_grid_persist(Args<T, D> a, uint32
 
 // ---- G2P -------------------------------------------------------------------
 
+// What the particle equations read of a particle, loaded before the sums: a load
+// issued after the first stores would wait for them.
+template <typename T, int D>
+struct ParticleIn {
+  T v[D], x[D], F[D * D];
+  __device__ __forceinline__ ParticleIn(const Args<T, D>& a, int64_t p) {
+    get_row(a.p_rows, a.v, p, v);
+    get_row(a.p_rows, a.x, p, x);
+    get_row(a.p_rows, a.F, p, F);
+  }
+};
+
 // Particle equations of the README @G2P block (README.md:81-86) after the sums.
 template <typename T, int D>
-__device__ __forceinline__ void particle_update(const Args<T, D>& a, int64_t p, int64_t dst, const T* dv, const T* L,
-                                                const T* dx) {
+__device__ __forceinline__ void particle_update(const Args<T, D>& a, const ParticleIn<T, D>& in, int64_t p, int64_t dst,
+                                                const T* dv, const T (&L)[D * D], const T* dx) {
   const T dt = a.dt;
-#pragma unroll
-  for (int c = 0; c < D; ++c) a.ov(dst, c) = a.v(p, c) + dv[c];
-#pragma unroll
-  for (int k = 0; k < D * D; ++k) a.ogradv(dst, k) = L[k];
+  const bool rows = a.p_rows;
+  T vn[D], xn[D], M[D * D], Fn[D * D];
 #pragma unroll
   for (int c = 0; c < D; ++c) {
-    const T x = a.x(p, c);
-    if (a.x_keep) a.x_keep[dst * D + c] = x;
-    a.ox(dst, c) = x + dx[c];
+    vn[c] = in.v[c] + dv[c];
+    xn[c] = in.x[c] + dx[c];
+    if (a.x_keep) a.x_keep[dst * D + c] = in.x[c];
   }
-  T Fo[D * D], M[D * D], Fn[D * D];
-#pragma unroll
-  for (int k = 0; k < D * D; ++k) Fo[k] = a.F(p, k);
+  put_row(rows, a.ov, dst, vn);
+  put_row(rows, a.ogradv, dst, L);
+  put_row(rows, a.ox, dst, xn);
 #pragma unroll
   for (int b = 0; b < D; ++b)
 #pragma unroll
@@ -2414,28 +2489,31 @@ __device__ __forceinline__ void particle_update(const Args<T, D>& a, int64_t p, 
   for (int b = 0; b < D; ++b)
 #pragma unroll
     for (int r = 0; r < D; ++r) {
-      T s = M[r] * Fo[D * b];
+      T s = M[r] * in.F[D * b];
 #pragma unroll
-      for (int k = 1; k < D; ++k) s = s + M[r + D * k] * Fo[k + D * b];
+      for (int k = 1; k < D; ++k) s = s + M[r + D * k] * in.F[k + D * b];
       Fn[r + D * b] = s;
     }
-#pragma unroll
-  for (int k = 0; k < D * D; ++k) a.oF(dst, k) = Fn[k];
+  put_row(rows, a.oF, dst, Fn);
   T sg[D * D], Vn;
   neo_hookean<T, D>(Fn, a.lambda, a.mu, a.V0, a.logE.p != nullptr, a.logE.p ? a.logE(p) : T(0), sg, Vn);
-#pragma unroll
-  for (int k = 0; k < D * D; ++k) a.osigma(dst, k) = sg[k];
+  put_row(rows, a.osigma, dst, sg);
   a.oV(dst) = Vn;
 }
 
-// One wave per tile, lanes own the tile's classes as in P2G (the walk is
-// coalesced when particles are stored in the layered order).  The footprint's
-// vⁿ and v are staged in LDS once per tile.
+// Stored and general corrected weights.  The waves of a tile walk its particles
+// in turns of 64, in class or sorted order as k_g2p_fast does; the footprint's
+// vⁿ and v are staged in LDS once per tile.  Bound as k_p2g_tile is; on the same
+// particles one wave per tile took 83 and 356 us, four take 78 and 130 us, and 52
+// and 105 us with everything loaded ahead and in 16-byte words.
+constexpr int G2P_TILE_WAVES = 4;  // (8: 51 us instead of 52)
+
 template <typename T, int D, int BASIS, bool STORED, bool CORR = false>
-__global__ __launch_bounds__(64) void k_g2p_tile(Args<T, D> a, const uint32_t* __restrict__ skeys) {
+__global__ __launch_bounds__(64 * G2P_TILE_WAVES) void k_g2p_tile(Args<T, D> a, const uint32_t* __restrict__ skeys) {
   using G = Geo<D>;
-  constexpr int SW = support_width(BASIS);
-  const int lane = threadIdx.x;
+  constexpr int SW = support_width(BASIS), NW = G2P_TILE_WAVES;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   const int64_t j = xcd_remap(blockIdx.x, a.n_active);
   if (j >= a.n_active) return;
   const uint32_t tile = a.active[j];
@@ -2449,7 +2527,7 @@ __global__ __launch_bounds__(64) void k_g2p_tile(Args<T, D> a, const uint32_t* _
   __shared__ T s_v[D][G::NFOOT];
   __shared__ T s_nodex[D][G::TS];
   __shared__ uint32_t s_cnt[64];
-  for (int q = lane; q < G::NFOOT; q += 64) {
+  for (int q = int(threadIdx.x); q < G::NFOOT; q += 64 * NW) {
     int I[D], r = q;
     bool in = true;
 #pragma unroll
@@ -2466,28 +2544,35 @@ __global__ __launch_bounds__(64) void k_g2p_tile(Args<T, D> a, const uint32_t* _
       s_v[c][q] = in ? a.gv(i, c) : T(0);
     }
   }
-  for (int q = lane; q < D * G::TS; q += 64) {
+  for (int q = int(threadIdx.x); q < D * G::TS; q += 64 * NW) {
     const int d = q / G::TS, k = q % G::TS;
     s_nodex[d][k] = a.mesh.node(d, origin[d] + k);
   }
   int ccount, coff, maxcnt;
-  tile_class_counts(skeys, start, cnt, s_cnt, ccount, coff, maxcnt);  // contains the barrier after staging
-  int ccoord[D];
-  {
-    int r = lane;
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      ccoord[d] = r % G::BW;
-      r /= G::BW;
-    }
-  }
+  __shared__ uint32_t s_pid[PID_CAP], s_key[PID_CAP];
+  // contains the barrier after staging
+  tile_class_counts<NW>(skeys, start, cnt, s_cnt, ccount, coff, maxcnt, a.perm, 0, s_pid, s_key, PID_CAP);
+  const int n_sorted = (cnt + 63) / 64;
+  const bool by_sorted = 3 * n_sorted < 2 * maxcnt;
+  const int kend = by_sorted ? n_sorted : maxcnt;
   const T hinv = a.mesh.h_inv, dt = a.dt;
-  for (int k = 0; k < maxcnt; ++k) {
-    if (k >= ccount) continue;
-    const uint32_t pid = a.perm[start + coff + k];
+  for (int k = wave; k < kend; k += NW) {
+    const int at = by_sorted ? k * 64 + lane : coff + k;
+    if (by_sorted ? at >= cnt : k >= ccount) continue;
+    const uint32_t pid = cnt <= PID_CAP ? s_pid[at] : a.perm[start + uint32_t(at)];
+    int ccoord[D];  // class coordinates
+    {
+      uint32_t r = by_sorted ? (cnt <= PID_CAP ? s_key[at] : skeys[start + uint32_t(at)]) & 63u : uint32_t(lane);
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        ccoord[d] = int(r % G::BW);
+        r /= G::BW;
+      }
+    }
     T x[D], l;
     int lo[D], hi[D];
     particle_window<T, D, BASIS, STORED>(a, pid, x, l, lo, hi, nullptr);
+    const ParticleIn<T, D> in(a, pid);
     int ext[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) ext[d] = hi[d] - lo[d];
@@ -2506,9 +2591,14 @@ __global__ __launch_bounds__(64) void k_g2p_tile(Args<T, D> a, const uint32_t* _
     }
 #pragma unroll
     for (int q = 0; q < D * D; ++q) L[q] = T(0);
-    // column-major walk of the window (eachindex(window))
+    // column-major walk of the window (eachindex(window)); stored weights are
+    // loaded a row at a time
+    T sw[STORED ? SW : 1], sg[STORED ? SW : 1][D];
 #pragma unroll
     for (int o = 0; o < Pow<SW, D>::v; ++o) {
+      if constexpr (STORED) {
+        if (o % SW == 0) stored_weights<T, D, Pow<SW, D>::v>(a, pid, o, sw, sg);
+      }
       int aa[D], r = o;
       bool ok = true;
 #pragma unroll
@@ -2520,10 +2610,9 @@ __global__ __launch_bounds__(64) void k_g2p_tile(Args<T, D> a, const uint32_t* _
       if (!ok) continue;
       T w, g[D];
       if constexpr (STORED) {
-        const int64_t e = int64_t(o) + int64_t(Pow<SW, D>::v) * pid;
-        w = a.w(e);
+        w = sw[o % SW];
 #pragma unroll
-        for (int c = 0; c < D; ++c) g[c] = a.gw(e, c);
+        for (int c = 0; c < D; ++c) g[c] = sg[o % SW][c];
       } else if (CORR && cs.mode == CORR_GENERAL) {
         cs.node(val, aa, filter_pass<D>(a.filter, a.mesh.dims, lo, aa), hinv, w, g);
       } else {
@@ -2556,7 +2645,7 @@ __global__ __launch_bounds__(64) void k_g2p_tile(Args<T, D> a, const uint32_t* _
 #pragma unroll
       for (int c = 0; c < D; ++c) dx[c] += (w * vi[c]) * dt;
     }
-    particle_update<T, D>(a, pid, pid, dv, L, dx);
+    particle_update<T, D>(a, in, pid, pid, dv, L, dx);
   }
 }
 
@@ -2578,10 +2667,18 @@ __global__ __launch_bounds__(256) void k_g2p_outside(Args<T, D> a, const uint32_
   }
 #pragma unroll
   for (int k = 0; k < D * D; ++k) L[k] = T(0);
-  particle_update<T, D>(a, pid, a.dest ? a.dest[j] : pid, dv, L, dx);
+  particle_update<T, D>(a, ParticleIn<T, D>(a, pid), pid, a.dest ? a.dest[j] : pid, dv, L, dx);
 }
 
 // ---- host side ----------------------------------------------------------------
+
+// True when every particle field is Julia-native AoS (components contiguous,
+// element stride = component count), the layout the vectorised kernels assume.
+inline bool julia_layout(const tess_particles& P, int D) {
+  auto ok = [](const tess_field& f, int nc) { return !f.ptr || (f.comp_stride == 1 && f.elem_stride == nc) ||
+                                                      (nc == 1 && f.elem_stride == 1); };
+  return ok(P.x, D) && ok(P.v, D) && ok(P.V, 1) && ok(P.grad_v, D * D) && ok(P.F, D * D) && ok(P.sigma, D * D);
+}
 
 template <typename T, int D>
 Args<T, D> make_args(const tess_mesh& mesh, const tess_grid* G, const tess_particles& P, const tess_weights* W,
@@ -2608,7 +2705,9 @@ Args<T, D> make_args(const tess_mesh& mesh, const tess_grid* G, const tess_parti
     a.window = W->window;
     a.w = dfield<T>(W->w);
     a.gw = dfield<T>(W->grad_w);
+    a.w_rows = W->w.elem_stride == 1 && W->grad_w.elem_stride == D && W->grad_w.comp_stride == 1;
   }
+  a.p_rows = julia_layout(P, D);
   write_in_place(a);
   a.n = P.n;
   if (prm) {
@@ -2654,14 +2753,6 @@ template <typename T, int D, bool STORED>
 void set_correction(tess_ctx* ctx, Args<T, D>& a) {
   a.corr = STORED ? 0 : ctx->corr;
   a.filter = STORED ? nullptr : ctx->corr_filter;
-}
-
-// True when every particle field is Julia-native AoS (components contiguous,
-// element stride = component count), the layout the vectorised kernels assume.
-inline bool julia_layout(const tess_particles& P, int D) {
-  auto ok = [](const tess_field& f, int nc) { return !f.ptr || (f.comp_stride == 1 && f.elem_stride == nc) ||
-                                                      (nc == 1 && f.elem_stride == 1); };
-  return ok(P.x, D) && ok(P.v, D) && ok(P.V, 1) && ok(P.grad_v, D * D) && ok(P.F, D * D) && ok(P.sigma, D * D);
 }
 
 inline bool grid_julia_layout(const tess_grid& G, int D) {
@@ -3045,11 +3136,12 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
     // algorithmic bytes: x, v, V, σ per particle
     const int tok = prof_begin(ctx, "k_p2g_tile", double(b.n_inside) * sizeof(T) * (2 * D + 1 + D * D));
     const uint32_t* sk = static_cast<const uint32_t*>(ctx->keys_sorted.ptr);
+    const dim3 tile_block(64 * NPASS * P2G_TILE_SPLIT<D, NPASS>);
     if constexpr (STORED) {
-      hipLaunchKernelGGL((k_p2g_tile<T, D, BASIS, STORED, NPASS>), dim3(xcd_grid(b.n_active)), dim3(64), 0,
+      hipLaunchKernelGGL((k_p2g_tile<T, D, BASIS, STORED, NPASS>), dim3(xcd_grid(b.n_active)), tile_block, 0,
                          ctx->stream, a, sk, misplaced);
     } else if (a.corr && !separable_correction(a.corr, BASIS, a.filter != nullptr)) {
-      hipLaunchKernelGGL((k_p2g_tile<T, D, BASIS, false, NPASS, true>), dim3(xcd_grid(b.n_active)), dim3(64), 0,
+      hipLaunchKernelGGL((k_p2g_tile<T, D, BASIS, false, NPASS, true>), dim3(xcd_grid(b.n_active)), tile_block, 0,
                          ctx->stream, a, sk, misplaced);
     } else {
       // 3D: one wave per offset along z; 2D: one wave while the stencil fits
@@ -3132,6 +3224,7 @@ void g2p_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
     a.oF = dfield<T>(out->F);
     a.osigma = dfield<T>(out->sigma);
     a.dest = dest;
+    a.p_rows = a.p_rows && julia_layout(*out, D);
   }
   fill_binning_ptrs<T, D>(ctx, a);
   set_sparse<T, D>(a, mesh, sp);
@@ -3155,11 +3248,11 @@ void g2p_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
                                double(b.n_inside) * sizeof(T) * per_p + nodes * sizeof(T) * 2 * D);
     const uint32_t* sk = static_cast<const uint32_t*>(ctx->keys_sorted.ptr);
     if constexpr (STORED) {
-      hipLaunchKernelGGL((k_g2p_tile<T, D, BASIS, STORED>), dim3(xcd_grid(b.n_active)), dim3(64), 0, ctx->stream, a,
-                         sk);
-    } else if (generic) {
-      hipLaunchKernelGGL((k_g2p_tile<T, D, BASIS, false, true>), dim3(xcd_grid(b.n_active)), dim3(64), 0,
+      hipLaunchKernelGGL((k_g2p_tile<T, D, BASIS, STORED>), dim3(xcd_grid(b.n_active)), dim3(64 * G2P_TILE_WAVES), 0,
                          ctx->stream, a, sk);
+    } else if (generic) {
+      hipLaunchKernelGGL((k_g2p_tile<T, D, BASIS, false, true>), dim3(xcd_grid(b.n_active)), dim3(64 * G2P_TILE_WAVES),
+                         0, ctx->stream, a, sk);
     } else {
       constexpr int NW = TESS_G2P_WAVES_PER_TILE;
       const dim3 grid(xcd_grid(b.n_active)), block(64 * NW);
