@@ -4,6 +4,8 @@
 // a thread-local message.  No exception crosses this boundary.
 #include <hip/hip_runtime.h>
 
+#include <cstring>
+
 #include <atomic>
 #include <cmath>
 #include <cstdio>
@@ -273,6 +275,7 @@ tess_ctx* ctx_new(int device, hipStream_t stream) {
     check_hip(e, "hipHostMalloc");
   }
   c->counters_host = static_cast<int64_t*>(pinned);
+  std::memset(pinned, 0, 512 * sizeof(int64_t));  // no report has a number yet
   try {
     // device counters start at zero (the binning reads slots written by the previous P2G)
     TESS_HIP(hipMemset(c->counters.get(64 * sizeof(uint32_t)), 0, 64 * sizeof(uint32_t)));

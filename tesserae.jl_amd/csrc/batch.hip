@@ -139,13 +139,14 @@ void batch_bin_run(tess_ctx* ctx, tess_batch& B, bool keys_from_g2p) {
   uint32_t* counters = ctx->counters.as<uint32_t>(64);
   const uint32_t* hc = reinterpret_cast<const uint32_t*>(ctx->counters_host);
   const size_t m = size_t(std::max<int64_t>(n, 1));
-  const TabArgs tab = batch_tables(ctx, B);
+  TabArgs tab = batch_tables(ctx, B);
   const int tok = prof_begin(ctx, "binning", 0.0);
   if (incremental) {
     // the last G2P wrote the keys and counted the particles whose key changed;
     // with none the previous order and tile lists stand
-    build_tables(ctx, tab);
-    TESS_HIP(hipStreamSynchronize(ctx->stream));
+    const uint32_t seq = build_tables(ctx, tab);
+    MergeArgs merge = merge_ahead(ctx, n, int64_t(ntiles), b.n_active);
+    wait_report(ctx, seq);
     take_report(ctx);
     ctx->last_active_nodes = int64_t(hc[CNT_NODES]);
     if (hc[CNT_MOVED] == 0) {
@@ -154,7 +155,7 @@ void batch_bin_run(tess_ctx* ctx, tess_batch& B, bool keys_from_g2p) {
       prof_end(ctx, tok);
       return;
     }
-    merge_moves(ctx, n, int64_t(ntiles), b.n_active, b.n_inside);
+    merge_finish(ctx, merge, b.n_inside);
   } else {
     Args<T, D> a = batch_args<T, D>(ctx, B);
     uint32_t* skeys = ctx->keys_sorted.as<uint32_t>(m);
@@ -167,8 +168,7 @@ void batch_bin_run(tess_ctx* ctx, tess_batch& B, bool keys_from_g2p) {
       radix_sort_pairs(ctx, keys, nullptr, skeys, perm, n, key_bits_for(ntiles * 64));
     }
     launch_tile_counts(ctx->stream, skeys, n, int64_t(ntiles), tab.stay, tab.tin);
-    build_tables(ctx, tab);
-    TESS_HIP(hipStreamSynchronize(ctx->stream));
+    wait_report(ctx, build_tables(ctx, tab));
     take_report(ctx);
     ctx->last_active_nodes = int64_t(hc[CNT_NODES]);  // written by the previous step's gather
   }

@@ -152,6 +152,12 @@ __global__ __launch_bounds__(TAB_THREADS) void k_tab_prefix(uint32_t* __restrict
   }
 }
 
+// A thread's part of the report is in host memory: its number, for wait_report.
+__device__ __forceinline__ void reported(const TabArgs& a, int reporter) {
+  __threadfence_system();
+  if (a.seq) __hip_atomic_store(&a.host[CNT_SEQ + reporter], a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The tables of a workgroup's tiles from the sums of the workgroups before it.
 // Workgroup 0 also sums the lane counters (particles whose key changed, broken
 // layered pairs, nodes with mass), the last one holds the totals; both report
@@ -218,7 +224,7 @@ __global__ __launch_bounds__(TAB_THREADS) void k_tab_scan(TabArgs a) {
     a.host[CNT_NB] = nb;
     a.host[CNT_OUTIN] = out_in;
     a.host[CNT_ARRIVE] = arrive + out_in;
-    __threadfence_system();
+    reported(a, LANE_GROUPS);
   }
   if (blockIdx.x == 0) {
     // one wave per group of lanes
@@ -233,14 +239,16 @@ __global__ __launch_bounds__(TAB_THREADS) void k_tab_scan(TabArgs a) {
     for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off, 64);
     if (i == 0 && g < LANE_GROUPS) {
       a.host[g == LANE_MOVED ? CNT_MOVED : g == LANE_BROKEN ? CNT_MISPLACED : CNT_NODES] = x;
+      if (g == LANE_MOVED) a.counters[CNT_MOVED] = x;
       if (g == LANE_NODES) {
         a.counters[CNT_NODES] = x;
+        a.counters[CNT_REENTERED] = a.counters[CNT_REENTER];
         a.host[CNT_ERR] = a.counters[CNT_ERR];
         a.host[CNT_REENTER] = a.counters[CNT_REENTER];
         if (!a.keep_err) a.counters[CNT_ERR] = 0u;
         a.counters[CNT_REENTER] = 0u;
       }
-      __threadfence_system();
+      reported(a, g);
     }
   }
 }
@@ -270,11 +278,19 @@ __global__ __launch_bounds__(256) void k_tile_counts(const uint32_t* __restrict_
   tin[t] = 0u;
 }
 
+// A merge launched before the host has read the report: nothing to do when no key
+// changed, or when particles came back into the mesh (the host sorts them all).
+__device__ __forceinline__ bool merge_gated(const MergeArgs& a) {
+  if (!a.gate) return false;
+  const uint32_t moved = a.gate[CNT_MOVED], reentered = a.gate[CNT_REENTERED];  // read together
+  return (moved == 0u) | (reentered != 0u);
+}
+
 // The leavers of each previously active tile into the arrival segments of the
 // tiles they enter (a leaver's rank there was drawn when its key was computed).
 __global__ __launch_bounds__(64) void k_scatter_out(MergeArgs a) {
   const int64_t j = blockIdx.x;
-  if (j >= int64_t(a.old_count ? *a.old_count : a.old_active_n)) return;
+  if (j >= int64_t(a.old_count ? *a.old_count : a.old_active_n) || merge_gated(a)) return;
   const uint32_t t = a.old_active[j];
   const uint32_t start = a.old_start[t], cnt = a.old_end[t] - start;
   const uint32_t leave = cnt - a.stay[t];
@@ -372,11 +388,11 @@ __global__ __launch_bounds__(64 * NW) void k_merge_tiles(MergeArgs a) {
   __shared__ uint2 s_raw[CAP], s_in[CAP];
   __shared__ uint32_t s_hist[256], s_wc[MERGE_WAVES][256];
   __shared__ uint32_t s_base[MERGE_WAVES][64], s_low;
-  const int64_t jt = blockIdx.x;
-  if (jt >= int64_t(a.new_count ? *a.new_count : a.new_active_n)) return;
+  const int64_t jt = a.first_tile + int64_t(blockIdx.x);
+  const uint32_t t = a.new_active[jt];  // (ntiles entries: in range whether or not jt is active)
+  if (jt >= int64_t(a.new_count ? *a.new_count : a.new_active_n) || merge_gated(a)) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  const uint32_t t = a.new_active[jt];
   const uint32_t os = a.old_start[t], oc = a.old_end[t] - os;
   const uint32_t ns = a.new_start[t], k = a.new_end[t] - ns - a.stay[t];
   const uint2* in = s_in;
@@ -556,17 +572,23 @@ void launch_merge(hipStream_t st, const MergeArgs& a, bool arrivals, unsigned ou
     hipLaunchKernelGGL(k_scatter_out, dim3(unsigned(a.old_active_n)), dim3(64), 0, st, a);
     TESS_HIP(hipGetLastError());
   }
-  if (a.new_active_n > 0) {
-    if (a.small_tiles)
-      hipLaunchKernelGGL(k_merge_tiles<1>, dim3(unsigned(a.new_active_n)), dim3(64), 0, st, a);
-    else
-      hipLaunchKernelGGL(k_merge_tiles<4>, dim3(unsigned(a.new_active_n)), dim3(256), 0, st, a);
-    TESS_HIP(hipGetLastError());
-  }
-  if (outside_blocks > 0) {
-    hipLaunchKernelGGL(k_merge_outside, dim3(outside_blocks), dim3(256), 0, st, a);
-    TESS_HIP(hipGetLastError());
-  }
+  launch_merge_tiles(st, a, a.new_active_n);
+  if (outside_blocks > 0) launch_merge_outside(st, a, outside_blocks);
+}
+
+// The tiles from a.first_tile on, one workgroup each.
+void launch_merge_tiles(hipStream_t st, const MergeArgs& a, int64_t tiles) {
+  if (tiles <= 0) return;
+  if (a.small_tiles)
+    hipLaunchKernelGGL(k_merge_tiles<1>, dim3(unsigned(tiles)), dim3(64), 0, st, a);
+  else
+    hipLaunchKernelGGL(k_merge_tiles<4>, dim3(unsigned(tiles)), dim3(256), 0, st, a);
+  TESS_HIP(hipGetLastError());
+}
+
+void launch_merge_outside(hipStream_t st, const MergeArgs& a, unsigned blocks) {
+  hipLaunchKernelGGL(k_merge_outside, dim3(blocks), dim3(256), 0, st, a);
+  TESS_HIP(hipGetLastError());
 }
 
 }  // namespace tess

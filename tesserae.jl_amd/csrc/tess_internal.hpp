@@ -111,8 +111,11 @@ namespace tess {
 enum {
   CNT_INSIDE = 0, CNT_ACTIVE = 1, CNT_NB = 2, CNT_ERR = 3, CNT_BIN_SLOTS = 4,
   CNT_MISPLACED = 8, CNT_NODES = 9, CNT_ARRIVE = 10, CNT_P2GERR = 11, CNT_MOVED = 12, CNT_OUTIN = 13, CNT_REENTER = 14,
-  CNT_PREV_ACTIVE = 15, CNT_SLOTS = 16
+  CNT_PREV_ACTIVE = 15, CNT_SLOTS = 16,
+  CNT_REENTERED = 16,  // device: CNT_REENTER of the last report
+  CNT_SEQ = 17         // host: the report's number, once by each of its REPORTERS
 };
+constexpr int REPORTERS = 4;
 // Kernels count into lanes, one per 128-byte line, chosen by workgroup (no
 // single contended address): particles whose key changed, layered neighbour
 // pairs not consecutive in storage, nodes with m > 0.
@@ -145,6 +148,7 @@ struct TabArgs {
   uint32_t* lanes;
   uint32_t* counters;
   uint32_t* host;
+  uint32_t seq;  // the report's number (0: nobody waits for it by number)
   int32_t keep_err;
 };
 
@@ -155,6 +159,7 @@ struct MergeArgs {
   const uint32_t* old_count;  // device counts for launches sized by an upper bound, or nullptr
   const uint32_t* new_count;
   int64_t old_active_n, new_active_n;
+  int64_t first_tile;  // of new_active, for the launch's first workgroup
   const uint32_t* stay;
   const uint32_t* nk;
   const uint32_t* perm_old;
@@ -163,6 +168,7 @@ struct MergeArgs {
   uint2 *seg, *seg_alt;
   uint32_t *keys_new, *perm_new;
   const uint32_t* counters;  // device count of arrivals outside the mesh, or nullptr: out_in
+  const uint32_t* gate;      // device counters: do nothing where they call for no merge, or nullptr
   uint32_t out_in;
   int32_t pos_bits;
   int32_t small_tiles;  // one wave per tile
@@ -200,6 +206,7 @@ struct tess_ctx {
   const uint8_t* corr_filter = nullptr;
   tess::Buffer lanes;      // counts spread over cache lines (LANE_GROUPS groups of LANES)
   tess::Buffer host_pinned_dummy;
+  uint32_t report_seq = 0;           // number of the last report asked for by number
   int64_t* counters_host = nullptr;  // pinned readback slots
   tess::Binning bin;
   // zeroing bookkeeping for the grid of the previous P2G
@@ -328,6 +335,8 @@ int64_t tab_blocks(int64_t ntiles);
 void launch_tables(hipStream_t st, const TabArgs& a);
 void launch_tile_counts(hipStream_t st, const uint32_t* skeys, int64_t n, int64_t ntiles, uint32_t* stay, uint32_t* tin);
 void launch_merge(hipStream_t st, const MergeArgs& a, bool arrivals, unsigned outside_blocks);
+void launch_merge_tiles(hipStream_t st, const MergeArgs& a, int64_t tiles);
+void launch_merge_outside(hipStream_t st, const MergeArgs& a, unsigned blocks);
 
 // ---- reference-layout weights and partition (partition.hip) ----
 void launch_update_weights(tess_ctx* ctx, int basis, const tess_mesh& mesh, const tess_particles& P,

@@ -2805,8 +2805,10 @@ inline TabArgs table_args(tess_ctx* ctx, int64_t ntiles) {
 }
 
 // Builds the tables into the alternate set, whose node-block list the stale
-// zeroing may still need.
-inline void build_tables(tess_ctx* ctx, const TabArgs& t) {
+// zeroing may still need.  Returns the number of the report it enqueued.
+inline uint32_t build_tables(tess_ctx* ctx, TabArgs& t) {
+  if (++ctx->report_seq == 0) ctx->report_seq = 1;
+  t.seq = ctx->report_seq;
   if (ctx->prev_list == tess_ctx::PrevList::Alternate && ctx->prev_nodeblocks > 0) {
     uint32_t* keep = ctx->nb_list_prev.as<uint32_t>(size_t(ctx->prev_nodeblocks));
     TESS_HIP(hipMemcpyAsync(keep, ctx->alt_nb_list.ptr, size_t(ctx->prev_nodeblocks) * sizeof(uint32_t),
@@ -2814,6 +2816,7 @@ inline void build_tables(tess_ctx* ctx, const TabArgs& t) {
     ctx->prev_list = tess_ctx::PrevList::Copied;
   }
   launch_tables(ctx->stream, t);
+  return t.seq;
 }
 
 // The alternate tables become the current ones.
@@ -2837,11 +2840,35 @@ inline void take_report(tess_ctx* ctx) {
   ctx->nodes_pending = false;
 }
 
-// The merge of the particles whose key changed (counts in the report, tables
-// built in the alternate set): (keys_sorted, vals) and the tables become the
-// new ones.
-inline void merge_moves(tess_ctx* ctx, int64_t n, int64_t ntiles, int64_t old_active, int64_t old_inside) {
+// Waits for report number seq: its words arrive in pinned memory while the
+// kernel that writes them still runs, which the end of the stream's work would
+// tell 5-10 us later.  The stream is asked now and then, so that a failed launch
+// or a report that never comes ends the wait.
+inline void wait_report(tess_ctx* ctx, uint32_t seq) {
   const uint32_t* hc = reinterpret_cast<const uint32_t*>(ctx->counters_host);
+  auto there = [&]() {
+    bool all = true;
+    for (int r = 0; r < REPORTERS; ++r) all = all && __atomic_load_n(hc + CNT_SEQ + r, __ATOMIC_ACQUIRE) == seq;
+    return all;
+  };
+  for (uint32_t spin = 1; !there(); ++spin) {
+    if (spin % 4096 != 0) {
+      __builtin_ia32_pause();
+      continue;
+    }
+    const hipError_t e = hipStreamQuery(ctx->stream);
+    if (e == hipErrorNotReady) {
+      (void)hipGetLastError();
+      continue;
+    }
+    TESS_HIP(e);
+    if (!there()) raise(TESS_ERR_STATE, "the binning's report did not arrive");
+  }
+}
+
+// The merge of the particles whose key changed, from the current tables to the
+// alternate ones (which build_tables has enqueued).
+inline MergeArgs merge_args(tess_ctx* ctx, int64_t n, int64_t ntiles, int64_t old_active) {
   const size_t m = size_t(std::max<int64_t>(n, 1));
   MergeArgs g;
   std::memset(static_cast<void*>(&g), 0, sizeof(g));
@@ -2854,7 +2881,6 @@ inline void merge_moves(tess_ctx* ctx, int64_t n, int64_t ntiles, int64_t old_ac
   g.new_start = static_cast<const uint32_t*>(ctx->alt_start.ptr);
   g.new_end = static_cast<const uint32_t*>(ctx->alt_end.ptr);
   g.old_active_n = old_active;
-  g.new_active_n = int64_t(hc[CNT_ACTIVE]);
   g.stay = static_cast<const uint32_t*>(ctx->tile_stay.ptr);
   g.nk = static_cast<const uint32_t*>(ctx->inc_nk.ptr);
   g.perm_old = static_cast<const uint32_t*>(ctx->vals.ptr);
@@ -2864,12 +2890,33 @@ inline void merge_moves(tess_ctx* ctx, int64_t n, int64_t ntiles, int64_t old_ac
   g.seg_alt = ctx->inc_seg2.as<uint2>(m);
   g.keys_new = ctx->skeys2.as<uint32_t>(m);
   g.perm_new = ctx->perm2.as<uint32_t>(m);
-  g.out_in = hc[CNT_OUTIN];
   g.pos_bits = key_bits_for(uint64_t(m));
-  g.small_tiles = n < 256 * g.new_active_n;
-  const int64_t outside = n - int64_t(hc[CNT_INSIDE]);
-  launch_merge(ctx->stream, g, hc[CNT_ARRIVE] != 0,
-               outside > 0 ? unsigned(std::min<int64_t>(blocks_for(n - old_inside, 256), 2048)) : 0u);
+  return g;
+}
+
+// Launches the merge behind the tables, before the host has their report: its
+// launches and the wait overlap.  The counts are the device's, and the launch
+// guesses an eighth more active tiles than before; merge_finish adds the rest.
+inline MergeArgs merge_ahead(tess_ctx* ctx, int64_t n, int64_t ntiles, int64_t old_active) {
+  MergeArgs g = merge_args(ctx, n, ntiles, old_active);
+  const uint32_t* counters = static_cast<const uint32_t*>(ctx->counters.ptr);
+  g.gate = counters;
+  g.new_count = counters + CNT_ACTIVE;
+  g.new_active_n = std::min(ntiles, old_active + old_active / 8 + 64);
+  g.small_tiles = n < 256 * std::max<int64_t>(old_active, 1);
+  launch_merge(ctx->stream, g, true, 0);
+  return g;
+}
+
+// After the report of a merge launched ahead: the particles outside the mesh, and
+// (keys_sorted, vals) become the new ones.
+inline void merge_finish(tess_ctx* ctx, MergeArgs& g, int64_t old_inside) {
+  const uint32_t* hc = reinterpret_cast<const uint32_t*>(ctx->counters_host);
+  g.out_in = hc[CNT_OUTIN];
+  g.first_tile = g.new_active_n;
+  launch_merge_tiles(ctx->stream, g, int64_t(hc[CNT_ACTIVE]) - g.first_tile);
+  if (g.n > int64_t(hc[CNT_INSIDE]))
+    launch_merge_outside(ctx->stream, g, unsigned(std::min<int64_t>(blocks_for(g.n - old_inside, 256), 2048)));
   std::swap(ctx->keys_sorted, ctx->skeys2);
   std::swap(ctx->vals, ctx->perm2);
 }
@@ -2983,8 +3030,9 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
         TESS_HIP(hipGetLastError());
       }
     }
-    build_tables(ctx, tab);
-    TESS_HIP(hipStreamSynchronize(ctx->stream));
+    const uint32_t seq = build_tables(ctx, tab);
+    MergeArgs merge = merge_ahead(ctx, n, int64_t(ntiles), b.n_active);
+    wait_report(ctx, seq);
     take_report(ctx);
     ctx->last_movers = int64_t(hc[CNT_MOVED]);
     const bool same_kind = b.tile_log2 == Geo<D>::LT && b.basis == BASIS && b.dtype == mesh.dtype;
@@ -3004,7 +3052,7 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
       std::swap(ctx->keys_sorted, ctx->skeys2);
       std::swap(ctx->vals, ctx->perm2);
     } else if (ctx->last_movers > 0) {
-      merge_moves(ctx, n, int64_t(ntiles), b.n_active, b.n_inside);
+      merge_finish(ctx, merge, b.n_inside);
     }
   } else {
     uint32_t* skeys = ctx->keys_sorted.as<uint32_t>(m);
@@ -3018,8 +3066,7 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
     }
     ctx->last_movers = -1;
     launch_tile_counts(ctx->stream, skeys, n, int64_t(ntiles), tab.stay, tab.tin);
-    build_tables(ctx, tab);
-    TESS_HIP(hipStreamSynchronize(ctx->stream));
+    wait_report(ctx, build_tables(ctx, tab));
     take_report(ctx);
   }
   prof_end(ctx, tok);

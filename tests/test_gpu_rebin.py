@@ -137,3 +137,30 @@ def test_reorders_of_a_g2p2g_loop(layout, passes):
     for k in a:
         assert rel_err(b[k][ib], a[k][ia]) <= 1e-9, k
     assert rel_err(gb["m"], ga["m"]) <= 1e-12
+
+
+@pytest.mark.parametrize("n", [700, 3000])
+def test_rebinning_spreads_over_many_tiles(n):
+    """Particles of one tile spread over some 900 at once and gather again: far more active tiles than the merge launched
+    behind the tables allows for, then far fewer; P2G equals a fresh context's to Float64 rounding."""
+    sc = random_box(2, n, 7, th.BSpline(th.Quadratic()), dtype=torch.float64, h=0.004)
+    mesh, P, G = to_gpu(sc)
+    ctx = th.Context(library=_abi.DEBUG_LIB_PATH)
+    spread = 0.01 + 0.98 * (sc.x - sc.x.min(0)) / (sc.x.max(0) - sc.x.min(0))
+    for k, x in enumerate((0.5 + 0.02 * spread, spread, 0.3 + 0.02 * spread, spread[::-1].copy())):
+        P.set("x", x)
+        th.P2G(G, P, sc.basis, sc.params, ctx=ctx)
+        ctx.sync()
+        got, stats = grid_np(G), ctx.stats()
+        mesh2, P2, G2 = to_gpu(sc)
+        P2.set("x", x)
+        ref_ctx = th.Context()
+        th.P2G(G2, P2, sc.basis, sc.params, ctx=ref_ctx)
+        ref_ctx.sync()
+        ref = grid_np(G2)
+        for f in ref:
+            assert rel_err(got[f], ref[f]) <= 1e-12, (k, f)
+        assert stats["active_tiles"] == ref_ctx.stats()["active_tiles"]
+        assert (stats["active_tiles"] > 400) == (k % 2 == 1)
+        ref_ctx.close()
+    ctx.close()
