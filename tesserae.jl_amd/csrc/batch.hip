@@ -208,7 +208,7 @@ __global__ __launch_bounds__(256) void k_batch_new_index(Args<T, D> a, const uin
   const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (j < a.n) {
     const uint32_t g = a.perm[j];
-    const int s = scene_of(a.scene_poff, a.nscenes, int64_t(g));
+    const int s = scene_near(a.scene_poff, a.nscenes, int64_t(g));
     const int64_t p0 = a.scene_poff[s], p1 = a.scene_poff[s + 1];
     const uint32_t dst = j < a.n_inside ? uint32_t(int64_t(layered[j]) + int64_t(R[p0]))
                                         : uint32_t(p1 - int64_t(R[p1] - R[p0]) + int64_t(R[g] - R[p0]));
@@ -217,52 +217,50 @@ __global__ __launch_bounds__(256) void k_batch_new_index(Args<T, D> a, const uin
   }
 }
 
-template <typename T, int D>
-__device__ __forceinline__ DField<T> scene_field(const SceneRec<T, D>& r, int fid) {
-  switch (fid) {
-    case 0: return r.x;
-    case 1: return r.v;
-    case 2: return r.V;
-    case 3: return r.gradv;
-    case 4: return r.F;
-    case 5: return r.sigma;
-    case 6: return r.l;
-    default: return r.logE;
-  }
-}
-
-// components of the particle fields x, v, V, ∇v, F, σ, l, log E
-template <int D>
-constexpr int kFieldComps[8] = {D, D, 1, D * D, D * D, D * D, 1, 1};
+// scalars of a particle's fields x, v, V, ∇v, F, σ, l, log E
 template <int D>
 constexpr int kStateWidth = 2 * D + 2 + 3 * D * D + 1;
 
 // With `order`: every field of particle order[i] into row i of the packed
 // scratch (field-major: field f's rows start at its component offset times n).
-// Without: row i back into particle i.  One scene lookup per particle.
+// Without: row i back into particle i.  A particle's fields are all loaded before
+// the first is stored, contiguous ones in words of up to 16 bytes: scalar by
+// scalar, a field's loads behind the previous one's stores, the two launches took
+// 547 us each on 9.7 M 2D Float32 particles.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void k_batch_state(Args<T, D> a, T* __restrict__ scratch,
                                                      const uint32_t* __restrict__ order) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= a.n) return;
-  const int s = scene_of(a.scene_poff, a.nscenes, i);
+  const int s = scene_near(a.scene_poff, a.nscenes, i);
   const SceneRec<T, D>& r = a.scenes[s];
   const int64_t li = (order ? int64_t(order[i]) : i) - r.poff;  // the permutation stays within the scene
-  int64_t off = 0;
-#pragma unroll
-  for (int fid = 0; fid < 8; ++fid) {
-    const int nc = kFieldComps<D>[fid];
-    const DField<T> f = scene_field<T, D>(r, fid);
-    if (f.p) {
-      T* row = scratch + off * a.n + i * nc;
-      if (order) {
-        for (int c = 0; c < nc; ++c) row[c] = f(li, c);
-      } else {
-        for (int c = 0; c < nc; ++c) f(li, c) = row[c];
-      }
-    }
-    off += nc;
-  }
+  T x[D], v[D], V[1], gradv[D * D], F[D * D], sigma[D * D], l[1], logE[1];
+  auto each = [&](auto&& f) {
+    int64_t off = 0;
+    auto field = [&](const DField<T>& d, auto& val) {
+      constexpr int NC = int(sizeof(val) / sizeof(T));
+      if (d.p) f(d, val, off * a.n + i * NC);
+      off += NC;
+    };
+    field(r.x, x);
+    field(r.v, v);
+    field(r.V, V);
+    field(r.gradv, gradv);
+    field(r.F, F);
+    field(r.sigma, sigma);
+    field(r.l, l);
+    field(r.logE, logE);
+  };
+  auto rows = [](const DField<T>& d, int nc) { return d.es == nc && (nc == 1 || d.cs == 1); };
+  each([&](const DField<T>& d, auto& val, int64_t at) {
+    if (order) get_row(rows(d, int(sizeof(val) / sizeof(T))), d, li, val);
+    else __builtin_memcpy(val, scratch + at, sizeof(val));
+  });
+  each([&](const DField<T>& d, auto& val, int64_t at) {
+    if (order) __builtin_memcpy(scratch + at, val, sizeof(val));
+    else put_row(rows(d, int(sizeof(val) / sizeof(T))), d, li, val);
+  });
 }
 
 // Reorders the scenes' particles when the batch's contiguity score is below

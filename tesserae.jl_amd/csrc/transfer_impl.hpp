@@ -192,6 +192,15 @@ __device__ __forceinline__ int scene_of(const int64_t* __restrict__ off, int ns,
   return lo;
 }
 
+// The same for lanes whose places lie close together: one search by scalar loads
+// for the wave's first lane, which nearly every lane shares.
+__device__ __forceinline__ int scene_near(const int64_t* __restrict__ off, int ns, int64_t g) {
+  const int64_t g0 = (int64_t(__builtin_amdgcn_readfirstlane(int(g >> 32))) << 32) |
+                     int64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(g)))));
+  const int s = scene_of(off, ns, g0);
+  return off[s] <= g && g < off[s + 1] ? s : scene_of(off, ns, g);
+}
+
 // Replace the scene-dependent part of a by scene s of the batch.
 template <typename T, int D>
 __device__ __forceinline__ const SceneRec<T, D>& bind_scene(Args<T, D>& a, int s) {
@@ -402,7 +411,7 @@ __global__ __launch_bounds__(256) void k_bin_keys(Args<T, D> a, uint32_t* __rest
   const int64_t p = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (p >= a.n) return;
   if constexpr (BATCH) {  // batch: scene-local key, shifted to the scene's first global tile
-    const SceneRec<T, D>& r = bind_scene(a, scene_of(a.scene_poff, a.nscenes, p));
+    const SceneRec<T, D>& r = bind_scene(a, scene_near(a.scene_poff, a.nscenes, p));
     uint32_t nl = 1;
 #pragma unroll
     for (int d = 0; d < D; ++d) nl *= uint32_t(r.ntiles[d]);
