@@ -176,10 +176,17 @@ __global__ __launch_bounds__(256) void k_update_weights(WArgs<T, D> a) {
 
 // key = colour * nblocks + linear block id (cpu_block_strategy.jl:197-219: groups
 // by colour, blocks in linear order inside a group), or `outside` past the end.
+// The launch also clears the blocks' runs (fills of their own took 2-3 us each,
+// of the 75 us that a partition of 51 k particles took).
 template <typename T, int D>
 __global__ __launch_bounds__(256) void k_partition_keys(DMesh<T, D> mesh, DField<T> X, int64_t n, int L,
-                                                         int3 nb, uint32_t nbt, uint32_t* __restrict__ keys) {
+                                                         int3 nb, uint32_t nbt, uint32_t* __restrict__ keys,
+                                                         int32_t* __restrict__ starts, int32_t* __restrict__ stops) {
   const int64_t p = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  for (int64_t b = p; b < int64_t(nbt); b += int64_t(gridDim.x) * blockDim.x) {
+    starts[b] = 0;
+    stops[b] = 0;
+  }
   if (p >= n) return;
   const int nbd[3] = {nb.x, nb.y, nb.z};
   uint32_t lin = 0, color = 0;
@@ -357,6 +364,11 @@ void update_weights_typed(tess_ctx* ctx, int basis, const tess_mesh& mesh, const
   }
 }
 
+// workgroups for n keys and the clearing of nbt runs
+inline unsigned partition_grid(int64_t n, uint64_t nbt) {
+  return nblk(std::max(n, int64_t(std::min<uint64_t>(nbt, 1u << 20))), 256);
+}
+
 template <typename T, int D>
 void partition_typed(tess_ctx* ctx, const tess_mesh& mesh, tess_field x, int64_t n, int32_t* pidx, int32_t* starts,
                      int32_t* stops, int64_t* nassigned) {
@@ -370,29 +382,25 @@ void partition_typed(tess_ctx* ctx, const tess_mesh& mesh, tess_field x, int64_t
   const uint64_t outside = (uint64_t(1) << D) * nbt;
   if (outside >= uint64_t(UINT32_MAX) || n >= int64_t(INT32_MAX))
     raise(TESS_ERR_ARGUMENT, "Partition block count exceeds packed block id capacity.");
-  TESS_HIP(hipMemsetAsync(starts, 0, nbt * sizeof(int32_t), ctx->stream));
-  TESS_HIP(hipMemsetAsync(stops, 0, nbt * sizeof(int32_t), ctx->stream));
-  uint32_t* cnt = ctx->counters.as<uint32_t>(4);
-  TESS_HIP(hipMemsetAsync(cnt, 0, sizeof(uint32_t), ctx->stream));
+  uint32_t* hc = reinterpret_cast<uint32_t*>(ctx->counters_host);
+  uint32_t* keys = ctx->keys.as<uint32_t>(size_t(std::max<int64_t>(n, 1)));
+  hipLaunchKernelGGL((k_partition_keys<T, D>), dim3(partition_grid(n, nbt)), dim3(256), 0, ctx->stream, dmesh<T, D>(mesh),
+                     dfield<T>(x), n, L, make_int3(nbd[0], nbd[1], nbd[2]), uint32_t(nbt), keys, starts, stops);
+  TESS_HIP(hipGetLastError());
   if (n > 0) {
-    uint32_t* keys = ctx->keys.as<uint32_t>(size_t(n));
     uint32_t* skeys = ctx->keys_sorted.as<uint32_t>(size_t(n));
     uint32_t* vals = ctx->vals.as<uint32_t>(size_t(n));
-    hipLaunchKernelGGL((k_partition_keys<T, D>), dim3(nblk(n, 256)), dim3(256), 0, ctx->stream, dmesh<T, D>(mesh),
-                       dfield<T>(x), n, L, make_int3(nbd[0], nbd[1], nbd[2]), uint32_t(nbt), keys);
-    TESS_HIP(hipGetLastError());
     int bits = 0;
     while ((uint64_t(1) << bits) <= outside) ++bits;
     radix_sort_pairs(ctx, keys, nullptr, skeys, vals, n, bits);
+    // exactly one thread writes the count, to pinned memory
     hipLaunchKernelGGL(k_partition_runs, dim3(nblk(n, 256)), dim3(256), 0, ctx->stream, skeys, vals, n,
-                       uint32_t(nbt), uint32_t(outside), pidx, starts, stops, cnt);
+                       uint32_t(nbt), uint32_t(outside), pidx, starts, stops, hc);
     TESS_HIP(hipGetLastError());
     // the internal tile binning used the same buffers
     ctx->bin.valid = false;
     ctx->bin.state_valid = false;
   }
-  uint32_t* hc = reinterpret_cast<uint32_t*>(ctx->counters_host);
-  TESS_HIP(hipMemcpyAsync(hc, cnt, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
   TESS_HIP(hipStreamSynchronize(ctx->stream));
   *nassigned = n > 0 ? int64_t(hc[0]) : 0;
 }
@@ -419,11 +427,6 @@ static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices] = {};
-
-__global__ void k_fill_i32(int32_t* __restrict__ a, int64_t n, int32_t v) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = v;
-}
 
 __global__ void k_store_nassigned(const uint32_t* __restrict__ count, int64_t n, int64_t* __restrict__ out) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *out = n > 0 ? int64_t(*count) : 0;
@@ -460,15 +463,10 @@ void partition_noalloc_typed(const tess_mesh& mesh, tess_field x, int64_t n, int
     raise(TESS_ERR_STATE, "the sort's histograms exceed the fixed work area");
   w.hist = reinterpret_cast<uint32_t*>(take(kNoAllocHistBytes));
   uint32_t* cnt = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t)));
-  // fill kernels rather than memset nodes, so that a captured graph replays them
-  hipLaunchKernelGGL(k_fill_i32, dim3(nblk(int64_t(nbt), 256)), dim3(256), 0, stream, starts, int64_t(nbt), 0);
-  TESS_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_fill_i32, dim3(nblk(int64_t(nbt), 256)), dim3(256), 0, stream, stops, int64_t(nbt), 0);
+  hipLaunchKernelGGL((k_partition_keys<T, D>), dim3(partition_grid(n, nbt)), dim3(256), 0, stream, dmesh<T, D>(mesh),
+                     dfield<T>(x), n, L, make_int3(nbd[0], nbd[1], nbd[2]), uint32_t(nbt), keys, starts, stops);
   TESS_HIP(hipGetLastError());
   if (n > 0) {
-    hipLaunchKernelGGL((k_partition_keys<T, D>), dim3(nblk(n, 256)), dim3(256), 0, stream, dmesh<T, D>(mesh),
-                       dfield<T>(x), n, L, make_int3(nbd[0], nbd[1], nbd[2]), uint32_t(nbt), keys);
-    TESS_HIP(hipGetLastError());
     int bits = 0;
     while ((uint64_t(1) << bits) <= outside) ++bits;
     radix_sort_pairs_ws(w, keys, nullptr, skeys, vals, n, bits);

@@ -2,7 +2,7 @@
 // uint32) used for particle binning.  Integer-only, so results are
 // deterministic; ranking inside a workgroup is stable (index order).
 //
-// Sort pass structure (one digit of 8 to 10 bits per pass):
+// Sort pass structure (one digit of 8 to 10 bits per pass, sort_digit_bits):
 //   1. k_radix_hist   per-workgroup digit histogram of a chunk, stored
 //                     digit-major: hist[digit * nchunks + chunk]
 //   2. k_radix_rows   one workgroup per digit: exclusive scan of its row, and
@@ -12,13 +12,12 @@
 //                     ballots and running counts per wave, no barrier between
 //                     rounds), and writes (key, value) to offset + rank.
 //
-// What bounds it: at a million particles the launches and the few hundred
-// workgroups, each a serial chain of rounds; at ten million the scattered
-// writes of 4 bytes.  1.67 M particles with 20-bit keys, unsorted: a pass took
-// 12 us for the histogram, 14 us for a scan of three launches and 22 us with
-// four barriers per 256 keys, and there were three; now there are two of 12 + 5
-// + 31 us (10-bit digits scatter wider), and the block partition that they
-// serve takes 139 us instead of 188.
+// What bounds it: up to a million particles the launches and the few hundred
+// workgroups, each a serial chain of rounds; past that the scattered writes of 4
+// bytes.  1.67 M particles with 20-bit keys, unsorted: three passes took 12 us for
+// the histogram, 14 us for a scan of three launches and 22 us with four barriers
+// per 256 keys each; now they take 8 + 4 + 15 us, and the block partition that
+// they serve 115 us instead of 188.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -42,10 +41,18 @@ constexpr int64_t SORT_LARGE = int64_t(4) << 20;
 inline int64_t sort_chunk(int64_t n) {
   return int64_t(SORT_THREADS) * (n >= SORT_LARGE ? SORT_ROUNDS_LARGE : SORT_ROUNDS_SMALL);
 }
-// Digit bits: as few passes as 10-bit digits give, of equal width.
-inline int sort_passes(int key_bits) { return key_bits <= 0 ? 1 : (key_bits + RADIX_BITS_MAX - 1) / RADIX_BITS_MAX; }
-inline int sort_digit_bits(int key_bits) {
-  const int p = sort_passes(key_bits);
+// Digit bits: as few passes as 10-bit digits give, of equal width, while launches
+// are what a pass costs; 8-bit digits from SORT_NARROW keys on, where a wider
+// digit leaves a chunk two keys of each and its writes share no line.  A block
+// partition of particles in no order, 10-bit and 8-bit digits: 0.05 M 68 and 79 us,
+// 0.8 M 84 and 102, 1.67 M 137 and 133, 3.3 M 205 and 182.
+constexpr int64_t SORT_NARROW = int64_t(1) << 20;
+inline int sort_passes(int key_bits, int64_t n) {
+  const int widest = n < SORT_NARROW ? RADIX_BITS_MAX : 8;
+  return key_bits <= 0 ? 1 : (key_bits + widest - 1) / widest;
+}
+inline int sort_digit_bits(int key_bits, int64_t n) {
+  const int p = sort_passes(key_bits, n);
   const int b = (key_bits + p - 1) / p;
   return b < 8 ? 8 : b;
 }
@@ -417,7 +424,7 @@ void radix_sort_pairs_ws(const SortWork& w, const uint32_t* keys_in, const uint3
                          uint32_t* vals_out, int64_t n, int key_bits, const uint32_t* n_dev) {
   if (n <= 0) return;
   if (n > int64_t(UINT32_MAX)) raise(TESS_ERR_ARGUMENT, "radix sort: more than 2^32-1 elements");
-  const int passes = sort_passes(key_bits), bits = sort_digit_bits(key_bits);
+  const int passes = sort_passes(key_bits, n), bits = sort_digit_bits(key_bits, n);
   const int64_t nchunks = ceil_div(n, sort_chunk(n));
   const bool large = n >= SORT_LARGE;
   // ping-pong so that the last pass writes (keys_out, vals_out)
