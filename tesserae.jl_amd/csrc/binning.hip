@@ -305,24 +305,23 @@ __global__ __launch_bounds__(64) void k_scatter_out(MergeArgs a) {
   }
 }
 
-// The merge runs one workgroup per tile, of 4 waves, or of one where tiles hold
-// few particles (the batch's 256 uneven scenes, 110 per active tile: 227 us with
-// four waves per tile).  Arrivals up to the LDS list are sorted there.
-template <int NW>
-constexpr int MERGE_CAP = NW == 1 ? 128 : 512;
+// The merge runs one workgroup per tile, of 4 waves also where tiles hold few
+// particles: one wave for each of the batch's 215 k tiles of 45 particles made a
+// call of 8 steps 0.26 ms longer, and a binning of the two disks 3 us.  Arrivals
+// up to the LDS list are sorted there.
+constexpr int MERGE_WAVES = 4, MERGE_THREADS = 64 * MERGE_WAVES;
+constexpr uint32_t MERGE_CAP = 512;
 
 // Sorts k (key, position) pairs of a segment by position with one workgroup:
 // 8-bit digits of the position, `bits` low bits, between seg and alt; returns
 // the buffer that holds the result.  For segments past the LDS list.
-template <int NW>
 __device__ uint2* segment_sort(uint2* seg, uint2* alt, uint32_t k, int bits, uint32_t* s_hist, uint32_t (*s_wc)[256]) {
-  constexpr int NT = 64 * NW;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int shift = 0; shift < bits; shift += 8) {
     __syncthreads();
-    for (int d = int(threadIdx.x); d < 256; d += NT) s_hist[d] = 0;
+    for (int d = int(threadIdx.x); d < 256; d += MERGE_THREADS) s_hist[d] = 0;
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < k; i += NT) atomicAdd(&s_hist[(seg[i].y >> shift) & 255u], 1u);
+    for (uint32_t i = threadIdx.x; i < k; i += MERGE_THREADS) atomicAdd(&s_hist[(seg[i].y >> shift) & 255u], 1u);
     __syncthreads();
     if (wave == 0) {  // exclusive prefix of the 256 digits, four per lane
       uint32_t h[4], tot = 0;
@@ -339,14 +338,14 @@ __device__ uint2* segment_sort(uint2* seg, uint2* alt, uint32_t k, int bits, uin
       }
     }
     __syncthreads();
-    for (uint32_t b = 0; b < k; b += NT) {
+    for (uint32_t b = 0; b < k; b += MERGE_THREADS) {
       const uint32_t i = b + threadIdx.x;
       const bool valid = i < k;
       const uint2 e = valid ? seg[i] : make_uint2(0u, 0u);
       const uint32_t d = (e.y >> shift) & 255u;
-      for (int q = int(threadIdx.x); q < 256; q += NT)
+      for (int q = int(threadIdx.x); q < 256; q += MERGE_THREADS)
 #pragma unroll
-        for (int w = 0; w < NW; ++w) s_wc[w][q] = 0;
+        for (int w = 0; w < MERGE_WAVES; ++w) s_wc[w][q] = 0;
       __syncthreads();
       uint64_t peers = __ballot(valid);
 #pragma unroll
@@ -364,10 +363,10 @@ __device__ uint2* segment_sort(uint2* seg, uint2* alt, uint32_t k, int bits, uin
         alt[pos] = e;
       }
       __syncthreads();
-      for (int q = int(threadIdx.x); q < 256; q += NT) {
+      for (int q = int(threadIdx.x); q < 256; q += MERGE_THREADS) {
         uint32_t add = 0;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) add += s_wc[w][q];
+        for (int w = 0; w < MERGE_WAVES; ++w) add += s_wc[w][q];
         s_hist[q] += add;
       }
       __syncthreads();
@@ -385,11 +384,8 @@ __device__ uint2* segment_sort(uint2* seg, uint2* alt, uint32_t k, int bits, uin
 // stable counting sort, by class, of a sequence in order of previous position:
 // arrivals from below its old run, the old run without its leavers, arrivals
 // from above.  The waves take consecutive parts of the sequence.
-template <int NW>
-__global__ __launch_bounds__(64 * NW) void k_merge_tiles(MergeArgs a) {
-  constexpr int MERGE_THREADS = 64 * NW, MERGE_WAVES = NW;
-  constexpr uint32_t CAP = MERGE_CAP<NW>;
-  __shared__ uint2 s_raw[CAP], s_in[CAP];
+__global__ __launch_bounds__(MERGE_THREADS) void k_merge_tiles(MergeArgs a) {
+  __shared__ uint2 s_raw[MERGE_CAP], s_in[MERGE_CAP];
   __shared__ uint32_t s_hist[256], s_wc[MERGE_WAVES][256];
   __shared__ uint32_t s_base[MERGE_WAVES][64], s_low;
   const int64_t jt = a.first_tile + int64_t(blockIdx.x);
@@ -402,7 +398,7 @@ __global__ __launch_bounds__(64 * NW) void k_merge_tiles(MergeArgs a) {
   const uint2* in = s_in;
   if (threadIdx.x == 0) s_low = 0;
   s_base[wave][lane] = 0;
-  if (k > 0 && k <= CAP) {
+  if (k > 0 && k <= MERGE_CAP) {
     const uint2* seg = a.seg + a.seg_off[t];
     for (uint32_t i = threadIdx.x; i < k; i += MERGE_THREADS) s_raw[i] = seg[i];
     __syncthreads();
@@ -413,7 +409,7 @@ __global__ __launch_bounds__(64 * NW) void k_merge_tiles(MergeArgs a) {
       s_in[r] = e;
     }
   } else if (k > 0) {
-    in = segment_sort<NW>(a.seg + a.seg_off[t], a.seg_alt + a.seg_off[t], k, a.pos_bits, s_hist, s_wc);
+    in = segment_sort(a.seg + a.seg_off[t], a.seg_alt + a.seg_off[t], k, a.pos_bits, s_hist, s_wc);
   }
   __syncthreads();
   if (k > 0) {
@@ -522,14 +518,13 @@ __global__ __launch_bounds__(64 * NW) void k_merge_tiles(MergeArgs a) {
 // Particles outside the mesh: those that were outside keep their order behind
 // the arrivals (whose previous positions are all lower).  Workgroup 0 places
 // the arrivals, sorted by previous position.
-__global__ __launch_bounds__(256) void k_merge_outside(MergeArgs a) {
-  constexpr int MERGE_THREADS = 256, MERGE_WAVES = 4;
+__global__ __launch_bounds__(MERGE_THREADS) void k_merge_outside(MergeArgs a) {
   __shared__ uint32_t s_hist[256], s_wc[MERGE_WAVES][256];
   const uint32_t k = a.counters ? a.counters[CNT_OUTIN] : a.out_in;
   const uint32_t ns = a.new_start[a.ntiles], os = a.old_start[a.ntiles];
   if (blockIdx.x == 0 && k > 0) {
     const uint32_t off = a.seg_off[a.ntiles];
-    const uint2* in = segment_sort<4>(a.seg + off, a.seg_alt + off, k, a.pos_bits, s_hist, s_wc);
+    const uint2* in = segment_sort(a.seg + off, a.seg_alt + off, k, a.pos_bits, s_hist, s_wc);
     for (uint32_t i = threadIdx.x; i < k; i += MERGE_THREADS) {
       a.keys_new[ns + i] = in[i].x;
       a.perm_new[ns + i] = a.perm_old[in[i].y];
@@ -588,10 +583,7 @@ void launch_merge(hipStream_t st, const MergeArgs& a, bool arrivals, unsigned ou
 // The tiles from a.first_tile on, one workgroup each.
 void launch_merge_tiles(hipStream_t st, const MergeArgs& a, int64_t tiles) {
   if (tiles <= 0) return;
-  if (a.small_tiles)
-    hipLaunchKernelGGL(k_merge_tiles<1>, dim3(unsigned(tiles)), dim3(64), 0, st, a);
-  else
-    hipLaunchKernelGGL(k_merge_tiles<4>, dim3(unsigned(tiles)), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(k_merge_tiles, dim3(unsigned(tiles)), dim3(MERGE_THREADS), 0, st, a);
   TESS_HIP(hipGetLastError());
 }
 

@@ -171,7 +171,6 @@ struct MergeArgs {
   const uint32_t* gate;      // device counters: do nothing where they call for no merge, or nullptr
   uint32_t out_in;
   int32_t pos_bits;
-  int32_t small_tiles;  // one wave per tile
 };
 
 }  // namespace tess

@@ -2912,7 +2912,6 @@ inline MergeArgs merge_ahead(tess_ctx* ctx, int64_t n, int64_t ntiles, int64_t o
   g.gate = counters;
   g.new_count = counters + CNT_ACTIVE;
   g.new_active_n = std::min(ntiles, old_active + old_active / 8 + 64);
-  g.small_tiles = n < 256 * std::max<int64_t>(old_active, 1);
   launch_merge(ctx->stream, g, true, 0);
   return g;
 }
