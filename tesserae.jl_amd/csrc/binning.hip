@@ -109,6 +109,14 @@ __device__ __forceinline__ bool touched(const TabArgs& a, int64_t t) {
 // walking the 27 neighbours of four tiles in turn (22 us).
 __global__ __launch_bounds__(TAB_THREADS) void k_tab_reduce(TabArgs a) {
   __shared__ uint32_t s[TAB_WAVES];
+  if (a.may_keep) {
+    // a step in which no key changed needs the report alone: without this, the
+    // two launches took 20 us over the 275 k tiles of a 256^3 mesh
+    const int i = int(threadIdx.x & 63);
+    const bool keep = __ballot(i < LANES && a.lanes[(LANE_MOVED * LANES + (i & (LANES - 1))) * LANE_STRIDE] != 0u) == 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.counters[CNT_KEEP] = keep ? 1u : 0u;
+    if (keep) return;  // uniform
+  }
   const int64_t t = int64_t(blockIdx.x) * TAB_THREADS + threadIdx.x;
   uint32_t c = 0, in = 0, pk = 0;
   if (t < a.ntiles) {
@@ -169,6 +177,12 @@ template <bool ALONE>
 __global__ __launch_bounds__(TAB_THREADS) void k_tab_scan(TabArgs a) {
   __shared__ uint32_t s[TAB_WAVES];
   uint32_t pre[4] = {0, 0, 0, 0};
+  bool keep = false;
+  if constexpr (!ALONE) {
+    keep = a.may_keep && a.counters[CNT_KEEP] != 0u;
+    if (keep && blockIdx.x != 0) return;
+  }
+  if (!keep) {
   if constexpr (!ALONE) {
     if (gridDim.x > SUMS_DIRECT) {
 #pragma unroll
@@ -227,6 +241,9 @@ __global__ __launch_bounds__(TAB_THREADS) void k_tab_scan(TabArgs a) {
     a.host[CNT_OUTIN] = out_in;
     a.host[CNT_ARRIVE] = arrive + out_in;
     reported(a, LANE_GROUPS);
+  }
+  } else if (threadIdx.x == 0) {
+    reported(a, LANE_GROUPS);  // the totals of the last report stand
   }
   if (blockIdx.x == 0) {
     // one wave per group of lanes

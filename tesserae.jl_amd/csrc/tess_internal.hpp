@@ -113,6 +113,7 @@ enum {
   CNT_MISPLACED = 8, CNT_NODES = 9, CNT_ARRIVE = 10, CNT_P2GERR = 11, CNT_MOVED = 12, CNT_OUTIN = 13, CNT_REENTER = 14,
   CNT_PREV_ACTIVE = 15, CNT_SLOTS = 16,
   CNT_REENTERED = 16,  // device: CNT_REENTER of the last report
+  CNT_KEEP = 21,       // device: the tables being scanned are not wanted
   CNT_SEQ = 17         // host: the report's number, once by each of its REPORTERS
 };
 constexpr int REPORTERS = 4;
@@ -150,6 +151,7 @@ struct TabArgs {
   uint32_t* host;
   uint32_t seq;  // the report's number (0: nobody waits for it by number)
   int32_t keep_err;
+  int32_t may_keep;  // with no changed key the old tables stand: build none (CNT_KEEP)
 };
 
 // The merge of the particles whose key changed into the previous order.

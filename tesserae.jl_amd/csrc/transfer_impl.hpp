@@ -3038,12 +3038,18 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
         TESS_HIP(hipGetLastError());
       }
     }
+    const bool same_kind = b.tile_log2 == Geo<D>::LT && b.basis == BASIS && b.dtype == mesh.dtype;
+    tab.may_keep = same_kind ? 1 : 0;
     const uint32_t seq = build_tables(ctx, tab);
-    MergeArgs merge = merge_ahead(ctx, n, int64_t(ntiles), b.n_active);
+    // (over many tiles, whose workgroups cost 0.2 ns each to find nothing to do,
+    // not ahead while the last binning found no changed key)
+    const bool ahead = ctx->last_movers != 0 || b.n_active <= 8192;
+    MergeArgs merge;
+    if (ahead) merge = merge_ahead(ctx, n, int64_t(ntiles), b.n_active);
     wait_report(ctx, seq);
     take_report(ctx);
     ctx->last_movers = int64_t(hc[CNT_MOVED]);
-    const bool same_kind = b.tile_log2 == Geo<D>::LT && b.basis == BASIS && b.dtype == mesh.dtype;
+    if (!ahead && ctx->last_movers > 0 && !hc[CNT_REENTER]) merge = merge_ahead(ctx, n, int64_t(ntiles), b.n_active);
     if (ctx->last_movers == 0 && same_kind && !(hc[CNT_ERR] & ERR_GIMP_LENGTH)) {
       // no particle changed its key: the previous order and tile lists stand
       ctx->last_misplaced = (ctx->misplaced_x_ptr == P.x.ptr && ctx->misplaced_n == n) ? ctx->broken_count : -1;
