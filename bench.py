@@ -182,8 +182,9 @@ def traffic_record(fetch_dir, write_dir):
     alg = {"k_g2p_fast": 196 * 13434880, "k_p2g_fast": 64 * 13434880, "k_gather_grid": None}
     out = {}
     for key, label in (("k_g2p_fast", "k_g2p_tile"), ("k_p2g_fast", "k_p2g_tile"), ("k_gather_grid", "k_gather_grid")):
-        name = next((k for k in fetch if key + "<float, 3" in k), None)
-        if name is None or name not in write:
+        # the form with the most dispatches (G2P's first step of a scene stores plainly, the rest stream)
+        name = max((k for k in fetch if key + "<float, 3" in k), key=lambda k: len(fetch[k]), default=None)
+        if name is None or len(fetch[name]) < 2 or len(write.get(name, ())) < 2:
             continue
         fr, wr = fetch[name][1:], write[name][1:]
         rd = sum(fr) / len(fr) * 1024 * fscale
