@@ -2790,8 +2790,21 @@ inline MoveOut move_out(tess_ctx* ctx, int64_t n, int64_t ntiles) {
 }
 inline MoveOut no_moves() { return MoveOut{nullptr, nullptr, nullptr, nullptr, nullptr}; }
 
-// Arguments that build the tables of ntiles tiles into the alternate set.
+// The node-block list of the last P2G, where it is in the alternate set (the
+// stale zeroing may still need it), into a buffer of its own.
+inline void save_prev_list(tess_ctx* ctx) {
+  if (ctx->prev_list != tess_ctx::PrevList::Alternate || ctx->prev_nodeblocks == 0) return;
+  uint32_t* keep = ctx->nb_list_prev.as<uint32_t>(size_t(ctx->prev_nodeblocks));
+  TESS_HIP(hipMemcpyAsync(keep, ctx->alt_nb_list.ptr, size_t(ctx->prev_nodeblocks) * sizeof(uint32_t),
+                          hipMemcpyDeviceToDevice, ctx->stream));
+  ctx->prev_list = tess_ctx::PrevList::Copied;
+}
+
+// Arguments that build the tables of ntiles tiles into the alternate set, whose
+// buffers grow here where the mesh has more tiles than they hold (and lose what
+// they held).
 inline TabArgs table_args(tess_ctx* ctx, int64_t ntiles) {
+  save_prev_list(ctx);
   TabArgs t;
   std::memset(static_cast<void*>(&t), 0, sizeof(t));
   const size_t nt = size_t(ntiles) + 1;
@@ -2813,17 +2826,11 @@ inline TabArgs table_args(tess_ctx* ctx, int64_t ntiles) {
   return t;
 }
 
-// Builds the tables into the alternate set, whose node-block list the stale
-// zeroing may still need.  Returns the number of the report it enqueued.
+// Builds the tables of table_args into the alternate set.  Returns the number of
+// the report it enqueued.
 inline uint32_t build_tables(tess_ctx* ctx, TabArgs& t) {
   if (++ctx->report_seq == 0) ctx->report_seq = 1;
   t.seq = ctx->report_seq;
-  if (ctx->prev_list == tess_ctx::PrevList::Alternate && ctx->prev_nodeblocks > 0) {
-    uint32_t* keep = ctx->nb_list_prev.as<uint32_t>(size_t(ctx->prev_nodeblocks));
-    TESS_HIP(hipMemcpyAsync(keep, ctx->alt_nb_list.ptr, size_t(ctx->prev_nodeblocks) * sizeof(uint32_t),
-                            hipMemcpyDeviceToDevice, ctx->stream));
-    ctx->prev_list = tess_ctx::PrevList::Copied;
-  }
   launch_tables(ctx->stream, t);
   return t.seq;
 }

@@ -1,0 +1,58 @@
+"""What a P2G leaves on a grid is its own: the node blocks that an earlier P2G on the same grid wrote and this one does
+not touch are zero again, whatever the context did in between.
+
+Each case moves the particles to another part of the mesh and compares every grid field with that of a fresh context
+and a fresh grid (Float64; the particles may be summed in another order: 1e-12)."""
+import numpy as np
+import pytest
+import torch
+
+import tesserae_hip as th
+from gpu_util import grid_np, rel_err, to_gpu
+from tesserae_hip.scenes import random_box, uniform01
+
+pytestmark = pytest.mark.gpu
+
+QUADRATIC = th.BSpline(th.Quadratic())
+
+
+def _p2g_alone(sc, x):
+    """The grid of one P2G at x on a context and a grid of its own."""
+    _, P, G = to_gpu(sc)
+    P.set("x", x)
+    ctx = th.Context()
+    th.P2G(G, P, sc.basis, sc.params, ctx=ctx)
+    ctx.sync()
+    out = grid_np(G)
+    ctx.close()
+    return out
+
+
+def _equal_grids(got, ref, what):
+    for name in ref:
+        assert rel_err(got[name], ref[name]) <= 1e-12, (what, name)
+        assert not np.any(got[name][ref[name] == 0.0]), (what, name)
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("fine", [1, 4], ids=["same-tiles", "more-tiles"])
+@pytest.mark.parametrize("between", [1, 2, 3])
+def test_g2p_on_another_mesh_between_two_p2g(dim, fine, between):
+    """P2G(A), G2P(B) some times, P2G(A): no P2G on B tells the context that the grid changed, and B's tables (of as
+    many tiles as A's, or of more than A's buffers hold) are built in the sets that held the node blocks of A."""
+    h = 0.02 if dim == 2 else 0.05
+    a = random_box(dim, 700, 3, QUADRATIC, h=h, lo=0.1, hi=0.3)
+    b = random_box(dim, 900, 5, QUADRATIC, h=h / fine, lo=0.1, hi=0.9, vscale=30.0)
+    _, Pa, Ga = to_gpu(a)
+    _, Pb, Gb = to_gpu(b)
+    ctx = th.Context()
+    th.P2G(Ga, Pa, a.basis, a.params, ctx=ctx)
+    for k in range(between):
+        Pb.set("x", 0.1 + 0.8 * uniform01(40 + k, b.n * dim).reshape(b.n, dim))
+        th.G2P(Gb, Pb, b.basis, b.params, ctx=ctx)
+    x = a.x + 0.5
+    Pa.set("x", x)
+    th.P2G(Ga, Pa, a.basis, a.params, ctx=ctx)
+    ctx.sync()
+    _equal_grids(grid_np(Ga), _p2g_alone(a, x), between)
+    ctx.close()
