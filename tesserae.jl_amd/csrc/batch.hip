@@ -178,7 +178,6 @@ void batch_bin_run(tess_ctx* ctx, tess_batch& B, bool keys_from_g2p) {
   b.n_inside = int64_t(hc[CNT_INSIDE]);
   b.n_active = int64_t(hc[CNT_ACTIVE]);
   b.n_nodeblocks = int64_t(hc[CNT_NB]);
-  b.generation += 1;
   b.ntiles = int64_t(ntiles);
   b.n = n;
   b.valid = true;

@@ -60,8 +60,6 @@ struct Binning {
   // the last G2P wrote the next keys at the sorted positions and the counts
   // and leavers of every tile
   bool keys_ready = false;
-  // counts the binnings that built new tile lists
-  uint64_t generation = 0;
 };
 
 // Per-kernel timing with HIP events on the context's stream.  Disabled by
@@ -213,10 +211,9 @@ struct tess_ctx {
   // zeroing bookkeeping for the grid of the previous P2G
   const void* last_grid_m = nullptr;
   int64_t prev_nodeblocks = 0;
-  // the binning of the last P2G, and where its node-block list is: in the
-  // current tables, in the alternate set they were swapped with, or copied out
-  // before that set was built again
-  uint64_t prev_generation = 0;
+  // where the node-block list of the last P2G is: in the current tables, in the
+  // alternate set they were swapped with, or copied out before that set was
+  // built again
   enum class PrevList { Current, Alternate, Copied } prev_list = PrevList::Copied;
   int32_t prev_tile_log2 = -1;
   int64_t prev_ntiles = -1;

@@ -3100,7 +3100,6 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
   ctx->last_misplaced = (ctx->misplaced_x_ptr == P.x.ptr && ctx->misplaced_n == n) ? ctx->broken_count : -1;
   b.n_active = int64_t(hc[CNT_ACTIVE]);
   b.n_nodeblocks = int64_t(hc[CNT_NB]);
-  b.generation += 1;
   b.x_ptr = P.x.ptr;
   b.n = n;
   b.dim = D;
@@ -3167,9 +3166,9 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
       TESS_HIP(hipGetLastError());
     }
   };
-  // stale node blocks are zeroed by the gather's launch (a binning that kept
-  // its layout left none)
-  const bool stale = !sp && !fresh && ctx->prev_nodeblocks > 0 && ctx->prev_generation != ctx->bin.generation;
+  // stale node blocks are zeroed by the gather's launch; there are none while
+  // the tables are still those of the last P2G (no binning since has swapped them)
+  const bool stale = !sp && !fresh && ctx->prev_nodeblocks > 0 && ctx->prev_list != tess_ctx::PrevList::Current;
   if (stale) {
     a.stale_list = static_cast<const uint32_t*>(ctx->prev_list == tess_ctx::PrevList::Alternate ? ctx->alt_nb_list.ptr
                                                                                                 : ctx->nb_list_prev.ptr);
@@ -3255,7 +3254,6 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
   }
   // this call's node blocks are what the next call's stale zeroing looks at
   ctx->prev_nodeblocks = b.n_nodeblocks;
-  ctx->prev_generation = b.generation;
   ctx->prev_list = tess_ctx::PrevList::Current;
   ctx->last_grid_m = sp ? nullptr : G.m.ptr;  // a dense grid after an SpGrid call starts from a full zero
   ctx->prev_tile_log2 = Gm::LT;

@@ -56,3 +56,28 @@ def test_g2p_on_another_mesh_between_two_p2g(dim, fine, between):
     ctx.sync()
     _equal_grids(grid_np(Ga), _p2g_alone(a, x), between)
     ctx.close()
+
+
+@pytest.mark.parametrize("nsteps,every,repeats", [(2, 10, 1), (3, 10, 1), (2, 1, 2), (21, 10, 2), (11, 10, 3)])
+def test_p2g_after_a_pullback(nsteps, every, repeats):
+    """A rollout whose steps re-bin, its pullback, then a P2G elsewhere on the same grid: the pullback works from kept
+    binnings of other steps, which say nothing about what the rollout's last P2G wrote."""
+    sc = random_box(2, 600, 7, QUADRATIC, h=0.02, lo=0.1, hi=0.3)
+    sc.v[:] = (5.0, 3.0)  # a quarter of a cell per step: some particles change their cell in every step
+    _, P, G = to_gpu(sc)
+    ctx = th.Context()
+    adj = th.Adjoint(sc.n, 2)
+    for r in range(repeats):
+        P.set("x", sc.x)
+        P.set("v", sc.v)
+        P.set("F", sc.F)
+        th.rollout(G, P, sc.basis, sc.params, nsteps, checkpoint_every=every, ctx=ctx)
+        adj.x.fill_(1.0)
+        th.rollout_adjoint(G, sc.basis, sc.params, adj, ctx=ctx)
+        _, P0, _ = to_gpu(sc)
+        x = sc.x + 0.5 - 0.1 * r
+        P0.set("x", x)
+        th.P2G(G, P0, sc.basis, sc.params, ctx=ctx)
+        ctx.sync()
+        _equal_grids(grid_np(G), _p2g_alone(sc, x), r)
+    ctx.close()
