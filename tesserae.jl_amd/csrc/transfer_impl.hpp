@@ -3708,15 +3708,23 @@ void step_impl(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const t
       const bool last = s + 1 == nsteps;
       if (done) *done = s;
       if (hook) (*hook)(0, s);
-      if (sp) {
-        // update_sparsity!(grid, xₚ) at the top of the SpGrid loop (src/Grids/grid.jl:97-101);
-        // the binning's readback brings its totals too
-        run_sparsity_update(ctx, mesh, mp.now().x, P.n, *sp, nullptr, true);
-      }
       // from the second step on, the previous G2P wrote the keys (same call, so
       // nothing else moved the particles in between)
-      bin_particles<T, D, BASIS, false>(ctx, mesh, mp.now(), nullptr, s > 0);
-      if (sp) {
+      auto bin = [&]() { bin_particles<T, D, BASIS, false>(ctx, mesh, mp.now(), nullptr, s > 0); };
+      if (!sp) {
+        bin();
+      } else {
+        // update_sparsity!(grid, xₚ) at the top of the SpGrid loop (src/Grids/grid.jl:97-101);
+        // the binning's readback brings its totals too.  A binning that fails leaves
+        // the new numbering, whose storage length later calls check against: sp
+        // takes it before the error goes on
+        run_sparsity_update(ctx, mesh, mp.now().x, P.n, *sp, nullptr, true);
+        try {
+          bin();
+        } catch (...) {
+          if (hipStreamSynchronize(ctx->stream) == hipSuccess) take_sparsity(ctx, mesh, *sp, nullptr);
+          throw;
+        }
         take_sparsity(ctx, mesh, *sp, nullptr);
         if (sp->storage_len > sp->capacity)
           raise(TESS_ERR_STATE, "SpGrid storage holds " + std::to_string(sp->capacity) + " nodes but the active blocks need " +
