@@ -216,8 +216,7 @@ struct tess_ctx {
   // built again
   enum class PrevList { Current, Alternate, Copied } prev_list = PrevList::Copied;
   int32_t prev_tile_log2 = -1;
-  int64_t prev_ntiles = -1;
-  int64_t prev_nnodes = -1;
+  int64_t prev_dims[3] = {-1, -1, -1};
   // reorder scratch and the layout score of the last step's P2G
   tess::Buffer reorder_tmp, reorder_cnt;
   const void* misplaced_x_ptr = nullptr;

@@ -3045,7 +3045,9 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
         TESS_HIP(hipGetLastError());
       }
     }
-    const bool same_kind = b.tile_log2 == Geo<D>::LT && b.basis == BASIS && b.dtype == mesh.dtype;
+    // (meshes of as many tiles with other axes give equal keys, not equal node blocks)
+    bool same_kind = b.tile_log2 == Geo<D>::LT && b.basis == BASIS && b.dtype == mesh.dtype;
+    for (int d = 0; d < D; ++d) same_kind = same_kind && b.ntiles_axis[d] == a.ntiles[d];
     tab.may_keep = same_kind ? 1 : 0;
     const uint32_t seq = build_tables(ctx, tab);
     // (over many tiles, whose workgroups cost 0.2 ns each to find nothing to do,
@@ -3144,8 +3146,8 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
   // zero what this call will not overwrite: everything on first use of a
   // grid, else the node blocks that were written last time and are not now.
   // An SpGrid's storage is zeroed whole (its numbering may have changed).
-  const bool fresh = ctx->last_grid_m != G.m.ptr || ctx->prev_tile_log2 != Gm::LT ||
-                     ctx->prev_ntiles != ctx->bin.ntiles || ctx->prev_nnodes != nnodes;
+  bool fresh = ctx->last_grid_m != G.m.ptr || ctx->prev_tile_log2 != Gm::LT;
+  for (int d = 0; d < D; ++d) fresh = fresh || ctx->prev_dims[d] != mesh.dims[d];
   // The numbering was built from these particles (fresh_numbering): with blocks
   // of at least two nodes every class window lies within the activated blocks,
   // and there is nothing to check.
@@ -3257,8 +3259,7 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
   ctx->prev_list = tess_ctx::PrevList::Current;
   ctx->last_grid_m = sp ? nullptr : G.m.ptr;  // a dense grid after an SpGrid call starts from a full zero
   ctx->prev_tile_log2 = Gm::LT;
-  ctx->prev_ntiles = b.ntiles;
-  ctx->prev_nnodes = nnodes;
+  for (int d = 0; d < D; ++d) ctx->prev_dims[d] = mesh.dims[d];
   if (check) {
     uint32_t* hc = reinterpret_cast<uint32_t*>(ctx->counters_host);
     TESS_HIP(hipMemcpyAsync(hc + CNT_P2GERR, counters + CNT_P2GERR, sizeof(uint32_t), hipMemcpyDeviceToHost,

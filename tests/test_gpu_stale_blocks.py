@@ -81,3 +81,34 @@ def test_p2g_after_a_pullback(nsteps, every, repeats):
         ctx.sync()
         _equal_grids(grid_np(G), _p2g_alone(sc, x), r)
     ctx.close()
+
+
+def _on_mesh(sc, mesh):
+    out = sc.copy()
+    out.mesh = mesh
+    return out
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("shared", [False, True], ids=["own-grid", "shared-grid"])
+def test_meshes_of_equal_counts(dim, shared):
+    """Two meshes with as many nodes and tiles, their axes exchanged: the particles' keys are the same numbers on both
+    (they lie in the first tile), but not the node blocks around them.  With `shared` the second mesh takes over the
+    arrays of the first one's grid."""
+    h = 1.0 / 32
+    ends = (1.0, 2.0) if dim == 2 else (0.5, 1.0, 0.75)
+    mesh_a = th.CartesianMesh(h, *[(0.0, e) for e in ends], dtype=torch.float64)
+    mesh_b = th.CartesianMesh(h, *[(0.0, e) for e in ends[::-1]], dtype=torch.float64)
+    assert mesh_a.nnodes() == mesh_b.nnodes() and tuple(mesh_a.size()) != tuple(mesh_b.size())
+    sc = random_box(dim, 500, 3, QUADRATIC, h=h, lo=0.01, hi=0.09 if dim == 3 else 0.23)
+    a, b = _on_mesh(sc, mesh_a), _on_mesh(sc, mesh_b)
+    _, P, Ga = to_gpu(a)
+    _, _, Gb = to_gpu(b)
+    if shared:
+        Gb.tensors = Ga.tensors
+    ctx = th.Context()
+    for s, G in ((a, Ga), (b, Gb), (a, Ga)):
+        th.P2G(G, P, s.basis, s.params, ctx=ctx)
+        ctx.sync()
+        _equal_grids(grid_np(G), _p2g_alone(s, sc.x), "a" if s is a else "b")
+    ctx.close()
