@@ -140,12 +140,16 @@ void batch_bin_run(tess_ctx* ctx, tess_batch& B, bool keys_from_g2p) {
   const uint32_t* hc = reinterpret_cast<const uint32_t*>(ctx->counters_host);
   const size_t m = size_t(std::max<int64_t>(n, 1));
   TabArgs tab = batch_tables(ctx, B);
+  tab.tile_max = merge_tile_max(n);
   const int tok = prof_begin(ctx, "binning", 0.0);
   if (incremental) {
     // the last G2P wrote the keys and counted the particles whose key changed;
     // with none the previous order and tile lists stand
+    tab.crowd = merge_crowd(n);
+    tab.many = merge_many(n);
     const uint32_t seq = build_tables(ctx, tab);
-    MergeArgs merge = merge_ahead(ctx, n, int64_t(ntiles), b.n_active);
+    MergeArgs merge;
+    if (!b.crowded) merge = merge_ahead(ctx, n, int64_t(ntiles), b.n_active);
     wait_report(ctx, seq);
     take_report(ctx);
     ctx->last_active_nodes = int64_t(hc[CNT_NODES]);
@@ -155,7 +159,8 @@ void batch_bin_run(tess_ctx* ctx, tess_batch& B, bool keys_from_g2p) {
       prof_end(ctx, tok);
       return;
     }
-    merge_finish(ctx, merge, b.n_inside);
+    if (b.crowded || hc[CNT_RESORT] || hc[CNT_ARRIVE] > tab.many) resort_keys(ctx, n, key_bits_for(ntiles * 64));
+    else merge_finish(ctx, merge, b.n_inside);
   } else {
     Args<T, D> a = batch_args<T, D>(ctx, B);
     uint32_t* skeys = ctx->keys_sorted.as<uint32_t>(m);
@@ -178,6 +183,7 @@ void batch_bin_run(tess_ctx* ctx, tess_batch& B, bool keys_from_g2p) {
   b.n_inside = int64_t(hc[CNT_INSIDE]);
   b.n_active = int64_t(hc[CNT_ACTIVE]);
   b.n_nodeblocks = int64_t(hc[CNT_NB]);
+  b.crowded = (hc[CNT_RESORT] & RESORT_TILE) != 0;
   b.ntiles = int64_t(ntiles);
   b.n = n;
   b.valid = true;

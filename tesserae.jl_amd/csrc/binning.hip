@@ -16,7 +16,9 @@
 //                              (arrivals from lower positions, those that
 //                              stay, arrivals from higher positions)
 // The result is the stable sort of the previous order by the new keys, the
-// order a full radix sort of (new key, previous order) gives.
+// order a full radix sort of (new key, previous order) gives.  The sort takes the
+// merge's place where one tile, or all together, have too many changed keys
+// (CNT_RESORT, CNT_MANY): the device says so before the merge runs.
 //
 // What bounds it: each kernel moves 8-20 bytes per particle or per tile and is
 // short, so launches and the one readback bound it below about a million
@@ -103,6 +105,12 @@ __device__ __forceinline__ bool touched(const TabArgs& a, int64_t t) {
   return any != 0;
 }
 
+// Why a merge should not take a tile (with the last one also the outside).
+__device__ __forceinline__ uint32_t crowded(const TabArgs& a, int64_t t, uint32_t arrivals, uint32_t count) {
+  const bool in = arrivals > a.crowd || (t == a.ntiles - 1 && a.tin[a.ntiles] > a.crowd);
+  return (in ? uint32_t(RESORT_CROWD) : 0u) | (count > a.tile_max ? uint32_t(RESORT_TILE) : 0u);
+}
+
 // Per workgroup of TAB_THREADS tiles: particles, arrivals, active tiles and
 // touched node blocks; writes the touched flags.  One tile per thread: four per
 // thread left a mesh of 36 k tiles on 36 workgroups of 256 threads, each thread
@@ -122,6 +130,8 @@ __global__ __launch_bounds__(TAB_THREADS) void k_tab_reduce(TabArgs a) {
   if (t < a.ntiles) {
     in = a.tin[t];
     c = a.stay[t] + in;
+    const uint32_t why = crowded(a, t, in, c);
+    if (why) atomicOr(a.counters + CNT_RESORT, why);
     const bool f = c != 0 || touched(a, t);
     a.nb_flag[t] = f ? 1u : 0u;
     pk = (c ? 1u : 0u) | (f ? 0x10000u : 0u);
@@ -177,6 +187,7 @@ template <bool ALONE>
 __global__ __launch_bounds__(TAB_THREADS) void k_tab_scan(TabArgs a) {
   __shared__ uint32_t s[TAB_WAVES];
   uint32_t pre[4] = {0, 0, 0, 0};
+  uint32_t why = 0u;  // ALONE: what k_tab_reduce would have marked
   bool keep = false;
   if constexpr (!ALONE) {
     keep = a.may_keep && a.counters[CNT_KEEP] != 0u;
@@ -200,11 +211,16 @@ __global__ __launch_bounds__(TAB_THREADS) void k_tab_scan(TabArgs a) {
   const uint32_t ti = ok ? a.tin[t] : 0u, ct = ok ? a.stay[t] + ti : 0u;
   uint32_t fl = 0u;
   if constexpr (ALONE) {
+    uint32_t w = 0u;
     if (ok) {
       fl = ct != 0 || touched(a, t) ? 1u : 0u;
       a.nb_flag[t] = fl;
+      w = crowded(a, t, ti, ct);
     }
-    __syncthreads();  // the neighbours' arrivals have been read; they are reset below
+    // (a barrier: the neighbours' arrivals have been read; they are reset below)
+    if (__syncthreads_or(w != 0u))
+      why = (__syncthreads_or(w & RESORT_CROWD) ? uint32_t(RESORT_CROWD) : 0u) |
+            (__syncthreads_or(w & RESORT_TILE) ? uint32_t(RESORT_TILE) : 0u);
   } else {
     fl = ok ? a.nb_flag[t] : 0u;
   }
@@ -235,6 +251,7 @@ __global__ __launch_bounds__(TAB_THREADS) void k_tab_scan(TabArgs a) {
     a.counters[CNT_ACTIVE] = act;
     a.counters[CNT_NB] = nb;
     a.counters[CNT_OUTIN] = out_in;
+    a.counters[CNT_MANY] = arrive + out_in > a.many ? 1u : 0u;
     a.host[CNT_INSIDE] = inside;
     a.host[CNT_ACTIVE] = act;
     a.host[CNT_NB] = nb;
@@ -248,7 +265,11 @@ __global__ __launch_bounds__(TAB_THREADS) void k_tab_scan(TabArgs a) {
   if (blockIdx.x == 0) {
     // one wave per group of lanes
     const int g = int(threadIdx.x >> 6), i = int(threadIdx.x & 63);
-    uint32_t x = 0;
+    uint32_t x = 0, err = 0, resort = 0;
+    if (g == LANE_NODES && i == 0) {  // loaded with the lanes
+      err = a.counters[CNT_ERR];
+      resort = a.counters[CNT_RESORT] | why;
+    }
     if (g < LANE_GROUPS && i < LANES) {
       uint32_t* lane = a.lanes + (g * LANES + i) * LANE_STRIDE;
       x = *lane;
@@ -261,11 +282,12 @@ __global__ __launch_bounds__(TAB_THREADS) void k_tab_scan(TabArgs a) {
       if (g == LANE_MOVED) a.counters[CNT_MOVED] = x;
       if (g == LANE_NODES) {
         a.counters[CNT_NODES] = x;
-        a.counters[CNT_REENTERED] = a.counters[CNT_REENTER];
-        a.host[CNT_ERR] = a.counters[CNT_ERR];
-        a.host[CNT_REENTER] = a.counters[CNT_REENTER];
+        a.counters[CNT_RESORTED] = resort;
+        a.counters[CNT_RESORT] = 0u;
+        a.counters[CNT_SCATTERED] = 0u;
+        a.host[CNT_ERR] = err;
+        a.host[CNT_RESORT] = resort;
         if (!a.keep_err) a.counters[CNT_ERR] = 0u;
-        a.counters[CNT_REENTER] = 0u;
       }
       reported(a, g);
     }
@@ -298,11 +320,11 @@ __global__ __launch_bounds__(256) void k_tile_counts(const uint32_t* __restrict_
 }
 
 // A merge launched before the host has read the report: nothing to do when no key
-// changed, or when particles came back into the mesh (the host sorts them all).
+// changed, or when the host sorts them all (CNT_RESORT, CNT_MANY).
 __device__ __forceinline__ bool merge_gated(const MergeArgs& a) {
   if (!a.gate) return false;
-  const uint32_t moved = a.gate[CNT_MOVED], reentered = a.gate[CNT_REENTERED];  // read together
-  return (moved == 0u) | (reentered != 0u);
+  const uint32_t moved = a.gate[CNT_MOVED], resort = a.gate[CNT_RESORTED] | a.gate[CNT_MANY];  // read together
+  return (moved == 0u) | (resort != 0u);
 }
 
 // The leavers of each previously active tile into the arrival segments of the

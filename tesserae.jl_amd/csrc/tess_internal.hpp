@@ -53,6 +53,7 @@ struct Binning {
   int64_t n_inside = 0;     // particles with a non-empty window (host copy)
   int64_t n_active = 0;     // tiles holding >= 1 particle (host copy)
   int64_t n_nodeblocks = 0; // node blocks touched by some tile footprint (host copy)
+  bool crowded = false;     // some tile holds more than merge_tile_max particles
   // the sorted (key, perm) arrays are a valid previous order for incremental re-binning
   bool state_valid = false;
   int64_t state_n = -1, state_ntiles = -1;
@@ -108,9 +109,11 @@ namespace tess {
 // counters_host): totals of a binning, error flags, and sums over the lanes
 enum {
   CNT_INSIDE = 0, CNT_ACTIVE = 1, CNT_NB = 2, CNT_ERR = 3, CNT_BIN_SLOTS = 4,
-  CNT_MISPLACED = 8, CNT_NODES = 9, CNT_ARRIVE = 10, CNT_P2GERR = 11, CNT_MOVED = 12, CNT_OUTIN = 13, CNT_REENTER = 14,
+  CNT_MISPLACED = 8, CNT_NODES = 9, CNT_ARRIVE = 10, CNT_P2GERR = 11, CNT_MOVED = 12, CNT_OUTIN = 13, CNT_RESORT = 14,
   CNT_PREV_ACTIVE = 15, CNT_SLOTS = 16,
-  CNT_REENTERED = 16,  // device: CNT_REENTER of the last report
+  CNT_RESORTED = 16,   // device: CNT_RESORT of the last report
+  CNT_MANY = 22,       // device: the last report's arrivals are too many to merge
+  CNT_SCATTERED = 23,  // device: waves of k_rekey nearly all of whose particles left their tiles
   CNT_KEEP = 21,       // device: the tables being scanned are not wanted
   CNT_SEQ = 17         // host: the report's number, once by each of its REPORTERS
 };
@@ -133,6 +136,13 @@ struct MoveOut {
   uint32_t* lanes;
 };
 
+// Why a re-binning sorts every key instead of merging the changed ones (bits of
+// CNT_RESORT): the per-tile counts are not complete (particles came back into the
+// mesh, or nearly all were put elsewhere) and the tables wait for a count of the
+// sorted keys; one tile has more arrivals, or holds more particles, than its
+// workgroup should take alone.
+enum { RESORT_RECOUNT = 1, RESORT_CROWD = 2, RESORT_TILE = 4 };
+
 // The tile tables of a binning, from the per-tile counts (binning.hip).
 struct TabArgs {
   uint32_t* stay;  // ntiles + 1: particles that stay, the last entry those outside the mesh
@@ -150,6 +160,9 @@ struct TabArgs {
   uint32_t seq;  // the report's number (0: nobody waits for it by number)
   int32_t keep_err;
   int32_t may_keep;  // with no changed key the old tables stand: build none (CNT_KEEP)
+  uint32_t crowd;    // more arrivals in one tile than this ask for a sort (RESORT_CROWD),
+  uint32_t many;     // and more in all (CNT_MANY)
+  uint32_t tile_max; // and more particles in one tile (RESORT_TILE)
 };
 
 // The merge of the particles whose key changed into the previous order.

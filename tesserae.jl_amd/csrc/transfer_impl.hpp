@@ -446,6 +446,49 @@ __device__ __forceinline__ void next_key(const MoveOut& mo, uint32_t key, uint32
   }
 }
 
+// next_key for particles that may all have been put elsewhere, in one tile or
+// outside the mesh: a wave draws the ranks of those that enter the tile of its
+// first leaver with one atomic, and those of the ones outside (tile ntiles) are
+// the workgroup's own, counted in s_out (outside_ranks makes them global).
+// (8 M particles put outside: 1.7 ms with one atomic per wave on the one word, 0.54
+// so.)
+__device__ __forceinline__ void next_key_anywhere(const MoveOut& mo, uint32_t key, uint32_t old_key, uint32_t jj,
+                                                  uint32_t tile, uint32_t start, uint32_t ntiles, TileMoves* s_mv,
+                                                  uint32_t* s_out, uint32_t& moved) {
+  mo.nk[jj] = key;
+  if (key == old_key) return;
+  ++moved;
+  const uint32_t to = key >> 6;
+  if (to == tile) return;
+  uint32_t r = 0;
+  if (to == ntiles) {
+    r = atomicAdd(s_out, 1u);
+  } else {
+    const bool mine = to == uint32_t(__builtin_amdgcn_readfirstlane(int(to)));
+    const uint64_t same = __ballot(mine);
+    const uint32_t below = uint32_t(__popcll(same & ((uint64_t(1) << (threadIdx.x & 63)) - 1)));
+    if (!mine || below == 0) r = atomicAdd(&mo.tin[to], mine ? uint32_t(__popcll(same)) : 1u);
+    const uint32_t first = uint32_t(__builtin_amdgcn_readfirstlane(int(r)));
+    if (mine) r = first + below;
+  }
+  mo.out[start + atomicAdd(&s_mv->leave, 1u)] = make_uint2(jj, r);
+}
+
+// The ranks outside the mesh of a workgroup's particles, by every thread of it
+// after tile_moves_end (whose barrier orders the list and its length).
+__device__ __forceinline__ void outside_ranks(const MoveOut& mo, uint32_t start, uint32_t ntiles, const TileMoves* s_mv,
+                                              uint32_t* s_out) {
+  if (*s_out == 0) return;  // uniform
+  const uint32_t leave = s_mv->leave;
+  __syncthreads();
+  if (threadIdx.x == 0) *s_out = atomicAdd(&mo.tin[ntiles], *s_out);
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < leave; i += blockDim.x) {
+    uint2& o = mo.out[start + i];
+    if ((mo.nk[o.x] >> 6) == ntiles) o.y += *s_out;
+  }
+}
+
 // The tile's counts, by every thread of the workgroup after its last key.
 __device__ __forceinline__ void tile_moves_end(const MoveOut& mo, uint32_t tile, int cnt, TileMoves* s_mv,
                                                uint32_t moved) {
@@ -466,37 +509,86 @@ template <typename T, int D, int BASIS, bool STORED>
 __global__ __launch_bounds__(256) void k_rekey(Args<T, D> a, const uint32_t* __restrict__ skeys, uint32_t ntiles,
                                                MoveOut mo, uint32_t* __restrict__ counters) {
   __shared__ TileMoves s_mv;
+  __shared__ uint32_t s_out;
   const int64_t j = xcd_remap(blockIdx.x, a.n_active);
   if (j >= a.n_active) return;
   const uint32_t tile = a.active[j];
   const uint32_t start = a.tile_start[tile];
   const int cnt = int(a.tile_end[tile] - start);
-  if (threadIdx.x == 0) s_mv = TileMoves{0u, 0u};
+  if (threadIdx.x == 0) {
+    s_mv = TileMoves{0u, 0u};
+    s_out = 0u;
+  }
   __syncthreads();
   uint32_t moved = 0;
-  for (int i = int(threadIdx.x); i < cnt; i += 256) {
-    const uint32_t jj = start + uint32_t(i);
-    const uint32_t key = particle_key<T, D, BASIS, STORED>(a, a.perm[jj], ntiles, counters + CNT_ERR);
-    next_key(mo, key, skeys[jj], jj, tile, start, &s_mv, moved);
+  auto key_at = [&](int i) {
+    return particle_key<T, D, BASIS, STORED>(a, a.perm[start + uint32_t(i)], ntiles, counters + CNT_ERR);
+  };
+  auto take = [&](int i) {
+    const uint32_t jj = start + uint32_t(i), key = key_at(i);
+    next_key_anywhere(mo, key, skeys[jj], jj, tile, start, ntiles, &s_mv, &s_out, moved);
+    return (key >> 6) != tile;
+  };
+  int i = int(threadIdx.x);
+  const bool left = i < cnt && take(i);
+  i += 256;
+  if (cnt > 256 && __popcll(__ballot(left)) >= 48) {
+    // particles put elsewhere altogether: once an eighth of the waves has lost
+    // three quarters of its first 64, the others leave the ranks to the sort and
+    // the tables to a count of the sorted keys (8 M particles spread anew, one
+    // atomic each on 2,200 words: 2.11 ms, so 1.63 ms)
+    uint32_t before = 0u;
+    if ((threadIdx.x & 63) == 0) before = atomicAdd(counters + CNT_SCATTERED, 1u);
+    if (int64_t(__builtin_amdgcn_readfirstlane(int(before))) >= a.n_active / 2) {
+      if ((threadIdx.x & 63) == 0) atomicOr(counters + CNT_RESORT, uint32_t(RESORT_RECOUNT));
+      for (; i < cnt; i += 256) {
+        const uint32_t jj = start + uint32_t(i), key = key_at(i);
+        mo.nk[jj] = key;
+        moved += key != skeys[jj] ? 1u : 0u;
+      }
+    }
   }
+  for (; i < cnt; i += 256) take(i);
   tile_moves_end(mo, tile, cnt, &s_mv, moved);
+  outside_ranks(mo, start, ntiles, &s_mv, &s_out);
+}
+
+// A workgroup's changed keys into its lane, by every thread of the workgroup.
+__device__ __forceinline__ void count_moved(uint32_t* lanes, bool moved) {
+  const int k = __syncthreads_count(moved);
+  if (threadIdx.x == 0 && k > 0) atomicAdd(lane_of(lanes, LANE_MOVED), uint32_t(k));
+}
+
+// Next keys from the positions where some tile is too full for one workgroup (or
+// the host sorts anyway): one particle per thread, no per-tile counts.
+template <typename T, int D, int BASIS, bool STORED>
+__global__ __launch_bounds__(256) void k_rekey_flat(Args<T, D> a, const uint32_t* __restrict__ skeys, uint32_t ntiles,
+                                                    MoveOut mo, uint32_t* __restrict__ counters) {
+  const int64_t jj = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  bool moved = false;
+  if (jj < a.n) {
+    const uint32_t key = particle_key<T, D, BASIS, STORED>(a, a.perm[jj], ntiles, counters + CNT_ERR);
+    mo.nk[jj] = key;
+    moved = key != skeys[jj];
+  }
+  count_moved(mo.lanes, moved);
 }
 
 // The same for the particles that were outside the mesh; one that came back is
-// reported (the caller then sorts every key again).
+// reported (the caller then sorts every key and counts the tiles again).
 template <typename T, int D, int BASIS, bool STORED>
 __global__ __launch_bounds__(256) void k_rekey_outside(Args<T, D> a, uint32_t ntiles, MoveOut mo,
                                                        uint32_t* __restrict__ counters) {
   const int64_t jj = a.n_inside + int64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (jj >= a.n) return;
-  const uint32_t key = particle_key<T, D, BASIS, STORED>(a, a.perm[jj], ntiles, counters + CNT_ERR);
-  mo.nk[jj] = key;
-  if ((key >> 6) != ntiles) {
-    atomicAdd(&mo.tin[key >> 6], 1u);
-    atomicSub(&mo.stay[ntiles], 1u);
-    atomicAdd(lane_of(mo.lanes, LANE_MOVED), 1u);
-    atomicOr(counters + CNT_REENTER, 1u);
+  bool back = false;
+  if (jj < a.n) {
+    const uint32_t key = particle_key<T, D, BASIS, STORED>(a, a.perm[jj], ntiles, counters + CNT_ERR);
+    mo.nk[jj] = key;
+    back = (key >> 6) != ntiles;
   }
+  count_moved(mo.lanes, back);
+  if (__syncthreads_or(back) && threadIdx.x == 0 && !(__atomic_load_n(counters + CNT_RESORT, __ATOMIC_RELAXED) & RESORT_RECOUNT))
+    atomicOr(counters + CNT_RESORT, uint32_t(RESORT_RECOUNT));
 }
 
 template <typename T, int D>
@@ -2777,6 +2869,20 @@ int key_bits_for(uint64_t maxkey) {
   return b;
 }
 
+// Where a re-binning of n particles sorts every key instead of merging the changed
+// ones.  The sort takes some 60 us and 0.12 ns per key.  The merge takes little per
+// particle, but one workgroup works on a tile's arrivals at some 25 ns each, and on
+// a tile's run (and its leavers) at some 20 ns per particle: the lines lie near
+// where such a workgroup alone takes as long as the sort.  P2G on 3D Float32 particles,
+// always merged and now: 2 M put outside the mesh 53 and 0.32 ms, a tenth of them
+// 5.4 and 0.53 ms; 1 M spread from one 2D tile 25 and 0.25 ms; 200 k in eight tiles
+// 5.1 and 2.1 ms.
+inline uint32_t merge_crowd(int64_t n) { return uint32_t(2048 + n / 256); }     // arrivals of a tile
+inline uint32_t merge_tile_max(int64_t n) { return uint32_t(4096 + n / 128); }  // particles of a tile
+// arrivals in all: 8 M particles, all in other tiles, 2.55 ms merged and 2.11 ms
+// sorted, 2 M 0.59 and 0.55, 0.2 M 0.146 and 0.161
+inline uint32_t merge_many(int64_t n) { return uint32_t((512 << 10) + n / 2); }
+
 // The re-binning's buffers for n particles and the context's current tables.
 inline MoveOut move_out(tess_ctx* ctx, int64_t n, int64_t ntiles) {
   const size_t m = size_t(std::max<int64_t>(n, 1));
@@ -2823,6 +2929,7 @@ inline TabArgs table_args(tess_ctx* ctx, int64_t ntiles) {
   t.lanes = lane_counters(ctx);
   t.counters = ctx->counters.as<uint32_t>(64);
   t.host = reinterpret_cast<uint32_t*>(ctx->counters_host);
+  t.crowd = t.many = t.tile_max = UINT32_MAX;
   return t;
 }
 
@@ -2936,6 +3043,14 @@ inline void merge_finish(tess_ctx* ctx, MergeArgs& g, int64_t old_inside) {
   std::swap(ctx->vals, ctx->perm2);
 }
 
+// Every next key sorted in the previous order, which is what the merge gives too.
+inline void resort_keys(tess_ctx* ctx, int64_t n, int key_bits) {
+  radix_sort_pairs(ctx, static_cast<const uint32_t*>(ctx->inc_nk.ptr), static_cast<const uint32_t*>(ctx->vals.ptr),
+                   ctx->skeys2.as<uint32_t>(size_t(n)), ctx->perm2.as<uint32_t>(size_t(n)), n, key_bits);
+  std::swap(ctx->keys_sorted, ctx->skeys2);
+  std::swap(ctx->vals, ctx->perm2);
+}
+
 // Debug builds (-DTESS_DEBUG=1, `make debug`): after every binning the host
 // reads the binning back and checks its invariants (the permutation, sorted
 // keys, each tile's run of keys, the active-tile list), raising
@@ -3026,20 +3141,28 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
   b.keys_ready = false;
   TabArgs tab = table_args(ctx, int64_t(ntiles));
   for (int d = 0; d < 3; ++d) tab.nt[d] = d < D ? a.ntiles[d] : 1;
+  tab.tile_max = merge_tile_max(n);
   const uint32_t* hc = reinterpret_cast<const uint32_t*>(ctx->counters_host);
+  uint32_t err = 0;
   if (incremental) {
     // keys in the previous sorted order, from the previous G2P of the same step
     // loop or from the positions; the tables they give; one readback
     const MoveOut mo = move_out(ctx, n, int64_t(ntiles));
+    const bool flat = !precomputed && b.crowded;
     if (!precomputed) {
       fill_binning_ptrs<T, D>(ctx, a);
       const uint32_t* skeys = static_cast<const uint32_t*>(ctx->keys_sorted.ptr);
-      if (b.n_active > 0) {
+      if (flat) {
+        hipLaunchKernelGGL((k_rekey_flat<T, D, BASIS, STORED>), dim3(blocks_for(n, 256)), dim3(256), 0, ctx->stream, a,
+                           skeys, uint32_t(ntiles), mo, counters);
+        TESS_HIP(hipGetLastError());
+      }
+      if (!flat && b.n_active > 0) {
         hipLaunchKernelGGL((k_rekey<T, D, BASIS, STORED>), dim3(xcd_grid(b.n_active)), dim3(256), 0, ctx->stream, a,
                            skeys, uint32_t(ntiles), mo, counters);
         TESS_HIP(hipGetLastError());
       }
-      if (n > b.n_inside) {
+      if (!flat && n > b.n_inside) {
         hipLaunchKernelGGL((k_rekey_outside<T, D, BASIS, STORED>), dim3(blocks_for(n - b.n_inside, 256)), dim3(256),
                            0, ctx->stream, a, uint32_t(ntiles), mo, counters);
         TESS_HIP(hipGetLastError());
@@ -3049,17 +3172,22 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
     bool same_kind = b.tile_log2 == Geo<D>::LT && b.basis == BASIS && b.dtype == mesh.dtype;
     for (int d = 0; d < D; ++d) same_kind = same_kind && b.ntiles_axis[d] == a.ntiles[d];
     tab.may_keep = same_kind ? 1 : 0;
+    tab.crowd = merge_crowd(n);
+    tab.many = merge_many(n);
     const uint32_t seq = build_tables(ctx, tab);
     // (over many tiles, whose workgroups cost 0.2 ns each to find nothing to do,
     // not ahead while the last binning found no changed key)
-    const bool ahead = ctx->last_movers != 0 || b.n_active <= 8192;
+    const bool ahead = !b.crowded && (ctx->last_movers != 0 || b.n_active <= 8192);
     MergeArgs merge;
     if (ahead) merge = merge_ahead(ctx, n, int64_t(ntiles), b.n_active);
     wait_report(ctx, seq);
     take_report(ctx);
     ctx->last_movers = int64_t(hc[CNT_MOVED]);
-    if (!ahead && ctx->last_movers > 0 && !hc[CNT_REENTER]) merge = merge_ahead(ctx, n, int64_t(ntiles), b.n_active);
-    if (ctx->last_movers == 0 && same_kind && !(hc[CNT_ERR] & ERR_GIMP_LENGTH)) {
+    err = hc[CNT_ERR];
+    const bool recount = flat || (hc[CNT_RESORT] & RESORT_RECOUNT);
+    const bool resort = ctx->last_movers > 0 && (recount || b.crowded || hc[CNT_RESORT] || hc[CNT_ARRIVE] > tab.many);
+    if (!ahead && ctx->last_movers > 0 && !resort) merge = merge_ahead(ctx, n, int64_t(ntiles), b.n_active);
+    if (ctx->last_movers == 0 && same_kind && !(err & ERR_GIMP_LENGTH)) {
       // no particle changed its key: the previous order and tile lists stand
       ctx->last_misplaced = (ctx->misplaced_x_ptr == P.x.ptr && ctx->misplaced_n == n) ? ctx->broken_count : -1;
       ctx->kept_binnings += 1;
@@ -3068,14 +3196,17 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
       prof_end(ctx, tok);
       return;
     }
-    if (hc[CNT_REENTER]) {
-      // particles came back into the mesh: every key sorted in the previous order
-      radix_sort_pairs(ctx, mo.nk, static_cast<const uint32_t*>(ctx->vals.ptr), ctx->skeys2.as<uint32_t>(m),
-                       ctx->perm2.as<uint32_t>(m), n, kbits);
-      std::swap(ctx->keys_sorted, ctx->skeys2);
-      std::swap(ctx->vals, ctx->perm2);
+    if (resort) {
+      resort_keys(ctx, n, kbits);
     } else if (ctx->last_movers > 0) {
       merge_finish(ctx, merge, b.n_inside);
+    }
+    if (recount) {
+      // (the tables above had no counts of these keys; the ones of this report stand)
+      tab.may_keep = 0;
+      launch_tile_counts(ctx->stream, static_cast<const uint32_t*>(ctx->keys_sorted.ptr), n, int64_t(ntiles), tab.stay,
+                         tab.tin);
+      wait_report(ctx, build_tables(ctx, tab));
     }
   } else {
     uint32_t* skeys = ctx->keys_sorted.as<uint32_t>(m);
@@ -3091,10 +3222,11 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
     launch_tile_counts(ctx->stream, skeys, n, int64_t(ntiles), tab.stay, tab.tin);
     wait_report(ctx, build_tables(ctx, tab));
     take_report(ctx);
+    err = hc[CNT_ERR];
   }
   prof_end(ctx, tok);
-  if (hc[CNT_ERR] & ERR_GIMP_LENGTH) raise(TESS_ERR_ARGUMENT, "uGIMP requires 0 ≤ pt.l ≤ spacing(mesh)");
-  if (hc[CNT_ERR] & ERR_WINDOW)
+  if (err & ERR_GIMP_LENGTH) raise(TESS_ERR_ARGUMENT, "uGIMP requires 0 ≤ pt.l ≤ spacing(mesh)");
+  if (err & ERR_WINDOW)
     raise(TESS_ERR_DIMENSION, "stored support window is larger than the basis support width");
   swap_tables(ctx);
   b.n_inside = int64_t(hc[CNT_INSIDE]);
@@ -3102,6 +3234,7 @@ void bin_particles_run(tess_ctx* ctx, const tess_mesh& mesh, const tess_particle
   ctx->last_misplaced = (ctx->misplaced_x_ptr == P.x.ptr && ctx->misplaced_n == n) ? ctx->broken_count : -1;
   b.n_active = int64_t(hc[CNT_ACTIVE]);
   b.n_nodeblocks = int64_t(hc[CNT_NB]);
+  b.crowded = (hc[CNT_RESORT] & RESORT_TILE) != 0;
   b.x_ptr = P.x.ptr;
   b.n = n;
   b.dim = D;
