@@ -63,6 +63,25 @@ void* Buffer::get(size_t need) {
   return ptr;
 }
 
+bool Buffer::fits(size_t need) {
+  if (need <= bytes) return true;
+  if (ptr) TESS_HIP(hipDeviceSynchronize());
+  release();
+  const size_t cap = need + need / 8;
+  void* p = nullptr;
+  const hipError_t e = hipMalloc(&p, cap);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (e == hipSuccess) {
+    ptr = p;
+    bytes = cap;
+  }
+  TESS_HIP(e);
+  return true;
+}
+
 void Buffer::release() {
   if (ptr) (void)hipFree(ptr);
   ptr = nullptr;

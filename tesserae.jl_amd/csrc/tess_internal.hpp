@@ -35,6 +35,7 @@ struct Buffer {
   void* ptr = nullptr;
   size_t bytes = 0;
   void* get(size_t need);  // (re)allocates when need > bytes; contents undefined
+  bool fits(size_t need);  // get, but false where the device has no memory for it
   void release();
   template <typename U>
   U* as(size_t count) { return static_cast<U*>(get(count * sizeof(U))); }

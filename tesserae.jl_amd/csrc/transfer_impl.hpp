@@ -3581,10 +3581,12 @@ void layered_reorder(tess_ctx* ctx, const tess_mesh& mesh, const tess_particles&
 // place of the second set, at no cost), and only a reorder in that last step,
 // or an error, leaves a copy to make.
 //
-// Moving the 31 scalars of a particle before the step took a gather and a
+// Moving the 34 scalars of a particle before the step took a gather and a
 // write-back pass: 3.3 ms for 13.4 M particles (Float32), beside 1.5 ms for the
 // step.  What is left is the pair of maps (0.1 ms) and the copy of at most one
-// reorder per call (0.6 ms).
+// reorder per call (0.6 ms).  The second set (34 scalars per particle in 3D, and an
+// eighth) stays with the context; where the device has no memory for it the loop
+// moves the particles before the step, through one field's scratch.
 class MovingParticles {
  public:
   // allowed: the step's G2P is the one that can write elsewhere
@@ -3598,16 +3600,19 @@ class MovingParticles {
       can_ = can_ && a.ptr && (aos || soa);
     }
   }
-  bool can_move() const { return can_; }
+  // asked before a reordering step's work is enqueued: whether there is, or can
+  // be, a second set (without it the particles are moved where they are stored)
+  bool can_move() {
+    if (can_ && home()) can_ = ctx_->moved.fits(bytes());
+    return can_;
+  }
   const tess_particles& now() const { return cur_; }
   bool home() const { return cur_.x.ptr == home_.x.ptr; }
   // the set the particles are not in (same layout)
   tess_particles other() {
     if (!home()) return home_;
     tess_particles q = home_;
-    size_t off = 0;
-    for (int f = 0; f < 6; ++f) off += span(f);
-    char* p = static_cast<char*>(ctx_->moved.get(off));
+    char* p = static_cast<char*>(ctx_->moved.get(bytes()));
     for (int f = 0; f < 6; ++f) {
       const_cast<tess_field&>(field(q, f)).ptr = p;
       p += span(f);
@@ -3643,6 +3648,11 @@ class MovingParticles {
   }
   int comps(int f) const { return f < 2 ? D_ : f == 2 ? 1 : D_ * D_; }
   size_t span(int f) const { return (size_t(home_.n) * size_t(comps(f)) * scalar_ + 255) & ~size_t(255); }
+  size_t bytes() const {
+    size_t b = 0;
+    for (int f = 0; f < 6; ++f) b += span(f);
+    return b;
+  }
   void rename(const void* from, const void* to) {
     if (ctx_->bin.x_ptr == from) ctx_->bin.x_ptr = to;
     if (ctx_->misplaced_x_ptr == from) ctx_->misplaced_x_ptr = to;

@@ -1,0 +1,55 @@
+"""A loop whose reorder finds no memory for the second set of particle arrays moves the particles where they are stored:
+the same states, bit for bit, and no error."""
+import numpy as np
+import pytest
+import torch
+
+import tesserae_hip as th
+from gpu_util import particles_np, to_gpu
+from tesserae_hip.scenes import random_box
+
+pytestmark = pytest.mark.gpu
+
+QUADRATIC = th.BSpline(th.Quadratic())
+
+
+def test_reorder_without_room_for_a_second_set():
+    """The second set of 2 M 3D Float64 particles takes some 600 MB.  The step loops' other buffers exist already and
+    500 MB of the device stay free: room for the scratch of one field (160 MB), not for the set."""
+    free, total = torch.cuda.mem_get_info()
+    if free < 8 << 30:
+        pytest.skip("the device's memory is in use")
+    n = 1 << 21
+    sc = random_box(3, n, 3, QUADRATIC, h=1 / 32, vscale=1.0, lo=0.1, hi=0.9)
+
+    def run(ctx, hold):
+        _, P, G = to_gpu(sc)
+        th.step(G, P, sc.basis, sc.params, nsteps=1, ctx=ctx)  # the buffers that every loop needs
+        ctx.sync()
+        held = []
+        if hold:
+            torch.cuda.empty_cache()
+            free, _ = torch.cuda.mem_get_info()
+            held.append(torch.empty(free - (500 << 20), dtype=torch.uint8, device="cuda"))
+        th.step(G, P, sc.basis, sc.params, nsteps=3, reorder_threshold=1.0, ctx=ctx)
+        ctx.sync()
+        left = torch.cuda.mem_get_info()[0]
+        del held
+        torch.cuda.empty_cache()
+        assert ctx.stats()["reorders"] == 3
+        return particles_np(P), left
+
+    # a general correction reorders in place too: its kernels are loaded before memory runs short
+    warm = random_box(3, 100, 3, th.WLS(QUADRATIC), h=0.1)
+    _, P, G = to_gpu(warm)
+    th.step(G, P, warm.basis, warm.params, nsteps=2, reorder_threshold=1.0, ctx=th.Context())
+    torch.cuda.synchronize()
+    short = th.Context()
+    got, left = run(short, True)
+    short.close()
+    assert left < 500 << 20
+    ctx = th.Context()
+    ref, _ = run(ctx, False)
+    ctx.close()
+    for name in ref:
+        np.testing.assert_array_equal(got[name], ref[name], err_msg=name)
