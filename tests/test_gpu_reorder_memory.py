@@ -1,5 +1,7 @@
 """A loop whose reorder finds no memory for the second set of particle arrays moves the particles where they are stored:
 the same states, bit for bit, and no error."""
+import gc
+
 import numpy as np
 import pytest
 import torch
@@ -14,8 +16,8 @@ QUADRATIC = th.BSpline(th.Quadratic())
 
 
 def test_reorder_without_room_for_a_second_set():
-    """The second set of 2 M 3D Float64 particles takes some 600 MB.  The step loops' other buffers exist already and
-    500 MB of the device stay free: room for the scratch of one field (160 MB), not for the set."""
+    """The second set of 2 M 3D Float64 particles takes some 640 MB.  The step loops' other buffers exist already and
+    six pieces of 64 MB stay free on the device: room for the scratch of one field (170 MB), not for the set."""
     free, total = torch.cuda.mem_get_info()
     if free < 8 << 30:
         pytest.skip("the device's memory is in use")
@@ -28,9 +30,18 @@ def test_reorder_without_room_for_a_second_set():
         ctx.sync()
         held = []
         if hold:
+            gc.collect()  # (contexts that other tests dropped)
             torch.cuda.empty_cache()
+            # (the free memory that the runtime reports is not exact: until an allocation fails)
             free, _ = torch.cuda.mem_get_info()
-            held.append(torch.empty(free - (500 << 20), dtype=torch.uint8, device="cuda"))
+            held.append(torch.empty(free - (2000 << 20), dtype=torch.uint8, device="cuda"))
+            try:
+                for _ in range(100):
+                    held.append(torch.empty(64 << 20, dtype=torch.uint8, device="cuda"))
+            except torch.cuda.OutOfMemoryError:
+                pass
+            del held[-6:]
+            torch.cuda.empty_cache()
         th.step(G, P, sc.basis, sc.params, nsteps=3, reorder_threshold=1.0, ctx=ctx)
         ctx.sync()
         left = torch.cuda.mem_get_info()[0]
@@ -47,9 +58,10 @@ def test_reorder_without_room_for_a_second_set():
     short = th.Context()
     got, left = run(short, True)
     short.close()
-    assert left < 500 << 20
     ctx = th.Context()
     ref, _ = run(ctx, False)
     ctx.close()
     for name in ref:
         np.testing.assert_array_equal(got[name], ref[name], err_msg=name)
+    if left > 600 << 20:
+        pytest.skip("memory came back during the loop: nothing shown")
