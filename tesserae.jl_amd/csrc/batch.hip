@@ -636,7 +636,7 @@ void batch_graph_step(tess_ctx* g, tess_batch& B, bool full, int in) {
     g2.perm_new = cur.perm;
     g2.counters = counters;
     g2.pos_bits = key_bits_for(uint64_t(m));
-    launch_merge(st, g2, true, n > 0 ? unsigned(std::min<int64_t>(blocks_for(n, 256), 512)) : 0u);
+    launch_merge(st, g2, n > 0 ? unsigned(std::min<int64_t>(blocks_for(n, 256), 512)) : 0u);
   }
   // grids: the previous step's stale node blocks, P2G, the grid-node half
   hipLaunchKernelGGL((k_zero_stale_persist<T, D>), dim3(B.grid_zero), dim3(64), 0, st, a,

@@ -607,10 +607,10 @@ void launch_tile_counts(hipStream_t st, const uint32_t* skeys, int64_t n, int64_
 // dispatch each), 16 k that walk them 19 us
 constexpr int64_t SCATTER_GRID = 16384;
 
-// arrivals: whether any particle entered a tile; the launch counts are those of
-// the host, or upper bounds of the device counts the args point at.
-void launch_merge(hipStream_t st, const MergeArgs& a, bool arrivals, unsigned outside_blocks) {
-  if (arrivals && a.old_active_n > 0) {
+// The launch counts are those of the host, or upper bounds of the device counts
+// the args point at.
+void launch_merge(hipStream_t st, const MergeArgs& a, unsigned outside_blocks) {
+  if (a.old_active_n > 0) {
     hipLaunchKernelGGL(k_scatter_out, dim3(unsigned(std::min<int64_t>(a.old_active_n, SCATTER_GRID))), dim3(64), 0, st,
                        a);
     TESS_HIP(hipGetLastError());

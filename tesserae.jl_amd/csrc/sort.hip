@@ -158,15 +158,11 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t digit, bool valid) {
   return peers;
 }
 
-// n_dev (when set): the element count read on the device, at most n; chunks
-// past it hold an empty histogram.
 template <int RB, int ROUNDS>
 __global__ __launch_bounds__(SORT_THREADS) void k_radix_hist(const uint32_t* __restrict__ keys, int64_t n, int shift,
-                                                              uint32_t* __restrict__ hist, int64_t nchunks,
-                                                              const uint32_t* __restrict__ n_dev) {
+                                                              uint32_t* __restrict__ hist, int64_t nchunks) {
   constexpr int RADIX = 1 << RB;
   __shared__ uint32_t s_hist[RADIX];
-  if (n_dev) n = int64_t(*n_dev);
   const int64_t base = int64_t(blockIdx.x) * (SORT_THREADS * ROUNDS);
   uint32_t k[ROUNDS];
 #pragma unroll
@@ -221,15 +217,13 @@ __global__ __launch_bounds__(SORT_THREADS) void k_radix_scatter(const uint32_t* 
                                                                  uint32_t* __restrict__ vals_out, int64_t n,
                                                                  int shift, const uint32_t* __restrict__ rows,
                                                                  const uint32_t* __restrict__ totals,
-                                                                 int64_t nchunks, const uint32_t* __restrict__ n_dev) {
+                                                                 int64_t nchunks) {
   constexpr int RADIX = 1 << RB, PER = RADIX / SORT_THREADS;
   __shared__ uint32_t s_cnt[SORT_WAVES][RADIX];
   __shared__ uint32_t s_wave[SORT_THREADS / 64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  if (n_dev) n = int64_t(*n_dev);
   const int64_t base = int64_t(blockIdx.x) * (SORT_THREADS * ROUNDS);
-  if (base >= n) return;  // uniform
   // wave w takes the keys [w*64*ROUNDS, (w+1)*64*ROUNDS) of the chunk in order
   const int64_t first = base + int64_t(wave) * (64 * ROUNDS) + lane;
   uint32_t k[ROUNDS], v[ROUNDS], rank[ROUNDS];
@@ -407,21 +401,21 @@ size_t sort_hist_words(int64_t n) {
 namespace {
 template <int RB, int ROUNDS>
 void sort_pass(const SortWork& w, const uint32_t* kin, const uint32_t* vin, uint32_t* kout, uint32_t* vout, int64_t n,
-               int shift, int64_t nchunks, const uint32_t* n_dev) {
+               int shift, int64_t nchunks) {
   uint32_t* totals = w.hist + (nchunks << RB);
   hipLaunchKernelGGL((k_radix_hist<RB, ROUNDS>), dim3(unsigned(nchunks)), dim3(SORT_THREADS), 0, w.stream, kin, n, shift,
-                     w.hist, nchunks, n_dev);
+                     w.hist, nchunks);
   TESS_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_radix_rows, dim3(1u << RB), dim3(SORT_THREADS), 0, w.stream, w.hist, nchunks, totals);
   TESS_HIP(hipGetLastError());
   hipLaunchKernelGGL((k_radix_scatter<RB, ROUNDS>), dim3(unsigned(nchunks)), dim3(SORT_THREADS), 0, w.stream, kin, vin,
-                     kout, vout, n, shift, w.hist, totals, nchunks, n_dev);
+                     kout, vout, n, shift, w.hist, totals, nchunks);
   TESS_HIP(hipGetLastError());
 }
 }  // namespace
 
 void radix_sort_pairs_ws(const SortWork& w, const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out,
-                         uint32_t* vals_out, int64_t n, int key_bits, const uint32_t* n_dev) {
+                         uint32_t* vals_out, int64_t n, int key_bits) {
   if (n <= 0) return;
   if (n > int64_t(UINT32_MAX)) raise(TESS_ERR_ARGUMENT, "radix sort: more than 2^32-1 elements");
   const int passes = sort_passes(key_bits, n), bits = sort_digit_bits(key_bits, n);
@@ -436,8 +430,8 @@ void radix_sort_pairs_ws(const SortWork& w, const uint32_t* keys_in, const uint3
     uint32_t* vout = to_out ? vals_out : w.vals_alt;
     auto run = [&](auto rb) {
       constexpr int RB = decltype(rb)::value;
-      if (large) sort_pass<RB, SORT_ROUNDS_LARGE>(w, kin, vin, kout, vout, n, p * bits, nchunks, n_dev);
-      else sort_pass<RB, SORT_ROUNDS_SMALL>(w, kin, vin, kout, vout, n, p * bits, nchunks, n_dev);
+      if (large) sort_pass<RB, SORT_ROUNDS_LARGE>(w, kin, vin, kout, vout, n, p * bits, nchunks);
+      else sort_pass<RB, SORT_ROUNDS_SMALL>(w, kin, vin, kout, vout, n, p * bits, nchunks);
     };
     if (bits == 8) run(std::integral_constant<int, 8>{});
     else if (bits == 9) run(std::integral_constant<int, 9>{});
@@ -448,7 +442,7 @@ void radix_sort_pairs_ws(const SortWork& w, const uint32_t* keys_in, const uint3
 }
 
 void radix_sort_pairs(tess_ctx* ctx, const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out,
-                      uint32_t* vals_out, int64_t n, int key_bits, const uint32_t* n_dev) {
+                      uint32_t* vals_out, int64_t n, int key_bits) {
   if (n <= 0) return;
   if (n > int64_t(UINT32_MAX)) raise(TESS_ERR_ARGUMENT, "radix sort: more than 2^32-1 elements");
   SortWork w;
@@ -456,7 +450,7 @@ void radix_sort_pairs(tess_ctx* ctx, const uint32_t* keys_in, const uint32_t* va
   w.hist = ctx->hist.as<uint32_t>(sort_hist_words(n));
   w.keys_alt = ctx->keys_alt.as<uint32_t>(size_t(n));
   w.vals_alt = ctx->vals_alt.as<uint32_t>(size_t(n));
-  radix_sort_pairs_ws(w, keys_in, vals_in, keys_out, vals_out, n, key_bits, n_dev);
+  radix_sort_pairs_ws(w, keys_in, vals_in, keys_out, vals_out, n, key_bits);
 }
 
 }  // namespace tess

@@ -109,7 +109,7 @@ namespace tess {
 // device counters (words of tess_ctx::counters, reported to the same words of
 // counters_host): totals of a binning, error flags, and sums over the lanes
 enum {
-  CNT_INSIDE = 0, CNT_ACTIVE = 1, CNT_NB = 2, CNT_ERR = 3, CNT_BIN_SLOTS = 4,
+  CNT_INSIDE = 0, CNT_ACTIVE = 1, CNT_NB = 2, CNT_ERR = 3,
   CNT_MISPLACED = 8, CNT_NODES = 9, CNT_ARRIVE = 10, CNT_P2GERR = 11, CNT_MOVED = 12, CNT_OUTIN = 13, CNT_RESORT = 14,
   CNT_PREV_ACTIVE = 15, CNT_SLOTS = 16,
   CNT_RESORTED = 16,   // device: CNT_RESORT of the last report
@@ -324,10 +324,8 @@ void exclusive_scan_u32(tess_ctx* ctx, uint32_t* data, int64_t n, uint32_t* tota
 void sum_u32(tess_ctx* ctx, const uint32_t* v, int64_t n, uint32_t* out);
 // Stable LSD radix sort of (key, value) pairs on the low key_bits of key.
 // vals_in == nullptr means values 0..n-1.  Result lands in (keys_out, vals_out).
-// With n_dev the element count is read on the device (at most n, which sizes
-// the launches), so the sort can be captured in a graph.
 void radix_sort_pairs(tess_ctx* ctx, const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out,
-                      uint32_t* vals_out, int64_t n, int key_bits, const uint32_t* n_dev = nullptr);
+                      uint32_t* vals_out, int64_t n, int key_bits);
 // The same sort over caller-provided work buffers on a stream (no allocation):
 // hist holds sort_hist_words(n) words, keys_alt/vals_alt n words each.
 struct SortWork {
@@ -339,13 +337,13 @@ struct SortWork {
 size_t sort_hist_words(int64_t n);
 size_t scan_work_bytes(int64_t n);
 void radix_sort_pairs_ws(const SortWork& w, const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out,
-                         uint32_t* vals_out, int64_t n, int key_bits, const uint32_t* n_dev = nullptr);
+                         uint32_t* vals_out, int64_t n, int key_bits);
 
 // ---- tile tables and the merge between two steps (binning.hip) ----
 int64_t tab_blocks(int64_t ntiles);
 void launch_tables(hipStream_t st, const TabArgs& a);
 void launch_tile_counts(hipStream_t st, const uint32_t* skeys, int64_t n, int64_t ntiles, uint32_t* stay, uint32_t* tin);
-void launch_merge(hipStream_t st, const MergeArgs& a, bool arrivals, unsigned outside_blocks);
+void launch_merge(hipStream_t st, const MergeArgs& a, unsigned outside_blocks);
 void launch_merge_tiles(hipStream_t st, const MergeArgs& a, int64_t tiles);
 void launch_merge_outside(hipStream_t st, const MergeArgs& a, unsigned blocks);
 

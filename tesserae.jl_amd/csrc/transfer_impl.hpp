@@ -1091,15 +1091,6 @@ __device__ __forceinline__ void st_g2p(T& dst, T v) {
   if constexpr (NT) __builtin_nontemporal_store(v, &dst);
   else dst = v;
 }
-// P2G's particle reads (x, v, V, σ): 0 plain, 1 non-temporal
-#ifndef TESS_P2G_STREAM
-#define TESS_P2G_STREAM 0
-#endif
-template <typename T>
-__device__ __forceinline__ T ld_p2g(T& src) {
-  if constexpr (TESS_P2G_STREAM >= 1) return __builtin_nontemporal_load(&src);
-  else return src;
-}
 
 // 1-D jets at the window nodes lo..lo+SW-1 of one axis; entries past the
 // (truncated) window are zero.  Derivatives are returned times h⁻¹.
@@ -1190,12 +1181,12 @@ template <typename T, int D, int BASIS, bool AOS>
 __device__ __forceinline__ void p2g_load(const Args<T, D>& a, uint32_t pid, P2GIn<T, D>& in) {
   in.pid = pid;
 #pragma unroll
-  for (int d = 0; d < D; ++d) in.x[d] = ld_p2g(fldw<T, D, AOS>(a.x, pid, d));
+  for (int d = 0; d < D; ++d) in.x[d] = fldw<T, D, AOS>(a.x, pid, d);
 #pragma unroll
-  for (int d = 0; d < D; ++d) in.v[d] = ld_p2g(fldw<T, D, AOS>(a.v, pid, d));
-  in.V = ld_p2g(a.V(pid));
+  for (int d = 0; d < D; ++d) in.v[d] = fldw<T, D, AOS>(a.v, pid, d);
+  in.V = a.V(pid);
 #pragma unroll
-  for (int q = 0; q < D * D; ++q) in.S[q] = ld_p2g(fldw<T, D * D, AOS>(a.sigma, pid, q));
+  for (int q = 0; q < D * D; ++q) in.S[q] = fldw<T, D * D, AOS>(a.sigma, pid, q);
   in.l = T(0);
   if constexpr (BASIS == TESS_UGIMP) in.l = a.l(pid) / a.mesh.h;
 }
@@ -1407,7 +1398,6 @@ template <typename T, int D, int BASIS, int NPASS, bool AOS, bool BATCH, bool SE
 __device__ __forceinline__ void k_p2g_fast_body(Args<T, D>& a, const uint32_t* __restrict__ skeys,
                                                           uint32_t* __restrict__ misplaced, const int64_t j) {
   using G = Geo<D>;
-  using PT = Part<D, support_width(BASIS)>;
   constexpr int SW = support_width(BASIS);
   constexpr int NV = 1 + 2 * D;
   constexpr int KN = SW / NPASS;                       // last-axis offsets per pass
@@ -3026,7 +3016,7 @@ inline MergeArgs merge_ahead(tess_ctx* ctx, int64_t n, int64_t ntiles, int64_t o
   g.gate = counters;
   g.new_count = counters + CNT_ACTIVE;
   g.new_active_n = std::min(ntiles, old_active + old_active / 8 + 64);
-  launch_merge(ctx->stream, g, true, 0);
+  launch_merge(ctx->stream, g, 0);
   return g;
 }
 
