@@ -552,9 +552,10 @@ inline BinSet bin_set(tess_ctx* g, int64_t n, int64_t ntiles, int which) {
 // One step of the batch on context g, every launch size fixed and every count
 // on the device.  full: the binning sorts every particle's key into set 0
 // (the step that starts each call); else it merges the particles whose key
-// the previous step's G2P changed (written with the stayer flags at the
-// sorted positions of set `in`) into set 1-in, the form that is captured.
-// Either way the G2P writes the next keys and stayer flags.
+// the previous step's G2P changed (MoveOut, over the sorted positions and tiles
+// of set `in`) into set 1-in, the form that is captured, whatever their number:
+// no host is there to sort them instead.  Either way the G2P writes the next keys
+// and each tile's counts and leavers.
 template <typename T, int D, int BASIS>
 void batch_graph_step(tess_ctx* g, tess_batch& B, bool full, int in) {
   constexpr int SW = support_width(BASIS);
@@ -674,8 +675,8 @@ void batch_graph_step(tess_ctx* g, tess_batch& B, bool full, int in) {
   hipLaunchKernelGGL(k_save_list, dim3(unsigned(std::min<int64_t>(blocks_for(int64_t(ntiles), 256), 1024))), dim3(256),
                      0, st, nblist, n_nb, prev_list, prev_count);
   TESS_HIP(hipGetLastError());
-  // G2P over the active tiles (next keys and stayer flags at the sorted
-  // positions), then the particles outside every mesh
+  // G2P over the active tiles (with the next keys and each tile's counts and
+  // leavers), then the particles outside every mesh
   const uint32_t nt32 = uint32_t(ntiles);
   const int nw = (B.variant & 4) ? 1 : (B.variant & 2) ? 2 : 4;
   auto g2p = [&](auto nwc) {
