@@ -287,8 +287,10 @@ tess_ctx* ctx_new(int device, hipStream_t stream) {
   c->stream = stream;
   c->seen_epoch = error_epoch();
   void* pinned = nullptr;
-  // pinned readback slots: the device counters' words 0-63
-  hipError_t e = hipHostMalloc(&pinned, 512 * sizeof(int64_t), hipHostMallocDefault);
+  // pinned readback slots: the device counters' words 0-63.  Coherent by request,
+  // not as the environment has it (HIP_HOST_COHERENT): the host reads reports while
+  // the kernel that writes them runs, by the order of their words
+  hipError_t e = hipHostMalloc(&pinned, 512 * sizeof(int64_t), hipHostMallocCoherent);
   if (e != hipSuccess) {
     delete c;
     check_hip(e, "hipHostMalloc");
