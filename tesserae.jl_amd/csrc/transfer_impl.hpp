@@ -828,31 +828,45 @@ __device__ __forceinline__ void stored_weights(const Args<T, D>& a, uint32_t pid
 // particles by class (window start relative to the footprint origin), so lane c
 // owns class c: it walks its particles, accumulates their contributions to the
 // sw^dim nodes of the class window in registers, and adds them into the LDS
-// tile.  Lanes hold distinct classes, so every LDS add instruction touches each
-// node at most once; the waves add in turn, so the order of the adds is fixed.
+// tile.  Lanes hold distinct classes, so the adds of one offset touch each node at
+// most once; the waves add in turn, so the order of the adds is fixed.
 //
-// A tile has NPASS x NK waves: wave w accumulates the offsets of pass w % NPASS
-// over every NK-th particle of each class.  What bounds it is the latency of the
+// A tile has WP x NK waves: wave w accumulates the offsets of the passes w % WP,
+// w % WP + WP, ... over every NK-th particle of each class (WP is NPASS, or 1).  What bounds it is the latency of the
 // particle loads (each waits for its id) and, for particles in no order, the
 // lines they touch.  168k particles at random places, 2D Float64 quadratic with
 // stored weights, about 250 and up to 1400 particles per tile: one wave per tile
 // 58 and 239 us; four, ids in LDS, 58 and 106 us; with the weights in 16-byte
 // words 46 and 67 us.
+// The waves add by reading, adding and writing back: LDS add instructions made the
+// four waves' adds the longest part in Float32 (1.44 M ordered 2D particles, stored
+// quadratic: 408 us with them, 361 us for one wave with them, 149 us so).
 template <int D, int NPASS>
 constexpr int P2G_TILE_SPLIT = NPASS == 1 ? 4 : (D == 2 ? 2 : 1);  // NK
 
-template <typename T, int D, int BASIS, bool STORED, int NPASS, bool CORR = false>
-__global__ __launch_bounds__((64 * NPASS * P2G_TILE_SPLIT<D, NPASS>)) void k_p2g_tile(
+// A general corrected basis in Float64 fills the registers of a SIMD with one or
+// two waves.  Where the tiles alone fill the chip, a tile takes one wave per pass
+// (2D), or one wave for its three passes (3D: three waves leave every fourth SIMD
+// idle).  WLS quadratic, random places, split and so: 2D 57.6 k particles (400
+// tiles) 68 and 70 us, 360 k (2,500) 160 and 116, 1.44 M 459 and 276; 3D 64 k (500
+// tiles) 181 and 182 us, 125 k (730) 257 and 193, 1 M 1225 and 651.
+template <typename T, int D, int NPASS>
+constexpr bool P2G_TILE_SOLO = sizeof(T) == 8 && (D == 2 || NPASS == 3);
+constexpr int64_t P2G_SOLO_TILES = 512;
+
+template <typename T, int D, int BASIS, bool STORED, int NPASS, bool CORR = false, int WP = NPASS,
+          int NK = P2G_TILE_SPLIT<D, NPASS>>
+__global__ __launch_bounds__((64 * WP * NK)) void k_p2g_tile(
     Args<T, D> a, const uint32_t* __restrict__ skeys, uint32_t* __restrict__ misplaced) {
   using G = Geo<D>;
   constexpr int SW = support_width(BASIS);
   constexpr int NV = 1 + 2 * D;
   constexpr int NOFF = Pow<SW, D>::v;
   constexpr int NSL = NOFF / NPASS;  // offsets per pass (NPASS is 1 or SW)
-  constexpr int NK = P2G_TILE_SPLIT<D, NPASS>, NW = NPASS * NK;
+  constexpr int NW = WP * NK;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  const int pass = wave % NPASS, part = wave / NPASS;
+  const int part = wave / WP;
   const int64_t j = xcd_remap(blockIdx.x, a.n_active);
   if (j >= a.n_active) return;
   const uint32_t tile = a.active[j];
@@ -896,7 +910,7 @@ __global__ __launch_bounds__((64 * NPASS * P2G_TILE_SPLIT<D, NPASS>)) void k_p2g
     if (lane == 0 && bad) atomicAdd(lane_of(misplaced, LANE_BROKEN), bad);
   }
   const T mp = a.mp, hinv = a.mesh.h_inv;
-  {
+  for (int pass = wave % WP; pass < NPASS; pass += WP) {
     T acc[NSL][NV];
 #pragma unroll
     for (int s2 = 0; s2 < NSL; ++s2)
@@ -988,8 +1002,12 @@ __global__ __launch_bounds__((64 * NPASS * P2G_TILE_SPLIT<D, NPASS>)) void k_p2g
           r /= SW;
           mul *= G::TS;
         }
+        T t[NV];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) atomicAdd(&s_tile[q][v], acc[s2][v]);
+        for (int v = 0; v < NV; ++v) t[v] = s_tile[q][v];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) s_tile[q][v] = t[v] + acc[s2][v];
+        __asm__ volatile("" ::: "memory");  // the LDS executes one wave's accesses in order
       }
       }
       __syncthreads();
@@ -3337,8 +3355,18 @@ void p2g_launch(tess_ctx* ctx, const tess_mesh& mesh, const tess_grid& G, const 
       hipLaunchKernelGGL((k_p2g_tile<T, D, BASIS, STORED, NPASS>), dim3(xcd_grid(b.n_active)), tile_block, 0,
                          ctx->stream, a, sk, misplaced);
     } else if (a.corr && !separable_correction(a.corr, BASIS, a.filter != nullptr)) {
-      hipLaunchKernelGGL((k_p2g_tile<T, D, BASIS, false, NPASS, true>), dim3(xcd_grid(b.n_active)), tile_block, 0,
-                         ctx->stream, a, sk, misplaced);
+      bool solo = false;
+      if constexpr (P2G_TILE_SOLO<T, D, NPASS>) {
+        if (b.n_active >= P2G_SOLO_TILES) {
+          constexpr int WP = D == 2 ? NPASS : 1;
+          hipLaunchKernelGGL((k_p2g_tile<T, D, BASIS, false, NPASS, true, WP, 1>), dim3(xcd_grid(b.n_active)),
+                             dim3(64 * WP), 0, ctx->stream, a, sk, misplaced);
+          solo = true;
+        }
+      }
+      if (!solo)
+        hipLaunchKernelGGL((k_p2g_tile<T, D, BASIS, false, NPASS, true>), dim3(xcd_grid(b.n_active)), tile_block, 0,
+                           ctx->stream, a, sk, misplaced);
     } else {
       // 3D: one wave per offset along z; 2D: one wave while the stencil fits
       constexpr int NPF = (D == 3 || Pow<SW, D>::v * NV * int(sizeof(T)) / 4 > 96) ? SW : 1;
