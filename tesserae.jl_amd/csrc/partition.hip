@@ -123,7 +123,10 @@ __global__ __launch_bounds__(256) void k_update_weights(WArgs<T, D> a) {
   // stored in 16-byte words (a lane's weights lie apart from its neighbours', and
   // each store instruction costs a request per lane: 168k particles, 2D Float64
   // quadratic, 29 us scalar by scalar, 19 us so)
-  const bool rows = whole && a.rows;
+  // (not the Float64 uGIMP ones in 3D, many of which are not whole: 1 M particles,
+  // 518 us with the words, 490 without)
+  constexpr bool WORDS = !(BASIS == TESS_UGIMP && D == 3 && sizeof(T) == 8);
+  const bool rows = WORDS && whole && a.rows;
 #pragma unroll
   for (int o0 = 0; o0 < IPow<SW, D>::v; o0 += SW) {
     T w[SW], g[SW][D];
