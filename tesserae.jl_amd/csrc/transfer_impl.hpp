@@ -559,8 +559,8 @@ __device__ __forceinline__ void count_moved(uint32_t* lanes, bool moved) {
   if (threadIdx.x == 0 && k > 0) atomicAdd(lane_of(lanes, LANE_MOVED), uint32_t(k));
 }
 
-// Next keys from the positions where some tile is too full for one workgroup (or
-// the host sorts anyway): one particle per thread, no per-tile counts.
+// Next keys from the positions where some tile is too full for one workgroup: one
+// particle per thread, no per-tile counts.
 template <typename T, int D, int BASIS, bool STORED>
 __global__ __launch_bounds__(256) void k_rekey_flat(Args<T, D> a, const uint32_t* __restrict__ skeys, uint32_t ntiles,
                                                     MoveOut mo, uint32_t* __restrict__ counters) {
@@ -587,8 +587,10 @@ __global__ __launch_bounds__(256) void k_rekey_outside(Args<T, D> a, uint32_t nt
     back = (key >> 6) != ntiles;
   }
   count_moved(mo.lanes, back);
-  if (__syncthreads_or(back) && threadIdx.x == 0 && !(__atomic_load_n(counters + CNT_RESORT, __ATOMIC_RELAXED) & RESORT_RECOUNT))
-    atomicOr(counters + CNT_RESORT, uint32_t(RESORT_RECOUNT));
+  if (__syncthreads_or(back) && threadIdx.x == 0) {
+    const uint32_t marked = __atomic_load_n(counters + CNT_RESORT, __ATOMIC_RELAXED);
+    if (!(marked & RESORT_RECOUNT)) atomicOr(counters + CNT_RESORT, uint32_t(RESORT_RECOUNT));
+  }
 }
 
 template <typename T, int D>
@@ -832,12 +834,14 @@ __device__ __forceinline__ void stored_weights(const Args<T, D>& a, uint32_t pid
 // most once; the waves add in turn, so the order of the adds is fixed.
 //
 // A tile has WP x NK waves: wave w accumulates the offsets of the passes w % WP,
-// w % WP + WP, ... over every NK-th particle of each class (WP is NPASS, or 1).  What bounds it is the latency of the
-// particle loads (each waits for its id) and, for particles in no order, the
-// lines they touch.  168k particles at random places, 2D Float64 quadratic with
-// stored weights, about 250 and up to 1400 particles per tile: one wave per tile
-// 58 and 239 us; four, ids in LDS, 58 and 106 us; with the weights in 16-byte
-// words 46 and 67 us; with the adds below 38 us (the first).
+// w % WP + WP, ... over every NK-th particle of each class (WP is NPASS, or 1).
+// What bounds it is the latency of the particle loads (each waits for its id) and,
+// for particles in no order, the lines they touch.  168k particles at random
+// places, 2D Float64 quadratic with stored weights, about 250 and up to 1400
+// particles per tile: one wave per tile 58 and 239 us; four, ids in LDS, 58 and
+// 106 us; with the weights in 16-byte words 46 and 67 us; with the adds below 38 us
+// (the first).
+//
 // The waves add by reading, adding and writing back: LDS add instructions made the
 // four waves' adds the longest part in Float32 (1.44 M ordered 2D particles, stored
 // quadratic: 408 us with them, 361 us for one wave with them, 149 us so).
@@ -2885,10 +2889,10 @@ int key_bits_for(uint64_t maxkey) {
 // ones.  The sort takes some 60 us and 0.12 ns per key.  The merge takes little per
 // particle, but one workgroup works on a tile's arrivals at some 25 ns each, and on
 // a tile's run (and its leavers) at some 20 ns per particle: the lines lie near
-// where such a workgroup alone takes as long as the sort.  P2G on 3D Float32 particles,
-// always merged and now: 2 M put outside the mesh 53 and 0.32 ms, a tenth of them
-// 5.4 and 0.53 ms; 1 M spread from one 2D tile 25 and 0.25 ms; 200 k in eight tiles
-// 5.1 and 2.1 ms.
+// where such a workgroup alone takes as long as the sort.  P2G on 3D Float32
+// particles, always merged and now: 2 M put outside the mesh 53 and 0.32 ms, a tenth
+// of them 5.4 and 0.53 ms; 1 M spread from one 2D tile 25 and 0.25 ms; 200 k in eight
+// tiles 5.1 and 2.1 ms.
 inline uint32_t merge_crowd(int64_t n) { return uint32_t(2048 + n / 256); }     // arrivals of a tile
 inline uint32_t merge_tile_max(int64_t n) { return uint32_t(4096 + n / 128); }  // particles of a tile
 // arrivals in all: 8 M particles, all in other tiles, 2.55 ms merged and 2.11 ms
