@@ -428,77 +428,72 @@ __global__ __launch_bounds__(256) void k_bin_keys(Args<T, D> a, uint32_t* __rest
 
 // The counters of a workgroup that computes its tile's next keys.
 struct TileMoves {
-  uint32_t leave, moved;
+  uint32_t leave, moved, out;  // out: those that leave the mesh, where next_key counts them (OWN)
 };
+
+// A leaver's rank among the arrivals of tile `to`: a wave draws the ranks of those
+// that enter the tile of its first leaver with one atomic.  Where many leave in one
+// step they mostly go to one place, and an atomic each on the one word takes 5.6 ns.
+__device__ __forceinline__ uint32_t arrival_rank(const MoveOut& mo, uint32_t to) {
+  const bool mine = to == uint32_t(__builtin_amdgcn_readfirstlane(int(to)));
+  const uint64_t same = __ballot(mine);
+  const uint32_t below = uint32_t(__popcll(same & ((uint64_t(1) << (threadIdx.x & 63)) - 1)));
+  uint32_t r = 0;
+  if (!mine || below == 0) r = atomicAdd(&mo.tin[to], mine ? uint32_t(__popcll(same)) : 1u);
+  const uint32_t first = uint32_t(__builtin_amdgcn_readfirstlane(int(r)));
+  return mine ? first + below : r;
+}
 
 // One particle's next key at sorted position jj of the tile whose run starts at
 // `start`: written out, counted, and listed with its rank among the arrivals
-// when it enters another tile (or leaves the mesh: tile ntiles).
+// when it enters another tile (or leaves the mesh: tile ntiles).  OWN: of those
+// that leave the mesh the rank is the workgroup's own, until tile_moves_end makes
+// it global.  WAVE: the ranks by arrival_rank.
+// k_rekey does both (8 M particles put outside: 1.7 ms by the wave, 0.54 so).  G2P
+// draws by the wave but in 3D Float64, whose registers are full (the Taylor rod, five
+// steps: 2,590 and 2,690 us by the wave, 2,570 and 2,580 us OWN).  Five steps whose
+// first takes every particle out of the mesh, an atomic each and now: 2 M 3D Float32
+// 24.8 and 2.7 ms, Float64 25.4 and 3.3 ms, 800 k 2D Float32 9.8 and 0.97 ms.
+template <bool OWN, bool WAVE>
 __device__ __forceinline__ void next_key(const MoveOut& mo, uint32_t key, uint32_t old_key, uint32_t jj, uint32_t tile,
-                                         uint32_t start, TileMoves* s_mv, uint32_t& moved) {
+                                         uint32_t start, uint32_t ntiles, TileMoves* s_mv, uint32_t& moved) {
   mo.nk[jj] = key;
   if (key != old_key) {
     ++moved;
-    if ((key >> 6) != tile) {
-      const uint32_t r = atomicAdd(&mo.tin[key >> 6], 1u);
+    const uint32_t to = key >> 6;
+    if (to != tile) {
+      uint32_t r;
+      if (OWN && to == ntiles)
+        r = atomicAdd(&s_mv->out, 1u);
+      else if constexpr (WAVE)
+        r = arrival_rank(mo, to);
+      else
+        r = atomicAdd(&mo.tin[to], 1u);
       mo.out[start + atomicAdd(&s_mv->leave, 1u)] = make_uint2(jj, r);
     }
   }
 }
 
-// next_key for particles that may all have been put elsewhere, in one tile or
-// outside the mesh: a wave draws the ranks of those that enter the tile of its
-// first leaver with one atomic, and those of the ones outside (tile ntiles) are
-// the workgroup's own, counted in s_out (outside_ranks makes them global).
-// (8 M particles put outside: 1.7 ms with one atomic per wave on the one word, 0.54
-// so.)
-__device__ __forceinline__ void next_key_anywhere(const MoveOut& mo, uint32_t key, uint32_t old_key, uint32_t jj,
-                                                  uint32_t tile, uint32_t start, uint32_t ntiles, TileMoves* s_mv,
-                                                  uint32_t* s_out, uint32_t& moved) {
-  mo.nk[jj] = key;
-  if (key == old_key) return;
-  ++moved;
-  const uint32_t to = key >> 6;
-  if (to == tile) return;
-  uint32_t r = 0;
-  if (to == ntiles) {
-    r = atomicAdd(s_out, 1u);
-  } else {
-    const bool mine = to == uint32_t(__builtin_amdgcn_readfirstlane(int(to)));
-    const uint64_t same = __ballot(mine);
-    const uint32_t below = uint32_t(__popcll(same & ((uint64_t(1) << (threadIdx.x & 63)) - 1)));
-    if (!mine || below == 0) r = atomicAdd(&mo.tin[to], mine ? uint32_t(__popcll(same)) : 1u);
-    const uint32_t first = uint32_t(__builtin_amdgcn_readfirstlane(int(r)));
-    if (mine) r = first + below;
-  }
-  mo.out[start + atomicAdd(&s_mv->leave, 1u)] = make_uint2(jj, r);
-}
-
-// The ranks outside the mesh of a workgroup's particles, by every thread of it
-// after tile_moves_end (whose barrier orders the list and its length).
-__device__ __forceinline__ void outside_ranks(const MoveOut& mo, uint32_t start, uint32_t ntiles, const TileMoves* s_mv,
-                                              uint32_t* s_out) {
-  if (*s_out == 0) return;  // uniform
-  const uint32_t leave = s_mv->leave;
-  __syncthreads();
-  if (threadIdx.x == 0) *s_out = atomicAdd(&mo.tin[ntiles], *s_out);
-  __syncthreads();
-  for (uint32_t i = threadIdx.x; i < leave; i += blockDim.x) {
-    uint2& o = mo.out[start + i];
-    if ((mo.nk[o.x] >> 6) == ntiles) o.y += *s_out;
-  }
-}
-
-// The tile's counts, by every thread of the workgroup after its last key.
-__device__ __forceinline__ void tile_moves_end(const MoveOut& mo, uint32_t tile, int cnt, TileMoves* s_mv,
-                                               uint32_t moved) {
+// The tile's counts, and its ranks outside the mesh, by every thread of the
+// workgroup after its last key.
+__device__ __forceinline__ void tile_moves_end(const MoveOut& mo, uint32_t tile, uint32_t start, int cnt,
+                                               uint32_t ntiles, TileMoves* s_mv, uint32_t moved) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) moved += __shfl_xor(moved, off, 64);
   if ((threadIdx.x & 63) == 0 && moved) atomicAdd(&s_mv->moved, moved);
   __syncthreads();
+  const uint32_t leave = s_mv->leave, out = s_mv->out;
   if (threadIdx.x == 0) {
-    mo.stay[tile] = uint32_t(cnt) - s_mv->leave;
+    mo.stay[tile] = uint32_t(cnt) - leave;
     if (s_mv->moved) atomicAdd(lane_of(mo.lanes, LANE_MOVED), s_mv->moved);
+  }
+  if (out == 0) return;  // uniform
+  __syncthreads();
+  if (threadIdx.x == 0) s_mv->out = atomicAdd(&mo.tin[ntiles], out);
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < leave; i += blockDim.x) {
+    uint2& o = mo.out[start + i];
+    if ((mo.nk[o.x] >> 6) == ntiles) o.y += s_mv->out;
   }
 }
 
@@ -509,16 +504,12 @@ template <typename T, int D, int BASIS, bool STORED>
 __global__ __launch_bounds__(256) void k_rekey(Args<T, D> a, const uint32_t* __restrict__ skeys, uint32_t ntiles,
                                                MoveOut mo, uint32_t* __restrict__ counters) {
   __shared__ TileMoves s_mv;
-  __shared__ uint32_t s_out;
   const int64_t j = xcd_remap(blockIdx.x, a.n_active);
   if (j >= a.n_active) return;
   const uint32_t tile = a.active[j];
   const uint32_t start = a.tile_start[tile];
   const int cnt = int(a.tile_end[tile] - start);
-  if (threadIdx.x == 0) {
-    s_mv = TileMoves{0u, 0u};
-    s_out = 0u;
-  }
+  if (threadIdx.x == 0) s_mv = TileMoves{0u, 0u, 0u};
   __syncthreads();
   uint32_t moved = 0;
   auto key_at = [&](int i) {
@@ -526,7 +517,7 @@ __global__ __launch_bounds__(256) void k_rekey(Args<T, D> a, const uint32_t* __r
   };
   auto take = [&](int i) {
     const uint32_t jj = start + uint32_t(i), key = key_at(i);
-    next_key_anywhere(mo, key, skeys[jj], jj, tile, start, ntiles, &s_mv, &s_out, moved);
+    next_key<true, true>(mo, key, skeys[jj], jj, tile, start, ntiles, &s_mv, moved);
     return (key >> 6) != tile;
   };
   int i = int(threadIdx.x);
@@ -549,8 +540,7 @@ __global__ __launch_bounds__(256) void k_rekey(Args<T, D> a, const uint32_t* __r
     }
   }
   for (; i < cnt; i += 256) take(i);
-  tile_moves_end(mo, tile, cnt, &s_mv, moved);
-  outside_ranks(mo, start, ntiles, &s_mv, &s_out);
+  tile_moves_end(mo, tile, start, cnt, ntiles, &s_mv, moved);
 }
 
 // A workgroup's changed keys into its lane, by every thread of the workgroup.
@@ -1959,7 +1949,8 @@ __device__ __forceinline__ void g2p_particle(const Args<T, D>& a, const G2PIn<T,
     for (int d = 0; d < D; ++d) nl *= uint32_t(a.ntiles[d]);
     const uint32_t kl = key_of_position<T, D, BASIS>(a, xn, cur.l, nl);
     const uint32_t key = kl == nl * 64u ? ntiles * 64u : kl + (tile - ltile) * 64u;
-    if (!ROWS || act) next_key(mo, key, cur.key, jj, tile, start, s_mv, moved);
+    constexpr bool OWN = D == 3 && sizeof(T) == 8;
+    if (!ROWS || act) next_key<OWN, !OWN>(mo, key, cur.key, jj, tile, start, ntiles, s_mv, moved);
   }
   T Fn[D * D];
 #pragma unroll
@@ -2013,7 +2004,7 @@ __device__ __forceinline__ void k_g2p_fast_body(Args<T, D>& a, const uint32_t* _
   __shared__ uint32_t s_cnt[64];
   __shared__ TileMoves s_mv;
   uint32_t moved = 0;
-  if (threadIdx.x == 0) s_mv = TileMoves{0u, 0u};  // before the barriers below
+  if (threadIdx.x == 0) s_mv = TileMoves{0u, 0u, 0u};  // before the barriers below
   G2PStage<T, D, 64 * NW> stage;
   g2p_stage_load<T, D, 64 * NW>(a, origin, stage);
   int ccount, coff, maxcnt;
@@ -2099,7 +2090,7 @@ __device__ __forceinline__ void k_g2p_fast_body(Args<T, D>& a, const uint32_t* _
     walk(std::true_type{});
   else
     walk(std::false_type{});
-  if (mo.nk) tile_moves_end(mo, tile, cnt, &s_mv, moved);
+  if (mo.nk) tile_moves_end(mo, tile, start, cnt, ntiles, &s_mv, moved);
 }
 
 template <typename T, int D, int BASIS, bool AOS, int NW, bool BATCH = false, bool SEP = false, bool NT = false>
@@ -2215,7 +2206,7 @@ __device__ __forceinline__ void k_g2p2g_fast_body(Args<T, D>& a, const uint32_t*
   __shared__ uint32_t s_pid[PID_CAP], s_key[PID_CAP];
   __shared__ TileMoves s_mv;
   uint32_t moved = 0;
-  if (threadIdx.x == 0) s_mv = TileMoves{0u, 0u};  // before the barriers below
+  if (threadIdx.x == 0) s_mv = TileMoves{0u, 0u, 0u};  // before the barriers below
   // [round parity][producer][row][class lane]; after the last round the
   // tile's node sums take its place: the consumers' slabs (several consumers)
   // or one array per component over the footprint (one)
@@ -2409,7 +2400,7 @@ __device__ __forceinline__ void k_g2p2g_fast_body(Args<T, D>& a, const uint32_t*
     p2g_write_partial_slabs<T, D, SW, KN, NC, NT>(a, j, s_xraw);
   else
     p2g_write_partial<T, D, SW, NT>(a, j, s_tile);
-  if (mo.nk) tile_moves_end(mo, tile, cnt, &s_mv, moved);
+  if (mo.nk) tile_moves_end(mo, tile, start, cnt, ntiles, &s_mv, moved);
 }
 
 template <typename T, int D, int BASIS, bool AOS, int NP, int NC>
