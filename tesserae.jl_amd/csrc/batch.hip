@@ -636,6 +636,7 @@ void batch_graph_step(tess_ctx* g, tess_batch& B, bool full, int in) {
     g2.keys_new = cur.keys;
     g2.perm_new = cur.perm;
     g2.counters = counters;
+    g2.crowd = merge_crowd(n);
     g2.pos_bits = key_bits_for(uint64_t(m));
     launch_merge(st, g2, n > 0 ? unsigned(std::min<int64_t>(blocks_for(n, 256), 512)) : 0u);
   }

@@ -554,14 +554,73 @@ __global__ __launch_bounds__(MERGE_THREADS) void k_merge_tiles(MergeArgs a) {
   }
 }
 
+// Arrivals outside the mesh, many of them, in order of previous position: each of
+// `parts` workgroups counts those at positions before its part (reading them all,
+// so that no workgroup waits for another) and places its own.
+constexpr uint32_t OUTSIDE_PARTS = 128;
+__device__ void place_outside(const MergeArgs& a, uint32_t ns, uint32_t os, uint32_t parts, uint32_t* s_sum) {
+  constexpr uint32_t STEP = 4 * MERGE_THREADS;  // positions of a workgroup at a time, four a thread
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t out = uint32_t(a.ntiles);
+  const uint32_t part = ((os + parts - 1) / parts + STEP - 1) / STEP * STEP;
+  const uint32_t lo = blockIdx.x * part, hi = min(os, lo + part);
+  if (lo >= os) return;  // uniform
+  const uint4* nk4 = reinterpret_cast<const uint4*>(a.nk);
+  uint32_t before = 0;
+#pragma unroll 4
+  for (uint32_t i = threadIdx.x; i < lo / 4; i += MERGE_THREADS) {
+    const uint4 q = nk4[i];
+    before += (q.x >> 6 == out) + (q.y >> 6 == out) + (q.z >> 6 == out) + (q.w >> 6 == out);
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) before += __shfl_xor(before, off, 64);
+  if (lane == 0) s_sum[wave] = before;
+  __syncthreads();
+  uint32_t at = ns;
+#pragma unroll
+  for (int w = 0; w < MERGE_WAVES; ++w) at += s_sum[w];
+  for (uint32_t b = lo; b < hi; b += STEP) {
+    const uint32_t i = b + 4 * threadIdx.x;
+    uint32_t key[4], mine = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q) {
+      key[q] = i + q < hi ? a.nk[i + q] : 0u;
+      mine += i + q < hi && key[q] >> 6 == out ? 1u : 0u;
+    }
+    const uint32_t incl = wave_scan_incl(mine);
+    __syncthreads();  // the sums have been read
+    if (lane == 63) s_sum[wave] = incl;
+    __syncthreads();
+    uint32_t r = at + incl - mine;
+#pragma unroll
+    for (int w = 0; w < MERGE_WAVES; ++w) {
+      if (w < wave) r += s_sum[w];
+      at += s_sum[w];
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q) {
+      if (i + q < hi && key[q] >> 6 == out) {
+        a.keys_new[r] = key[q];
+        a.perm_new[r++] = a.perm_old[i + q];
+      }
+    }
+  }
+}
+
 // Particles outside the mesh: those that were outside keep their order behind
 // the arrivals (whose previous positions are all lower).  Workgroup 0 places
-// the arrivals, sorted by previous position.
+// the arrivals, sorted by previous position; a captured step, which merges
+// whatever their number, shares many among its workgroups from where the host would
+// sort every key (six steps, 800 k particles that leave in three of them: 2D 13.0
+// and 1.8 ms, 3D 13.7 and 1.6 ms).
 __global__ __launch_bounds__(MERGE_THREADS) void k_merge_outside(MergeArgs a) {
   __shared__ uint32_t s_hist[256], s_wc[MERGE_WAVES][256];
   const uint32_t k = a.counters ? a.counters[CNT_OUTIN] : a.out_in;
   const uint32_t ns = a.new_start[a.ntiles], os = a.old_start[a.ntiles];
-  if (blockIdx.x == 0 && k > 0) {
+  const uint32_t parts = min(gridDim.x, OUTSIDE_PARTS);
+  if (k > a.crowd) {
+    if (blockIdx.x < parts) place_outside(a, ns, os, parts, s_hist);
+  } else if (blockIdx.x == 0 && k > 0) {
     const uint32_t off = a.seg_off[a.ntiles];
     const uint2* in = segment_sort(a.seg + off, a.seg_alt + off, k, a.pos_bits, s_hist, s_wc);
     for (uint32_t i = threadIdx.x; i < k; i += MERGE_THREADS) {

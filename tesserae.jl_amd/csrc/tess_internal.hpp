@@ -184,6 +184,7 @@ struct MergeArgs {
   const uint32_t* counters;  // device count of arrivals outside the mesh, or nullptr: out_in
   const uint32_t* gate;      // device counters: do nothing where they call for no merge, or nullptr
   uint32_t out_in;
+  uint32_t crowd;  // more arrivals outside the mesh than this are placed by several workgroups
   int32_t pos_bits;
 };
 

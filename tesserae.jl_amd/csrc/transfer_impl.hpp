@@ -3020,6 +3020,7 @@ inline MergeArgs merge_args(tess_ctx* ctx, int64_t n, int64_t ntiles, int64_t ol
   g.seg_alt = ctx->inc_seg2.as<uint2>(m);
   g.keys_new = ctx->skeys2.as<uint32_t>(m);
   g.perm_new = ctx->perm2.as<uint32_t>(m);
+  g.crowd = merge_crowd(n);
   g.pos_bits = key_bits_for(uint64_t(m));
   return g;
 }

@@ -75,3 +75,50 @@ def test_steps_that_lose_particles_take_no_longer(dim, n, h):
         t[shift] = _time(lambda: th.step(G, P, QUADRATIC, sc.params, nsteps=5, ctx=ctx), reset, ctx.sync)
         ctx.close()
     assert t[1.0] <= 2.5 * t[0.3 * h], t
+
+
+@pytest.mark.skipif(not os.path.exists(_abi.DEBUG_LIB_PATH), reason="debug build not made")
+@pytest.mark.parametrize("dim,h", [(2, 0.02), (3, 0.1)])
+@pytest.mark.parametrize("n", [2000, 2200, 9000, 40001])
+def test_batches_that_lose_particles(dim, h, n):
+    """Eager steps of a batch equal its captured steps bit for bit, on both sides of 2048 + n/256 arrivals outside."""
+    out = []
+    for variant in (0, 8):
+        members = []
+        for k, shift in ((n, 0.5), (n // 3, 0.1), (n // 2, 0.02)):
+            sc = _scene(dim, k, torch.float64, h, shift)
+            _, P, G = to_gpu(sc)
+            members.append((G, P, sc.params))
+        ctx = th.Context(library=_abi.DEBUG_LIB_PATH)
+        b = th.Batch(members, QUADRATIC, ctx=ctx)
+        b.set_variant(variant)
+        b.step(6)
+        ctx.sync()
+        out.append([(particles_np(P), grid_np(G)) for G, P, _ in members])
+        b.close()
+        ctx.close()
+    for (pa, ga), (pb, gb) in zip(*out):
+        for a, b in ((pa, pb), (ga, gb)):
+            for k in a:
+                assert np.array_equal(a[k], b[k], equal_nan=True), k
+
+
+@pytest.mark.parametrize("dim,n,h", [(2, 800000, 1 / 256), (3, 800000, 1 / 64)])
+def test_captured_steps_that_lose_particles_take_no_longer(dim, n, h):
+    t = {}
+    for shift in (0.3 * h, 1.0):
+        sc = _scene(dim, n, torch.float32, h, shift)
+        _, P, G = to_gpu(sc)
+        x = P.x.clone()
+        ctx = th.Context()
+        b = th.Batch([(G, P, sc.params)], QUADRATIC, ctx=ctx)
+        b.set_variant(8)
+
+        def reset():
+            P.x.copy_(x)
+            P.set("v", sc.v)
+
+        t[shift] = _time(lambda: b.step(6), reset, ctx.sync)
+        b.close()
+        ctx.close()
+    assert t[1.0] <= 2.5 * t[0.3 * h], t
